@@ -114,8 +114,9 @@ int64_t rbg_fw_workspace_bytes(int64_t n, int32_t elem_bytes);
 int64_t rbg_fw_tri_workspace_bytes(int64_t n, int32_t elem_bytes);
 /* No counterpart in the reference (test hook): the longest wait of one
  * persistent work item, in device wall-clock ticks, for the closures
- * launched after the call (single-matrix and batched); 0 restores the
- * default of two seconds.  A wait that runs out ends every workgroup of that
+ * launched after the call (single-matrix and batched), which take the
+ * persistent launch where they could do without its waits (rbg_fw_rows_*
+ * closes nothing meanwhile); 0 restores the default of two seconds.  A wait that runs out ends every workgroup of that
  * closure and flags it RBG_F_STALLED | RBG_F_NEED_GENERAL.  Returns the
  * previous override. */
 int64_t rbg_fw_flow_wait_limit(int64_t ticks);
@@ -169,6 +170,26 @@ int rbg_fw_load_i32(const int32_t *A, int64_t n, int64_t lda, int32_t *W, int64_
                     rbg_stream_t stream);
 int rbg_fw_load_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_t npad, rbg_status *st,
                     rbg_stream_t stream);
+/* No counterpart in the reference: the closure of a lower triangular matrix
+ * from its rows' direct entries, for matrices with few of them (pedigrees:
+ * two a row).  Reads A (n x n, row stride lda) once; when every off-diagonal
+ * entry lies below the diagonal, the values pass rbg_fw_precheck_*, every row
+ * has at most max(8, min(n / 64, 128)) off-diagonal entries and the graph at
+ * most 64 levels, writes the closure (natural values) into columns [0, n) of
+ * rows [0, n) of W (row stride npad, a multiple of 128, 16-byte aligned; the
+ * rest of W is unspecified), sets st->aux[5] = 1 and st->diameter_max = the
+ * max trajectory value; RBG_F_NEED_GENERAL then asks for mode 1 as for
+ * rbg_fw_dense_*.  Otherwise st->aux[5] = 0, W is untouched, st->flags may
+ * hold RBG_F_PRECOND_FAIL (mode 1), and the caller goes on with
+ * rbg_fw_load_*.  Writes the whole status block (no rbg_status_init needed);
+ * nothing is read by the host.  workspace: rbg_fw_rows_workspace_bytes(n,
+ * element size) bytes, 256-byte aligned; n <= rbg_fw_rows_max_n(). */
+int64_t rbg_fw_rows_max_n(void);
+int64_t rbg_fw_rows_workspace_bytes(int64_t n, int32_t elem_bytes);
+int rbg_fw_rows_i32(const int32_t *A, int64_t n, int64_t lda, int32_t *W, int64_t npad, void *workspace,
+                    int64_t workspace_bytes, rbg_status *st, rbg_stream_t stream);
+int rbg_fw_rows_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_t npad, void *workspace,
+                    int64_t workspace_bytes, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_precheck_i32(const int32_t *W, int64_t n, int64_t ld, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_precheck_i64(const int64_t *W, int64_t n, int64_t ld, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_dense_i32(int32_t *W, int64_t n, int64_t ld, int32_t width, int32_t is_unsigned, int32_t mode,

@@ -64,6 +64,10 @@ SIGNATURES = {
                                  ctypes.POINTER(ctypes.c_double)]),
     "rbg_fw_prof_read": (I32, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int64),
                                ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int64)]),
+    "rbg_fw_rows_max_n": (I64, []),
+    "rbg_fw_rows_workspace_bytes": (I64, [I64, I32]),
+    "rbg_fw_rows_i32": (I32, [P, I64, I64, P, I64, P, I64, P, P]),
+    "rbg_fw_rows_i64": (I32, [P, I64, I64, P, I64, P, I64, P, P]),
     "rbg_fw_precheck_i32": (I32, [P, I64, I64, P, P]),
     "rbg_fw_precheck_i64": (I32, [P, I64, I64, P, P]),
     "rbg_fw_load_i32": (I32, [P, I64, I64, P, I64, P, P]),

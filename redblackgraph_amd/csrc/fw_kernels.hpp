@@ -119,7 +119,7 @@ __device__ void capture_block(rbg_status* st, const T* colT, const T* rowS, int6
   }
 }
 
-static __global__ void k_status_init(rbg_status* st) {
+__device__ inline void status_clear(rbg_status* st) {
   st->events = 0;
   st->flags = 0;
   st->cycle_count = 0;
@@ -132,6 +132,8 @@ static __global__ void k_status_init(rbg_status* st) {
   st->diameter_max = 0;
   for (int i = 0; i < 8; i++) st->aux[i] = 0;
 }
+
+static __global__ void k_status_init(rbg_status* st) { status_clear(st); }
 
 // Precondition of the fast kernels: every value >= -1, no off-diagonal +-1,
 // every diagonal value in {-1, 0, 1}.  With such diagonals the products that

@@ -135,18 +135,7 @@ static inline int lines_groups(int npad) { return (2 * npad + NT - 1) / NT; }
 static __global__ void k_bfw_init(const BComp* comps, int32_t count) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= count) return;
-  rbg_status* st = comps[c].st;
-  st->events = 0;
-  st->flags = 0;
-  st->cycle_count = 0;
-  st->cycle_first_key = ~0ull;
-  st->cycle_last_key = 0;
-  st->ov_first_key = ~0ull;
-  st->ov_last_key = 0;
-  st->cycle_first_a = st->cycle_first_b = st->cycle_last_a = st->cycle_last_b = 0;
-  st->ov_last_a = st->ov_last_b = 0;
-  st->diameter_max = 0;
-  for (int i = 0; i < 8; i++) st->aux[i] = 0;
+  status_clear(comps[c].st);
 }
 
 // Domain conversion of one 128 x 128 chunk, four cells per thread and pass.

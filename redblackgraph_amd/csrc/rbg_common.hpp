@@ -23,7 +23,8 @@ namespace rbg {
 // While enabled, selected launches are bracketed by hipEvents on their stream
 // (bench and profiling only).  Kinds: 0 FW panel, 1 FW tile (128 x 128 for
 // int32), 2 DAG level, 3 SpGEMM rows, 4 batched FW, 5 FW tile (64 x 64 int32
-// tiles of the small-matrix and triangular schedules).  Each launch may
+// tiles of the small-matrix and triangular schedules), 6 persistent closure,
+// 7 closure from the rows' entries (its close pass).  Each launch may
 // carry a count of the work it does (relaxations for the tiles).
 constexpr int PROF_KINDS = 8;
 struct Prof {

@@ -12,6 +12,7 @@ from . import _lib
 from ._dtypes import ElemType, msb
 
 FW_TILE = 128
+ROWS_MAX_N = 32768  # rbg_fw_rows_max_n(): the largest order rbg_fw_rows_* takes
 _tls = threading.local()
 
 
@@ -20,17 +21,35 @@ def _workspace(npad: int, elem: int):
     threads run closures on their own streams and must not share it)."""
     t = _lib.torch()
     dev = _lib.device()
-    cache = getattr(_tls, "ws_cache", None)
+    return _cached_bytes("ws_cache", (dev.index, npad, elem),
+                         lambda: int(_lib.load().rbg_fw_tri_workspace_bytes(npad, elem)), t, dev)
+
+
+def _cached_bytes(name: str, key: tuple, nbytes, t, dev):
+    """The calling thread's byte buffer for ``key``; another key replaces it."""
+    cache = getattr(_tls, name, None)
     if cache is None:
-        cache = _tls.ws_cache = {}
-    key = (dev.index, npad, elem)
+        cache = {}
+        setattr(_tls, name, cache)
     ws = cache.get(key)
     if ws is None:
-        nbytes = int(_lib.load().rbg_fw_tri_workspace_bytes(npad, elem))
-        ws = t.empty(nbytes, dtype=t.uint8, device=dev)
+        ws = t.empty(nbytes(), dtype=t.uint8, device=dev)
         cache.clear()
         cache[key] = ws
     return ws
+
+
+def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
+    """rbg_fw_rows_*: the closure from the rows' direct entries, where the
+    matrix allows it (status aux[5])."""
+    t = _lib.torch()
+    dev = _lib.device()
+    elem = work.element_size()
+    ws = _cached_bytes("rows_cache", (dev.index, n, elem),
+                       lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev)
+    _lib.call("rbg_fw_rows_i32" if elem == 4 else "rbg_fw_rows_i64", _lib.ptr(src), n, src.stride(0), _lib.ptr(work),
+              npad, _lib.ptr(ws), ws.numel(), st.p, _lib.stream_handle(stream))
+    return st.read(stream)
 
 
 def padded_order(n: int) -> int:
@@ -86,7 +105,9 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
     schedule when the precheck finds every off-diagonal entry on one side of
     the diagonal (a pedigree numbered parents first is lower triangular), else
     the full one; "full" forces the full schedule (the results are the same).
-    A lower triangular closure runs as one persistent launch; "steps" keeps
+    With "auto" a lower triangular matrix of few entries per row (a pedigree)
+    is closed from its rows' direct entries (rbg_fw_rows_*).  Other lower
+    triangular closures run as one persistent launch; "steps" keeps
     one launch per pivot step there (the same results again).
     """
     if schedule not in ("auto", "full", "steps"):
@@ -103,13 +124,24 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
         return w
 
     st = status()
-    st.reset(stream)
     fast = et.native and not force_general
     sched = "full"
     if fast:
-        # one pass: copy, fast-domain check and encoding (rbg_fw_load_*)
         src = W if (W.stride(1) == 1 and W.stride(0) >= n) else W.contiguous()
         work = t.empty((npad, npad), dtype=W.dtype, device=W.device)
+        if schedule == "auto" and 0 < n <= ROWS_MAX_N:
+            s = _rows_closure(src, work, n, npad, st, stream)
+            if s.aux[5]:
+                sched = "lower"
+                s.aux[5] = 0
+                if not s.flags & _lib.F_NEED_GENERAL:
+                    return work[:n, :n], FwOutcome(s, npad, "fast", sched)
+                fast = False
+            elif s.flags & _lib.F_PRECOND_FAIL:
+                fast = False
+    st.reset(stream)
+    if fast:
+        # one pass: copy, fast-domain check and encoding (rbg_fw_load_*)
         fn = "rbg_fw_load_i32" if work.dtype == t.int32 else "rbg_fw_load_i64"
         _lib.call(fn, _lib.ptr(src), n, src.stride(0), _lib.ptr(work), npad, st.p, _lib.stream_handle(stream))
         s = st.read(stream)

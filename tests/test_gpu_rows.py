@@ -1,0 +1,141 @@
+"""The dense closure from the rows' direct entries (rbg_fw_rows_*): which
+matrices it takes, and W, diameter and status against the oracle's naive loop
+and the blocked full schedule, at the edges of its slabs, slots and levels."""
+import numpy as np
+import pytest
+
+from redblackgraph_amd import _lib, dense, synth
+from redblackgraph_amd._dtypes import elem_type
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(A, lda=None):
+    """(closed, W, status) of one rbg_fw_rows_* call."""
+    t = _lib.torch()
+    n = A.shape[0]
+    big = np.zeros((n, lda or n), dtype=A.dtype)
+    big[:, :n] = A
+    src = _lib.to_device(big)[:, :n]
+    npad = dense.padded_order(n)
+    work = t.full((npad, npad), 77, dtype=src.dtype, device=src.device)
+    s = dense._rows_closure(src, work, n, npad, dense.status(), None)
+    return int(s.aux[5]), work[:n, :n].cpu().numpy(), s
+
+
+def _full(A):
+    W, out = dense.fw_closure(_lib.to_device(A), elem_type(A.dtype), schedule="full")
+    return W.cpu().numpy(), out
+
+
+def _slots(n):
+    return max(8, min(n // 64, 128))
+
+
+def _with_extra_entries(n, per_row, dt, seed):
+    """A lower triangular matrix with ``per_row`` entries in every row that has
+    room for them, values 2..5, and few levels: entries lie in the first half."""
+    rng = np.random.default_rng(seed)
+    A = np.zeros((n, n), dtype=dt)
+    A[np.arange(n), np.arange(n)] = rng.choice([-1, 0, 1], n)
+    for i in range(n // 2, n):
+        A[i, rng.choice(n // 2, per_row, replace=False)] = rng.integers(2, 6, per_row)
+    for i in range(1, n // 2):
+        A[i, rng.integers(0, max(1, i // 2))] = 2
+    return A
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("n,lda", [(1, None), (2, None), (17, None), (31, 33), (32, 32), (33, 36), (129, None),
+                                   (300, 301), (513, 516), (1100, None)])
+def test_rows_closure_vs_oracle(orc, dt, n, lda):
+    A = synth.dense_pedigree(synth.PedigreeSpec(n, min(n, 12), 0.8, 3), 3 + n, dtype=dt)
+    if n > 20:
+        A[7, 7] = 0  # a vertex without a colour
+    closed, W, s = _rows(A, lda)
+    ref = orc.warshall(A)
+    assert closed == 1 and s.flags == 0 and s.events == 0 and s.cycle_count == 0
+    np.testing.assert_array_equal(W, ref.W)
+    Wf, out = _full(A)
+    np.testing.assert_array_equal(W, Wf)
+    assert s.diameter_max == out.status.diameter_max
+    assert dense.msb(s.diameter_max) == ref.diameter
+
+
+@pytest.mark.parametrize("dt,n", [(np.int32, 256), (np.int32, 1500), (np.int64, 640)])
+def test_rows_closure_slot_limit(dt, n):
+    """Rows with as many entries as there are slots are closed here, one more
+    sends the matrix to the blocked schedules; the results are the same."""
+    full = _with_extra_entries(n, _slots(n), dt, 1)
+    closed, W, s = _rows(full)
+    Wf, out = _full(full)
+    assert closed == 1 and s.diameter_max == out.status.diameter_max
+    np.testing.assert_array_equal(W, Wf)
+    over = _with_extra_entries(n, _slots(n) + 1, dt, 1)
+    closed, W, _ = _rows(over)
+    assert closed == 0 and (W == 77).all()
+    W2, out2 = dense.fw_closure(_lib.to_device(over), elem_type(dt))
+    Wf, outf = _full(over)
+    assert out2.schedule == "lower" and out2.status.diameter_max == outf.status.diameter_max
+    np.testing.assert_array_equal(W2.cpu().numpy(), Wf)
+
+
+def _chain(n, dt):
+    A = np.diag(np.full(n, -1, dtype=dt))
+    A[np.arange(1, n), np.arange(n - 1)] = 2
+    return A
+
+
+def _shortcut_chain(n, dt):
+    """A chain whose every row also names vertex i - 2, i - 4, ...: n levels,
+    values that stay small."""
+    A = _chain(n, dt)
+    for i in range(n):
+        for q in range(1, 7):
+            if i - (1 << q) >= 0:
+                A[i, i - (1 << q)] = 2
+    return A
+
+
+def test_rows_closure_level_limit():
+    for n, closed_ref in ((63, 1), (64, 1), (65, 0)):
+        A = _shortcut_chain(n, np.int64)
+        closed, W, s = _rows(A)
+        assert closed == closed_ref
+        Wf, out = _full(A)
+        W2, out2 = dense.fw_closure(_lib.to_device(A), elem_type(np.int64))
+        np.testing.assert_array_equal(W2.cpu().numpy(), Wf)
+        assert out2.status.diameter_max == out.status.diameter_max and out2.schedule == "lower"
+
+
+@pytest.mark.parametrize("dt,bits", [(np.int32, 32), (np.int64, 64)])
+def test_rows_closure_overflow_guard(dt, bits):
+    """The longest chain whose values fit is closed; one vertex more overflows
+    and comes out of general mode with its events."""
+    fits, over = _chain(bits - 1, dt), _chain(bits, dt)
+    closed, W, s = _rows(fits)
+    Wf, out = _full(fits)
+    assert closed == 1 and s.flags == 0
+    np.testing.assert_array_equal(W, Wf)
+    closed, _, s = _rows(over)
+    assert s.flags & _lib.F_NEED_GENERAL
+    W2, out2 = dense.fw_closure(_lib.to_device(over), elem_type(dt))
+    Wf, outf = _full(over)
+    assert out2.mode == outf.mode == "general" and out2.status.events == outf.status.events != 0
+    np.testing.assert_array_equal(W2.cpu().numpy(), Wf)
+
+
+@pytest.mark.parametrize("i,j,v", [(40, 3, 1), (40, 3, -1), (40, 3, -5), (40, 40, 2), (40, 40, -3)])
+def test_rows_closure_declines_values(i, j, v):
+    A = synth.dense_pedigree(synth.PedigreeSpec(70, 6, 0.8, 3), 1)
+    A[i, j] = v
+    closed, W, s = _rows(A)
+    assert closed == 0 and s.flags & _lib.F_PRECOND_FAIL and (W == 77).all()
+
+
+def test_rows_closure_declines_other_sides():
+    A = synth.dense_pedigree(synth.PedigreeSpec(140, 7, 0.8, 3), 1)
+    B = A.copy()
+    B[3, 90] = 2
+    closed, W, s = _rows(B)
+    assert closed == 0 and (W == 77).all()
