@@ -16,11 +16,12 @@
 // of the blocked schedules, almost all of which have an absent operand: the
 // closure is bound by reading the input and writing the result.
 //
-// Three launches, no waits between workgroups and nothing read by the host:
+// Four launches, no waits between workgroups and nothing read by the host:
 //   scan    one wave per row: reads the matrix once, checks the fast domain,
 //           keeps each row's off-diagonal entries in ascending column order;
 //   levels  one workgroup: each row's level (1 + the largest level among its
-//           entries' rows), rows sorted by level;
+//           entries' rows) and its position in level order;
+//   place   the rows' records in level order;
 //   close   one workgroup per slab of columns (128 bytes wide, a cache line a
 //           row).  A column depends on itself alone, so a workgroup needs only
 //           its own barrier between levels.
@@ -38,7 +39,7 @@
 namespace rbg {
 
 constexpr int ROWS_MAX_LEVELS = 64;
-constexpr int64_t ROWS_MAX_N = 32768;  // one byte of LDS per row in the level pass
+constexpr int64_t ROWS_MAX_N = 32640;  // rows in 15 bits; a byte of LDS per row in the level pass
 constexpr int ROWS_LEVEL_NT = 1024;
 constexpr int ROWS_CLOSE_NT = 1024;
 
@@ -47,23 +48,30 @@ __host__ __device__ inline int rows_slots(int64_t n) {
   return (int)(s < 8 ? 8 : (s > 128 ? 128 : s));
 }
 
-// head word of a row: entries | (diagonal + 1) << 16 | ROW_* flags
+// A row for the level pass: entry 0's column | entry 1's column << 16
+// (ROW_NONE where there is none) | ROW_MORE when it has more entries.  A row
+// that keeps the matrix from being closed here is ROW_STOP | why.
 enum : uint32_t {
-  ROW_BAD = 1u << 20,    // a value outside the fast domain
-  ROW_LOWER = 1u << 21,  // an entry below the diagonal
-  ROW_UPPER = 1u << 22,  // an entry above it
-  ROW_WIDE = 1u << 23,   // more than rows_slots(n) entries
+  ROW_NONE = 0x7fff,
+  ROW_MORE = 1u << 15,
+  ROW_STOP = 1u << 31,
+  STOP_UPPER = 4,  // an entry above the diagonal
+  STOP_BAD = 8,    // a value outside the fast domain
+  STOP_WIDE = 16,  // more than rows_slots(n) entries
 };
+__host__ __device__ inline int rec_cnt(uint32_t w) { return (int)((w >> 16) & 0xff); }
 
-// A row in level order: its first two entries inline (a pedigree's father and
-// mother), the rest in the row's slots.
+// A row's first two entries (a pedigree's father and mother) inline, the rest
+// in the row's slots.  Eight words; a quad of lanes loads two each.
 template <typename T>
 struct alignas(16) RowRec {
-  int32_t row;
-  int32_t head;  // entries | (diagonal + 1) << 16
-  int32_t c0, c1;
+  uint32_t row_c0;  // row | column of entry 0 << 16
+  uint32_t c1_p0;   // column of entry 1 | position of entry 0's row in level order << 16
+  uint32_t p1_cnt;  // position of entry 1's row | entries << 16 | (diagonal + 1) << 24
+  uint32_t pad;
   T v0, v1;
 };
+static_assert(sizeof(RowRec<int32_t>) == 32 && sizeof(RowRec<int64_t>) == 32, "a quad's two words per lane");
 
 // ctl words: [0] the side the close pass takes (0: not closed here, 1 lower),
 // [1] levels, [CTL_START + l] first position of level l
@@ -72,8 +80,10 @@ constexpr int CTL_START = 8;
 template <typename T>
 struct RowsWork {
   int32_t* ctl;
-  uint32_t* head;
-  RowRec<T>* rec;
+  uint32_t* entries;  // the level pass's word per row (scan)
+  uint16_t* pos;      // each row's position in level order (levels)
+  RowRec<T>* rec0;    // in row order (scan)
+  RowRec<T>* rec;     // in level order (place)
   int32_t* ecol;  // row i's entries at [i * slots]
   T* eval;
   int slots;
@@ -91,11 +101,13 @@ static inline int64_t rows_layout(int64_t n, char* base, RowsWork<T>* w) {
     return base + at;
   };
   char* ctl = take(4 * (CTL_START + ROWS_MAX_LEVELS + 1));
-  char* head = take(4 * n);
+  char* entries = take(4 * (n + 3));  // read four at a time
+  char* pos = take(2 * (n + 3));
+  char* rec0 = take((int64_t)sizeof(RowRec<T>) * n);
   char* rec = take((int64_t)sizeof(RowRec<T>) * n);
   char* ecol = take(4 * n * slots);
   char* eval = take((int64_t)sizeof(T) * n * slots);
-  if (w) *w = RowsWork<T>{(int32_t*)ctl, (uint32_t*)head, (RowRec<T>*)rec, (int32_t*)ecol, (T*)eval, slots};
+  if (w) *w = RowsWork<T>{(int32_t*)ctl, (uint32_t*)entries, (uint16_t*)pos, (RowRec<T>*)rec0, (RowRec<T>*)rec, (int32_t*)ecol, (T*)eval, slots};
   return o;
 }
 
@@ -111,8 +123,10 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
   const uint64_t below = ((uint64_t)1 << lane) - 1;
   int32_t* ecol = w.ecol + i * w.slots;
   T* eval = w.eval + i * w.slots;
+  RowRec<T>& rec = w.rec0[i];
+  uint32_t c0 = ROW_NONE, c1 = ROW_NONE;
   int cnt = 0;
-  bool bad = false, lo = false, up = false;
+  bool bad = false, up = false;
   T diag = 0;
   auto emit = [&](int64_t j, const T* v) {
     bool keep[V];
@@ -127,7 +141,6 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
       }
       if (keep[x]) {
         bad |= v[x] < (T)2;
-        lo |= j + x < i;
         up |= j + x > i;
       }
       const uint64_t m = __ballot(keep[x]);
@@ -142,6 +155,8 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
           ecol[p] = (int32_t)(j + x);
           eval[p] = v[x];
         }
+        if (p == 0) c0 = (uint32_t)(j + x), rec.v0 = v[x];
+        if (p == 1) c1 = (uint32_t)(j + x), rec.v1 = v[x];
         p++;
       }
     cnt += total;
@@ -195,117 +210,182 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
       }
     }
   }
+  // the lanes that met entries 0 and 1 hold their columns
+  const uint64_t h0 = __ballot(c0 != ROW_NONE), h1 = __ballot(c1 != ROW_NONE);
+  if (h0) c0 = (uint32_t)__builtin_amdgcn_readlane((int)c0, __ffsll((unsigned long long)h0) - 1);
+  if (h1) c1 = (uint32_t)__builtin_amdgcn_readlane((int)c1, __ffsll((unsigned long long)h1) - 1);
   const uint32_t d = __any(diag == (T)1) ? 2u : (__any(diag == (T)-1) ? 0u : 1u);
-  const uint32_t f = (__any(bad) ? (uint32_t)ROW_BAD : 0u) | (__any(lo) ? (uint32_t)ROW_LOWER : 0u) |
-                     (__any(up) ? (uint32_t)ROW_UPPER : 0u) | (cnt > w.slots ? (uint32_t)ROW_WIDE : 0u);
-  if (lane == 0) w.head[i] = (uint32_t)(cnt < w.slots ? cnt : w.slots) | d << 16 | f;
+  const uint32_t stop = (__any(bad) ? (uint32_t)STOP_BAD : 0u) | (__any(up) ? (uint32_t)STOP_UPPER : 0u) |
+                        (cnt > w.slots ? (uint32_t)STOP_WIDE : 0u);
+  if (lane == 0) {
+    rec.row_c0 = (uint32_t)i | c0 << 16;
+    rec.c1_p0 = c1;
+    rec.p1_cnt = (uint32_t)(cnt < w.slots ? cnt : w.slots) << 16 | d << 24;
+    w.entries[i] = stop ? ROW_STOP | stop : c0 | c1 << 16 | (cnt > 2 ? (uint32_t)ROW_MORE : 0u);
+  }
 }
 
 struct LevelShared {
-  int hist[ROWS_MAX_LEVELS + 1];
+  int hist[ROWS_MAX_LEVELS];
   int next[ROWS_MAX_LEVELS];
-  uint32_t flags;
-  int deep;
+  int marks[4];
 };
 
-// Levels and level order of a lower triangular matrix's rows, by one
-// workgroup.  Rows go in chunks of a thread each; a row's entries lie in
-// earlier chunks (final) or its own, where the levels only grow, so a chunk
-// repeats until no level changed: as many passes as the chunk is deep.
-// Returns the flags of all rows.
+// Level and position of every row of a lower triangular matrix, by one
+// workgroup of at least 64 threads; lev: n + 1 bytes of LDS.  Eight rows a
+// thread (four neighbours, twice) in registers, in blocks of rows; a row's
+// entries lie in earlier blocks (final) or its own, where the levels only
+// grow, so a block is swept until no level changed, one barrier a sweep, at
+// most as many sweeps as the block is deep.  One workgroup runs its code
+// once, so its time is instruction fetches, barriers and LDS reads: short
+// loops and few of them count for more here than loads in flight
+// (N = 8192, 18 levels: 28 us against 93 us with one row per thread and pass,
+// chunk by chunk, and 66 us with the records moved here, eight unrolled; N =
+// 512: 12 us).  Returns the STOP_* reasons (0: positions are in w.pos).
 template <typename T>
-__device__ inline uint32_t rows_levels(RowsWork<T> w, int64_t n, LevelShared& L, uint8_t* lev, bool allowed) {
-  const int tid = threadIdx.x, nthreads = blockDim.x;
-  if (tid == 0) {
-    L.flags = 0;
-    L.deep = 0;
-  }
-  if (tid <= ROWS_MAX_LEVELS) L.hist[tid] = 0;
+__device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev) {
+  const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, n = (int)n64;
+  if (tid < 4) L.marks[tid] = 0;
+  if (tid < ROWS_MAX_LEVELS) L.hist[tid] = 0;
+  if (tid == 0) lev[n] = 255;  // an absent entry's level: below 0
   __syncthreads();
-  uint32_t f = 0;
-  for (int64_t i = tid; i < n; i += nthreads) f |= w.head[i];
-  f &= ROW_BAD | ROW_LOWER | ROW_UPPER | ROW_WIDE;
-  if (f) atomicOr(&L.flags, f);
-  __syncthreads();
-  f = L.flags;
-  if (!allowed || (f & (ROW_BAD | ROW_WIDE | ROW_UPPER))) {
-    if (tid == 0) w.ctl[0] = 0;
-    return f;
-  }
-  for (int64_t b = 0; b < n; b += nthreads) {
-    const int64_t i = b + tid;
-    const bool on = i < n;
-    const int cnt = on ? (int)(w.head[i] & 0xffff) : 0;
-    const int32_t* ec = w.ecol + i * w.slots;
-    const int c0 = cnt > 0 ? ec[0] : 0, c1 = cnt > 1 ? ec[1] : 0;
-    int lv = 0;
-    if (on) lev[i] = 0;
+  int it = 0;  // sweeps so far: sweep it marks marks[it & 3]
+  for (int b = 0; b < n; b += 8 * nt) {
+    uint32_t e[8];
+    int row[2];
+    uint32_t lv[2] = {0, 0};  // four levels each
+    int stop = 0;
+    bool more = false;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      row[h] = b + 4 * (h * nt + tid);
+      uint4 q = make_uint4(0, 0, 0, 0);
+      if (row[h] < n) {
+        q = *(const uint4*)(w.entries + row[h]);
+        *(uint32_t*)(lev + row[h]) = 0;
+      }
+      e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
+    }
     __syncthreads();
-    for (;;) {
-      int nl = 0;
-      if (cnt > 0) nl = lev[c0] + 1;
-      if (cnt > 1) nl = nl > lev[c1] + 1 ? nl : lev[c1] + 1;
-      for (int e = 2; e < cnt; e++) {
-        const int x = lev[ec[e]] + 1;
-        nl = nl > x ? nl : x;
-      }
-      bool changed = nl > lv;
-      if (nl >= ROWS_MAX_LEVELS) {
-        L.deep = 1;
-        changed = false;
-      }
-      if (changed) {
-        lv = nl;
-        lev[i] = (uint8_t)nl;
-      }
-      if (!__syncthreads_or(changed)) break;
+    if (tid == 0) lev[n] = 255;  // the words above may cover it
+#pragma unroll
+    for (int x = 0; x < 8; x++) {
+      const bool on = row[x / 4] + x % 4 < n;
+      if (!on) e[x] = ROW_NONE | ROW_NONE << 16;
+      if (e[x] & ROW_STOP) stop |= (int)(e[x] & 0xff);
+      more |= (e[x] & ROW_MORE) != 0;
+      const uint32_t c0 = e[x] & 0x7fff, c1 = (e[x] >> 16) & 0x7fff;
+      e[x] = (e[x] & ROW_STOP) ? (uint32_t)n | (uint32_t)n << 16
+                               : (c0 == ROW_NONE ? (uint32_t)n : c0) | (c1 == ROW_NONE ? (uint32_t)n : c1) << 16 |
+                                     (e[x] & ROW_MORE) << 16;
     }
-    if (L.deep) {  // written before the barrier above
-      if (tid == 0) w.ctl[0] = 0;
-      return f;
+    __syncthreads();
+    for (;; it++) {
+      uint32_t nv[2] = {0, 0};
+      int worst = 0;
+#pragma unroll
+      for (int x = 0; x < 8; x++) {
+        const int l0 = (uint8_t)(lev[e[x] & 0xffff] + 1), l1 = (uint8_t)(lev[(e[x] >> 16) & 0x7fff] + 1);
+        int nl = l0 > l1 ? l0 : l1;
+        if (more && e[x] >> 31) {
+          const int i = row[x / 4] + x % 4, cnt = rec_cnt(w.rec0[i].p1_cnt);
+          const int32_t* ec = w.ecol + (int64_t)i * w.slots;
+          for (int k = 2; k < cnt; k++) {
+            const int y = lev[ec[k]] + 1;
+            nl = nl > y ? nl : y;
+          }
+        }
+        worst = nl > worst ? nl : worst;
+        nv[x / 4] |= (uint32_t)nl << (8 * (x % 4));
+      }
+      bool changed = false;
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        if (nv[h] != lv[h]) {
+          lv[h] = nv[h];
+          changed = true;
+          if (row[h] + 3 < n)
+            *(uint32_t*)(lev + row[h]) = nv[h];
+          else
+            for (int x = 0; row[h] + x < n; x++) lev[row[h] + x] = (uint8_t)(nv[h] >> (8 * x));
+        }
+      const int mark = (__any(changed) ? 1 : 0) | (__any(worst >= ROWS_MAX_LEVELS) ? 2 : 0) |
+                       (__any(stop & STOP_UPPER) ? STOP_UPPER : 0) | (__any(stop & STOP_BAD) ? STOP_BAD : 0) |
+                       (__any(stop & STOP_WIDE) ? STOP_WIDE : 0);
+      if (mark && lane == 0) atomicOr(&L.marks[it & 3], mark);
+      if (tid == 0) L.marks[(it + 2) & 3] = 0;  // read two sweeps ago, marked two sweeps on
+      __syncthreads();
+      const int marks = L.marks[it & 3];  // the same for every thread: the branches below are uniform
+      if (marks & ~1) return marks & ~1;
+      if (!marks) break;
     }
-    if (on) atomicAdd(&L.hist[lv], 1);
+    it++;
+#pragma unroll
+    for (int x = 0; x < 8; x++)
+      if (row[x / 4] + x % 4 < n) atomicAdd(&L.hist[(lv[x / 4] >> (8 * (x % 4))) & 0xff], 1);
   }
   __syncthreads();
-  if (tid == 0) {
-    int at = 0, levels = 0;
-    for (int l = 0; l < ROWS_MAX_LEVELS; l++) {
-      L.next[l] = at;
-      w.ctl[CTL_START + l] = at;
-      if (L.hist[l]) levels = l + 1;
-      at += L.hist[l];
+  if (tid < ROWS_MAX_LEVELS) {  // the first wave: an exclusive scan of the level sizes
+    const int c = L.hist[tid];
+    int incl = c;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d, 64);
+      if (tid >= d) incl += o;
     }
-    w.ctl[CTL_START + ROWS_MAX_LEVELS] = at;
-    w.ctl[1] = levels;
-    w.ctl[0] = 1;
+    L.next[tid] = incl - c;
+    w.ctl[CTL_START + tid] = incl - c;
+    const uint64_t some = __ballot(c != 0);
+    if (tid == 0) {
+      w.ctl[CTL_START + ROWS_MAX_LEVELS] = n;
+      w.ctl[1] = 64 - __clzll(some);
+    }
   }
   __syncthreads();
-  for (int64_t i = tid; i < n; i += nthreads) {
-    const uint32_t h = w.head[i];
-    const int cnt = (int)(h & 0xffff);
-    const int32_t* ec = w.ecol + i * w.slots;
-    const T* ev = w.eval + i * w.slots;
-    RowRec<T> r{(int32_t)i, (int32_t)(h & 0x3ffff), 0, 0, 0, 0};
-    if (cnt > 0) r.c0 = ec[0], r.v0 = ev[0];
-    if (cnt > 1) r.c1 = ec[1], r.v1 = ev[1];
-    w.rec[atomicAdd(&L.next[lev[i]], 1)] = r;
+  for (int i = 4 * tid; i < n; i += 4 * nt) {
+    uint16_t at[4];
+#pragma unroll
+    for (int x = 0; x < 4; x++) at[x] = i + x < n ? (uint16_t)atomicAdd(&L.next[lev[i + x]], 1) : (uint16_t)0;
+    *(ushort4*)(w.pos + i) = make_ushort4(at[0], at[1], at[2], at[3]);
   }
-  return f;
+  return 0;
+}
+static_assert(ROWS_MAX_LEVELS == 64, "one wave scans the level sizes");
+
+// Row i's record to its place in level order, with its entries' places.
+template <typename T>
+__device__ inline void rows_place(RowsWork<T> w, int64_t i) {
+  const uint4* p = (const uint4*)(w.rec0 + i);
+  uint4 a = p[0];
+  const uint4 v = p[1];
+  const int cnt = rec_cnt(a.z);
+  if (cnt > 0) a.y = (a.y & 0xffff) | (uint32_t)w.pos[a.x >> 16] << 16;
+  if (cnt > 1) a.z |= w.pos[a.y & 0xffff];
+  uint4* o = (uint4*)(w.rec + w.pos[i]);
+  o[0] = a;
+  o[1] = v;
 }
 
-// Left operand a of a lane's V cells: a (x) y for the cells y of the entry's
-// row.  A cell below 2 is no operand (absent, or the diagonal's identity).
+// Left operand a on a lane's V cells y of the entry's row: cells are kept as
+// value - 1 with all ones for an absent one, so that the sum is an unsigned
+// min and the stored value cell + 1.  A y below 2 is no operand (absent, or
+// the diagonal's identity).  top: largest y met (for the overflow guard);
+// tmax: largest cell (all ones counts as -1).
 template <typename T, int V>
-__device__ inline void rows_relax(typename unsigned_of<T>::type (&cur)[V], T a, const T (&y)[V], int& guard, T& tmax) {
+__device__ inline void rows_relax(typename unsigned_of<T>::type (&cur)[V], T a, const T (&y)[V], T& top, T& tmax) {
   using U = typename unsigned_of<T>::type;
-  const int ma = msb_u((U)a);
+  constexpr int HI = 8 * (int)sizeof(T) - 1;
+  const U am = (U)(a - 1);
 #pragma unroll
   for (int x = 0; x < V; x++) {
-    const bool present = y[x] > (T)1;
-    const int m = present ? msb_u((U)y[x]) : 0;
-    const U p = present ? ((U)(a - 1) << m) + (U)y[x] : ~(U)0;
-    guard = present && ma + m > guard ? ma + m : guard;
+    int z;  // leading zeros; y = 0 gives some number, dropped below
+    if constexpr (sizeof(T) == 4)
+      z = __builtin_clz((U)y[x]);
+    else
+      z = __builtin_clzll((U)y[x]);
+    const U q = (am << ((HI - z) & HI)) + (U)(y[x] - 1);
+    const U p = y[x] > (T)1 ? q : ~(U)0;
     cur[x] = p < cur[x] ? p : cur[x];
+    top = y[x] > top ? y[x] : top;
     tmax = (T)cur[x] > tmax ? (T)cur[x] : tmax;
   }
 }
@@ -329,31 +409,70 @@ __device__ inline void rows_st(T* p, const T (&y)[V]) {
     *(ulonglong2*)p = make_ulonglong2((unsigned long long)y[0], (unsigned long long)y[1]);
 }
 
-constexpr int ROWS_LANES = 8;  // lanes of 16 bytes per row segment: one 128-byte line
+// 16 bytes of zeros that nothing here reads again
+template <typename T>
+__device__ inline void rows_st_stream(T* p) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  __builtin_nontemporal_store(u32x4{0, 0, 0, 0}, (u32x4*)p);
+}
+
+constexpr int ROWS_LANES = 4;  // lanes of 16 bytes per row segment
 template <typename T>
 __host__ __device__ inline int64_t rows_slab() {
   return ROWS_LANES * (16 / (int64_t)sizeof(T));
 }
 
+constexpr int ROWS_RING = 1024;  // 64 KB: two workgroups per CU
+template <typename T>
 struct CloseShared {
+  T ring[ROWS_RING][ROWS_LANES][16 / sizeof(T)];
   int start[ROWS_MAX_LEVELS + 1];
   long long top;
   int guard;
 };
 
-// One slab of columns through every level.  W rows are 16-byte aligned (ld a
-// multiple of 128).  Eight lanes hold one row's segment; two rows per lane
-// group are in flight so that the four loads of their entries' rows overlap.
+// Word `lane` of a quad, to all four lanes.
+template <int LANE>
+__device__ inline uint32_t quad_bcast(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, LANE * 0x55, 0xf, 0xf, false);
+}
 template <typename T>
-__device__ inline void rows_close_slab(CloseShared& L, RowsWork<T> w, T* W, int64_t ld, int64_t slab, int width,
+__device__ inline RowRec<T> rec_of_quad(uint2 q) {
+  RowRec<T> r;
+  r.row_c0 = quad_bcast<0>(q.x);
+  r.c1_p0 = quad_bcast<0>(q.y);
+  r.p1_cnt = quad_bcast<1>(q.x);
+  if constexpr (sizeof(T) == 4) {
+    r.v0 = (T)quad_bcast<2>(q.x);
+    r.v1 = (T)quad_bcast<2>(q.y);
+  } else {
+    r.v0 = (T)((uint64_t)quad_bcast<2>(q.x) | (uint64_t)quad_bcast<2>(q.y) << 32);
+    r.v1 = (T)((uint64_t)quad_bcast<3>(q.x) | (uint64_t)quad_bcast<3>(q.y) << 32);
+  }
+  return r;
+}
+
+// One slab of columns through every level.  W rows are 16-byte aligned (ld a
+// multiple of 128).  A quad of lanes holds one row's segment.  Entries' rows
+// are mostly of the last few levels (parents a few layers up), so the last
+// ROWS_RING rows in level order stay in LDS and only older ones are read back
+// from memory (N = 8192 int32: 130 us with every row read back, 128-byte
+// segments or 64; 93-101 us so, of which about 40 are the writes' own time;
+// 2048 rows with one workgroup per CU: 93 us).  The products are not the
+// bound: leaving them out changed nothing.  Rows above the slab's first column hold no entry there and
+// are never read again: their zeros go out as streaming stores.
+template <typename T, int UN>
+__device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, int64_t ld, int64_t slab, int width,
                                        rbg_status* st) {
   using U = typename unsigned_of<T>::type;
   constexpr int V = 16 / (int)sizeof(T);
-  constexpr int UN = 2;
-  const int tid = threadIdx.x, G = blockDim.x / ROWS_LANES;
+  const int tid = threadIdx.x, G = blockDim.x / ROWS_LANES, ql = tid % ROWS_LANES;
   const int g = tid / ROWS_LANES;
   const int j0 = (int)(slab * rows_slab<T>());
-  const int jl = j0 + (tid % ROWS_LANES) * V;
+  const int jl = j0 + ql * V;
+  // row offsets in 16-byte units: below 2^32 for ROWS_MAX_N, one 24-bit multiply each
+  const uint32_t ld16 = (uint32_t)(ld / V), jl16 = (uint32_t)(jl / V);
+  auto at = [&](int row) { return W + (size_t)(__umul24((uint32_t)row, ld16) + jl16) * V; };
   const int levels = w.ctl[1];
   if (tid <= levels) L.start[tid] = w.ctl[CTL_START + tid];
   if (tid == 0) {
@@ -361,90 +480,122 @@ __device__ inline void rows_close_slab(CloseShared& L, RowsWork<T> w, T* W, int6
     L.guard = 0;
   }
   __syncthreads();
-  int guard = 0;
-  T tmax = 0;
-  for (int l = 0; l < levels; l++) {
-    const int end = L.start[l + 1];
-    for (int p = L.start[l] + g; p < end; p += UN * G) {
-      RowRec<T> r[UN];
-      T y0[UN][V], y1[UN][V];
-      int cnt[UN];
+  int guard = 0;  // largest MSB(left) + MSB(right) of a product
+  T tmax = -1;
+  uint2 qr[UN];  // this lane's words of the records
+  auto fetch = [&](int p, int end, uint2& q) {
+    if (p < end) q = ((const uint2*)(w.rec + p))[ql];
+  };
+  int base = 0, end = L.start[1];  // this pass: positions base + g + u G of level l
 #pragma unroll
-      for (int u = 0; u < UN; u++) r[u] = w.rec[p + u * G < end ? p + u * G : p];
+  for (int u = 0; u < UN; u++) fetch(base + g + u * G, end, qr[u]);
+  for (int l = 0; l < levels;) {
+    const int kept = end - ROWS_RING;  // older positions have left the ring by the end of this level
+    RowRec<T> r[UN];
+    T y0[UN][V], y1[UN][V];
+    bool on[UN];
+    int cnt[UN], row[UN], c0[UN], c1[UN];
+    auto operand = [&](int c, int p, T(&y)[V]) {
+      if (p >= kept)
+        rows_ld<T, V>(L.ring[p & (ROWS_RING - 1)][ql], y);
+      else
+        rows_ld<T, V>(at(c), y);
+    };
 #pragma unroll
-      for (int u = 0; u < UN; u++) {
-        cnt[u] = r[u].head & 0xffff;
-        if (cnt[u] > 0 && r[u].c0 >= j0) {
-          rows_ld<T, V>(W + r[u].c0 * ld + jl, y0[u]);
-        } else {
+    for (int u = 0; u < UN; u++) {
+      on[u] = base + g + u * G < end;
+      r[u] = rec_of_quad<T>(qr[u]);
+      cnt[u] = on[u] ? rec_cnt(r[u].p1_cnt) : 0;
+      row[u] = (int)(r[u].row_c0 & 0xffff);
+      c0[u] = (int)(r[u].row_c0 >> 16);
+      c1[u] = (int)(r[u].c1_p0 & 0xffff);
 #pragma unroll
-          for (int x = 0; x < V; x++) y0[u][x] = 0;
-        }
-        if (cnt[u] > 1 && r[u].c1 >= j0) {
-          rows_ld<T, V>(W + r[u].c1 * ld + jl, y1[u]);
-        } else {
+      for (int x = 0; x < V; x++) y0[u][x] = y1[u][x] = 0;
+      if (cnt[u] > 0 && c0[u] >= j0) operand(c0[u], (int)(r[u].c1_p0 >> 16), y0[u]);
+      if (cnt[u] > 1 && c1[u] >= j0) operand(c1[u], (int)(r[u].p1_cnt & 0xffff), y1[u]);
+    }
+    // the pass after this one: the same level's, or the next level's first
+    int bn = base + UN * G, ln = l, en = end;
+    if (bn >= end) {
+      ln = l + 1;
+      bn = end;
+      en = ln < levels ? L.start[ln + 1] : end;
+    }
 #pragma unroll
-          for (int x = 0; x < V; x++) y1[u][x] = 0;
-        }
+    for (int u = 0; u < UN; u++) fetch(bn + g + u * G, en, qr[u]);
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      if (!on[u]) continue;
+      T* out = at(row[u]);
+      if (row[u] < j0) {
+        rows_st_stream<T>(out);
+        continue;
       }
+      U cur[V];
 #pragma unroll
-      for (int u = 0; u < UN; u++) {
-        if (p + u * G >= end) break;
-        const int row = r[u].row;
-        U cur[V];
-        const T d = (T)((r[u].head >> 16) & 3) - 1;
+      for (int x = 0; x < V; x++) cur[x] = ~(U)0;
+      const int32_t* ec = w.ecol + (int64_t)row[u] * w.slots;
+      const T* ev = w.eval + (int64_t)row[u] * w.slots;
+      // the input's cells in this lane's columns, and the diagonal's identity
+      T one = 0;
+      const bool here = (unsigned)(row[u] - jl) < (unsigned)V || (cnt[u] > 0 && (unsigned)(c0[u] - jl) < (unsigned)V) ||
+                        (cnt[u] > 1 && (unsigned)(c1[u] - jl) < (unsigned)V) || cnt[u] > 2;
+      if (here) {
 #pragma unroll
         for (int x = 0; x < V; x++) {
-          cur[x] = ~(U)0;
-          if (row == jl + x) cur[x] = (U)e_enc<T>(d);
-          if (cnt[u] > 0 && r[u].c0 == jl + x) cur[x] = (U)r[u].v0;
-          if (cnt[u] > 1 && r[u].c1 == jl + x) cur[x] = (U)r[u].v1;
+          if (row[u] == jl + x) one = (T)((r[u].p1_cnt >> 24) & 3) - 1;
+          if (cnt[u] > 0 && c0[u] == jl + x) cur[x] = (U)r[u].v0 - 1;
+          if (cnt[u] > 1 && c1[u] == jl + x) cur[x] = (U)r[u].v1 - 1;
         }
-        if (cnt[u] > 2) {
-          const int32_t* ec = w.ecol + (int64_t)row * w.slots;
-          const T* ev = w.eval + (int64_t)row * w.slots;
-          for (int e = 2; e < cnt[u]; e++) {
-            const int x = ec[e] - jl;
-            if (x >= 0 && x < V) {
+        for (int e = 2; e < cnt[u]; e++) {
+          const int c = ec[e] - jl;
 #pragma unroll
-              for (int c = 0; c < V; c++)
-                if (x == c) cur[c] = (U)ev[e];
-            }
-          }
+          for (int x = 0; x < V; x++)
+            if (c == x) cur[x] = (U)ev[e] - 1;
         }
 #pragma unroll
         for (int x = 0; x < V; x++) tmax = (T)cur[x] > tmax ? (T)cur[x] : tmax;
-        if (cnt[u] > 0) rows_relax<T, V>(cur, r[u].v0, y0[u], guard, tmax);
-        if (cnt[u] > 1) rows_relax<T, V>(cur, r[u].v1, y1[u], guard, tmax);
-        if (cnt[u] > 2) {
-          const int32_t* ec = w.ecol + (int64_t)row * w.slots;
-          const T* ev = w.eval + (int64_t)row * w.slots;
-          for (int e = 2; e < cnt[u]; e += 4) {
-            T y[4][V], a[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-              const int c = e + q < cnt[u] ? ec[e + q] : -1;
-              a[q] = e + q < cnt[u] ? ev[e + q] : (T)2;
-              if (c >= j0) {
-                rows_ld<T, V>(W + c * ld + jl, y[q]);
-              } else {
-#pragma unroll
-                for (int x = 0; x < V; x++) y[q][x] = 0;
-              }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) rows_relax<T, V>(cur, a[q], y[q], guard, tmax);
-          }
-        }
-        T o[V];
-#pragma unroll
-        for (int x = 0; x < V; x++) o[x] = e_dec<T>((T)cur[x]);
-        rows_st<T, V>(W + row * ld + jl, o);
+        if (one == (T)1 && tmax < 0) tmax = 0;
       }
+      auto relax = [&](T a, const T(&y)[V]) {
+        T top = 1;
+        rows_relax<T, V>(cur, a, y, top, tmax);
+        const int m = top > 1 ? msb_u((U)top) + msb_u((U)a) : 0;
+        guard = m > guard ? m : guard;
+      };
+      if (cnt[u] > 0) relax(r[u].v0, y0[u]);
+      if (cnt[u] > 1) relax(r[u].v1, y1[u]);
+      for (int e = 2; e < cnt[u]; e += 4) {
+        T y[4][V], a[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int c = e + q < cnt[u] ? ec[e + q] : -1;
+          a[q] = e + q < cnt[u] ? ev[e + q] : (T)2;
+#pragma unroll
+          for (int x = 0; x < V; x++) y[q][x] = 0;
+          if (c >= j0) rows_ld<T, V>(at(c), y[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) relax(a[q], y[q]);
+      }
+      T o[V];
+#pragma unroll
+      for (int x = 0; x < V; x++) o[x] = (T)(cur[x] + 1);
+      if (one != 0) {  // the lane of the diagonal; no product reaches that cell
+#pragma unroll
+        for (int x = 0; x < V; x++)
+          if (row[u] == jl + x) o[x] = one;
+      }
+      rows_st<T, V>(out, o);
+      const int p = base + g + u * G;
+      if (p >= kept) rows_st<T, V>(L.ring[p & (ROWS_RING - 1)][ql], o);
     }
-    __syncthreads();  // the level's rows are read by the next ones of this workgroup alone
+    if (ln != l) __syncthreads();  // the level's rows are read by the next ones of this workgroup alone
+    l = ln;
+    base = bn;
+    end = en;
   }
-  const long long t = wave_max_i64(tmax);
+  const long long t = wave_max_i64((int64_t)tmax + 1);
   if ((tid & 63) == 0 && t > 0) atomicMax(&L.top, t);
   if (guard > width - 2) atomicMax(&L.guard, guard);
   __syncthreads();

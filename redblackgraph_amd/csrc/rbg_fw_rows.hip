@@ -1,4 +1,4 @@
-// Closure of one triangular matrix from its rows' direct entries: the three
+// Closure of one triangular matrix from its rows' direct entries: the
 // launches of fw_rows.hpp and the C ABI.
 #include "fw_rows.hpp"
 
@@ -10,32 +10,47 @@ static __global__ __launch_bounds__(NT) void k_rows_scan(const T* A, int64_t n, 
   if (i < n) rows_scan_row<T>(A + i * lda, n, i, vec, w);
 }
 
-// Also writes the whole status block: the flags the scan found, and aux[5] =
-// 1 when the close pass will close the matrix.
+// Also writes the whole status block: aux[5] = 1 when the next launches close
+// the matrix.
 template <typename T>
 static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n, RowsWork<T> w, bool allowed,
                                                                      rbg_status* st) {
-  extern __shared__ uint8_t lev[];
+  extern __shared__ __align__(16) uint8_t lev[];
   __shared__ LevelShared L;
-  const uint32_t f = rows_levels<T>(w, n, L, lev, allowed);
+  const int stop = allowed ? rows_levels<T>(w, n, L, lev) : 1;
   if (threadIdx.x == 0) {
     status_clear(st);
-    const bool closed = w.ctl[0] != 0;
-    // a closed matrix's flags are clean, as the blocked closure leaves them
-    st->flags = closed ? 0
-                       : ((f & ROW_BAD) ? (uint32_t)RBG_F_PRECOND_FAIL : 0u) |
-                             ((f & ROW_LOWER) ? (uint32_t)RBG_F_HAS_LOWER : 0u) |
-                             ((f & ROW_UPPER) ? (uint32_t)RBG_F_HAS_UPPER : 0u);
-    st->aux[5] = w.ctl[0];
+    if (stop & STOP_BAD) st->flags = RBG_F_PRECOND_FAIL;
+    w.ctl[0] = st->aux[5] = stop == 0;
   }
 }
 
 template <typename T>
-static __global__ __launch_bounds__(ROWS_CLOSE_NT) void k_rows_close(RowsWork<T> w, T* W, int64_t ld, int width,
+static __global__ __launch_bounds__(NT) void k_rows_place(int64_t n, RowsWork<T> w) {
+  const int64_t i = blockIdx.x * (int64_t)NT + threadIdx.x;
+  if (w.ctl[0] && i < n) rows_place<T>(w, i);
+}
+
+// Workgroup -> slab, `count` of them.  Slabs cost less from left to right
+// (their columns' rows start lower); two workgroups share a CU, the first 512
+// all start at once and the second 256 of them join the first 256 CU by CU, so
+// those take the cheapest slabs.  The XCDs take turns at workgroups: eight
+// neighbouring slabs (512 bytes of a row) go to one XCD's L2.
+__device__ inline int rows_slab_of(int b, int count) {
+  auto grouped = [&](int q) {
+    return (q | 63) < count && (q | 63) < 256 ? (q & ~63) + (q & 7) * 8 + ((q & 63) >> 3) : q;
+  };
+  if (b < 256) return grouped(b);
+  if (b < 512) return count - 1 - (b - 256);
+  return b - 256;
+}
+
+template <typename T>
+static __global__ __launch_bounds__(ROWS_CLOSE_NT, 8) void k_rows_close(RowsWork<T> w, T* W, int64_t ld, int width,
                                                                     rbg_status* st) {
-  __shared__ CloseShared L;
+  __shared__ CloseShared<T> L;
   if (w.ctl[0] != 1) return;
-  rows_close_slab<T>(L, w, W, ld, blockIdx.x, width, st);
+  rows_close_slab<T, 1>(L, w, W, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
 }
 
 template <typename T>
@@ -52,7 +67,9 @@ static int fw_rows(const T* A, int64_t n, int64_t lda, T* W, int64_t npad, void*
   RBG_CHECK_LAUNCH();
   // a forced wait limit asks for the persistent closure (rbg_fw_flow_wait_limit)
   const bool allowed = g_flow_limit_override.load() == 0;
-  hipLaunchKernelGGL((k_rows_levels<T>), dim3(1), dim3(ROWS_LEVEL_NT), (size_t)n, s, n, w, allowed, st);
+  hipLaunchKernelGGL((k_rows_levels<T>), dim3(1), dim3(ROWS_LEVEL_NT), (size_t)(n + 4), s, n, w, allowed, st);
+  RBG_CHECK_LAUNCH();
+  hipLaunchKernelGGL((k_rows_place<T>), dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, s, n, w);
   RBG_CHECK_LAUNCH();
   const int p = prof_start(s);
   hipLaunchKernelGGL((k_rows_close<T>), dim3((unsigned)((n + rows_slab<T>() - 1) / rows_slab<T>())),

@@ -12,7 +12,7 @@ from . import _lib
 from ._dtypes import ElemType, msb
 
 FW_TILE = 128
-ROWS_MAX_N = 32768  # rbg_fw_rows_max_n(): the largest order rbg_fw_rows_* takes
+ROWS_MAX_N = 32640  # rbg_fw_rows_max_n(): the largest order rbg_fw_rows_* takes
 _tls = threading.local()
 
 
