@@ -170,26 +170,35 @@ int rbg_fw_load_i32(const int32_t *A, int64_t n, int64_t lda, int32_t *W, int64_
                     rbg_stream_t stream);
 int rbg_fw_load_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_t npad, rbg_status *st,
                     rbg_stream_t stream);
-/* No counterpart in the reference: the closure of a lower triangular matrix
- * from its rows' direct entries, for matrices with few of them (pedigrees:
- * two a row).  Reads A (n x n, row stride lda) once; when every off-diagonal
- * entry lies below the diagonal, the values pass rbg_fw_precheck_*, every row
- * has at most max(8, min(n / 64, 128)) off-diagonal entries and the graph at
- * most 64 levels, writes the closure (natural values) into columns [0, n) of
- * rows [0, n) of W (row stride npad, a multiple of 128, 16-byte aligned; the
- * rest of W is unspecified), sets st->aux[5] = 1 and st->diameter_max = the
- * max trajectory value; RBG_F_NEED_GENERAL then asks for mode 1 as for
- * rbg_fw_dense_*.  Otherwise st->aux[5] = 0, W is untouched, st->flags may
- * hold RBG_F_PRECOND_FAIL (mode 1), and the caller goes on with
- * rbg_fw_load_*.  Writes the whole status block (no rbg_status_init needed);
- * nothing is read by the host.  workspace: rbg_fw_rows_workspace_bytes(n,
- * element size) bytes, 256-byte aligned; n <= rbg_fw_rows_max_n(). */
+/* No counterpart in the reference: the closure of an acyclic matrix from its
+ * rows' direct entries, for matrices with few of them (pedigrees: two a row).
+ * Reads A (n x n, row stride lda) once; when the values pass
+ * rbg_fw_precheck_*, every row has at most max(8, min(n / 64, 128))
+ * off-diagonal entries and the graph is acyclic with at most 64 levels,
+ * st->aux[5] = 1 (every off-diagonal entry below the diagonal), 2 (above) or 3
+ * (both), and with
+ *   1  the closure (natural values) is written into columns [0, n) of rows
+ *      [0, n) of W (row stride npad, a multiple of 128, 16-byte aligned; the
+ *      rest of W is unspecified) and st->diameter_max = the max trajectory
+ *      value; RBG_F_NEED_GENERAL then asks for mode 1 as for rbg_fw_dense_*;
+ *   2, 3  rbg_fw_rows_any_*, with the same W, workspace and st, writes them.
+ *      W2 is a second matrix like W (scratch).  st->aux[6] != 0 or
+ *      RBG_F_NEED_GENERAL: not closed.
+ * Otherwise st->aux[5] = 0 and st->flags may hold RBG_F_PRECOND_FAIL (mode 1).
+ * A matrix not closed goes on with rbg_fw_load_*.  rbg_fw_rows_* writes the
+ * whole status block (no rbg_status_init needed).  workspace:
+ * rbg_fw_rows_workspace_bytes(n, element size) bytes, 256-byte aligned;
+ * n <= rbg_fw_rows_max_n() (2 and 3: n <= 16384). */
 int64_t rbg_fw_rows_max_n(void);
 int64_t rbg_fw_rows_workspace_bytes(int64_t n, int32_t elem_bytes);
 int rbg_fw_rows_i32(const int32_t *A, int64_t n, int64_t lda, int32_t *W, int64_t npad, void *workspace,
                     int64_t workspace_bytes, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_rows_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_t npad, void *workspace,
                     int64_t workspace_bytes, rbg_status *st, rbg_stream_t stream);
+int rbg_fw_rows_any_i32(int64_t n, int32_t *W, int32_t *W2, int64_t npad, void *workspace, int64_t workspace_bytes,
+                        rbg_status *st, rbg_stream_t stream);
+int rbg_fw_rows_any_i64(int64_t n, int64_t *W, int64_t *W2, int64_t npad, void *workspace, int64_t workspace_bytes,
+                        rbg_status *st, rbg_stream_t stream);
 int rbg_fw_precheck_i32(const int32_t *W, int64_t n, int64_t ld, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_precheck_i64(const int64_t *W, int64_t n, int64_t ld, rbg_status *st, rbg_stream_t stream);
 int rbg_fw_dense_i32(int32_t *W, int64_t n, int64_t ld, int32_t width, int32_t is_unsigned, int32_t mode,

@@ -68,6 +68,8 @@ SIGNATURES = {
     "rbg_fw_rows_workspace_bytes": (I64, [I64, I32]),
     "rbg_fw_rows_i32": (I32, [P, I64, I64, P, I64, P, I64, P, P]),
     "rbg_fw_rows_i64": (I32, [P, I64, I64, P, I64, P, I64, P, P]),
+    "rbg_fw_rows_any_i32": (I32, [I64, P, P, I64, P, I64, P, P]),
+    "rbg_fw_rows_any_i64": (I32, [I64, P, P, I64, P, I64, P, P]),
     "rbg_fw_precheck_i32": (I32, [P, I64, I64, P, P]),
     "rbg_fw_precheck_i64": (I32, [P, I64, I64, P, P]),
     "rbg_fw_load_i32": (I32, [P, I64, I64, P, I64, P, P]),

@@ -1,5 +1,5 @@
 #pragma once
-// Dense closure of a triangular matrix from its rows' direct entries.
+// Dense closure of a matrix from its rows' direct entries.
 //
 // In a lower triangular matrix of the fast domain (fw_kernels.hpp) a product
 // W[i][k] (x) W[k][j] is present only for i > k > j (the pivot cell's products
@@ -40,6 +40,8 @@ namespace rbg {
 
 constexpr int ROWS_MAX_LEVELS = 64;
 constexpr int64_t ROWS_MAX_N = 32640;  // rows in 15 bits; a byte of LDS per row in the level pass
+constexpr int64_t ROWS_ANY_MAX_N = 16384;  // other numberings: two bytes of LDS per row (rows_first_value)
+constexpr int ROWS_MAX_CELLS = 4096;
 constexpr int ROWS_LEVEL_NT = 1024;
 constexpr int ROWS_CLOSE_NT = 1024;
 
@@ -55,9 +57,9 @@ enum : uint32_t {
   ROW_NONE = 0x7fff,
   ROW_MORE = 1u << 15,
   ROW_STOP = 1u << 31,
-  STOP_UPPER = 4,  // an entry above the diagonal
-  STOP_BAD = 8,    // a value outside the fast domain
-  STOP_WIDE = 16,  // more than rows_slots(n) entries
+  STOP_BAD = 8,          // a value outside the fast domain
+  STOP_WIDE = 16,        // more than rows_slots(n) entries
+  REC_UPPER = 1u << 26,  // in RowRec::p1_cnt: an entry above the diagonal
 };
 __host__ __device__ inline int rec_cnt(uint32_t w) { return (int)((w >> 16) & 0xff); }
 
@@ -86,6 +88,8 @@ struct RowsWork {
   RowRec<T>* rec;     // in level order (place)
   int32_t* ecol;  // row i's entries at [i * slots]
   T* eval;
+  T* slab_top;      // largest W2 value of each slab
+  uint32_t* cells;  // [0] number of cells with W2 > max W, then i | j << 16 of each
   int slots;
 };
 
@@ -107,7 +111,10 @@ static inline int64_t rows_layout(int64_t n, char* base, RowsWork<T>* w) {
   char* rec = take((int64_t)sizeof(RowRec<T>) * n);
   char* ecol = take(4 * n * slots);
   char* eval = take((int64_t)sizeof(T) * n * slots);
-  if (w) *w = RowsWork<T>{(int32_t*)ctl, (uint32_t*)entries, (uint16_t*)pos, (RowRec<T>*)rec0, (RowRec<T>*)rec, (int32_t*)ecol, (T*)eval, slots};
+  char* slab_top = take((int64_t)sizeof(T) * (n * (int64_t)sizeof(T) / 64 + 1));
+  char* cells = take(4 * (1 + ROWS_MAX_CELLS));
+  if (w) *w = RowsWork<T>{(int32_t*)ctl, (uint32_t*)entries, (uint16_t*)pos, (RowRec<T>*)rec0, (RowRec<T>*)rec, (int32_t*)ecol, (T*)eval,
+                     (T*)slab_top, (uint32_t*)cells, slots};
   return o;
 }
 
@@ -215,12 +222,12 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
   if (h0) c0 = (uint32_t)__builtin_amdgcn_readlane((int)c0, __ffsll((unsigned long long)h0) - 1);
   if (h1) c1 = (uint32_t)__builtin_amdgcn_readlane((int)c1, __ffsll((unsigned long long)h1) - 1);
   const uint32_t d = __any(diag == (T)1) ? 2u : (__any(diag == (T)-1) ? 0u : 1u);
-  const uint32_t stop = (__any(bad) ? (uint32_t)STOP_BAD : 0u) | (__any(up) ? (uint32_t)STOP_UPPER : 0u) |
-                        (cnt > w.slots ? (uint32_t)STOP_WIDE : 0u);
+  const uint32_t stop = (__any(bad) ? (uint32_t)STOP_BAD : 0u) | (cnt > w.slots ? (uint32_t)STOP_WIDE : 0u);
+  const uint32_t upper = __any(up) ? (uint32_t)REC_UPPER : 0u;
   if (lane == 0) {
     rec.row_c0 = (uint32_t)i | c0 << 16;
     rec.c1_p0 = c1;
-    rec.p1_cnt = (uint32_t)(cnt < w.slots ? cnt : w.slots) << 16 | d << 24;
+    rec.p1_cnt = (uint32_t)(cnt < w.slots ? cnt : w.slots) << 16 | d << 24 | upper;
     w.entries[i] = stop ? ROW_STOP | stop : c0 | c1 << 16 | (cnt > 2 ? (uint32_t)ROW_MORE : 0u);
   }
 }
@@ -231,99 +238,105 @@ struct LevelShared {
   int marks[4];
 };
 
-// Level and position of every row of a lower triangular matrix, by one
-// workgroup of at least 64 threads; lev: n + 1 bytes of LDS.  Eight rows a
-// thread (four neighbours, twice) in registers, in blocks of rows; a row's
-// entries lie in earlier blocks (final) or its own, where the levels only
-// grow, so a block is swept until no level changed, one barrier a sweep, at
-// most as many sweeps as the block is deep.  One workgroup runs its code
-// once, so its time is instruction fetches, barriers and LDS reads: short
-// loops and few of them count for more here than loads in flight
-// (N = 8192, 18 levels: 28 us against 93 us with one row per thread and pass,
-// chunk by chunk, and 66 us with the records moved here, eight unrolled; N =
-// 512: 12 us).  Returns the STOP_* reasons (0: positions are in w.pos).
-template <typename T>
-__device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev) {
+// Level and position of every row, by one workgroup of at least 64 threads
+// and n / (4 H) rows; lev: n + 4 bytes of LDS.  Each thread holds 4 H rows'
+// words (four neighbours, H times) in registers and sweeps them until no level
+// changed, one barrier a sweep: a row's level only grows, and the sweeps are
+// at most as many as the graph is deep (few more than one where the rows are
+// numbered parents first).  The levels of a cyclic graph grow past
+// ROWS_MAX_LEVELS.  One workgroup runs its code once, so its time is
+// instruction fetches, barriers and LDS reads: short loops and few of them
+// count for more here than loads in flight (N = 8192, 18 levels: 28 us against
+// 93 us with one row per thread and pass, chunk by chunk, and 66 us with the
+// records moved here, eight unrolled; N = 512: 12 us).  Returns the STOP_*
+// reasons (or 2: too deep); 0: positions are in w.pos and `sides` has 1 when
+// entries lie below the diagonal, 2 above.
+template <typename T, int H>
+__device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev, int& sides) {
   const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, n = (int)n64;
   if (tid < 4) L.marks[tid] = 0;
   if (tid < ROWS_MAX_LEVELS) L.hist[tid] = 0;
+  uint32_t e[4 * H];
+  uint32_t lv[H];  // four levels each
+#pragma unroll
+  for (int h = 0; h < H; h++) {
+    const int row = 4 * (h * nt + tid);
+    uint4 q = make_uint4(0, 0, 0, 0);
+    if (row < n) {
+      q = *(const uint4*)(w.entries + row);
+      *(uint32_t*)(lev + row) = 0;
+    }
+    e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
+    lv[h] = 0;
+  }
+  int facts = 0;  // STOP_* and sides << 5
+  bool more = false;
+#pragma unroll
+  for (int x = 0; x < 4 * H; x++) {
+    const int row = 4 * ((x / 4) * nt + tid) + x % 4;
+    if (row >= n) e[x] = ROW_NONE | ROW_NONE << 16;
+    const uint32_t c0 = e[x] & 0x7fff, c1 = (e[x] >> 16) & 0x7fff;
+    if (e[x] & ROW_STOP) {
+      facts |= (int)(e[x] & 0xff);
+      e[x] = (uint32_t)n | (uint32_t)n << 16;
+      continue;
+    }
+    const bool m = (e[x] & ROW_MORE) != 0;
+    more |= m;
+    if (c0 != ROW_NONE) facts |= (int)c0 < row ? 32 : 64;
+    if (c1 != ROW_NONE) facts |= (int)c1 < row ? 32 : 64;
+    if (m && (w.rec0[row].p1_cnt & REC_UPPER)) facts |= 64;
+    e[x] = (c0 == ROW_NONE ? (uint32_t)n : c0) | (c1 == ROW_NONE ? (uint32_t)n : c1) << 16 | (m ? 1u << 31 : 0u);
+  }
+  __syncthreads();
   if (tid == 0) lev[n] = 255;  // an absent entry's level: below 0
   __syncthreads();
-  int it = 0;  // sweeps so far: sweep it marks marks[it & 3]
-  for (int b = 0; b < n; b += 8 * nt) {
-    uint32_t e[8];
-    int row[2];
-    uint32_t lv[2] = {0, 0};  // four levels each
-    int stop = 0;
-    bool more = false;
+  for (int it = 0;; it++) {
+    bool changed = false;
+    int worst = 0;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      row[h] = b + 4 * (h * nt + tid);
-      uint4 q = make_uint4(0, 0, 0, 0);
-      if (row[h] < n) {
-        q = *(const uint4*)(w.entries + row[h]);
-        *(uint32_t*)(lev + row[h]) = 0;
-      }
-      e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
-    }
-    __syncthreads();
-    if (tid == 0) lev[n] = 255;  // the words above may cover it
+    for (int h = 0; h < H; h++) {
+      if (4 * h * nt >= n) continue;  // no row of any thread
+      const int row = 4 * (h * nt + tid);
+      uint32_t nv = 0;
 #pragma unroll
-    for (int x = 0; x < 8; x++) {
-      const bool on = row[x / 4] + x % 4 < n;
-      if (!on) e[x] = ROW_NONE | ROW_NONE << 16;
-      if (e[x] & ROW_STOP) stop |= (int)(e[x] & 0xff);
-      more |= (e[x] & ROW_MORE) != 0;
-      const uint32_t c0 = e[x] & 0x7fff, c1 = (e[x] >> 16) & 0x7fff;
-      e[x] = (e[x] & ROW_STOP) ? (uint32_t)n | (uint32_t)n << 16
-                               : (c0 == ROW_NONE ? (uint32_t)n : c0) | (c1 == ROW_NONE ? (uint32_t)n : c1) << 16 |
-                                     (e[x] & ROW_MORE) << 16;
-    }
-    __syncthreads();
-    for (;; it++) {
-      uint32_t nv[2] = {0, 0};
-      int worst = 0;
-#pragma unroll
-      for (int x = 0; x < 8; x++) {
-        const int l0 = (uint8_t)(lev[e[x] & 0xffff] + 1), l1 = (uint8_t)(lev[(e[x] >> 16) & 0x7fff] + 1);
+      for (int x = 0; x < 4; x++) {
+        const uint32_t ex = e[4 * h + x];
+        const int l0 = (uint8_t)(lev[ex & 0xffff] + 1), l1 = (uint8_t)(lev[(ex >> 16) & 0x7fff] + 1);
         int nl = l0 > l1 ? l0 : l1;
-        if (more && e[x] >> 31) {
-          const int i = row[x / 4] + x % 4, cnt = rec_cnt(w.rec0[i].p1_cnt);
-          const int32_t* ec = w.ecol + (int64_t)i * w.slots;
+        if (more && ex >> 31) {
+          const int cnt = rec_cnt(w.rec0[row + x].p1_cnt);
+          const int32_t* ec = w.ecol + (int64_t)(row + x) * w.slots;
           for (int k = 2; k < cnt; k++) {
             const int y = lev[ec[k]] + 1;
             nl = nl > y ? nl : y;
           }
         }
         worst = nl > worst ? nl : worst;
-        nv[x / 4] |= (uint32_t)nl << (8 * (x % 4));
+        nv |= (uint32_t)nl << (8 * x);
       }
-      bool changed = false;
-#pragma unroll
-      for (int h = 0; h < 2; h++)
-        if (nv[h] != lv[h]) {
-          lv[h] = nv[h];
-          changed = true;
-          if (row[h] + 3 < n)
-            *(uint32_t*)(lev + row[h]) = nv[h];
-          else
-            for (int x = 0; row[h] + x < n; x++) lev[row[h] + x] = (uint8_t)(nv[h] >> (8 * x));
-        }
-      const int mark = (__any(changed) ? 1 : 0) | (__any(worst >= ROWS_MAX_LEVELS) ? 2 : 0) |
-                       (__any(stop & STOP_UPPER) ? STOP_UPPER : 0) | (__any(stop & STOP_BAD) ? STOP_BAD : 0) |
-                       (__any(stop & STOP_WIDE) ? STOP_WIDE : 0);
-      if (mark && lane == 0) atomicOr(&L.marks[it & 3], mark);
-      if (tid == 0) L.marks[(it + 2) & 3] = 0;  // read two sweeps ago, marked two sweeps on
-      __syncthreads();
-      const int marks = L.marks[it & 3];  // the same for every thread: the branches below are uniform
-      if (marks & ~1) return marks & ~1;
-      if (!marks) break;
+      if (nv != lv[h]) {
+        lv[h] = nv;
+        changed = true;
+        if (row + 3 < n)
+          *(uint32_t*)(lev + row) = nv;
+        else
+          for (int x = 0; row + x < n; x++) lev[row + x] = (uint8_t)(nv >> (8 * x));
+      }
     }
-    it++;
-#pragma unroll
-    for (int x = 0; x < 8; x++)
-      if (row[x / 4] + x % 4 < n) atomicAdd(&L.hist[(lv[x / 4] >> (8 * (x % 4))) & 0xff], 1);
+    int mark = (__any(changed) ? 1 : 0) | (__any(worst >= ROWS_MAX_LEVELS) ? 2 : 0);
+    for (int k = 3; k < 7; k++) mark |= __any(facts & (1 << k)) ? 1 << k : 0;
+    if (mark && lane == 0) atomicOr(&L.marks[it & 3], mark);
+    if (tid == 0) L.marks[(it + 2) & 3] = 0;  // read two sweeps ago, marked two sweeps on
+    __syncthreads();
+    const int marks = L.marks[it & 3];  // the same for every thread: the branches below are uniform
+    sides = marks >> 5;
+    if (marks & (2 | STOP_BAD | STOP_WIDE)) return marks & (2 | STOP_BAD | STOP_WIDE);
+    if (!(marks & 1)) break;
   }
+#pragma unroll
+  for (int x = 0; x < 4 * H; x++)
+    if (4 * ((x / 4) * nt + tid) + x % 4 < n) atomicAdd(&L.hist[(lv[x / 4] >> (8 * (x % 4))) & 0xff], 1);
   __syncthreads();
   if (tid < ROWS_MAX_LEVELS) {  // the first wave: an exclusive scan of the level sizes
     const int c = L.hist[tid];
@@ -390,6 +403,18 @@ __device__ inline void rows_relax(typename unsigned_of<T>::type (&cur)[V], T a, 
   }
 }
 
+// The same product, keeping the largest (natural values, 0 absent).
+template <typename T, int V>
+__device__ inline void rows_relax_largest(T (&big)[V], T a, const T (&z)[V], T& top) {
+  using U = typename unsigned_of<T>::type;
+#pragma unroll
+  for (int x = 0; x < V; x++) {
+    const T p = z[x] > (T)1 ? (T)(((U)(a - 1) << msb_u((U)z[x])) + (U)z[x]) : (T)0;
+    big[x] = p > big[x] ? p : big[x];
+    top = z[x] > top ? z[x] : top;
+  }
+}
+
 template <typename T, int V>
 __device__ inline void rows_ld(const T* p, T (&y)[V]) {
   const uint4 q = *(const uint4*)p;
@@ -422,12 +447,15 @@ __host__ __device__ inline int64_t rows_slab() {
   return ROWS_LANES * (16 / (int64_t)sizeof(T));
 }
 
-constexpr int ROWS_RING = 1024;  // 64 KB: two workgroups per CU
-template <typename T>
+// 64 KB: two workgroups per CU
+template <bool LARGEST>
+constexpr int ROWS_RING = LARGEST ? 512 : 1024;
+template <typename T, bool LARGEST>
 struct CloseShared {
-  T ring[ROWS_RING][ROWS_LANES][16 / sizeof(T)];
+  T ring[ROWS_RING<LARGEST>][ROWS_LANES][16 / sizeof(T)];
+  T ring2[LARGEST ? ROWS_RING<LARGEST> : 1][ROWS_LANES][16 / sizeof(T)];
   int start[ROWS_MAX_LEVELS + 1];
-  long long top;
+  long long top, top2;
   int guard;
 };
 
@@ -461,9 +489,14 @@ __device__ inline RowRec<T> rec_of_quad(uint2 q) {
 // 2048 rows with one workgroup per CU: 93 us).  The products are not the
 // bound: leaving them out changed nothing.  Rows above the slab's first column hold no entry there and
 // are never read again: their zeros go out as streaming stores.
-template <typename T, int UN>
-__device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, int64_t ld, int64_t slab, int width,
-                                       rbg_status* st) {
+//
+// LARGEST: any numbering of the vertices.  The closure itself follows from the
+// rows' entries as above, level by level, but a cell's first value depends on
+// the numbering.  W2 takes the largest path value of every cell (no value a
+// cell ever holds is above it), and the slab's largest goes to w.slab_top.
+template <typename T, int UN, bool LARGEST>
+__device__ inline void rows_close_slab(CloseShared<T, LARGEST>& L, RowsWork<T> w, T* W, T* W2, int64_t ld,
+                                       int64_t slab, int width, rbg_status* st) {
   using U = typename unsigned_of<T>::type;
   constexpr int V = 16 / (int)sizeof(T);
   const int tid = threadIdx.x, G = blockDim.x / ROWS_LANES, ql = tid % ROWS_LANES;
@@ -472,16 +505,17 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
   const int jl = j0 + ql * V;
   // row offsets in 16-byte units: below 2^32 for ROWS_MAX_N, one 24-bit multiply each
   const uint32_t ld16 = (uint32_t)(ld / V), jl16 = (uint32_t)(jl / V);
-  auto at = [&](int row) { return W + (size_t)(__umul24((uint32_t)row, ld16) + jl16) * V; };
+  auto off = [&](int row) { return (size_t)(__umul24((uint32_t)row, ld16) + jl16) * V; };
+  constexpr int RING = ROWS_RING<LARGEST>;
   const int levels = w.ctl[1];
   if (tid <= levels) L.start[tid] = w.ctl[CTL_START + tid];
   if (tid == 0) {
-    L.top = 0;
+    L.top = L.top2 = 0;
     L.guard = 0;
   }
   __syncthreads();
   int guard = 0;  // largest MSB(left) + MSB(right) of a product
-  T tmax = -1;
+  T tmax = -1, tmax2 = 0;
   uint2 qr[UN];  // this lane's words of the records
   auto fetch = [&](int p, int end, uint2& q) {
     if (p < end) q = ((const uint2*)(w.rec + p))[ql];
@@ -490,16 +524,19 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
 #pragma unroll
   for (int u = 0; u < UN; u++) fetch(base + g + u * G, end, qr[u]);
   for (int l = 0; l < levels;) {
-    const int kept = end - ROWS_RING;  // older positions have left the ring by the end of this level
+    const int kept = end - RING;  // older positions have left the ring by the end of this level
     RowRec<T> r[UN];
-    T y0[UN][V], y1[UN][V];
+    T y0[UN][V], y1[UN][V], z0[UN][V], z1[UN][V];  // z: of W2
     bool on[UN];
     int cnt[UN], row[UN], c0[UN], c1[UN];
-    auto operand = [&](int c, int p, T(&y)[V]) {
-      if (p >= kept)
-        rows_ld<T, V>(L.ring[p & (ROWS_RING - 1)][ql], y);
-      else
-        rows_ld<T, V>(at(c), y);
+    auto operand = [&](int c, int p, T(&y)[V], T(&z)[V]) {
+      if (p >= kept) {
+        rows_ld<T, V>(L.ring[p & (RING - 1)][ql], y);
+        if (LARGEST) rows_ld<T, V>(L.ring2[p & (RING - 1)][ql], z);
+      } else {
+        rows_ld<T, V>(W + off(c), y);
+        if (LARGEST) rows_ld<T, V>(W2 + off(c), z);
+      }
     };
 #pragma unroll
     for (int u = 0; u < UN; u++) {
@@ -510,9 +547,9 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
       c0[u] = (int)(r[u].row_c0 >> 16);
       c1[u] = (int)(r[u].c1_p0 & 0xffff);
 #pragma unroll
-      for (int x = 0; x < V; x++) y0[u][x] = y1[u][x] = 0;
-      if (cnt[u] > 0 && c0[u] >= j0) operand(c0[u], (int)(r[u].c1_p0 >> 16), y0[u]);
-      if (cnt[u] > 1 && c1[u] >= j0) operand(c1[u], (int)(r[u].p1_cnt & 0xffff), y1[u]);
+      for (int x = 0; x < V; x++) y0[u][x] = y1[u][x] = z0[u][x] = z1[u][x] = 0;
+      if (cnt[u] > 0 && (LARGEST || c0[u] >= j0)) operand(c0[u], (int)(r[u].c1_p0 >> 16), y0[u], z0[u]);
+      if (cnt[u] > 1 && (LARGEST || c1[u] >= j0)) operand(c1[u], (int)(r[u].p1_cnt & 0xffff), y1[u], z1[u]);
     }
     // the pass after this one: the same level's, or the next level's first
     int bn = base + UN * G, ln = l, en = end;
@@ -526,14 +563,18 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
 #pragma unroll
     for (int u = 0; u < UN; u++) {
       if (!on[u]) continue;
-      T* out = at(row[u]);
-      if (row[u] < j0) {
+      T* out = W + off(row[u]);
+      if (!LARGEST && row[u] < j0) {
         rows_st_stream<T>(out);
         continue;
       }
       U cur[V];
+      T big[V];
 #pragma unroll
-      for (int x = 0; x < V; x++) cur[x] = ~(U)0;
+      for (int x = 0; x < V; x++) {
+        cur[x] = ~(U)0;
+        big[x] = 0;
+      }
       const int32_t* ec = w.ecol + (int64_t)row[u] * w.slots;
       const T* ev = w.eval + (int64_t)row[u] * w.slots;
       // the input's cells in this lane's columns, and the diagonal's identity
@@ -554,41 +595,64 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
             if (c == x) cur[x] = (U)ev[e] - 1;
         }
 #pragma unroll
-        for (int x = 0; x < V; x++) tmax = (T)cur[x] > tmax ? (T)cur[x] : tmax;
+        for (int x = 0; x < V; x++) {
+          if (LARGEST) big[x] = (T)(cur[x] + 1);
+          tmax = !LARGEST && (T)cur[x] > tmax ? (T)cur[x] : tmax;
+        }
         if (one == (T)1 && tmax < 0) tmax = 0;
       }
-      auto relax = [&](T a, const T(&y)[V]) {
+      auto relax = [&](T a, const T(&y)[V], const T(&z)[V]) {
         T top = 1;
-        rows_relax<T, V>(cur, a, y, top, tmax);
+        if (LARGEST) {
+          T none = 0;
+          rows_relax<T, V>(cur, a, y, none, none);
+          rows_relax_largest<T, V>(big, a, z, top);
+        } else {
+          rows_relax<T, V>(cur, a, y, top, tmax);
+        }
         const int m = top > 1 ? msb_u((U)top) + msb_u((U)a) : 0;
         guard = m > guard ? m : guard;
       };
-      if (cnt[u] > 0) relax(r[u].v0, y0[u]);
-      if (cnt[u] > 1) relax(r[u].v1, y1[u]);
-      for (int e = 2; e < cnt[u]; e += 4) {
-        T y[4][V], a[4];
+      if (cnt[u] > 0) relax(r[u].v0, y0[u], z0[u]);
+      if (cnt[u] > 1) relax(r[u].v1, y1[u], z1[u]);
+      constexpr int EN = LARGEST ? 2 : 4;  // further entries' rows in flight
+      for (int e = 2; e < cnt[u]; e += EN) {
+        T y[EN][V], z[EN][V], a[EN];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < EN; q++) {
           const int c = e + q < cnt[u] ? ec[e + q] : -1;
           a[q] = e + q < cnt[u] ? ev[e + q] : (T)2;
 #pragma unroll
-          for (int x = 0; x < V; x++) y[q][x] = 0;
-          if (c >= j0) rows_ld<T, V>(at(c), y[q]);
+          for (int x = 0; x < V; x++) y[q][x] = z[q][x] = 0;
+          if (c >= (LARGEST ? 0 : j0)) {
+            rows_ld<T, V>(W + off(c), y[q]);
+            if (LARGEST) rows_ld<T, V>(W2 + off(c), z[q]);
+          }
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) relax(a[q], y[q]);
+        for (int q = 0; q < EN; q++) relax(a[q], y[q], z[q]);
       }
       T o[V];
 #pragma unroll
-      for (int x = 0; x < V; x++) o[x] = (T)(cur[x] + 1);
+      for (int x = 0; x < V; x++) {
+        o[x] = (T)(cur[x] + 1);
+        if (LARGEST) {
+          tmax = (T)cur[x] > tmax ? (T)cur[x] : tmax;
+          tmax2 = big[x] > tmax2 ? big[x] : tmax2;
+        }
+      }
       if (one != 0) {  // the lane of the diagonal; no product reaches that cell
 #pragma unroll
         for (int x = 0; x < V; x++)
           if (row[u] == jl + x) o[x] = one;
       }
       rows_st<T, V>(out, o);
+      if (LARGEST) rows_st<T, V>(W2 + off(row[u]), big);
       const int p = base + g + u * G;
-      if (p >= kept) rows_st<T, V>(L.ring[p & (ROWS_RING - 1)][ql], o);
+      if (p >= kept) {
+        rows_st<T, V>(L.ring[p & (RING - 1)][ql], o);
+        if (LARGEST) rows_st<T, V>(L.ring2[p & (RING - 1)][ql], big);
+      }
     }
     if (ln != l) __syncthreads();  // the level's rows are read by the next ones of this workgroup alone
     l = ln;
@@ -597,13 +661,124 @@ __device__ inline void rows_close_slab(CloseShared<T>& L, RowsWork<T> w, T* W, i
   }
   const long long t = wave_max_i64((int64_t)tmax + 1);
   if ((tid & 63) == 0 && t > 0) atomicMax(&L.top, t);
+  if (LARGEST) {
+    const long long t2 = wave_max_i64((int64_t)tmax2);
+    if ((tid & 63) == 0 && t2 > 0) atomicMax(&L.top2, t2);
+  }
   if (guard > width - 2) atomicMax(&L.guard, guard);
   __syncthreads();
   if (tid == 0) {
     if (L.top > __hip_atomic_load(&st->diameter_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       record_diameter(st, L.top);
+    if (LARGEST) w.slab_top[slab] = (T)L.top2;
     if (L.guard) atomicOr(&st->flags, (uint32_t)RBG_F_NEED_GENERAL);
   }
+}
+
+// ---- the trajectory maximum of any numbering --------------------------------
+// The largest value any cell ever held is the largest first value of a cell:
+// values only fall.  Every first value lies between the cell's final value (W)
+// and its largest path value (W2), so with top = max W only the cells with
+// W2 > top can hold more than top: none to some hundred (deep pedigrees of a
+// thousand vertices and more have 0 to 402).  k_rows_select lists them;
+// rows_first_value computes a cell's first value: its path whose largest
+// intermediate vertex K is smallest, and among the paths through vertices up
+// to K the smallest value -- two small shortest-path sweeps over the vertices
+// between i and j.
+constexpr int ROWS_MAX_BETWEEN = 1024;
+
+template <typename T>
+struct FirstShared {
+  int bound[ROWS_MAX_BETWEEN + 1];  // smallest largest-intermediate of a path to j
+  typename unsigned_of<T>::type value[ROWS_MAX_BETWEEN + 1];
+  uint16_t vid[ROWS_MAX_BETWEEN];
+  int m;
+};
+
+// By one workgroup; idx: n words of LDS (vertex -> place in vid).  0: the
+// vertices between are more than ROWS_MAX_BETWEEN.
+template <typename T>
+__device__ inline T rows_first_value(FirstShared<T>& F, uint16_t* idx, RowsWork<T> w, const T* W, int64_t ld, int n,
+                                     int i, int j) {
+  using U = typename unsigned_of<T>::type;
+  constexpr uint16_t NONE = 0xffff;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  if (tid == 0) F.m = 0;
+  __syncthreads();
+  for (int v = tid; v < n; v += nt) {
+    uint16_t at = NONE;
+    if (v != i && v != j && W[(int64_t)i * ld + v] > (T)1 && W[(int64_t)v * ld + j] > (T)1) {
+      const int p = atomicAdd(&F.m, 1);
+      if (p < ROWS_MAX_BETWEEN) {
+        F.vid[p] = (uint16_t)v;
+        at = (uint16_t)p;
+      }
+    }
+    idx[v] = at;
+  }
+  __syncthreads();
+  const int m = F.m;
+  if (m > ROWS_MAX_BETWEEN) {
+    __syncthreads();  // the next cell clears F.m
+    return 0;
+  }
+  for (int x = tid; x <= m; x += nt) {
+    F.bound[x] = n;
+    F.value[x] = ~(U)0;
+  }
+  __syncthreads();
+  // place m is i itself
+  bool changed;
+  do {
+    changed = false;
+    for (int x = tid; x <= m; x += nt) {
+      const int v = x == m ? i : (int)F.vid[x];
+      const int cnt = rec_cnt(w.rec0[v].p1_cnt);
+      int b = F.bound[x];
+      for (int e = 0; e < cnt; e++) {
+        const int c = w.ecol[(int64_t)v * w.slots + e];
+        if (c == j) {
+          b = -1;
+        } else if (idx[c] != NONE) {
+          const int through = F.bound[idx[c]];
+          const int k = through > c ? through : c;
+          b = k < b ? k : b;
+        }
+      }
+      if (b < F.bound[x]) {
+        F.bound[x] = b;
+        changed = true;
+      }
+    }
+  } while (__syncthreads_or(changed));
+  const int K = F.bound[m];
+  do {
+    changed = false;
+    for (int x = tid; x <= m; x += nt) {
+      const int v = x == m ? i : (int)F.vid[x];
+      const int cnt = rec_cnt(w.rec0[v].p1_cnt);
+      U best = F.value[x];
+      for (int e = 0; e < cnt; e++) {
+        const int c = w.ecol[(int64_t)v * w.slots + e];
+        const U a = (U)w.eval[(int64_t)v * w.slots + e];
+        U p = ~(U)0;
+        if (c == j) {
+          p = a;
+        } else if (idx[c] != NONE && c <= K) {
+          const U y = F.value[idx[c]];
+          if (y != ~(U)0) p = ((a - 1) << msb_u(y)) + y;
+        }
+        best = p < best ? p : best;
+      }
+      if (best < F.value[x]) {
+        F.value[x] = best;
+        changed = true;
+      }
+    }
+  } while (__syncthreads_or(changed));
+  const T first = (T)F.value[m];
+  __syncthreads();  // the next cell's sweeps write what this one read
+  return first;
 }
 
 }  // namespace rbg

@@ -1,4 +1,4 @@
-// Closure of one triangular matrix from its rows' direct entries: the
+// Closure of one matrix from its rows' direct entries: the
 // launches of fw_rows.hpp and the C ABI.
 #include "fw_rows.hpp"
 
@@ -10,18 +10,23 @@ static __global__ __launch_bounds__(NT) void k_rows_scan(const T* A, int64_t n, 
   if (i < n) rows_scan_row<T>(A + i * lda, n, i, vec, w);
 }
 
-// Also writes the whole status block: aux[5] = 1 when the next launches close
-// the matrix.
-template <typename T>
+// Also writes the whole status block.  ctl[0] and aux[5]: 0 the matrix is not
+// closed from its rows, 1 lower triangular, 2 upper, 3 entries on both sides.
+template <typename T, int H>
 static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n, RowsWork<T> w, bool allowed,
                                                                      rbg_status* st) {
   extern __shared__ __align__(16) uint8_t lev[];
   __shared__ LevelShared L;
-  const int stop = allowed ? rows_levels<T>(w, n, L, lev) : 1;
+  int sides = 0;
+  const int stop = allowed ? rows_levels<T, H>(w, n, L, lev, sides) : 1;
   if (threadIdx.x == 0) {
     status_clear(st);
     if (stop & STOP_BAD) st->flags = RBG_F_PRECOND_FAIL;
-    w.ctl[0] = st->aux[5] = stop == 0;
+    int code = stop ? 0 : (sides & 2 ? (sides & 1 ? 3 : 2) : 1);
+    if (code > 1 && n > ROWS_ANY_MAX_N) code = 0;
+    w.ctl[0] = code;
+    st->aux[5] = code;
+    w.cells[0] = 0;
   }
 }
 
@@ -45,37 +50,121 @@ __device__ inline int rows_slab_of(int b, int count) {
   return b - 256;
 }
 
+template <typename T, bool LARGEST>
+static __global__ __launch_bounds__(ROWS_CLOSE_NT, LARGEST ? 4 : 8) void k_rows_close(RowsWork<T> w, T* W, T* W2,
+                                                                                     int64_t ld, int width,
+                                                                                     rbg_status* st) {
+  __shared__ CloseShared<T, LARGEST> L;
+  if (LARGEST ? w.ctl[0] < 2 : w.ctl[0] != 1) return;
+  rows_close_slab<T, 1, LARGEST>(L, w, W, W2, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
+}
+
+// The slab's cells whose largest path value is above the largest final value.
 template <typename T>
-static __global__ __launch_bounds__(ROWS_CLOSE_NT, 8) void k_rows_close(RowsWork<T> w, T* W, int64_t ld, int width,
-                                                                    rbg_status* st) {
-  __shared__ CloseShared<T> L;
-  if (w.ctl[0] != 1) return;
-  rows_close_slab<T, 1>(L, w, W, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
+static __global__ __launch_bounds__(NT) void k_rows_select(int64_t n, RowsWork<T> w, const T* W2, int64_t ld,
+                                                          const rbg_status* st) {
+  constexpr int V = 16 / (int)sizeof(T);
+  const T top = (T)st->diameter_max;
+  if (w.ctl[0] < 2 || w.slab_top[blockIdx.x] <= top) return;
+  const int64_t j = blockIdx.x * rows_slab<T>() + (threadIdx.x % ROWS_LANES) * V;
+  for (int64_t i = threadIdx.x / ROWS_LANES; i < n; i += NT / ROWS_LANES) {
+    T z[V];
+    rows_ld<T, V>(W2 + i * ld + j, z);
+#pragma unroll
+    for (int x = 0; x < V; x++)
+      if (z[x] > top) {
+        const uint32_t at = atomicAdd(&w.cells[0], 1u);
+        if (at < ROWS_MAX_CELLS) w.cells[1 + at] = (uint32_t)i | (uint32_t)(j + x) << 16;
+      }
+  }
+}
+
+// First values of the listed cells.  aux[6] = 1: too many cells, or too many
+// vertices between one's ends (the trajectory maximum is then not known).
+template <typename T>
+static __global__ __launch_bounds__(NT) void k_rows_first(int64_t n, RowsWork<T> w, const T* W, int64_t ld,
+                                                         rbg_status* st) {
+  extern __shared__ uint16_t idx[];
+  __shared__ FirstShared<T> F;
+  if (w.ctl[0] < 2) return;
+  const uint32_t count = w.cells[0];
+  if (count > ROWS_MAX_CELLS) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->aux[6] = 1;
+    return;
+  }
+  for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
+    const uint32_t c = w.cells[1 + q];
+    const T first = rows_first_value<T>(F, idx, w, W, ld, (int)n, (int)(c & 0xffff), (int)(c >> 16));
+    if (threadIdx.x == 0) {
+      if (first == 0)
+        st->aux[6] = 1;
+      else
+        record_diameter(st, (int64_t)first);
+    }
+  }
+}
+
+template <typename T>
+static int rows_args(const void* A, int64_t n, const T* W, int64_t npad, void* wsp, int64_t ws_bytes,
+                     const rbg_status* st, RowsWork<T>* w) {
+  if (!A || !W || !wsp || !st || n <= 0 || n > ROWS_MAX_N || npad < n || npad % TILE || ((uintptr_t)W & 15) ||
+      ((uintptr_t)wsp & 255))
+    return RBG_E_ARG;
+  return ws_bytes < rows_layout<T>(n, (char*)wsp, w) ? RBG_E_WORKSPACE : 0;
+}
+
+template <typename T>
+static unsigned rows_slabs(int64_t n) {
+  return (unsigned)((n + rows_slab<T>() - 1) / rows_slab<T>());
 }
 
 template <typename T>
 static int fw_rows(const T* A, int64_t n, int64_t lda, T* W, int64_t npad, void* wsp, int64_t ws_bytes,
                    rbg_status* st, hipStream_t s) {
-  if (!A || !W || !wsp || !st || n <= 0 || n > ROWS_MAX_N || lda < n || npad < n || npad % TILE ||
-      ((uintptr_t)W & 15) || ((uintptr_t)wsp & 255))
-    return RBG_E_ARG;
   RowsWork<T> w;
-  if (ws_bytes < rows_layout<T>(n, (char*)wsp, &w)) return RBG_E_WORKSPACE;
+  const int rc = rows_args<T>(A, n, W, npad, wsp, ws_bytes, st, &w);
+  if (rc) return rc;
+  if (lda < n) return RBG_E_ARG;
   const bool vec = lda % (16 / (int64_t)sizeof(T)) == 0 && ((uintptr_t)A & 15) == 0;
   hipLaunchKernelGGL((k_rows_scan<T>), dim3((unsigned)((n + NT / 64 - 1) / (NT / 64))), dim3(NT), 0, s, A, n, lda, vec,
                      w);
   RBG_CHECK_LAUNCH();
   // a forced wait limit asks for the persistent closure (rbg_fw_flow_wait_limit)
   const bool allowed = g_flow_limit_override.load() == 0;
-  hipLaunchKernelGGL((k_rows_levels<T>), dim3(1), dim3(ROWS_LEVEL_NT), (size_t)(n + 4), s, n, w, allowed, st);
+  const size_t lds = (size_t)(n + 4);
+  if (n <= 8 * ROWS_LEVEL_NT)
+    hipLaunchKernelGGL((k_rows_levels<T, 2>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
+  else if (n <= 16 * ROWS_LEVEL_NT)
+    hipLaunchKernelGGL((k_rows_levels<T, 4>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
+  else
+    hipLaunchKernelGGL((k_rows_levels<T, 8>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
   RBG_CHECK_LAUNCH();
   hipLaunchKernelGGL((k_rows_place<T>), dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, s, n, w);
   RBG_CHECK_LAUNCH();
   const int p = prof_start(s);
-  hipLaunchKernelGGL((k_rows_close<T>), dim3((unsigned)((n + rows_slab<T>() - 1) / rows_slab<T>())),
-                     dim3(ROWS_CLOSE_NT), 0, s, w, W, npad, (int)sizeof(T) * 8, st);
+  hipLaunchKernelGGL((k_rows_close<T, false>), dim3(rows_slabs<T>(n)), dim3(ROWS_CLOSE_NT), 0, s, w, W, (T*)nullptr,
+                     npad, (int)sizeof(T) * 8, st);
   RBG_CHECK_LAUNCH();
   prof_stop(7, p, s, (double)n * n * sizeof(T));
+  return 0;
+}
+
+template <typename T>
+static int fw_rows_any(int64_t n, T* W, T* W2, int64_t npad, void* wsp, int64_t ws_bytes, rbg_status* st,
+                       hipStream_t s) {
+  RowsWork<T> w;
+  const int rc = rows_args<T>(W2, n, W, npad, wsp, ws_bytes, st, &w);
+  if (rc) return rc;
+  if (n > ROWS_ANY_MAX_N || ((uintptr_t)W2 & 15)) return RBG_E_ARG;
+  const int p = prof_start(s);
+  hipLaunchKernelGGL((k_rows_close<T, true>), dim3(rows_slabs<T>(n)), dim3(ROWS_CLOSE_NT), 0, s, w, W, W2, npad,
+                     (int)sizeof(T) * 8, st);
+  RBG_CHECK_LAUNCH();
+  prof_stop(7, p, s, (double)n * n * sizeof(T));
+  hipLaunchKernelGGL((k_rows_select<T>), dim3(rows_slabs<T>(n)), dim3(NT), 0, s, n, w, (const T*)W2, npad, st);
+  RBG_CHECK_LAUNCH();
+  hipLaunchKernelGGL((k_rows_first<T>), dim3(512), dim3(NT), (size_t)(2 * n), s, n, w, (const T*)W, npad, st);
+  RBG_CHECK_LAUNCH();
   return 0;
 }
 
@@ -98,6 +187,15 @@ int rbg_fw_rows_i32(const int32_t* A, int64_t n, int64_t lda, int32_t* W, int64_
 int rbg_fw_rows_i64(const int64_t* A, int64_t n, int64_t lda, int64_t* W, int64_t npad, void* workspace,
                     int64_t workspace_bytes, rbg_status* st, rbg_stream_t stream) {
   return fw_rows<int64_t>(A, n, lda, W, npad, workspace, workspace_bytes, st, (hipStream_t)stream);
+}
+
+int rbg_fw_rows_any_i32(int64_t n, int32_t* W, int32_t* W2, int64_t npad, void* workspace, int64_t workspace_bytes,
+                        rbg_status* st, rbg_stream_t stream) {
+  return fw_rows_any<int32_t>(n, W, W2, npad, workspace, workspace_bytes, st, (hipStream_t)stream);
+}
+int rbg_fw_rows_any_i64(int64_t n, int64_t* W, int64_t* W2, int64_t npad, void* workspace, int64_t workspace_bytes,
+                        rbg_status* st, rbg_stream_t stream) {
+  return fw_rows_any<int64_t>(n, W, W2, npad, workspace, workspace_bytes, st, (hipStream_t)stream);
 }
 
 }  // extern "C"

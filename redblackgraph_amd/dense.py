@@ -39,17 +39,33 @@ def _cached_bytes(name: str, key: tuple, nbytes, t, dev):
     return ws
 
 
+_ROWS_SIDES = {1: "lower", 2: "upper", 3: "full"}
+
+
 def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
-    """rbg_fw_rows_*: the closure from the rows' direct entries, where the
-    matrix allows it (status aux[5])."""
+    """rbg_fw_rows_* / rbg_fw_rows_any_*: the closure from the rows' direct
+    entries.  Returns (schedule the numbering stands for, or None when the
+    matrix is not closed this way; status)."""
     t = _lib.torch()
     dev = _lib.device()
     elem = work.element_size()
     ws = _cached_bytes("rows_cache", (dev.index, n, elem),
                        lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev)
-    _lib.call("rbg_fw_rows_i32" if elem == 4 else "rbg_fw_rows_i64", _lib.ptr(src), n, src.stride(0), _lib.ptr(work),
-              npad, _lib.ptr(ws), ws.numel(), st.p, _lib.stream_handle(stream))
-    return st.read(stream)
+    sfx = "i32" if elem == 4 else "i64"
+    sh = _lib.stream_handle(stream)
+    _lib.call(f"rbg_fw_rows_{sfx}", _lib.ptr(src), n, src.stride(0), _lib.ptr(work), npad, _lib.ptr(ws), ws.numel(),
+              st.p, sh)
+    s = st.read(stream)
+    side = int(s.aux[5])
+    if side > 1:
+        largest = t.empty_like(work)
+        _lib.call(f"rbg_fw_rows_any_{sfx}", n, _lib.ptr(work), _lib.ptr(largest), npad, _lib.ptr(ws), ws.numel(),
+                  st.p, sh)
+        s = st.read(stream)
+        if s.aux[6] or s.flags & _lib.F_NEED_GENERAL:
+            side = 0
+    s.aux[5] = s.aux[6] = 0
+    return _ROWS_SIDES.get(side), s
 
 
 def padded_order(n: int) -> int:
@@ -105,9 +121,10 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
     schedule when the precheck finds every off-diagonal entry on one side of
     the diagonal (a pedigree numbered parents first is lower triangular), else
     the full one; "full" forces the full schedule (the results are the same).
-    With "auto" a lower triangular matrix of few entries per row (a pedigree)
-    is closed from its rows' direct entries (rbg_fw_rows_*).  Other lower
-    triangular closures run as one persistent launch; "steps" keeps
+    With "auto" an acyclic matrix of few entries per row (a pedigree, in any
+    numbering) is closed from its rows' direct entries (rbg_fw_rows_*), with
+    the schedule its entries' sides stand for.  Other lower triangular
+    closures run as one persistent launch; "steps" keeps
     one launch per pivot step there (the same results again).
     """
     if schedule not in ("auto", "full", "steps"):
@@ -130,14 +147,10 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
         src = W if (W.stride(1) == 1 and W.stride(0) >= n) else W.contiguous()
         work = t.empty((npad, npad), dtype=W.dtype, device=W.device)
         if schedule == "auto" and 0 < n <= ROWS_MAX_N:
-            s = _rows_closure(src, work, n, npad, st, stream)
-            if s.aux[5]:
-                sched = "lower"
-                s.aux[5] = 0
-                if not s.flags & _lib.F_NEED_GENERAL:
-                    return work[:n, :n], FwOutcome(s, npad, "fast", sched)
-                fast = False
-            elif s.flags & _lib.F_PRECOND_FAIL:
+            side, s = _rows_closure(src, work, n, npad, st, stream)
+            if side and not s.flags & _lib.F_NEED_GENERAL:
+                return work[:n, :n], FwOutcome(s, npad, "fast", side)
+            if side or s.flags & _lib.F_PRECOND_FAIL:
                 fast = False
     st.reset(stream)
     if fast:

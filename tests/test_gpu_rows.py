@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _rows(A, lda=None):
-    """(closed, W, status) of one rbg_fw_rows_* call."""
+    """(schedule or None, W, status) of one closure from the rows."""
     t = _lib.torch()
     n = A.shape[0]
     big = np.zeros((n, lda or n), dtype=A.dtype)
@@ -19,8 +19,8 @@ def _rows(A, lda=None):
     src = _lib.to_device(big)[:, :n]
     npad = dense.padded_order(n)
     work = t.full((npad, npad), 77, dtype=src.dtype, device=src.device)
-    s = dense._rows_closure(src, work, n, npad, dense.status(), None)
-    return int(s.aux[5]), work[:n, :n].cpu().numpy(), s
+    side, s = dense._rows_closure(src, work, n, npad, dense.status(), None)
+    return side, work[:n, :n].cpu().numpy(), s
 
 
 def _full(A):
@@ -54,7 +54,7 @@ def test_rows_closure_vs_oracle(orc, dt, n, lda):
         A[7, 7] = 0  # a vertex without a colour
     closed, W, s = _rows(A, lda)
     ref = orc.warshall(A)
-    assert closed == 1 and s.flags == 0 and s.events == 0 and s.cycle_count == 0
+    assert closed == "lower" and s.flags == 0 and s.events == 0 and s.cycle_count == 0
     np.testing.assert_array_equal(W, ref.W)
     Wf, out = _full(A)
     np.testing.assert_array_equal(W, Wf)
@@ -69,11 +69,11 @@ def test_rows_closure_slot_limit(dt, n):
     full = _with_extra_entries(n, _slots(n), dt, 1)
     closed, W, s = _rows(full)
     Wf, out = _full(full)
-    assert closed == 1 and s.diameter_max == out.status.diameter_max
+    assert closed == "lower" and s.diameter_max == out.status.diameter_max
     np.testing.assert_array_equal(W, Wf)
     over = _with_extra_entries(n, _slots(n) + 1, dt, 1)
     closed, W, _ = _rows(over)
-    assert closed == 0 and (W == 77).all()
+    assert closed is None and (W == 77).all()
     W2, out2 = dense.fw_closure(_lib.to_device(over), elem_type(dt))
     Wf, outf = _full(over)
     assert out2.schedule == "lower" and out2.status.diameter_max == outf.status.diameter_max
@@ -98,7 +98,7 @@ def _shortcut_chain(n, dt):
 
 
 def test_rows_closure_level_limit():
-    for n, closed_ref in ((63, 1), (64, 1), (65, 0)):
+    for n, closed_ref in ((63, "lower"), (64, "lower"), (65, None)):
         A = _shortcut_chain(n, np.int64)
         closed, W, s = _rows(A)
         assert closed == closed_ref
@@ -115,7 +115,7 @@ def test_rows_closure_overflow_guard(dt, bits):
     fits, over = _chain(bits - 1, dt), _chain(bits, dt)
     closed, W, s = _rows(fits)
     Wf, out = _full(fits)
-    assert closed == 1 and s.flags == 0
+    assert closed == "lower" and s.flags == 0
     np.testing.assert_array_equal(W, Wf)
     closed, _, s = _rows(over)
     assert s.flags & _lib.F_NEED_GENERAL
@@ -130,12 +130,75 @@ def test_rows_closure_declines_values(i, j, v):
     A = synth.dense_pedigree(synth.PedigreeSpec(70, 6, 0.8, 3), 1)
     A[i, j] = v
     closed, W, s = _rows(A)
-    assert closed == 0 and s.flags & _lib.F_PRECOND_FAIL and (W == 77).all()
+    assert closed is None and s.flags & _lib.F_PRECOND_FAIL and (W == 77).all()
 
 
-def test_rows_closure_declines_other_sides():
+@pytest.mark.parametrize("dt,n,layers,lookback,seed", [
+    (np.int32, 5, 3, 1, 1), (np.int32, 130, 7, 3, 1), (np.int32, 150, 12, 3, 1), (np.int32, 300, 9, 1, 0),
+    (np.int64, 700, 18, 2, 1), (np.int32, 700, 18, 4, 1), (np.int64, 513, 30, 3, 2), (np.int32, 1100, 11, 4, 0)])
+@pytest.mark.parametrize("numbering", ["upper", "any"])
+def test_rows_closure_any_numbering_vs_oracle(orc, dt, n, layers, lookback, seed, numbering):
+    """Upper triangular and shuffled pedigrees: W, and the exact largest value
+    the naive loop's cells ever held (pedigrees with several paths between two
+    vertices, where it depends on the numbering)."""
+    A = synth.dense_pedigree(synth.PedigreeSpec(n, layers, 0.8, lookback), seed, dtype=dt)
+    A = synth.reverse_vertices(A) if numbering == "upper" else synth.shuffle_vertices(A, seed)
+    side, W, s = _rows(A)
+    assert side == ("upper" if not np.tril(A, -1).any() else "full") and s.flags == 0
+    ref = orc.warshall(A)
+    np.testing.assert_array_equal(W, ref.W)
+    Wf, out = _full(A)
+    assert s.diameter_max == out.status.diameter_max and dense.msb(s.diameter_max) == ref.diameter
+
+
+def _detour(n, long, dt):
+    """Two paths from the last vertex but one to vertex 0: ``long`` edges
+    through low numbers, found first, and two edges through the last vertex;
+    the other vertices stand alone."""
+    A = np.diag(np.full(n, -1, dtype=dt))
+    walk = [n - 2] + list(range(long - 1, 0, -1)) + [0]
+    for a, b in zip(walk[:-1], walk[1:]):
+        A[a, b] = 2
+    A[n - 2, n - 1] = 2
+    A[n - 1, 0] = 2
+    return A
+
+
+@pytest.mark.parametrize("dt,n,long", [(np.int32, 20, 6), (np.int32, 300, 20), (np.int64, 300, 40)])
+def test_rows_closure_any_first_value_above_final(orc, dt, n, long):
+    """A cell whose first value is the largest ever held and not its last."""
+    A = _detour(n, long, dt)
+    side, W, s = _rows(A)
+    ref = orc.warshall(A)
+    assert side == "full" and s.diameter_max == 1 << long > W.max()
+    np.testing.assert_array_equal(W, ref.W)
+    assert dense.msb(s.diameter_max) == ref.diameter == long
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+def test_rows_closure_any_random_acyclic(orc, dt):
+    """Random acyclic matrices, several paths between most vertices, in random
+    numberings."""
+    for seed in range(24):
+        rng = np.random.default_rng(seed)
+        n = int(rng.integers(9, 60))
+        A = np.tril((rng.random((n, n)) < 0.12) * rng.integers(2, 6, (n, n)), -1).astype(dt)
+        A[np.arange(n), np.arange(n)] = rng.choice([-1, 1], n)
+        A = synth.shuffle_vertices(A, seed)
+        side, W, s = _rows(A)
+        if side is None:  # more than eight entries in a row, or values past the guard
+            continue
+        np.testing.assert_array_equal(W, orc.warshall(A).W)
+        assert s.diameter_max == _full(A)[1].status.diameter_max
+
+
+def test_rows_closure_declines_cycles():
     A = synth.dense_pedigree(synth.PedigreeSpec(140, 7, 0.8, 3), 1)
-    B = A.copy()
-    B[3, 90] = 2
-    closed, W, s = _rows(B)
-    assert closed == 0 and (W == 77).all()
+    kid = int(np.nonzero(A[139, :139])[0][0])
+    A[kid, 139] = 2
+    side, _, s = _rows(A)
+    assert side is None
+    W2, out2 = dense.fw_closure(_lib.to_device(A), elem_type(np.int32))
+    Wf, outf = _full(A)
+    assert out2.mode == outf.mode == "general"
+    assert out2.status.cycle_last_key == outf.status.cycle_last_key
