@@ -173,8 +173,8 @@ int rbg_fw_load_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_
 /* No counterpart in the reference: the closure of an acyclic matrix from its
  * rows' direct entries, for matrices with few of them (pedigrees: two a row).
  * Reads A (n x n, row stride lda) once; when the values pass
- * rbg_fw_precheck_*, every row has at most max(8, min(n / 64, 128))
- * off-diagonal entries and the graph is acyclic with at most 64 levels,
+ * rbg_fw_precheck_*, every row has at most 8 to 200
+ * off-diagonal entries (by n: n / 12 up to 24, n / 40 from there) and the graph is acyclic with at most 64 levels,
  * st->aux[5] = 1 (every off-diagonal entry below the diagonal), 2 (above) or 3
  * (both), and with
  *   1  the closure (natural values) is written into columns [0, n) of rows
@@ -182,10 +182,11 @@ int rbg_fw_load_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_
  *      rest of W is unspecified) and st->diameter_max = the max trajectory
  *      value; RBG_F_NEED_GENERAL then asks for mode 1 as for rbg_fw_dense_*;
  *   2, 3  rbg_fw_rows_any_*, with the same W, workspace and st, writes them.
- *      W2 is a second matrix like W (scratch).  st->aux[6] != 0 or
+ *      W2 is a second matrix like W (scratch).  st->aux[5] = 0 after it, or
  *      RBG_F_NEED_GENERAL: not closed.
  * Otherwise st->aux[5] = 0 and st->flags may hold RBG_F_PRECOND_FAIL (mode 1).
- * A matrix not closed goes on with rbg_fw_load_*.  rbg_fw_rows_* writes the
+ * st->aux[6] = 1, 2 or 3: the sides, also of a matrix not closed (0: not looked
+ * at).  A matrix not closed goes on with rbg_fw_load_*.  rbg_fw_rows_* writes the
  * whole status block (no rbg_status_init needed).  workspace:
  * rbg_fw_rows_workspace_bytes(n, element size) bytes, 256-byte aligned;
  * n <= rbg_fw_rows_max_n() (2 and 3: n <= 16384). */

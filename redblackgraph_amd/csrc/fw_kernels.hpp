@@ -218,8 +218,11 @@ __global__ __launch_bounds__(NT) void k_fw_load(const T* A, int64_t n, int64_t l
                      (__any(upper) ? (uint32_t)RBG_F_HAS_UPPER : 0u);
   vmax = wave_max_i64(vmax);
   if ((threadIdx.x & 63) == 0) {
-    if (f) atomicOr(&st->flags, f);
-    if (vmax > 0) atomicMax((long long*)&st->aux[FW_AUX_INIT], (long long)vmax);
+    // thousands of waves with the same few facts: only the first ones' atomics
+    // (served one after another on one line) are needed
+    if (f & ~__hip_atomic_load(&st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&st->flags, f);
+    if (vmax > __hip_atomic_load(&st->aux[FW_AUX_INIT], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax((long long*)&st->aux[FW_AUX_INIT], (long long)vmax);
   }
 }
 

@@ -22,16 +22,18 @@
 //   levels  one workgroup: each row's level (1 + the largest level among its
 //           entries' rows) and its position in level order;
 //   place   the rows' records in level order;
-//   close   one workgroup per slab of columns (128 bytes wide, a cache line a
-//           row).  A column depends on itself alone, so a workgroup needs only
+//   close   one workgroup per slab of columns (64 bytes of a row).  A column depends on itself alone, so a workgroup needs only
 //           its own barrier between levels.
 //
 // Taken when every row has at most rows_slots(n) off-diagonal entries and the
 // graph has at most ROWS_MAX_LEVELS levels; a graph with more entries keeps
-// the blocked schedules (their cost does not grow with the entries).  Where
-// the lines lie: a close pass reads one line per row, slab and entry, so its
-// bytes are entries * n^2 / 2 * sizeof(T) from the L2s, level with the
-// blocked closure's time at about n / 50 entries a row; and a path of L edges
+// the blocked schedules, whose cost does not grow with the entries.  Where the
+// lines lie: the close pass reads a line per row, slab and entry, and with the
+// same number of entries in every row it measured (us, against the blocked
+// closure) 151 / 157 at n = 100 with 12, 231 / 246 at 300 with 24, 274 / 563
+// at 1000 with 25, 451 / 1489 at 2000 with 50, 1511 / 3747 at 4000 with 100
+// and 7603 / 10283 at 8000 with 200, each growing with the entries.  A matrix
+// not taken pays for the scan and the level pass, 2-20 us.  A path of L edges
 // has a value of L bits at least, so a graph deeper than 64 levels overflows
 // (general mode) unless it is full of shortcuts, which are entries.
 #include "fw_kernels.hpp"
@@ -46,8 +48,8 @@ constexpr int ROWS_LEVEL_NT = 1024;
 constexpr int ROWS_CLOSE_NT = 1024;
 
 __host__ __device__ inline int rows_slots(int64_t n) {
-  const int64_t s = n / 64;
-  return (int)(s < 8 ? 8 : (s > 128 ? 128 : s));
+  const int64_t few = n / 12 < 8 ? 8 : (n / 12 > 24 ? 24 : n / 12), s = n / 40;
+  return (int)(s < few ? few : (s > 200 ? 200 : s));
 }
 
 // A row for the level pass: entry 0's column | entry 1's column << 16
@@ -59,6 +61,8 @@ enum : uint32_t {
   ROW_STOP = 1u << 31,
   STOP_BAD = 8,          // a value outside the fast domain
   STOP_WIDE = 16,        // more than rows_slots(n) entries
+  ROW_BELOW = 32,        // with ROW_STOP: an entry below the diagonal
+  ROW_ABOVE = 64,        // above it
   REC_UPPER = 1u << 26,  // in RowRec::p1_cnt: an entry above the diagonal
 };
 __host__ __device__ inline int rec_cnt(uint32_t w) { return (int)((w >> 16) & 0xff); }
@@ -120,8 +124,8 @@ static inline int64_t rows_layout(int64_t n, char* base, RowsWork<T>* w) {
 
 // One row, by one wave.  Bound by reading the matrix: 16-byte loads, eight in
 // flight per lane; only vectors with an entry go through the ballots that
-// place the entries in column order.  A row past its slots is left at once
-// (the blocked schedules read the matrix again).
+// place the entries in column order.  A row past its slots is read to its
+// end all the same: the blocked schedules need the sides its entries lie on.
 template <typename T>
 __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t i, bool vec, RowsWork<T> w) {
   constexpr int V = 16 / (int)sizeof(T);
@@ -170,7 +174,7 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
   };
   if (vec) {
     const int64_t nv = n / V;
-    for (int64_t b = 0; b < nv && cnt <= w.slots; b += 64 * UN) {
+    for (int64_t b = 0; b < nv; b += 64 * UN) {
       uint4 q[UN];
 #pragma unroll
       for (int u = 0; u < UN; u++) {
@@ -201,7 +205,7 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
       emit(j, v);
     }
   } else {
-    for (int64_t b = 0; b < n && cnt <= w.slots; b += 64 * UN) {
+    for (int64_t b = 0; b < n; b += 64 * UN) {
       T s[UN];
 #pragma unroll
       for (int u = 0; u < UN; u++) {
@@ -228,7 +232,7 @@ __device__ inline void rows_scan_row(const T* __restrict__ a, int64_t n, int64_t
     rec.row_c0 = (uint32_t)i | c0 << 16;
     rec.c1_p0 = c1;
     rec.p1_cnt = (uint32_t)(cnt < w.slots ? cnt : w.slots) << 16 | d << 24 | upper;
-    w.entries[i] = stop ? ROW_STOP | stop : c0 | c1 << 16 | (cnt > 2 ? (uint32_t)ROW_MORE : 0u);
+    w.entries[i] = stop ? ROW_STOP | stop | ((int64_t)c0 < i ? ROW_BELOW : 0u) | (upper ? (uint32_t)ROW_ABOVE : 0u) : c0 | c1 << 16 | (cnt > 2 ? (uint32_t)ROW_MORE : 0u);
   }
 }
 
@@ -249,8 +253,8 @@ struct LevelShared {
 // count for more here than loads in flight (N = 8192, 18 levels: 28 us against
 // 93 us with one row per thread and pass, chunk by chunk, and 66 us with the
 // records moved here, eight unrolled; N = 512: 12 us).  Returns the STOP_*
-// reasons (or 2: too deep); 0: positions are in w.pos and `sides` has 1 when
-// entries lie below the diagonal, 2 above.
+// reasons (or 2: too deep), 0 when the positions are in w.pos; `sides` has 1
+// when entries lie below the diagonal, 2 above.
 template <typename T, int H>
 __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev, int& sides) {
   const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, n = (int)n64;
@@ -269,7 +273,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
     lv[h] = 0;
   }
-  int facts = 0;  // STOP_* and sides << 5
+  int facts = 0;  // STOP_*, ROW_BELOW, ROW_ABOVE
   bool more = false;
 #pragma unroll
   for (int x = 0; x < 4 * H; x++) {
@@ -283,9 +287,9 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     }
     const bool m = (e[x] & ROW_MORE) != 0;
     more |= m;
-    if (c0 != ROW_NONE) facts |= (int)c0 < row ? 32 : 64;
-    if (c1 != ROW_NONE) facts |= (int)c1 < row ? 32 : 64;
-    if (m && (w.rec0[row].p1_cnt & REC_UPPER)) facts |= 64;
+    if (c0 != ROW_NONE) facts |= (int)c0 < row ? ROW_BELOW : ROW_ABOVE;
+    if (c1 != ROW_NONE) facts |= (int)c1 < row ? ROW_BELOW : ROW_ABOVE;
+    if (m && (w.rec0[row].p1_cnt & REC_UPPER)) facts |= ROW_ABOVE;
     e[x] = (c0 == ROW_NONE ? (uint32_t)n : c0) | (c1 == ROW_NONE ? (uint32_t)n : c1) << 16 | (m ? 1u << 31 : 0u);
   }
   __syncthreads();

@@ -10,8 +10,9 @@ static __global__ __launch_bounds__(NT) void k_rows_scan(const T* A, int64_t n, 
   if (i < n) rows_scan_row<T>(A + i * lda, n, i, vec, w);
 }
 
-// Also writes the whole status block.  ctl[0] and aux[5]: 0 the matrix is not
-// closed from its rows, 1 lower triangular, 2 upper, 3 entries on both sides.
+// Also writes the whole status block.  aux[6]: 1 the matrix is lower
+// triangular, 2 upper, 3 has entries on both sides (0: not looked at).  ctl[0]
+// and aux[5]: the same where it is closed from its rows, else 0.
 template <typename T, int H>
 static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n, RowsWork<T> w, bool allowed,
                                                                      rbg_status* st) {
@@ -21,11 +22,12 @@ static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n,
   const int stop = allowed ? rows_levels<T, H>(w, n, L, lev, sides) : 1;
   if (threadIdx.x == 0) {
     status_clear(st);
+    const int side = sides & 2 ? (sides & 1 ? 3 : 2) : 1;
+    const int code = stop || (side > 1 && n > ROWS_ANY_MAX_N) ? 0 : side;
     if (stop & STOP_BAD) st->flags = RBG_F_PRECOND_FAIL;
-    int code = stop ? 0 : (sides & 2 ? (sides & 1 ? 3 : 2) : 1);
-    if (code > 1 && n > ROWS_ANY_MAX_N) code = 0;
     w.ctl[0] = code;
     st->aux[5] = code;
+    st->aux[6] = allowed ? side : 0;
     w.cells[0] = 0;
   }
 }
@@ -79,7 +81,7 @@ static __global__ __launch_bounds__(NT) void k_rows_select(int64_t n, RowsWork<T
   }
 }
 
-// First values of the listed cells.  aux[6] = 1: too many cells, or too many
+// First values of the listed cells.  aux[5] = 0: too many cells, or too many
 // vertices between one's ends (the trajectory maximum is then not known).
 template <typename T>
 static __global__ __launch_bounds__(NT) void k_rows_first(int64_t n, RowsWork<T> w, const T* W, int64_t ld,
@@ -89,7 +91,7 @@ static __global__ __launch_bounds__(NT) void k_rows_first(int64_t n, RowsWork<T>
   if (w.ctl[0] < 2) return;
   const uint32_t count = w.cells[0];
   if (count > ROWS_MAX_CELLS) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->aux[6] = 1;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->aux[5] = 0;
     return;
   }
   for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
@@ -97,7 +99,7 @@ static __global__ __launch_bounds__(NT) void k_rows_first(int64_t n, RowsWork<T>
     const T first = rows_first_value<T>(F, idx, w, W, ld, (int)n, (int)(c & 0xffff), (int)(c >> 16));
     if (threadIdx.x == 0) {
       if (first == 0)
-        st->aux[6] = 1;
+        st->aux[5] = 0;
       else
         record_diameter(st, (int64_t)first);
     }

@@ -44,8 +44,8 @@ _ROWS_SIDES = {1: "lower", 2: "upper", 3: "full"}
 
 def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
     """rbg_fw_rows_* / rbg_fw_rows_any_*: the closure from the rows' direct
-    entries.  Returns (schedule the numbering stands for, or None when the
-    matrix is not closed this way; status)."""
+    entries.  Returns (closed or not, the schedule the entries' sides stand
+    for or None when they are not known, status)."""
     t = _lib.torch()
     dev = _lib.device()
     elem = work.element_size()
@@ -56,16 +56,16 @@ def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
     _lib.call(f"rbg_fw_rows_{sfx}", _lib.ptr(src), n, src.stride(0), _lib.ptr(work), npad, _lib.ptr(ws), ws.numel(),
               st.p, sh)
     s = st.read(stream)
-    side = int(s.aux[5])
-    if side > 1:
+    if s.aux[5] > 1:
         largest = t.empty_like(work)
         _lib.call(f"rbg_fw_rows_any_{sfx}", n, _lib.ptr(work), _lib.ptr(largest), npad, _lib.ptr(ws), ws.numel(),
                   st.p, sh)
         s = st.read(stream)
-        if s.aux[6] or s.flags & _lib.F_NEED_GENERAL:
-            side = 0
+        if s.flags & _lib.F_NEED_GENERAL:
+            s.aux[5] = s.flags = 0
+    closed, sched = bool(s.aux[5]), _ROWS_SIDES.get(int(s.aux[6]))
     s.aux[5] = s.aux[6] = 0
-    return _ROWS_SIDES.get(side), s
+    return closed, sched, s
 
 
 def padded_order(n: int) -> int:
@@ -146,26 +146,30 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
     if fast:
         src = W if (W.stride(1) == 1 and W.stride(0) >= n) else W.contiguous()
         work = t.empty((npad, npad), dtype=W.dtype, device=W.device)
+        known = None  # the schedule, where the rows' scan has found it
         if schedule == "auto" and 0 < n <= ROWS_MAX_N:
-            side, s = _rows_closure(src, work, n, npad, st, stream)
-            if side and not s.flags & _lib.F_NEED_GENERAL:
-                return work[:n, :n], FwOutcome(s, npad, "fast", side)
-            if side or s.flags & _lib.F_PRECOND_FAIL:
+            closed, known, s = _rows_closure(src, work, n, npad, st, stream)
+            if closed and not s.flags & _lib.F_NEED_GENERAL:
+                return work[:n, :n], FwOutcome(s, npad, "fast", known)
+            if closed or s.flags & _lib.F_PRECOND_FAIL:
                 fast = False
     st.reset(stream)
     if fast:
         # one pass: copy, fast-domain check and encoding (rbg_fw_load_*)
         fn = "rbg_fw_load_i32" if work.dtype == t.int32 else "rbg_fw_load_i64"
         _lib.call(fn, _lib.ptr(src), n, src.stride(0), _lib.ptr(work), npad, st.p, _lib.stream_handle(stream))
-        s = st.read(stream)
-        if s.flags & _lib.F_PRECOND_FAIL:
-            fast = False
-            st.reset(stream)
-        elif schedule in ("auto", "steps"):
-            if not s.flags & _lib.F_HAS_UPPER:
-                sched = "lower" if schedule == "auto" else "lower-steps"
-            elif not s.flags & _lib.F_HAS_LOWER:
-                sched = "upper"
+        if known is not None:
+            sched = known
+        else:
+            s = st.read(stream)
+            if s.flags & _lib.F_PRECOND_FAIL:
+                fast = False
+                st.reset(stream)
+            elif schedule in ("auto", "steps"):
+                if not s.flags & _lib.F_HAS_UPPER:
+                    sched = "lower" if schedule == "auto" else "lower-steps"
+                elif not s.flags & _lib.F_HAS_LOWER:
+                    sched = "upper"
     if not fast:
         work = fresh()
         sched = "full"
