@@ -1,0 +1,24 @@
+"""The build's check of the device assembly.  CPU only."""
+from redblackgraph_amd.build import shift_hazards
+
+_ASM = """
+_Z3fooPl:
+\tv_lshlrev_b64 v[2:3], v{amount}, v[4:5]
+\ts_endpgm
+\t.amdhsa_kernel _Z3fooPl
+\t\t.amdhsa_next_free_vgpr {vgprs}
+\t\t.amdhsa_accum_offset {vgprs}
+\t.end_amdhsa_kernel
+"""
+
+
+def test_shift_by_last_vgpr_is_found():
+    assert shift_hazards(_ASM.format(amount=135, vgprs=136)) == ["_Z3fooPl"]
+    assert shift_hazards(_ASM.format(amount=7, vgprs=8)) == ["_Z3fooPl"]
+
+
+def test_other_shifts_pass():
+    assert shift_hazards(_ASM.format(amount=134, vgprs=136)) == []
+    assert shift_hazards(_ASM.format(amount=135, vgprs=144)) == []
+    assert shift_hazards(_ASM.format(amount=131, vgprs=132)) == []
+    assert shift_hazards(_ASM.replace("v{amount}", "s4").format(vgprs=136)) == []
