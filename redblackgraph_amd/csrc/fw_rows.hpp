@@ -97,10 +97,10 @@ struct RowsWork {
   int slots;
 };
 
-static inline int64_t rows_align(int64_t x) { return (x + 255) & ~(int64_t)255; }
+__host__ __device__ inline int64_t rows_align(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
 template <typename T>
-static inline int64_t rows_layout(int64_t n, char* base, RowsWork<T>* w) {
+__host__ __device__ inline int64_t rows_layout(int64_t n, char* base, RowsWork<T>* w) {
   const int slots = rows_slots(n);
   int64_t o = 0;
   auto take = [&](int64_t bytes) {

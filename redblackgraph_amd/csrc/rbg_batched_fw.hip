@@ -11,6 +11,9 @@
 // panel lines) and one tile launch per tile shape, each over the work of all
 // running components, so a launch carries the panels (or tiles) of thousands
 // of components at once.
+// Lower triangular components are first tried from their rows' direct entries
+// (fw_rows.hpp): four launches for all of them, in place of every step; the
+// launches after that leave the closed ones alone.
 // Lower triangular components whose workspace holds the persistent closure's
 // (rbg_batch_tri_snap_bytes) instead take one persistent launch for all of
 // them: the single-matrix persistent closure's work items (k_fw_flow), every
@@ -23,7 +26,7 @@
 #include <algorithm>
 #include <numeric>
 
-#include "fw_kernels.hpp"
+#include "fw_rows.hpp"
 
 namespace rbg {
 
@@ -38,6 +41,8 @@ struct BComp {
   // triangular, per-step launches: every diagonal block closed before the
   // steps (k_bfw_prewalk), its step snapshots here for the panels
   void* dsnap;
+  int32_t rows;  // 1: tried from its rows' entries first (their workspace is `snap`)
+  int32_t done;  // written by each run: closed from its rows' entries
 };
 
 // A component of the persistent launch: its matrix, snapshot workspace (with
@@ -49,6 +54,7 @@ struct BFlow {
   void* dsnap;
   rbg_status* st;
   int64_t n;
+  const int32_t* done;  // the component's BComp::done
 };
 
 // The persistent launch's components of one padded order and tile edge, in
@@ -132,10 +138,60 @@ constexpr int CHUNK = 128;  // precheck / domain conversion granule
 // columns and column-panel rows)
 static inline int lines_groups(int npad) { return (2 * npad + NT - 1) / NT; }
 
-static __global__ void k_bfw_init(const BComp* comps, int32_t count) {
+static __global__ void k_bfw_init(BComp* comps, int32_t count) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= count) return;
+  comps[c].done = 0;
   status_clear(comps[c].st);
+}
+
+// ---- closure from the rows' direct entries (fw_rows.hpp) --------------------
+constexpr int ROWS_SCAN_CHUNK = 16;  // rows per scan workgroup
+constexpr int ROWS_BATCH_NT = 512;   // level pass: components are small
+constexpr int64_t ROWS_BATCH_MAX_N = 8 * ROWS_BATCH_NT;
+
+__device__ inline RowsWork<int32_t> rows_work(const BComp& c) {
+  RowsWork<int32_t> w;
+  rows_layout<int32_t>(c.npad, (char*)c.snap, &w);
+  return w;
+}
+
+// item = (component, chunk of rows)
+static __global__ __launch_bounds__(NT) void k_bfw_rows_scan(const BComp* comps, const Item* items) {
+  const Item it = items[blockIdx.x];
+  const BComp c = comps[it.comp];
+  const RowsWork<int32_t> w = rows_work(c);
+  for (int r = threadIdx.x / 64; r < ROWS_SCAN_CHUNK; r += NT / 64) {
+    const int64_t i = (int64_t)it.bid * ROWS_SCAN_CHUNK + r;
+    rows_scan_row<int32_t>(c.W + i * c.npad, c.npad, i, true, w);
+  }
+}
+
+// item = component
+static __global__ __launch_bounds__(ROWS_BATCH_NT) void k_bfw_rows_levels(BComp* comps, const int32_t* list) {
+  __shared__ __align__(16) uint8_t lev[ROWS_BATCH_MAX_N + 4];
+  __shared__ LevelShared L;
+  const BComp c = comps[list[blockIdx.x]];
+  int sides = 0;
+  const int stop = rows_levels<int32_t, 2>(rows_work(c), c.npad, L, lev, sides);
+  if (threadIdx.x == 0) comps[list[blockIdx.x]].done = stop == 0 && !(sides & 2);
+}
+
+// item = (component, chunk of NT rows)
+static __global__ __launch_bounds__(NT) void k_bfw_rows_place(const BComp* comps, const Item* items) {
+  const Item it = items[blockIdx.x];
+  const BComp c = comps[it.comp];
+  const int64_t i = (int64_t)it.bid * NT + threadIdx.x;
+  if (c.done && i < c.npad) rows_place<int32_t>(rows_work(c), i);
+}
+
+// item = (component, slab), in place: the entries have left the matrix
+static __global__ __launch_bounds__(ROWS_CLOSE_NT, 8) void k_bfw_rows_close(const BComp* comps, const Item* items) {
+  __shared__ CloseShared<int32_t, false> L;
+  const Item it = items[blockIdx.x];
+  const BComp c = comps[it.comp];
+  if (!c.done) return;
+  rows_close_slab<int32_t, 1, false>(L, rows_work(c), c.W, nullptr, c.npad, it.bid, 32, c.st);
 }
 
 // Domain conversion of one 128 x 128 chunk, four cells per thread and pass.
@@ -148,6 +204,7 @@ template <bool ENC>
 static __global__ __launch_bounds__(NT) void k_bfw_convert(const BComp* comps, const Item* items) {
   const Item it = items[blockIdx.x];
   const BComp c = comps[it.comp];
+  if (c.done) return;
   const int nc = c.npad / CHUNK, ci = it.bid / nc, cj = it.bid % nc;
   const int64_t i0 = (int64_t)ci * CHUNK, j0 = (int64_t)cj * CHUNK;
   // a chunk wholly on a triangular component's absent side is never read or
@@ -188,6 +245,7 @@ static __global__ __launch_bounds__(NT) void k_bfw_convert(const BComp* comps, c
 static __global__ __launch_bounds__(NT) void k_bfw_panel(const BComp* comps, const Item* items, int64_t K) {
   const Item it = items[blockIdx.x];
   const BComp c = comps[it.comp];
+  if (c.done) return;
   FwWork ws{c.snap, c.npad, 4};
   __shared__ LinesShared<uint32_t> L;
   const int64_t n = c.npad;
@@ -211,6 +269,7 @@ static __global__ __launch_bounds__(NT) void k_bfw_panel(const BComp* comps, con
 static __global__ __launch_bounds__(PANEL_NT) void k_bfw_prewalk(const BComp* comps, const Item* items) {
   const Item it = items[blockIdx.x];
   const BComp c = comps[it.comp];
+  if (c.done) return;
   fw_diag_walk_body<int32_t>(c.W, c.npad, c.npad, (int32_t*)c.dsnap, 32, c.st, it.bid);
 }
 
@@ -218,6 +277,7 @@ template <int RC>
 static __global__ __launch_bounds__(NT, 3) void k_bfw_tile(const BComp* comps, const Item* items, int64_t K) {
   const Item it = items[blockIdx.x];
   const BComp c = comps[it.comp];
+  if (c.done) return;
   FwWork ws{c.snap, c.npad, 4};
   const int nt = c.npad / (16 * RC);
   __shared__ TileShared<uint32_t, 16 * RC, false> L;
@@ -230,6 +290,7 @@ static __global__ void k_bfw_capture(const BComp* comps, int32_t count) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= count) return;
   const BComp b = comps[c];
+  if (b.done) return;
   const int64_t nb = b.npad / BLK;
   FwWork ws{b.snap, b.npad, 4, b.flow ? 4 : 2};
   const int par = ws.slot(nb - 1);
@@ -242,6 +303,7 @@ static __global__ void k_bfw_capture(const BComp* comps, int32_t count) {
 static __global__ __launch_bounds__(PANEL_NT) void k_bfw_diag_walk(const BFlow* comps, const Item* items) {
   const Item it = items[blockIdx.x];
   const BFlow c = comps[it.comp];
+  if (*c.done) return;
   fw_diag_walk_body<int32_t>(c.W, c.n, c.n, (int32_t*)c.dsnap, 32, c.st, it.bid);
 }
 
@@ -269,6 +331,7 @@ static __global__ __launch_bounds__(NT, 3) void k_bfw_flow(const BFlow* comps, i
   const FlowCtl f{ctl + k.c[j].ctl + (int64_t)(comp - k.c[j].first) * k.c[j].words, n / BLK, n / edge, edge, 0};
   const FlowItem q = flow_unpack(items[k.c[j].items + local]);
   const BFlow c = comps[comp];
+  if (*c.done) return;  // all of the component's items: none waits for another
   FwWork ws{c.snap, n, 4, 4};
   ws.dsnap = c.dsnap;
   if (!DUAL || edge == 128)
@@ -299,6 +362,11 @@ struct rbg_batch {
   // triangular components' tiles 128, step by step | the same for tiles 64
   Item* d_items = nullptr;
   int64_t n_chunk = 0, n_panel = 0, n_t128 = 0, n_t64 = 0, n_tri128 = 0, n_tri64 = 0;
+  // components tried from their rows' entries: the components, then the scan,
+  // place and close items
+  int32_t* d_rows = nullptr;
+  Item* d_ritems = nullptr;
+  int64_t n_rows = 0, n_rscan = 0, n_rplace = 0, n_rclose = 0;
   Item* d_prewalk = nullptr;  // (component, block) of the per-step components with dsnap
   int64_t n_prewalk = 0;
   std::vector<int64_t> panel_cnt, t128_cnt, t64_cnt;  // per step: items of running components
@@ -312,6 +380,20 @@ static int batch_launch(rbg_batch* b, hipStream_t s) {
   const int cgrid = (b->count + 255) / 256;
   hipLaunchKernelGGL(k_bfw_init, dim3(cgrid), dim3(256), 0, s, b->d_comps, b->count);
   RBG_CHECK_LAUNCH();
+  // a forced wait limit asks for the persistent launch (rbg_fw_flow_wait_limit)
+  if (b->n_rows && g_flow_limit_override.load() == 0) {
+    const Item* scan = b->d_ritems;
+    const Item* place = scan + b->n_rscan;
+    const Item* close = place + b->n_rplace;
+    hipLaunchKernelGGL(k_bfw_rows_scan, dim3((unsigned)b->n_rscan), dim3(NT), 0, s, b->d_comps, scan);
+    RBG_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_bfw_rows_levels, dim3((unsigned)b->n_rows), dim3(ROWS_BATCH_NT), 0, s, b->d_comps, b->d_rows);
+    RBG_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_bfw_rows_place, dim3((unsigned)b->n_rplace), dim3(NT), 0, s, b->d_comps, place);
+    RBG_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_CLOSE_NT), 0, s, b->d_comps, close);
+    RBG_CHECK_LAUNCH();
+  }
   const Item* chunks = b->d_items;
   const Item* panels = chunks + b->n_chunk;
   const Item* t128 = panels + b->n_panel;
@@ -421,8 +503,10 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     // can be closed before the steps; the persistent launch takes lower ones
     const bool room = q.tri != 0 && q.snap_bytes >= flow_ctl_offset(q.npad, 4);
     const int flow = room && q.tri == 1 && q.persistent;
+    const int rows = q.tri == 1 && q.npad <= ROWS_BATCH_MAX_N && ((uintptr_t)q.snap & 255) == 0 &&
+                     q.snap_bytes >= rows_layout<int32_t>(q.npad, nullptr, nullptr);
     c[i] = BComp{q.W, q.snap, q.st, q.npad, q.tile, q.tri, flow,
-                 room && !flow ? (char*)q.snap + dsnap_offset(q.npad, 4) : nullptr};
+                 room && !flow ? (char*)q.snap + dsnap_offset(q.npad, 4) : nullptr, rows, 0};
   }
   // largest first: the components running at step K are a prefix
   std::stable_sort(c.begin(), c.end(), [](const BComp& a, const BComp& b) { return a.npad > b.npad; });
@@ -451,7 +535,7 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
       continue;
     }
     for (int K = 0; K < c[i].npad / BLK; K++) walk.push_back({(int)fl.size(), K});
-    fl.push_back(BFlow{c[i].W, c[i].snap, (char*)c[i].snap + dsnap_offset(c[i].npad, 4), c[i].st, c[i].npad});
+    fl.push_back(BFlow{c[i].W, c[i].snap, (char*)c[i].snap + dsnap_offset(c[i].npad, 4), c[i].st, c[i].npad, nullptr});
     b->flow_work += flow_relaxations(flow_ctl(c[i].npad, 4, nullptr, c[i].tile), c[i].npad);
   }
   b->n_flow = (int32_t)fl.size();
@@ -518,7 +602,34 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     if (c[i].dsnap)
       for (int q = 0; q < c[i].npad / BLK; q++) prewalk.push_back({i, q});
   b->n_prewalk = (int64_t)prewalk.size();
+  // the components tried from their rows' entries
+  std::vector<int32_t> rows;
+  std::vector<Item> rscan, rplace, rclose;
+  for (int i = 0; i < count; i++) {
+    if (!c[i].rows) continue;
+    rows.push_back(i);
+    for (int q = 0; q < c[i].npad / ROWS_SCAN_CHUNK; q++) rscan.push_back({i, q});
+    for (int q = 0; q < (c[i].npad + NT - 1) / NT; q++) rplace.push_back({i, q});
+    // slab counts are multiples of eight, and the XCDs take turns at
+    // workgroups: eight neighbouring slabs go to one XCD where there are 64
+    const int slabs = (int)(c[i].npad / rows_slab<int32_t>());
+    for (int q = 0; q < slabs; q++) rclose.push_back({i, (q | 63) < slabs ? (q & ~63) + (q & 7) * 8 + ((q & 63) >> 3) : q});
+  }
+  b->n_rows = (int64_t)rows.size();
+  b->n_rscan = (int64_t)rscan.size();
+  b->n_rplace = (int64_t)rplace.size();
+  b->n_rclose = (int64_t)rclose.size();
+  std::vector<Item> ritems(rscan);
+  ritems.insert(ritems.end(), rplace.begin(), rplace.end());
+  ritems.insert(ritems.end(), rclose.begin(), rclose.end());
   hipError_t e = hipMalloc((void**)&b->d_comps, sizeof(BComp) * count);
+  if (e == hipSuccess && b->n_rows) {
+    e = hipMalloc((void**)&b->d_rows, sizeof(int32_t) * rows.size());
+    if (e == hipSuccess) e = hipMalloc((void**)&b->d_ritems, sizeof(Item) * ritems.size());
+    if (e == hipSuccess) e = hipMemcpy(b->d_rows, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = hipMemcpy(b->d_ritems, ritems.data(), sizeof(Item) * ritems.size(), hipMemcpyHostToDevice);
+  }
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_items, sizeof(Item) * all.size());
   if (e == hipSuccess) e = hipMemcpy(b->d_comps, c.data(), sizeof(BComp) * count, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(b->d_items, all.data(), sizeof(Item) * all.size(), hipMemcpyHostToDevice);
@@ -527,6 +638,8 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     if (e == hipSuccess)
       e = hipMemcpy(b->d_prewalk, prewalk.data(), sizeof(Item) * prewalk.size(), hipMemcpyHostToDevice);
   }
+  for (int i = 0, j = 0; i < count; i++)
+    if (c[i].flow) fl[j++].done = &b->d_comps[i].done;
   if (e == hipSuccess && b->n_flow) {
     e = hipMalloc((void**)&b->d_flow, sizeof(BFlow) * fl.size());
     if (e == hipSuccess) e = hipMalloc((void**)&b->d_walk, sizeof(Item) * walk.size());
@@ -540,6 +653,8 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
   if (e != hipSuccess) {
     (void)hipFree(b->d_comps);
     (void)hipFree(b->d_items);
+    (void)hipFree(b->d_rows);
+    (void)hipFree(b->d_ritems);
     (void)hipFree(b->d_prewalk);
     (void)hipFree(b->d_flow);
     (void)hipFree(b->d_walk);
@@ -554,7 +669,7 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
 
 int rbg_batch_info(const rbg_batch* b, int64_t* info) {
   if (!b || !info) return RBG_E_ARG;
-  int64_t launches = 4 + (b->n_flow ? 3 : 0) + (b->n_prewalk ? 1 : 0);
+  int64_t launches = 4 + (b->n_rows ? 4 : 0) + (b->n_flow ? 3 : 0) + (b->n_prewalk ? 1 : 0);
   for (int K = 0; K < b->stepnb; K++)
     launches += (b->panel_cnt[K] > 0) + (b->t128_cnt[K] > 0) + (b->t64_cnt[K] > 0) +
                 (b->tri128_off[K + 1] > b->tri128_off[K]) + (b->tri64_off[K + 1] > b->tri64_off[K]);
@@ -616,6 +731,8 @@ int rbg_batch_destroy(rbg_batch* b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   (void)hipFree(b->d_comps);
   (void)hipFree(b->d_items);
+  (void)hipFree(b->d_rows);
+  (void)hipFree(b->d_ritems);
   (void)hipFree(b->d_prewalk);
   (void)hipFree(b->d_flow);
   (void)hipFree(b->d_walk);
