@@ -524,8 +524,8 @@ int rbg_batch_destroy(rbg_batch *b);
  * :15-81 (find_components): components of the graph with edges taken in
  * both directions.  labels[v] = the smallest vertex of v's component (the
  * reference numbers components by that vertex, in increasing order).
- * flags: two int32 of device scratch.  The host waits once per hooking round
- * (*rounds of them). */
+ * flags: two int32 of device scratch (not used any more).  *rounds = 1, the
+ * passes over the edges; nothing is read by the host. */
 int rbg_components(const int64_t *indptr, const int32_t *indices, int32_t n, int32_t *labels, int32_t *flags,
                    int32_t *rounds, rbg_stream_t stream);
 

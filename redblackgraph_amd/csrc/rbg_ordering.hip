@@ -16,7 +16,6 @@
 #include <rocprim/device/device_merge_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_segmented_radix_sort.hpp>
-#include <rocprim/iterator/counting_iterator.hpp>
 
 #include "rbg_common.hpp"
 
@@ -121,22 +120,35 @@ __global__ __launch_bounds__(ORD_NT) void k_ord_csr(const int64_t* __restrict__ 
   }
 }
 
-// The canonical order of two vertices.
+// A vertex's place in the canonical order.  The sort moves these records: a
+// merge sort of vertex numbers whose comparison gathers five arrays spends its
+// time on those loads (n = 300,007: @SORT@).
+struct OrdKey {
+  uint64_t comp;  // ~component size << 32 | component id
+  int64_t anc, maxrel, diag;
+  int32_t v;
+};
 struct OrdLess {
-  const int32_t* comp;
-  const int32_t* csize;
-  const int64_t* anc;
-  const int64_t* maxrel;
-  const int64_t* diag;
-  __device__ bool operator()(const int32_t a, const int32_t b) const {
-    if (csize[a] != csize[b]) return csize[a] > csize[b];
-    if (comp[a] != comp[b]) return comp[a] < comp[b];
-    if (anc[a] != anc[b]) return anc[a] > anc[b];
-    if (maxrel[a] != maxrel[b]) return maxrel[a] < maxrel[b];
-    if (diag[a] != diag[b]) return diag[a] > diag[b];
-    return a < b;
+  __device__ bool operator()(const OrdKey& a, const OrdKey& b) const {
+    if (a.comp != b.comp) return a.comp < b.comp;
+    if (a.anc != b.anc) return a.anc > b.anc;
+    if (a.maxrel != b.maxrel) return a.maxrel < b.maxrel;
+    if (a.diag != b.diag) return a.diag > b.diag;
+    return a.v < b.v;
   }
 };
+
+__global__ void k_ord_keys(const int32_t* __restrict__ comp, const int32_t* __restrict__ csize,
+                           const int64_t* __restrict__ anc, const int64_t* __restrict__ maxrel,
+                           const int64_t* __restrict__ diag, int32_t n, OrdKey* __restrict__ out) {
+  for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x)
+    out[v] = OrdKey{(uint64_t)(uint32_t)~csize[v] << 32 | (uint32_t)comp[v], anc[v], maxrel[v], diag[v], (int32_t)v};
+}
+
+__global__ void k_ord_perm(const OrdKey* __restrict__ keys, int32_t n, int32_t* __restrict__ perm) {
+  for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x)
+    perm[v] = keys[v].v;
+}
 
 // B[i][j] = A[p[i]][p[j]] (0 below the diagonal when `upper`)
 template <typename T>
@@ -447,11 +459,16 @@ static int permute_dense(const T* A, int64_t n, const int32_t* p, T* B, int uppe
   return 0;
 }
 
-static size_t order_sort_bytes(int32_t n) {
+static size_t order_merge_bytes(int32_t n) {
   size_t b = 0;
-  (void)rocprim::merge_sort((void*)nullptr, b, rocprim::counting_iterator<int32_t>(0), (int32_t*)nullptr,
-                            (size_t)n, OrdLess{}, (hipStream_t)0);
+  (void)rocprim::merge_sort((void*)nullptr, b, (OrdKey*)nullptr, (OrdKey*)nullptr, (size_t)n, OrdLess{},
+                            (hipStream_t)0);
   return b;
+}
+
+// the records, the sorted records, rocPRIM's storage
+static size_t order_sort_bytes(int32_t n) {
+  return 2 * align256(sizeof(OrdKey) * (size_t)n) + align256(order_merge_bytes(n)) + 256;
 }
 
 }  // namespace rbg
@@ -483,11 +500,22 @@ int rbg_order_sort(int32_t n, const int32_t* comp, const int32_t* comp_size, con
                    const int64_t* maxrel, const int64_t* diag, int32_t* perm, void* temp, int64_t temp_bytes,
                    rbg_stream_t stream) {
   if (n <= 0 || !comp || !comp_size || !anc || !maxrel || !diag || !perm || !temp) return RBG_E_ARG;
-  size_t b = order_sort_bytes(n);
-  if (temp_bytes < (int64_t)b) return RBG_E_WORKSPACE;
-  hipError_t e = rocprim::merge_sort(temp, b, rocprim::counting_iterator<int32_t>(0), perm, (size_t)n,
-                                     OrdLess{comp, comp_size, anc, maxrel, diag}, (hipStream_t)stream);
-  return e == hipSuccess ? 0 : (int)e;
+  if (temp_bytes < (int64_t)order_sort_bytes(n)) return RBG_E_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  char* w = (char*)(((uintptr_t)temp + 255) & ~(uintptr_t)255);
+  OrdKey* keys = (OrdKey*)w;
+  w += align256(sizeof(OrdKey) * (size_t)n);
+  OrdKey* sorted = (OrdKey*)w;
+  w += align256(sizeof(OrdKey) * (size_t)n);
+  const int g = (int)((n + ORD_NT - 1) / ORD_NT < 4096 ? (n + ORD_NT - 1) / ORD_NT : 4096);
+  hipLaunchKernelGGL(k_ord_keys, dim3(g), dim3(ORD_NT), 0, s, comp, comp_size, anc, maxrel, diag, n, keys);
+  RBG_CHECK_LAUNCH();
+  size_t b = order_merge_bytes(n);
+  hipError_t e = rocprim::merge_sort(w, b, keys, sorted, (size_t)n, OrdLess{}, s);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(k_ord_perm, dim3(g), dim3(ORD_NT), 0, s, (const OrdKey*)sorted, n, perm);
+  RBG_CHECK_LAUNCH();
+  return 0;
 }
 
 int rbg_permute_dense_i32(const int32_t* A, int64_t n, const int32_t* p, int32_t* B, int32_t upper,
