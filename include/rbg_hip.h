@@ -320,6 +320,13 @@ int rbg_edge_compose_inplace_i32(int32_t *W, int64_t n, int64_t alpha, int64_t b
                                  int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
 int rbg_edge_compose_inplace_i64(int64_t *W, int64_t n, int64_t alpha, int64_t beta, int64_t rel, void *scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
+/* `count` edges one after another, each as rbg_edge_compose_inplace_*: edges
+ * (host memory) holds alpha, beta and the relationship of each.  Two launches
+ * an edge; nothing is read by the host. */
+int rbg_edge_compose_many_i32(int32_t *W, int64_t n, const int64_t *edges, int64_t count, void *scratch,
+                              int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
+int rbg_edge_compose_many_i64(int64_t *W, int64_t n, const int64_t *edges, int64_t count, void *scratch,
+                              int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
 /* Vertex composition: out is (n+1) x (n+1).  On a cycle violation st->flags |=
  * RBG_F_CYCLE and st->aux[0..2] = {idx, u_idx, v_idx} of the first violation. */
 int rbg_vertex_compose_i32(const int32_t *u, const int32_t *R, const int32_t *v, int32_t color,

@@ -264,63 +264,109 @@ __global__ void k_zero_i64(int64_t* p, int64_t n) {
     p[i] = 0;
 }
 
-// In-place edge composition, step 2: the rows m with W[m][alpha] != 0 (the
-// vertices that reach alpha) are the only rows the update changes, and within
-// them only the columns where u is present.  The first kernel lists those
-// rows (one read of column alpha), the second updates them in place; every
-// other entry is left untouched, so a composition into a pedigree closure
-// costs its affected rows rather than the whole matrix.
+// Edge composition in place, two launches an edge (a composition into a
+// pedigree's closure changes a few rows only, so its time is its launches and
+// their round trips to memory, not bytes: n = 4095, 64 edges, @EDGE@).
+//
+// k_edge_compose: workgroup b computes the composed row u = lhs (x) W (lhs =
+// row alpha with entry beta replaced by the relationship) for columns [64 b,
+// 64 b + 64) and lists the rows m in [64 b, 64 b + 64) with W[m][alpha] != 0,
+// the vertices that reach alpha: the only rows the edge changes.  The present
+// lefts of up to EC_SPAN columns are gathered in LDS at a time (16 loads in
+// flight per thread) and dealt to the four waves.
+constexpr int EC_SPAN = 4096;
 template <typename T>
-__global__ __launch_bounds__(256) void k_edge_rows_hit(const T* __restrict__ W, int64_t n, int64_t alpha,
-                                                       int64_t* __restrict__ hit, int64_t* __restrict__ nhit) {
-  __shared__ int s_n;
-  __shared__ int64_t s_base;
-  __shared__ int64_t s_m[256];
-  if (threadIdx.x == 0) s_n = 0;
-  __syncthreads();
-  const int64_t m = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (m < n && m != alpha && W[m * n + alpha] != 0) s_m[atomicAdd(&s_n, 1)] = m;
-  __syncthreads();
-  if (threadIdx.x == 0 && s_n) s_base = (int64_t)atomicAdd((unsigned long long*)nhit, (unsigned long long)s_n);
-  __syncthreads();
-  if (threadIdx.x < s_n) hit[s_base + threadIdx.x] = s_m[threadIdx.x];
-}
-
-// One workgroup per listed row, four consecutive columns per lane; row alpha
-// takes u from the scratch row once every product is formed from it.
-template <typename T>
-__global__ __launch_bounds__(256) void k_edge_update_rows(T* __restrict__ W, int64_t n, int64_t alpha,
-                                                          const T* __restrict__ u, const int64_t* __restrict__ hit,
-                                                          const int64_t* __restrict__ nhit, int width, int is_uns,
-                                                          rbg_status* st) {
+__global__ __launch_bounds__(256) void k_edge_compose(const T* __restrict__ W, int64_t n, int64_t alpha, int64_t beta,
+                                                      T np, T* __restrict__ u, int32_t* __restrict__ hit,
+                                                      int32_t* __restrict__ nhit, int width, int is_uns,
+                                                      rbg_status* st) {
+  __shared__ int32_t s_idx[EC_SPAN];
+  __shared__ T s_lhs[EC_SPAN];
+  __shared__ T s_part[4][64];
+  __shared__ int s_cnt;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t p = (int64_t)blockIdx.x * 64 + lane;
+  if (wv == 0 && p < n && p != alpha && W[p * n + alpha] != 0) hit[atomicAdd(nhit, 1)] = (int32_t)p;
+  if (blockIdx.x == 0 && tid == 0 && W[beta * n + alpha] != 0) atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
+  T acc = 0;
   uint32_t evs = 0;
-  const int64_t nh = *nhit;
-  for (int64_t h = blockIdx.x; h < nh; h += gridDim.x) {
-    const int64_t m = hit[h];
-    T* Wm = W + m * n;
-    const T rma = Wm[alpha];  // unchanged by the update: u[alpha] is alpha's own diagonal
-    for (int64_t p0 = (int64_t)threadIdx.x * 4; p0 < n; p0 += 256 * 4) {
+  for (int64_t k0 = 0; k0 < n; k0 += EC_SPAN) {
+    if (tid == 0) s_cnt = 0;
+    __syncthreads();
+    T x[EC_SPAN / 256];
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int64_t p = p0 + q;
-        if (p < n) {
-          const T up = u[p];
-          if (up != 0) {
-            uint32_t ev = 0;
-            Wm[p] = avos_sum<T>(Wm[p], avos_product<T>(rma, up, width, is_uns != 0, ev));
-            evs |= ev;
-          }
-        }
+    for (int q = 0; q < EC_SPAN / 256; q++) {
+      const int64_t k = k0 + 256 * q + tid;
+      x[q] = k < n ? W[alpha * n + k] : (T)0;
+    }
+#pragma unroll
+    for (int q = 0; q < EC_SPAN / 256; q++) {
+      const int64_t k = k0 + 256 * q + tid;
+      if (k < n && k == beta && np != 0) x[q] = np;
+      if (x[q] != 0) {
+        const int at = atomicAdd(&s_cnt, 1);
+        s_idx[at] = (int32_t)k;
+        s_lhs[at] = x[q];
       }
     }
+    __syncthreads();
+    const int cnt = s_cnt;
+    if (p < n)
+      for (int e = wv; e < cnt; e += 16) {
+        T y[4], l[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const bool on = e + 4 * q < cnt;
+          l[q] = on ? s_lhs[e + 4 * q] : (T)0;
+          y[q] = on ? W[(int64_t)s_idx[e + 4 * q] * n + p] : (T)0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          uint32_t ev = 0;
+          if (y[q] != 0) acc = avos_sum<T>(acc, avos_product<T>(l[q], y[q], width, is_uns != 0, ev));
+          evs |= ev;
+        }
+      }
+    __syncthreads();  // the next span's lefts replace these
   }
+  s_part[wv][lane] = acc;
+  __syncthreads();
+  if (wv == 0 && p < n)
+    u[p] = avos_sum<T>(avos_sum<T>(acc, s_part[1][lane]), avos_sum<T>(s_part[2][lane], s_part[3][lane]));
   if (evs) atomicOr(&st->events, evs);
 }
 
+// The listed rows m: W[m][p] = W[m][p] (+) W[m][alpha] (x) u[p] where u is
+// present (relational_composition.c.in:110-137), and row alpha = u.
+// W[m][alpha] is unchanged by it: u[alpha] is alpha's own diagonal.  Also
+// clears the next edge's row counter.
 template <typename T>
-__global__ void k_edge_put_row(T* __restrict__ W, int64_t n, int64_t alpha, const T* __restrict__ u) {
-  for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x)
-    W[alpha * n + p] = u[p];
+__global__ __launch_bounds__(256) void k_edge_apply(T* __restrict__ W, int64_t n, int64_t alpha,
+                                                    const T* __restrict__ u, const int32_t* __restrict__ hit,
+                                                    const int32_t* __restrict__ nhit, int32_t* __restrict__ next_nhit,
+                                                    int width, int is_uns, rbg_status* st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *next_nhit = 0;
+  for (int64_t p = blockIdx.x * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)gridDim.x * 256) W[alpha * n + p] = u[p];
+  uint32_t evs = 0;
+  const int nh = *nhit;
+  for (int h = blockIdx.x; h < nh; h += gridDim.x) {
+    T* Wm = W + (int64_t)hit[h] * n;
+    const T rma = Wm[alpha];
+    for (int64_t p0 = threadIdx.x; p0 < n; p0 += 256 * 8) {
+      T up[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) up[q] = p0 + 256 * q < n ? u[p0 + 256 * q] : (T)0;
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (up[q] != 0) {
+          const int64_t p = p0 + 256 * q;
+          uint32_t ev = 0;
+          Wm[p] = avos_sum<T>(Wm[p], avos_product<T>(rma, up[q], width, is_uns != 0, ev));
+          evs |= ev;
+        }
+    }
+  }
+  if (evs) atomicOr(&st->events, evs);
 }
 
 // Vertex composition, steps 3-4 (relational_composition.c.in:223-266).
@@ -397,35 +443,36 @@ static int edge_compose(const T* R, int64_t n, int64_t alpha, int64_t beta, T re
   return 0;
 }
 
-// scratch: rbg_edge_compose_scratch_bytes(n) bytes (the composed row and the
-// list of affected rows)
+// `count` edges (alpha, beta, relationship) one after another.  scratch:
+// rbg_edge_compose_scratch_bytes(n) bytes (the composed row, two row counters
+// and the list of affected rows)
 template <typename T>
-static int edge_compose_inplace(T* W, int64_t n, int64_t alpha, int64_t beta, T rel, void* scratch, int width,
-                                int is_uns, rbg_status* st, hipStream_t s) {
-  if (!W || !scratch || !st || n <= 0 || alpha < 0 || alpha >= n || beta < 0 || beta >= n) return RBG_E_ARG;
-  using U = typename unsigned_of<T>::type;
+static int edge_compose_many(T* W, int64_t n, const int64_t* edges, int64_t count, void* scratch, int width,
+                             int is_uns, rbg_status* st, hipStream_t s) {
+  if (!W || !scratch || !st || n <= 0 || n > 0x7fffffff || count < 0 || (count && !edges)) return RBG_E_ARG;
+  for (int64_t e = 0; e < count; e++)
+    if (edges[3 * e] < 0 || edges[3 * e] >= n || edges[3 * e + 1] < 0 || edges[3 * e + 1] >= n) return RBG_E_ARG;
   char* base = (char*)(((uintptr_t)scratch + 255) & ~(uintptr_t)255);
-  U* ukey = (U*)base;
-  int64_t* nhit = (int64_t*)(base + ((n * (int64_t)sizeof(T) + 255) & ~(int64_t)255));
-  int64_t* hit = nhit + 32;
-  const unsigned cols = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL((k_edge_begin<T>), dim3(cols), dim3(256), 0, s, W, n, alpha, beta, ukey, st);
-  RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(32), 0, s, nhit, (int64_t)1);
-  RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL((k_edge_row<T>), dim3(cols, (unsigned)((n + EC_ROWS - 1) / EC_ROWS)), dim3(256), 0, s, W, n,
-                     alpha, beta, rel, ukey, width, is_uns, st);
-  RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL((k_edge_row_end<T>), dim3(cols), dim3(256), 0, s, ukey, n);
-  RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL((k_edge_rows_hit<T>), dim3(cols), dim3(256), 0, s, W, n, alpha, hit, nhit);
-  RBG_CHECK_LAUNCH();
-  const unsigned grid = (unsigned)(n < 2048 ? n : 2048);
-  hipLaunchKernelGGL((k_edge_update_rows<T>), dim3(grid), dim3(256), 0, s, W, n, alpha, (const T*)ukey, hit, nhit,
-                     width, is_uns, st);
-  RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL((k_edge_put_row<T>), dim3(cols), dim3(256), 0, s, W, n, alpha, (const T*)ukey);
-  RBG_CHECK_LAUNCH();
+  T* u = (T*)base;
+  int64_t* counters = (int64_t*)(base + ((n * (int64_t)sizeof(T) + 255) & ~(int64_t)255));
+  int32_t* hit = (int32_t*)(counters + 32);
+  if (count) {
+    hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(32), 0, s, counters, (int64_t)32);
+    RBG_CHECK_LAUNCH();
+  }
+  for (int64_t e = 0; e < count; e++) {
+    const int64_t alpha = edges[3 * e], beta = edges[3 * e + 1];
+    // on lines of their own: one is cleared while the other is read
+    int32_t* now = (int32_t*)(counters + 16 * (e & 1));
+    int32_t* next = (int32_t*)(counters + 16 * ((e + 1) & 1));
+    hipLaunchKernelGGL((k_edge_compose<T>), dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, W, n, alpha, beta,
+                       (T)edges[3 * e + 2], u, hit, now, width, is_uns, st);
+    RBG_CHECK_LAUNCH();
+    const unsigned grid = (unsigned)((n + 255) / 256 < 64 ? 64 : ((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048));
+    hipLaunchKernelGGL((k_edge_apply<T>), dim3(grid), dim3(256), 0, s, W, n, alpha, (const T*)u, (const int32_t*)hit,
+                       (const int32_t*)now, next, width, is_uns, st);
+    RBG_CHECK_LAUNCH();
+  }
   return 0;
 }
 
@@ -540,11 +587,21 @@ int64_t rbg_edge_compose_scratch_bytes(int64_t n) {
 }
 int rbg_edge_compose_inplace_i32(int32_t* W, int64_t n, int64_t alpha, int64_t beta, int32_t rel, void* scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
-  return edge_compose_inplace<int32_t>(W, n, alpha, beta, rel, scratch, width, is_unsigned, st, (hipStream_t)stream);
+  const int64_t edge[3] = {alpha, beta, rel};
+  return edge_compose_many<int32_t>(W, n, edge, 1, scratch, width, is_unsigned, st, (hipStream_t)stream);
+}
+int rbg_edge_compose_many_i32(int32_t* W, int64_t n, const int64_t* edges, int64_t count, void* scratch,
+                              int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
+  return edge_compose_many<int32_t>(W, n, edges, count, scratch, width, is_unsigned, st, (hipStream_t)stream);
 }
 int rbg_edge_compose_inplace_i64(int64_t* W, int64_t n, int64_t alpha, int64_t beta, int64_t rel, void* scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
-  return edge_compose_inplace<int64_t>(W, n, alpha, beta, rel, scratch, width, is_unsigned, st, (hipStream_t)stream);
+  const int64_t edge[3] = {alpha, beta, rel};
+  return edge_compose_many<int64_t>(W, n, edge, 1, scratch, width, is_unsigned, st, (hipStream_t)stream);
+}
+int rbg_edge_compose_many_i64(int64_t* W, int64_t n, const int64_t* edges, int64_t count, void* scratch,
+                              int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
+  return edge_compose_many<int64_t>(W, n, edges, count, scratch, width, is_unsigned, st, (hipStream_t)stream);
 }
 int rbg_vertex_compose_i32(const int32_t* u, const int32_t* R, const int32_t* v, int32_t color, int64_t n,
                            int32_t* out, int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {

@@ -5,6 +5,7 @@ core.py wraps these.
 """
 from __future__ import annotations
 
+import ctypes
 import threading
 from dataclasses import dataclass
 
@@ -269,13 +270,12 @@ def edge_compose_many(R, edges, et: ElemType, stream=None, inplace: bool = False
     n = R.shape[0]
     st = status()
     st.reset(stream)
-    fn = "rbg_edge_compose_inplace_i32" if R.dtype == t.int32 else "rbg_edge_compose_inplace_i64"
+    fn = "rbg_edge_compose_many_i32" if R.dtype == t.int32 else "rbg_edge_compose_many_i64"
     sh = _lib.stream_handle(stream)
     cur = R if (inplace and R.is_contiguous()) else R.contiguous().clone()
     scratch = t.empty(int(_lib.load().rbg_edge_compose_scratch_bytes(n)), dtype=t.uint8, device=R.device)
-    for a, b, rel in edges:
-        _lib.call(fn, _lib.ptr(cur), n, int(a), int(b), int(rel), _lib.ptr(scratch), et.width, int(et.unsigned),
-                  st.p, sh)
+    flat = (ctypes.c_int64 * (3 * len(edges)))(*(int(x) for edge in edges for x in edge))
+    _lib.call(fn, _lib.ptr(cur), n, flat, len(edges), _lib.ptr(scratch), et.width, int(et.unsigned), st.p, sh)
     return cur, st.read(stream)
 
 
