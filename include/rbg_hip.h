@@ -543,6 +543,26 @@ int rbg_components(const int64_t *indptr, const int32_t *indices, int32_t n, int
  * n + 1 row pointers when out_indices / out_data are NULL, and the entries
  * (into buffers of out_indptr[n] entries) when they are given. */
 int64_t rbg_glue_temp_bytes(int64_t n);
+/* One step of a squaring closure (gpu/transitive_closure.py:26-74): N = R
+ * merged with R (x) R, the product's entry replacing R's where its absolute
+ * value is smaller (what rbg_spgemm_rows_* and rbg_csr_add_* with min_abs
+ * give), for a canonical n x n CSR matrix.  upper: the product's entries below
+ * the diagonal are left out.  _count writes N's row pointers (n + 1), st->aux[0]
+ * != 0 when N differs from R and st->aux[1] = N's entries (whole status block;
+ * temp: rbg_glue_temp_bytes(n)); RBG_F_CAPACITY: a row of N has more than 768
+ * entries, and neither call's result holds.  _fill writes N's columns and values. */
+int rbg_csr_square_count_i32(const int64_t *ap, const int32_t *aj, const int32_t *ax, int32_t n, int32_t upper,
+                             int64_t *out_ptr, void *temp, int64_t temp_bytes, int32_t width, rbg_status *st,
+                             rbg_stream_t stream);
+int rbg_csr_square_count_i64(const int64_t *ap, const int32_t *aj, const int64_t *ax, int32_t n, int32_t upper,
+                             int64_t *out_ptr, void *temp, int64_t temp_bytes, int32_t width, rbg_status *st,
+                             rbg_stream_t stream);
+int rbg_csr_square_fill_i32(const int64_t *ap, const int32_t *aj, const int32_t *ax, int32_t n, int32_t upper,
+                            const int64_t *out_ptr, int32_t *out_idx, int32_t *out_val, int32_t width,
+                            rbg_status *st, rbg_stream_t stream);
+int rbg_csr_square_fill_i64(const int64_t *ap, const int32_t *aj, const int64_t *ax, int32_t n, int32_t upper,
+                            const int64_t *out_ptr, int32_t *out_idx, int64_t *out_val, int32_t width,
+                            rbg_status *st, rbg_stream_t stream);
 /* st->aux[0] += sum over A's entries (i, k) of |row k of B|: the candidate
  * count of A (x) B, an exact bound on its size (the symbolic count of
  * gpu/spgemm_symbolic.py:124-183).  m = rows of A. */

@@ -130,6 +130,10 @@ SIGNATURES = {
     "rbg_components": (I32, [P, P, I32, P, P, ctypes.POINTER(ctypes.c_int32), P]),
     "rbg_glue_temp_bytes": (I64, [I64]),
     "rbg_csr_expand_size": (I32, [P, P, I32, P, P, P]),
+    "rbg_csr_square_count_i32": (I32, [P, P, P, I32, I32, P, P, I64, I32, P, P]),
+    "rbg_csr_square_count_i64": (I32, [P, P, P, I32, I32, P, P, I64, I32, P, P]),
+    "rbg_csr_square_fill_i32": (I32, [P, P, P, I32, I32, P, P, P, I32, P, P]),
+    "rbg_csr_square_fill_i64": (I32, [P, P, P, I32, I32, P, P, P, I32, P, P]),
     "rbg_csr_max_abs_i32": (I32, [P, P, I32, P, P]),
     "rbg_csr_max_abs_i64": (I32, [P, P, I32, P, P]),
     "rbg_csr_to_dense_i32": (I32, [P, P, P, I32, I64, P, P]),

@@ -59,6 +59,235 @@ static int rows_to_ptr(const int64_t* cnt, int64_t n, int64_t* out, void* temp, 
   return e == hipSuccess ? 0 : (int)e;
 }
 
+// ---- one step of a squaring closure -------------------------------------------
+// N = R merged with R (x) R (gpu/transitive_closure.py:26-74: the product's
+// entry replaces R's where its absolute value is smaller), a workgroup per row:
+// the products A[i][k] (x) R[k][j] go into a hash table of the row's columns in
+// LDS (a swap claims a column's place, an atomic min keeps the AVOS sum, whose
+// terms have no order), then R's own row is merged in.  FILL = false counts the
+// rows of N and tells whether any entry differs from R's, so the last step of a
+// closure writes nothing; FILL writes the rows, each column at its rank.
+// Bound by the round trips to the rows R[k] (four in flight) and the table's
+// atomics.  Last steps of the closure of n = 11,012: 44 us to count and 42 to
+// write with two waves a row, 54 and 56 with four, 56 and 51 with one; the
+// product by folding lists and the merge took 277 + 81 us and the comparison
+// and three host waits came on top (whole closure 3.24 -> 0.62 ms).  A row with
+// more than SQ_COLUMNS columns sets RBG_F_CAPACITY.
+constexpr int SQ_SLOTS = 1024;
+constexpr int SQ_COLUMNS = 768;
+constexpr int SQ_NT = 128;
+
+template <typename T>
+struct SquareRow {
+  using U = typename unsigned_of<T>::type;
+  int32_t col[SQ_SLOTS];         // -1: free
+  U key[SQ_SLOTS];               // -1 -> 0, v -> v, nothing yet -> all ones
+  int32_t cols[SQ_COLUMNS + 4];  // the columns together
+  uint16_t slot[SQ_COLUMNS];
+  int total, m, full, changed;
+};
+
+template <typename T, bool FILL>
+__global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__ ap, const int32_t* __restrict__ aj,
+                                                     const T* __restrict__ ax, int32_t n, int upper,
+                                                     int64_t* __restrict__ len, const int64_t* __restrict__ op,
+                                                     int32_t* __restrict__ oj, T* __restrict__ ox, int width,
+                                                     rbg_status* st) {
+  using U = typename unsigned_of<T>::type;
+  __shared__ SquareRow<T> L;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t i = blockIdx.x;
+  const int64_t r0 = ap[i];
+  const int cnt = (int)(ap[i + 1] - r0);
+  if (tid == 0) L.total = L.m = L.full = L.changed = 0;
+  __syncthreads();
+  // the table's size from the row's products: at most three quarters full
+  // where they are few, else SQ_SLOTS
+  int mine = 0;
+  for (int e = tid; e < cnt; e += SQ_NT) {
+    const int32_t k = aj[r0 + e];
+    const int64_t l = 1 + ap[k + 1] - ap[k];
+    mine += l < SQ_SLOTS ? (int)l : SQ_SLOTS;
+    if (mine > SQ_SLOTS) mine = SQ_SLOTS;
+  }
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+  if (lane == 0 && mine) atomicAdd(&L.total, mine);
+  __syncthreads();
+  const int total = L.total;
+  int slots = 64;
+  while (slots < SQ_SLOTS && 4 * total > 3 * slots) slots <<= 1;
+  const int shift = __builtin_clz(slots) + 1;
+  for (int q = tid; q < slots; q += SQ_NT) {
+    L.col[q] = -1;
+    L.key[q] = ~(U)0;
+  }
+  __syncthreads();
+  bool full = false;
+  uint32_t evs = 0;
+  auto place = [&](int32_t c) {  // c's slot, claimed if new; -1 when the table is full
+    int h = (int)(((uint32_t)c * 0x9E3779B1u) >> shift);
+    for (int probe = 0; probe < slots; probe++) {
+      const int32_t old = atomicCAS(&L.col[h], -1, c);
+      if (old == -1 || old == c) return h;
+      h = (h + 1) & (slots - 1);
+    }
+    return -1;
+  };
+  auto term = [&](T a, int32_t c, T b) {
+    if (upper && c < i) return;
+    uint32_t ev = 0;
+    const T p = avos_product<T>(a, b, width, false, ev);
+    evs |= ev;
+    if (p == 0) return;
+    const int h = place(c);
+    if (h < 0)
+      full = true;
+    else
+      atomicMin(&L.key[h], p == (T)-1 ? (U)0 : (U)p);
+  };
+  // the waves take 16 of the row's entries at a time
+  for (int e0 = (tid >> 6) * 16; e0 < cnt; e0 += SQ_NT / 64 * 16) {
+    const bool on = lane < 16 && e0 + lane < cnt;
+    const int32_t k = on ? aj[r0 + e0 + lane] : 0;
+    const T a = on ? ax[r0 + e0 + lane] : (T)0;
+    const int64_t s = on ? ap[k] : 0;
+    const int l = on ? (int)(ap[k + 1] - s) : 0;
+    const int here = cnt - e0 < 16 ? cnt - e0 : 16;
+    for (int e = 0; e < here; e += 4) {
+      int le[4];
+      int64_t at[4];
+      T ae[4], b[4];
+      int32_t c[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int q = e + u < here ? e + u : e;
+        le[u] = e + u < here ? __shfl(l, q, 64) : 0;
+        at[u] = __shfl(s, q, 64) + lane;
+        ae[u] = __shfl(a, q, 64);
+        if (lane < le[u]) {
+          c[u] = aj[at[u]];
+          b[u] = ax[at[u]];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (lane < le[u]) term(ae[u], c[u], b[u]);
+        for (int t = 64; t < le[u]; t += 64)
+          if (t + lane < le[u]) term(ae[u], aj[at[u] + t], ax[at[u] + t]);
+      }
+    }
+  }
+  __syncthreads();
+  bool changed = false;
+  for (int e = tid; e < cnt; e += SQ_NT) {  // R's own entries, each column once
+    const T x = ax[r0 + e];
+    const int h = place(aj[r0 + e]);
+    if (h < 0) {
+      full = true;
+      continue;
+    }
+    const U k = L.key[h];
+    T v = x;
+    if (k != ~(U)0) {
+      const T y = k == 0 ? (T)-1 : (T)k;
+      const T mx = x < 0 ? -x : x, my = y < 0 ? -y : y;
+      v = my < mx ? y : x;
+    }
+    changed |= v != x;
+    L.key[h] = v == (T)-1 ? (U)0 : (U)v;
+  }
+  if (full) L.full = 1;
+  if (changed) L.changed = 1;
+  __syncthreads();
+  for (int q = tid; q < slots; q += SQ_NT) {  // the taken slots, together (slots: a multiple of a wave)
+    const int32_t c = L.col[q];
+    const uint64_t taken = __ballot(c >= 0);
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&L.m, __popcll(taken));
+    at = __shfl(at, 0, 64) + __popcll(taken & (((uint64_t)1 << lane) - 1));
+    if (c >= 0 && at < SQ_COLUMNS) {
+      L.cols[at] = c;
+      L.slot[at] = (uint16_t)q;
+    }
+  }
+  __syncthreads();
+  const int m = L.m;
+  if (L.full || m > SQ_COLUMNS) {
+    if (tid == 0) {
+      if (!FILL) len[i] = 0;
+      atomicOr(&st->flags, (uint32_t)RBG_F_CAPACITY);
+    }
+    return;
+  }
+  if (!FILL) {
+    if (tid == 0) {
+      len[i] = m;
+      if ((L.changed || m > cnt) && __hip_atomic_load(&st->aux[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+        atomicOr((unsigned long long*)&st->aux[0], 1ull);
+    }
+    return;
+  }
+  if (tid < 4) L.cols[m + tid] = 0x7fffffff;
+  __syncthreads();
+  const int64_t d = op[i];
+  for (int q = tid; q < m; q += SQ_NT) {
+    const int32_t c = L.cols[q];
+    int r = 0;
+    for (int x = 0; x < m; x += 4)
+      r += (int)(L.cols[x] < c) + (int)(L.cols[x + 1] < c) + (int)(L.cols[x + 2] < c) + (int)(L.cols[x + 3] < c);
+    const U k = L.key[L.slot[q]];
+    oj[d + r] = c;
+    ox[d + r] = k == 0 ? (T)-1 : (T)k;
+  }
+  if (evs) atomicOr(&st->events, evs);
+}
+
+__global__ void k_gl_total(const int64_t* __restrict__ ptr, int32_t n, rbg_status* st) { st->aux[1] = ptr[n]; }
+
+// Row pointers of n <= PTR_SMALL counts and their total (st->aux[1]) by one
+// workgroup, in place of four launches.
+constexpr int PTR_NT = 1024;
+constexpr int64_t PTR_SMALL = 64 * PTR_NT;
+__global__ __launch_bounds__(PTR_NT) void k_gl_ptr_small(const int64_t* __restrict__ cnt, int32_t n,
+                                                         int64_t* __restrict__ out, rbg_status* st) {
+  __shared__ int64_t wsum[PTR_NT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int64_t base = 0;
+  for (int32_t b = 0; b < n; b += 4 * PTR_NT) {
+    int64_t c[4], mine = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int32_t i = b + 4 * tid + q;
+      c[q] = i < n ? cnt[i] : 0;
+      mine += c[q];
+    }
+    int64_t incl = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t u = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += u;
+    }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    int64_t at = base + incl - mine;
+    for (int w = 0; w < PTR_NT / 64; w++) {
+      if (w < wv) at += wsum[w];
+      base += wsum[w];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int32_t i = b + 4 * tid + q;
+      if (i < n) out[i] = at;
+      at += c[q];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    out[n] = base;
+    st->aux[1] = base;
+  }
+}
+
 // ---- reductions -------------------------------------------------------------
 // aux[0] += sum over A's entries (i, k) of |row k of B|: the candidate count
 // of C = A (x) B (an exact bound on every row's output)
@@ -359,6 +588,43 @@ struct GlueTemp {
     return true;
   }
 };
+
+#define RBG_GL_SQUARE(SUF, T)                                                                                       \
+  int rbg_csr_square_count_##SUF(const int64_t* ap, const int32_t* aj, const T* ax, int32_t n, int32_t upper,       \
+                                 int64_t* out_ptr, void* temp, int64_t temp_bytes, int32_t width, rbg_status* st,   \
+                                 rbg_stream_t stream) {                                                             \
+    hipStream_t s = (hipStream_t)stream;                                                                            \
+    if (!ap || !aj || !ax || n <= 0 || !out_ptr || !st) return RBG_E_ARG;                                           \
+    GlueTemp t;                                                                                                     \
+    if (!GlueTemp::carve(temp, temp_bytes, n, &t)) return RBG_E_WORKSPACE;                                          \
+    int rc = rbg_status_init(st, stream);                                                                           \
+    if (rc) return rc;                                                                                              \
+    hipLaunchKernelGGL((k_gl_square<T, false>), dim3(n), dim3(SQ_NT), 0, s, ap, \
+                       aj, ax, n, upper, t.cnt, (const int64_t*)nullptr, (int32_t*)nullptr, (T*)nullptr, width, st); \
+    RBG_CHECK_LAUNCH();                                                                                             \
+    if (n <= PTR_SMALL) {                                                                                           \
+      hipLaunchKernelGGL(k_gl_ptr_small, dim3(1), dim3(PTR_NT), 0, s, (const int64_t*)t.cnt, n, out_ptr, st);       \
+      RBG_CHECK_LAUNCH();                                                                                           \
+      return 0;                                                                                                     \
+    }                                                                                                               \
+    rc = rows_to_ptr(t.cnt, n, out_ptr, t.store, t.store_bytes, s);                                                 \
+    if (rc) return rc;                                                                                              \
+    hipLaunchKernelGGL(k_gl_total, dim3(1), dim3(1), 0, s, (const int64_t*)out_ptr, n, st);                         \
+    RBG_CHECK_LAUNCH();                                                                                             \
+    return 0;                                                                                                       \
+  }                                                                                                                 \
+  int rbg_csr_square_fill_##SUF(const int64_t* ap, const int32_t* aj, const T* ax, int32_t n, int32_t upper,        \
+                                const int64_t* out_ptr, int32_t* out_idx, T* out_val, int32_t width,                \
+                                rbg_status* st, rbg_stream_t stream) {                                              \
+    if (!ap || !aj || !ax || n <= 0 || !out_ptr || !out_idx || !out_val || !st) return RBG_E_ARG;                   \
+    hipLaunchKernelGGL((k_gl_square<T, true>), dim3(n), dim3(SQ_NT), 0,         \
+                       (hipStream_t)stream, ap, aj, ax, n, upper, (int64_t*)nullptr, out_ptr, out_idx, out_val,     \
+                       width, st);                                                                                  \
+    RBG_CHECK_LAUNCH();                                                                                             \
+    return 0;                                                                                                       \
+  }
+RBG_GL_SQUARE(i32, int32_t)
+RBG_GL_SQUARE(i64, int64_t)
 
 int rbg_csr_expand_size(const int64_t* ap, const int32_t* aj, int32_t m, const int64_t* bp, rbg_status* st,
                         rbg_stream_t stream) {

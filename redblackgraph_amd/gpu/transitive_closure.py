@@ -62,9 +62,8 @@ def transitive_closure_gpu(A: CSRMatrixGPU, max_iterations: int = 64) -> Tuple[C
     tri = A.triangular
     diameter = 0
     for iteration in range(max_iterations):
-        R2, _ = sd.spgemm(R, R, mask_upper=tri)
-        Rn = sd.avos_sum_csr(R, R2, min_abs=True)
-        if sd.csr_equal(R, Rn):
+        Rn = sd.square_step(R, mask_upper=tri)
+        if Rn is None:
             break
         R = Rn
         diameter = iteration + 1

@@ -108,9 +108,8 @@ def transitive_closure_squaring(A, max_iterations=64) -> TransitiveClosure:
         return transitive_closure_dag_sparse(A)
     R = sd.canonicalize(sd.from_scipy(A, np.int32))
     for _ in range(max_iterations):
-        R2, _ev = sd.spgemm(R, R)
-        Rn = sd.avos_sum_csr(R, R2, min_abs=True)
-        if sd.csr_equal(R, Rn):
+        Rn = sd.square_step(R)
+        if Rn is None:
             break
         R = Rn
     c = sd.to_scipy(R)
