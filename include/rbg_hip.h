@@ -147,7 +147,8 @@ int64_t rbg_fw_flow_waits(int64_t n, int32_t elem_bytes, int32_t edge, int64_t *
  * durations (ms) and launch counts since the last read, then clears them. */
 int rbg_fw_prof_enable(int32_t on);
 /* Same facility for every timed launch kind: 0 FW panel, 1 FW tile, 5 FW small tile,
- * 6 FW persistent closure, 2 DAG level, 3 SpGEMM rows, 4 batched FW.  on = 1 starts recording afresh, 2
+ * 6 FW persistent closure, 2 DAG level, 3 SpGEMM rows, 4 batched FW, 7 closure
+ * from the rows' entries (single matrix and batch).  on = 1 starts recording afresh, 2
  * resumes and 0 pauses, both keeping what was recorded (so a caller can time
  * a sample of its launches).  rbg_prof_read returns (and clears) the summed
  * duration and count of one kind. */
@@ -155,7 +156,8 @@ int rbg_prof_enable(int32_t on);
 int rbg_prof_read(int32_t kind, double *total_ms, int64_t *launches);
 /* rbg_prof_read, also returning the work the launches recorded: relaxations
  * executed for the FW tile kinds (1: 128 x 128 tiles, 5: 64 x 64 int32 tiles
- * of the small-matrix and triangular schedules), 0 for the other kinds. */
+ * of the small-matrix and triangular schedules; 4), bytes of the matrix written
+ * (7, single matrix), 0 for the other kinds. */
 int rbg_prof_read_work(int32_t kind, double *total_ms, int64_t *launches, double *work);
 int rbg_fw_prof_read(double *panel_ms, int64_t *panel_launches, double *tile_ms, int64_t *tile_launches);
 /* No counterpart in the reference (the fast path's copy-in, one pass over the
@@ -522,6 +524,9 @@ int64_t rbg_batch_flow_tickets(const int32_t *npad, const int32_t *edge, int32_t
 int rbg_batch_create(const rbg_batch_comp *comps, int32_t count, rbg_batch **out);
 int rbg_batch_info(const rbg_batch *b, int64_t *info);
 int rbg_batch_run(rbg_batch *b, rbg_stream_t stream);
+/* closed[i] = 1 where the last run closed component i from its rows' entries
+ * (count entries, host memory); waits for the stream. */
+int rbg_batch_rows_closed(const rbg_batch *b, int32_t *closed, rbg_stream_t stream);
 int rbg_batch_capture(rbg_batch *b, rbg_stream_t stream);
 int rbg_batch_replay(rbg_batch *b, rbg_stream_t stream);
 int rbg_batch_destroy(rbg_batch *b);

@@ -124,6 +124,7 @@ SIGNATURES = {
     "rbg_batch_create": (I32, [P, I32, P]),
     "rbg_batch_info": (I32, [P, P]),
     "rbg_batch_run": (I32, [P, P]),
+    "rbg_batch_rows_closed": (I32, [P, P, P]),
     "rbg_batch_capture": (I32, [P, P]),
     "rbg_batch_replay": (I32, [P, P]),
     "rbg_batch_destroy": (I32, [P]),

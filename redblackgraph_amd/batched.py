@@ -164,6 +164,13 @@ class BatchedClosure:
         except Exception:
             pass
 
+    def rows_closed(self) -> np.ndarray:
+        """Per component, whether the last run closed it from its rows' entries."""
+        out = np.zeros(self.count, dtype=np.int32)
+        _lib.call("rbg_batch_rows_closed", self._h, out.ctypes.data_as(ctypes.c_void_p),
+                  _lib.stream_handle(self.stream))
+        return out.astype(bool)
+
     def info(self) -> dict:
         buf = (ctypes.c_int64 * 10)()
         _lib.call("rbg_batch_info", self._h, buf)

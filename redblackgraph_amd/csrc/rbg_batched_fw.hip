@@ -391,8 +391,10 @@ static int batch_launch(rbg_batch* b, hipStream_t s) {
     RBG_CHECK_LAUNCH();
     hipLaunchKernelGGL(k_bfw_rows_place, dim3((unsigned)b->n_rplace), dim3(NT), 0, s, b->d_comps, place);
     RBG_CHECK_LAUNCH();
+    int pr = prof_start(s);
     hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_CLOSE_NT), 0, s, b->d_comps, close);
     RBG_CHECK_LAUNCH();
+    prof_stop(7, pr, s, 0.0);
   }
   const Item* chunks = b->d_items;
   const Item* panels = chunks + b->n_chunk;
@@ -689,6 +691,14 @@ int rbg_batch_info(const rbg_batch* b, int64_t* info) {
 int rbg_batch_run(rbg_batch* b, rbg_stream_t stream) {
   if (!b) return RBG_E_ARG;
   return batch_launch(b, (hipStream_t)stream);
+}
+
+int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stream) {
+  if (!b || !closed) return RBG_E_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  const hipError_t e = hipMemcpy2DAsync(closed, sizeof(int32_t), &b->d_comps->done, sizeof(BComp), sizeof(int32_t),
+                                        (size_t)b->count, hipMemcpyDeviceToHost, s);
+  return e == hipSuccess ? (int)hipStreamSynchronize(s) : (int)e;
 }
 
 int rbg_batch_capture(rbg_batch* b, rbg_stream_t stream) {
