@@ -580,8 +580,8 @@ def _batched_persistent_leg(args, sizes, pristine, eager_result, stream):
         p.stream.synchronize()
         ms = (time.perf_counter() - t0) * 1e3 / args.steps
         identical = bool(t.equal(p.pool, eager_result))
-        frac = relax * OPS_PER_RELAX["int32"] / (launch_ms / 1e3) / PEAK_VALU_OPS
-        return {"ms_per_step": ms, "launch_ms": launch_ms, "frac": frac if left else None,
+        frac = relax * OPS_PER_RELAX["int32"] / (launch_ms / 1e3) / PEAK_VALU_OPS if left else None
+        return {"ms_per_step": ms, "launch_ms": launch_ms, "frac": frac,
                 "components_closed_from_rows": rows_closed, "relaxations_executed": relax if left else 0, "work_items": info["persistent_items"],
                 "launches_per_batch": info["launches"], "status_flags": flags,
                 "identical_to_per_step_launches": identical,

@@ -523,6 +523,9 @@ int64_t rbg_batch_flow_tickets(const int32_t *npad, const int32_t *edge, int32_t
                                int64_t cap);
 int rbg_batch_create(const rbg_batch_comp *comps, int32_t count, rbg_batch **out);
 int rbg_batch_info(const rbg_batch *b, int64_t *info);
+/* Queues one run.  Outside a capture the call may wait, for no longer than
+ * queueing every schedule's launches takes, for word that all components were
+ * closed from their rows' entries; the launches behind are then not queued. */
 int rbg_batch_run(rbg_batch *b, rbg_stream_t stream);
 /* closed[i] = 1 where the last run closed component i from its rows' entries
  * (count entries, host memory); waits for the stream. */

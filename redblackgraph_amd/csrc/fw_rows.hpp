@@ -451,13 +451,14 @@ __host__ __device__ inline int64_t rows_slab() {
   return ROWS_LANES * (16 / (int64_t)sizeof(T));
 }
 
-// 64 KB: two workgroups per CU
-template <bool LARGEST>
-constexpr int ROWS_RING = LARGEST ? 512 : 1024;
-template <typename T, bool LARGEST>
+// 64 KB: two workgroups of 1024 threads per CU; in place, 16 KB for eight of 256
+template <bool LARGEST, bool INPLACE>
+constexpr int ROWS_RING = INPLACE ? 256 : LARGEST ? 512 : 1024;
+template <typename T, bool LARGEST, bool INPLACE>
 struct CloseShared {
-  T ring[ROWS_RING<LARGEST>][ROWS_LANES][16 / sizeof(T)];
-  T ring2[LARGEST ? ROWS_RING<LARGEST> : 1][ROWS_LANES][16 / sizeof(T)];
+  static constexpr int ROWS = ROWS_RING<LARGEST, INPLACE>;
+  T ring[ROWS][ROWS_LANES][16 / sizeof(T)];
+  T ring2[LARGEST ? ROWS : 1][ROWS_LANES][16 / sizeof(T)];
   int start[ROWS_MAX_LEVELS + 1];
   long long top, top2;
   int guard;
@@ -498,8 +499,12 @@ __device__ inline RowRec<T> rec_of_quad(uint2 q) {
 // rows' entries as above, level by level, but a cell's first value depends on
 // the numbering.  W2 takes the largest path value of every cell (no value a
 // cell ever holds is above it), and the slab's largest goes to w.slab_top.
-template <typename T, int UN, bool LARGEST>
-__device__ inline void rows_close_slab(CloseShared<T, LARGEST>& L, RowsWork<T> w, T* W, T* W2, int64_t ld,
+//
+// INPLACE: W is the input, lower triangular.  No entry's cell is ever cleared,
+// so a segment whose result is all zero was all zero and is not written (128
+// components, 0.5 GB of matrices: 481 -> 345 us).
+template <typename T, int UN, bool LARGEST, bool INPLACE>
+__device__ inline void rows_close_slab(CloseShared<T, LARGEST, INPLACE>& L, RowsWork<T> w, T* W, T* W2, int64_t ld,
                                        int64_t slab, int width, rbg_status* st) {
   using U = typename unsigned_of<T>::type;
   constexpr int V = 16 / (int)sizeof(T);
@@ -510,7 +515,7 @@ __device__ inline void rows_close_slab(CloseShared<T, LARGEST>& L, RowsWork<T> w
   // row offsets in 16-byte units: below 2^32 for ROWS_MAX_N, one 24-bit multiply each
   const uint32_t ld16 = (uint32_t)(ld / V), jl16 = (uint32_t)(jl / V);
   auto off = [&](int row) { return (size_t)(__umul24((uint32_t)row, ld16) + jl16) * V; };
-  constexpr int RING = ROWS_RING<LARGEST>;
+  constexpr int RING = ROWS_RING<LARGEST, INPLACE>;
   const int levels = w.ctl[1];
   if (tid <= levels) L.start[tid] = w.ctl[CTL_START + tid];
   if (tid == 0) {
@@ -569,7 +574,7 @@ __device__ inline void rows_close_slab(CloseShared<T, LARGEST>& L, RowsWork<T> w
       if (!on[u]) continue;
       T* out = W + off(row[u]);
       if (!LARGEST && row[u] < j0) {
-        rows_st_stream<T>(out);
+        if (!INPLACE) rows_st_stream<T>(out);
         continue;
       }
       U cur[V];
@@ -650,7 +655,10 @@ __device__ inline void rows_close_slab(CloseShared<T, LARGEST>& L, RowsWork<T> w
         for (int x = 0; x < V; x++)
           if (row[u] == jl + x) o[x] = one;
       }
-      rows_st<T, V>(out, o);
+      T any = 0;
+#pragma unroll
+      for (int x = 0; x < V; x++) any |= o[x];
+      if (!INPLACE || any != 0) rows_st<T, V>(out, o);
       if (LARGEST) rows_st<T, V>(W2 + off(row[u]), big);
       const int p = base + g + u * G;
       if (p >= kept) {

@@ -24,6 +24,7 @@
 // is flagged in its status; the caller reruns it through the single-matrix
 // path.
 #include <algorithm>
+#include <chrono>
 #include <numeric>
 
 #include "fw_rows.hpp"
@@ -186,12 +187,32 @@ static __global__ __launch_bounds__(NT) void k_bfw_rows_place(const BComp* comps
 }
 
 // item = (component, slab), in place: the entries have left the matrix
-static __global__ __launch_bounds__(ROWS_CLOSE_NT, 8) void k_bfw_rows_close(const BComp* comps, const Item* items) {
-  __shared__ CloseShared<int32_t, false> L;
+// 256 threads: a level of a component has n / log2(n) rows or so, 64 a pass
+// (128 components of up to 4096 vertices: 345 us with 1024 threads and their
+// ring, 287 with 512, 264 with 256 or 128; then bound by the instructions of
+// the rows' decoding and products)
+constexpr int ROWS_BATCH_CLOSE_NT = 256;
+static __global__ __launch_bounds__(ROWS_BATCH_CLOSE_NT, 8) void k_bfw_rows_close(const BComp* comps,
+                                                                                  const Item* items) {
+  __shared__ CloseShared<int32_t, false, true> L;
   const Item it = items[blockIdx.x];
   const BComp c = comps[it.comp];
   if (!c.done) return;
-  rows_close_slab<int32_t, 1, false>(L, rows_work(c), c.W, nullptr, c.npad, it.bid, 32, c.st);
+  rows_close_slab<int32_t, 1, false, true>(L, rows_work(c), c.W, nullptr, c.npad, it.bid, 32, c.st);
+}
+
+// Tells the host whether every component is closed from its rows: the number
+// of the run, negative where one is not.
+static __global__ __launch_bounds__(NT) void k_bfw_rows_tell(const BComp* comps, int32_t count, int64_t* runs,
+                                                             int64_t* told) {
+  bool left = false;
+  for (int c = threadIdx.x; c < count; c += NT) left |= comps[c].done == 0;
+  left = __syncthreads_or(left);
+  if (threadIdx.x == 0) {
+    const int64_t run = *runs + 1;
+    *runs = run;
+    __hip_atomic_store(told, left ? -run : run, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // Domain conversion of one 128 x 128 chunk, four cells per thread and pass.
@@ -367,35 +388,82 @@ struct rbg_batch {
   int32_t* d_rows = nullptr;
   Item* d_ritems = nullptr;
   int64_t n_rows = 0, n_rscan = 0, n_rplace = 0, n_rclose = 0;
+  int64_t* told = nullptr;    // pinned: k_bfw_rows_tell's answer
+  int64_t* d_runs = nullptr;  // runs told of; `runs`: launched
+  int64_t runs = 0;
   Item* d_prewalk = nullptr;  // (component, block) of the per-step components with dsnap
   int64_t n_prewalk = 0;
   std::vector<int64_t> panel_cnt, t128_cnt, t64_cnt;  // per step: items of running components
   std::vector<int64_t> tri128_off, tri64_off;         // per step: [off[K], off[K + 1]) of the step lists
   std::vector<double> work;                           // per step: relaxations its tile launches execute
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  // captured: every launch of a run, or where rows are tried the launches up to
+  // theirs and, in graph 1, those behind
+  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
 };
 
-static int batch_launch(rbg_batch* b, hipStream_t s) {
-  const int cgrid = (b->count + 255) / 256;
-  hipLaunchKernelGGL(k_bfw_init, dim3(cgrid), dim3(256), 0, s, b->d_comps, b->count);
-  RBG_CHECK_LAUNCH();
-  // a forced wait limit asks for the persistent launch (rbg_fw_flow_wait_limit)
-  if (b->n_rows && g_flow_limit_override.load() == 0) {
-    const Item* scan = b->d_ritems;
-    const Item* place = scan + b->n_rscan;
-    const Item* close = place + b->n_rplace;
-    hipLaunchKernelGGL(k_bfw_rows_scan, dim3((unsigned)b->n_rscan), dim3(NT), 0, s, b->d_comps, scan);
-    RBG_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_bfw_rows_levels, dim3((unsigned)b->n_rows), dim3(ROWS_BATCH_NT), 0, s, b->d_comps, b->d_rows);
-    RBG_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_bfw_rows_place, dim3((unsigned)b->n_rplace), dim3(NT), 0, s, b->d_comps, place);
-    RBG_CHECK_LAUNCH();
-    int pr = prof_start(s);
-    hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_CLOSE_NT), 0, s, b->d_comps, close);
-    RBG_CHECK_LAUNCH();
-    prof_stop(7, pr, s, 0.0);
+// launches of the relaxation schedules, behind the rows' ones
+static int64_t batch_step_launches(const rbg_batch* b) {
+  int64_t launches = 3 + (b->n_flow ? 3 : 0) + (b->n_prewalk ? 1 : 0);
+  for (int K = 0; K < b->stepnb; K++)
+    launches += (b->panel_cnt[K] > 0) + (b->t128_cnt[K] > 0) + (b->t64_cnt[K] > 0) +
+                (b->tri128_off[K + 1] > b->tri128_off[K]) + (b->tri64_off[K + 1] > b->tri64_off[K]);
+  return launches;
+}
+
+// Whether every component is known to be closed from its rows, so that nothing
+// is left to launch.  The answer is there while the rows' last launch still
+// runs; it is awaited for about as long as queueing the idle launches would
+// take (4 us each), no longer: the call stays asynchronous where the stream is
+// busy (128 components, 260 idle launches: 1.75 -> 1.11 ms a replay).
+static bool batch_rows_told(const rbg_batch* b) {
+  const int64_t limit_us = 4 * batch_step_launches(b);
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    const int64_t v = __atomic_load_n(b->told, __ATOMIC_ACQUIRE);
+    if (v == b->runs || v == -b->runs) return v > 0;
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(limit_us)) return false;
   }
+}
+
+// a forced wait limit asks for the persistent launch (rbg_fw_flow_wait_limit)
+static bool batch_tries_rows(const rbg_batch* b) { return b->n_rows && g_flow_limit_override.load() == 0; }
+
+// A stream under capture has no host beside it: every launch is queued.
+static bool stream_captures(hipStream_t s) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capture) == hipSuccess) return capture != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+static int batch_init(rbg_batch* b, hipStream_t s) {
+  hipLaunchKernelGGL(k_bfw_init, dim3((b->count + 255) / 256), dim3(256), 0, s, b->d_comps, b->count);
+  RBG_CHECK_LAUNCH();
+  return 0;
+}
+
+static int batch_launch_rows(rbg_batch* b, hipStream_t s) {
+  const Item* scan = b->d_ritems;
+  const Item* place = scan + b->n_rscan;
+  const Item* close = place + b->n_rplace;
+  hipLaunchKernelGGL(k_bfw_rows_scan, dim3((unsigned)b->n_rscan), dim3(NT), 0, s, b->d_comps, scan);
+  RBG_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_bfw_rows_levels, dim3((unsigned)b->n_rows), dim3(ROWS_BATCH_NT), 0, s, b->d_comps, b->d_rows);
+  RBG_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_bfw_rows_place, dim3((unsigned)b->n_rplace), dim3(NT), 0, s, b->d_comps, place);
+  RBG_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_bfw_rows_tell, dim3(1), dim3(NT), 0, s, b->d_comps, b->count, b->d_runs, b->told);
+  RBG_CHECK_LAUNCH();
+  int pr = prof_start(s);
+  hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_BATCH_CLOSE_NT), 0, s, b->d_comps, close);
+  RBG_CHECK_LAUNCH();
+  prof_stop(7, pr, s, 0.0);
+  return 0;
+}
+
+static int batch_launch_steps(rbg_batch* b, hipStream_t s) {
+  const int cgrid = (b->count + 255) / 256;
   const Item* chunks = b->d_items;
   const Item* panels = chunks + b->n_chunk;
   const Item* t128 = panels + b->n_panel;
@@ -628,6 +696,10 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
   if (e == hipSuccess && b->n_rows) {
     e = hipMalloc((void**)&b->d_rows, sizeof(int32_t) * rows.size());
     if (e == hipSuccess) e = hipMalloc((void**)&b->d_ritems, sizeof(Item) * ritems.size());
+    if (e == hipSuccess) e = hipHostMalloc((void**)&b->told, sizeof(int64_t), hipHostMallocMapped | hipHostMallocCoherent);
+    if (e == hipSuccess) *b->told = 0;
+    if (e == hipSuccess) e = hipMalloc((void**)&b->d_runs, sizeof(int64_t));
+    if (e == hipSuccess) e = hipMemcpy(b->d_runs, b->told, sizeof(int64_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b->d_rows, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess)
       e = hipMemcpy(b->d_ritems, ritems.data(), sizeof(Item) * ritems.size(), hipMemcpyHostToDevice);
@@ -656,12 +728,14 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     (void)hipFree(b->d_comps);
     (void)hipFree(b->d_items);
     (void)hipFree(b->d_rows);
+    (void)hipFree(b->d_runs);
     (void)hipFree(b->d_ritems);
     (void)hipFree(b->d_prewalk);
     (void)hipFree(b->d_flow);
     (void)hipFree(b->d_walk);
     (void)hipFree(b->d_ctl);
     (void)hipFree(b->d_fitems);
+    if (b->told) (void)hipHostFree(b->told);
     delete b;
     return (int)e;
   }
@@ -671,10 +745,7 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
 
 int rbg_batch_info(const rbg_batch* b, int64_t* info) {
   if (!b || !info) return RBG_E_ARG;
-  int64_t launches = 4 + (b->n_rows ? 4 : 0) + (b->n_flow ? 3 : 0) + (b->n_prewalk ? 1 : 0);
-  for (int K = 0; K < b->stepnb; K++)
-    launches += (b->panel_cnt[K] > 0) + (b->t128_cnt[K] > 0) + (b->t64_cnt[K] > 0) +
-                (b->tri128_off[K + 1] > b->tri128_off[K]) + (b->tri64_off[K + 1] > b->tri64_off[K]);
+  const int64_t launches = 1 + (b->n_rows ? 5 : 0) + batch_step_launches(b);
   info[0] = b->count;
   info[1] = b->maxnb;
   info[2] = launches;
@@ -682,7 +753,7 @@ int rbg_batch_info(const rbg_batch* b, int64_t* info) {
   info[4] = b->n_t128 + b->n_tri128;
   info[5] = b->n_t64 + b->n_tri64;
   info[6] = b->n_chunk;
-  info[7] = b->exec != nullptr;
+  info[7] = b->exec[0] != nullptr;
   info[8] = b->n_flow;
   info[9] = b->classes.total;
   return 0;
@@ -690,7 +761,16 @@ int rbg_batch_info(const rbg_batch* b, int64_t* info) {
 
 int rbg_batch_run(rbg_batch* b, rbg_stream_t stream) {
   if (!b) return RBG_E_ARG;
-  return batch_launch(b, (hipStream_t)stream);
+  hipStream_t s = (hipStream_t)stream;
+  int rc = batch_init(b, s);
+  if (rc == 0 && batch_tries_rows(b)) {
+    rc = batch_launch_rows(b, s);
+    if (rc == 0 && !stream_captures(s)) {
+      b->runs++;
+      if (batch_rows_told(b)) return 0;
+    }
+  }
+  return rc ? rc : batch_launch_steps(b, s);
 }
 
 int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stream) {
@@ -701,53 +781,65 @@ int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stre
   return e == hipSuccess ? (int)hipStreamSynchronize(s) : (int)e;
 }
 
-int rbg_batch_capture(rbg_batch* b, rbg_stream_t stream) {
-  if (!b || !stream) return RBG_E_ARG;  // the legacy null stream cannot be captured
-  hipStream_t s = (hipStream_t)stream;
-  if (b->exec) {
-    (void)hipGraphExecDestroy(b->exec);
-    (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
+static void batch_drop_graphs(rbg_batch* b) {
+  for (int k = 0; k < 2; k++) {
+    if (b->exec[k]) (void)hipGraphExecDestroy(b->exec[k]);
+    if (b->graph[k]) (void)hipGraphDestroy(b->graph[k]);
+    b->exec[k] = nullptr;
+    b->graph[k] = nullptr;
   }
+}
+
+// part 0: the init and, where rows are tried, their launches; part 1: the
+// others; both in one graph where no rows are tried
+static int batch_capture_part(rbg_batch* b, hipStream_t s, bool rows, int part) {
   hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return (int)e;
-  int rc = batch_launch(b, s);
-  hipGraph_t g = nullptr;
-  e = hipStreamEndCapture(s, &g);
-  if (rc) {
-    if (g) (void)hipGraphDestroy(g);
-    return rc;
-  }
+  int rc = part ? 0 : batch_init(b, s);
+  if (rc == 0 && part == 0 && rows) rc = batch_launch_rows(b, s);
+  if (rc == 0 && (part || !rows)) rc = batch_launch_steps(b, s);
+  e = hipStreamEndCapture(s, &b->graph[part]);
+  if (rc) return rc;
   if (e != hipSuccess) return (int)e;
-  e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    (void)hipGraphDestroy(g);
-    return (int)e;
-  }
-  b->graph = g;
-  return 0;
+  return (int)hipGraphInstantiate(&b->exec[part], b->graph[part], nullptr, nullptr, 0);
+}
+
+int rbg_batch_capture(rbg_batch* b, rbg_stream_t stream) {
+  if (!b || !stream) return RBG_E_ARG;  // the legacy null stream cannot be captured
+  batch_drop_graphs(b);
+  const bool rows = batch_tries_rows(b);
+  int rc = batch_capture_part(b, (hipStream_t)stream, rows, 0);
+  if (rc == 0 && rows) rc = batch_capture_part(b, (hipStream_t)stream, rows, 1);
+  if (rc) batch_drop_graphs(b);
+  return rc;
 }
 
 int rbg_batch_replay(rbg_batch* b, rbg_stream_t stream) {
-  if (!b || !b->exec) return RBG_E_ARG;
-  hipError_t e = hipGraphLaunch(b->exec, (hipStream_t)stream);
-  return e == hipSuccess ? 0 : (int)e;
+  if (!b || !b->exec[0]) return RBG_E_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  hipError_t e = hipGraphLaunch(b->exec[0], s);
+  if (e != hipSuccess || !b->exec[1]) return (int)e;
+  if (!stream_captures(s)) {
+    b->runs++;
+    if (batch_rows_told(b)) return 0;
+  }
+  return (int)hipGraphLaunch(b->exec[1], s);
 }
 
 int rbg_batch_destroy(rbg_batch* b) {
   if (!b) return 0;
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
+  batch_drop_graphs(b);
   (void)hipFree(b->d_comps);
   (void)hipFree(b->d_items);
   (void)hipFree(b->d_rows);
+  (void)hipFree(b->d_runs);
   (void)hipFree(b->d_ritems);
   (void)hipFree(b->d_prewalk);
   (void)hipFree(b->d_flow);
   (void)hipFree(b->d_walk);
   (void)hipFree(b->d_ctl);
   (void)hipFree(b->d_fitems);
+  if (b->told) (void)hipHostFree(b->told);
   delete b;
   return 0;
 }

@@ -56,9 +56,9 @@ template <typename T, bool LARGEST>
 static __global__ __launch_bounds__(ROWS_CLOSE_NT, LARGEST ? 4 : 8) void k_rows_close(RowsWork<T> w, T* W, T* W2,
                                                                                      int64_t ld, int width,
                                                                                      rbg_status* st) {
-  __shared__ CloseShared<T, LARGEST> L;
+  __shared__ CloseShared<T, LARGEST, false> L;
   if (LARGEST ? w.ctl[0] < 2 : w.ctl[0] != 1) return;
-  rows_close_slab<T, 1, LARGEST>(L, w, W, W2, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
+  rows_close_slab<T, 1, LARGEST, false>(L, w, W, W2, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
 }
 
 // The slab's cells whose largest path value is above the largest final value.
