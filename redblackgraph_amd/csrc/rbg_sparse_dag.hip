@@ -1109,10 +1109,19 @@ __global__ __launch_bounds__(64) void k_lvl_units(const int32_t* __restrict__ in
     int totc, totl;
     const int pc = wave_excl_scan(cw, lane, totc) + cw;  // inclusive prefixes
     const int pl = wave_excl_scan(lw, lane, totl) + lw;
+    // a unit ends before a long row: its rows land from the unit's first
+    // reserved entry on, and would run into the long row's own range
+    const uint64_t longs = __ballot(lng);
     int s0 = 0;
     while (s0 < m) {
+      if ((longs >> s0) & 1) {
+        s0++;
+        continue;
+      }
+      const uint64_t after = longs >> s0;
+      const int stop = after ? s0 + __builtin_ctzll(after) : m;
       const int bc = s0 > 0 ? __shfl(pc, s0 - 1) : 0, bl = s0 > 0 ? __shfl(pl, s0 - 1) : 0;
-      const uint64_t fit = __ballot(lane >= s0 && lane < m && pc - bc <= LU_CAND && pl - bl <= LU_LISTS);
+      const uint64_t fit = __ballot(lane >= s0 && lane < stop && pc - bc <= LU_CAND && pl - bl <= LU_LISTS);
       const int e = fit ? 63 - __builtin_clzll(fit) : s0;  // last row of the sub-unit (a row always fits)
       const int mu = e - s0 + 1;
       // rows s0..e to lanes 0..mu-1
