@@ -439,6 +439,14 @@ int rbg_dag_gather_i32(void *workspace, int32_t n, const int32_t *arena_cols, co
 int rbg_dag_gather_i64(void *workspace, int32_t n, const int32_t *arena_cols, const int64_t *arena_vals,
                        int64_t *out_indptr, int32_t *out_indices, int64_t *out_data, int64_t out_cap,
                        rbg_status *st, rbg_stream_t stream);
+/* The rows alone, behind a gather that wrote out_indptr only (its size is known
+ * by then): out_cap entries of room, RBG_F_CAPACITY in st where they need more. */
+int rbg_dag_copy_rows_i32(void *workspace, int32_t n, const int32_t *arena_cols, const int32_t *arena_vals,
+                          const int64_t *out_indptr, int32_t *out_indices, int32_t *out_data, int64_t out_cap,
+                          rbg_status *st, rbg_stream_t stream);
+int rbg_dag_copy_rows_i64(void *workspace, int32_t n, const int32_t *arena_cols, const int64_t *arena_vals,
+                          const int64_t *out_indptr, int32_t *out_indices, int64_t *out_data, int64_t out_cap,
+                          rbg_status *st, rbg_stream_t stream);
 
 /* ---- AVOS SpGEMM (sparse/sparsetools/rbm_math.h:116-222, gpu/spgemm*.py) ---------- */
 /* Rows of C = A (x) B into the row arena (rbg_dag_workspace_bytes(m) workspace,

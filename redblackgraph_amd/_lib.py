@@ -112,6 +112,8 @@ SIGNATURES = {
     "rbg_dag_closure_i64": (I32, [P, P, P, I32, P, I64, P, P, I64, I32, P, I32, P, P]),
     "rbg_topological_sort": (I32, [P, P, I32, P, I64, P, P, P, P]),
     "rbg_csr_triangles": (I32, [P, P, I32, P, P]),
+    "rbg_dag_copy_rows_i32": (I32, [P, I32, P, P, P, P, P, I64, P, P]),
+    "rbg_dag_copy_rows_i64": (I32, [P, I32, P, P, P, P, P, I64, P, P]),
     "rbg_dag_gather_i32": (I32, [P, I32, P, P, P, P, P, I64, P, P]),
     "rbg_dag_gather_i64": (I32, [P, I32, P, P, P, P, P, I64, P, P]),
     "rbg_spgemm_rows_i32": (I32, [P, P, P, I32, P, P, P, I32, P, P, P, I64, P, P, I64, I32, I32, P, P]),

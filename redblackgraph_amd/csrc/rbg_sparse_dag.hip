@@ -15,6 +15,10 @@
 //     needs no host round trip; the final CSR is gathered at the end.
 #include "rbg_common.hpp"
 
+#include <chrono>
+#include <mutex>
+#include <vector>
+
 namespace rbg {
 
 constexpr int DAG_WAVES = 4;          // waves per workgroup in the merge kernel
@@ -201,7 +205,7 @@ static int scan_dev(const int64_t* in, int64_t* local, int64_t* sums, const int6
 // ---------------------------------------------------------------------------
 enum {
   C_PLACED = 0,   // vertices placed so far
-  C_UNUSED1 = 1,
+  C_DEEP = 1,     // small graphs: not taken (too deep, a cycle, or a workspace sized without the nnz)
   C_UNUSED2 = 2,
   C_LSTART = 3,   // first index in `order` of the current level (its size: C_PLACED - C_LSTART)
   C_LPREV = 4,    // first index in `order` of the previous level
@@ -1396,23 +1400,295 @@ __global__ __launch_bounds__(64) void k_lvl_pairs(const int32_t* __restrict__ in
   if (evs) atomicOr(&st->events, evs);
 }
 
-// Round r, step 4: the long rows step 3 left, one per workgroup at a time:
-// merged in LDS when they fit (LV_BIG candidates, LV_MAXD direct entries),
-// otherwise in their arena slot from the lists in global memory.
+// A row of one or two successor lists by a workgroup: pair_merge's merge path
+// over LV_NT threads.  Every candidate placed by a binary search in every other
+// list took 113 us a level on average where this takes 100 (n = 1,000,005, the
+// four levels with long rows: 317 us the last, 263 so): bound by the chain of a
+// row's loads, at four workgroups a CU.
+constexpr int PW_R = LV_BIG / LV_NT;  // merged positions per thread
+template <typename T>
+struct PairLds {
+  int32_t c[LV_BIG];
+  T v[LV_BIG];
+  int32_t l0c[LV_MAXD];
+  T l0v[LV_MAXD];
+  T first_v[LV_WAVES];  // each wave's first merged value and column, and its last column
+  int32_t first_c[LV_WAVES], last_c[LV_WAVES];
+  int sum[LV_WAVES];
+  int below[LV_MAXD];  // kept merged entries before each direct entry
+  uint32_t hit;        // direct entries whose column a list holds
+};
+
+template <typename T>
+__device__ inline int pair_merge_wg(const int32_t* __restrict__ indices, const T* __restrict__ data,
+                                    const DagArena<T>& ar, PairLds<T>& L, int64_t e0, int nd, int64_t ro1, int a_len,
+                                    T av1, int64_t ro2, int b_len, T av2, int width, T& cmax, T& fmax,
+                                    uint32_t& evs) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  auto seen = [&](T x) {
+    const T a = x < 0 ? (T)-x : x;
+    cmax = a > cmax ? a : cmax;
+  };
+  auto kept = [&](T x) {
+    const T a = x < 0 ? (T)-x : x;
+    if (a > 1 && a > fmax) fmax = a;
+  };
+  // stage both lists, eight loads in flight per thread
+  {
+    const int m = a_len + b_len;
+    int32_t c[PW_R];
+    T x[PW_R];
+#pragma unroll
+    for (int u = 0; u < PW_R; u++) {
+      const int q = tid + u * LV_NT;
+      if (q < m) {
+        const int64_t o = q < a_len ? ro1 + q : ro2 + (q - a_len);
+        c[u] = ar.cols[o];
+        x[u] = ar.vals[o];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PW_R; u++) {
+      const int q = tid + u * LV_NT;
+      if (q < m) {
+        uint32_t ev = 0;
+        const T y = avos_product<T>(q < a_len ? av1 : av2, x[u], width, false, ev);
+        evs |= ev;
+        L.c[q] = c[u];
+        L.v[q] = y;
+        seen(y);
+      }
+    }
+  }
+  if (tid < nd) {
+    L.l0c[tid] = indices[e0 + tid];
+    const T x = data[e0 + tid];
+    L.l0v[tid] = x;
+    L.below[tid] = 0;
+    seen(x);
+  }
+  if (tid == 0) L.hit = 0;
+  __syncthreads();
+  const int m = a_len + b_len, R = (m + LV_NT - 1) / LV_NT;
+  const int32_t* Bc = L.c + a_len;
+  const T* Bv = L.v + a_len;
+  const int d = tid * R < m ? tid * R : m;
+  int lo = d > b_len ? d - b_len : 0, hi = d < a_len ? d : a_len;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (L.c[mid] <= Bc[d - mid - 1]) lo = mid + 1;
+    else hi = mid;
+  }
+  int i = lo, j = d - lo;
+  int32_t ha = i < a_len ? L.c[i] : INT32_MAX, hb = j < b_len ? Bc[j] : INT32_MAX;
+  const int nv = m - d < R ? m - d : R;
+  int32_t oc[PW_R];
+  T ov[PW_R];
+  int32_t lastc = INT32_MIN;
+#pragma unroll
+  for (int q = 0; q < PW_R; q++) {
+    oc[q] = INT32_MAX;
+    ov[q] = 0;
+    if (q < nv) {
+      if (ha <= hb) {
+        oc[q] = ha;
+        ov[q] = L.v[i];
+        i++;
+        ha = i < a_len ? L.c[i] : INT32_MAX;
+      } else {
+        oc[q] = hb;
+        ov[q] = Bv[j];
+        j++;
+        hb = j < b_len ? Bc[j] : INT32_MAX;
+      }
+      lastc = oc[q];
+    }
+  }
+  if (lane == 0) {
+    L.first_c[wv] = oc[0];
+    L.first_v[wv] = ov[0];
+  }
+  if (lane == 63) L.last_c[wv] = lastc;
+  int32_t prevc = __shfl_up(lastc, 1), nextc = __shfl_down(oc[0], 1);
+  T nextv = __shfl_down(ov[0], 1);
+  __syncthreads();
+  if (lane == 0) prevc = wv > 0 ? L.last_c[wv - 1] : INT32_MIN;
+  if (lane == 63) {
+    nextc = wv + 1 < LV_WAVES ? L.first_c[wv + 1] : INT32_MAX;
+    nextv = wv + 1 < LV_WAVES ? L.first_v[wv + 1] : (T)0;
+  }
+  // of two equal columns the first takes the AVOS sum, the second drops
+  bool keep[PW_R];
+#pragma unroll
+  for (int q = 0; q < PW_R; q++) {
+    const int32_t pc = q == 0 ? prevc : oc[q == 0 ? 0 : q - 1];
+    const bool in = q + 1 < nv;
+    const int32_t nc = in ? oc[q + 1 < PW_R ? q + 1 : q] : nextc;
+    const T nx = in ? ov[q + 1 < PW_R ? q + 1 : q] : nextv;
+    keep[q] = q < nv && pc != oc[q];
+    if (keep[q] && nc == oc[q]) ov[q] = avos_sum<T>(ov[q], nx);
+  }
+  for (int k = 0; k < nd; k++) {
+    const int32_t ck = L.l0c[k];
+#pragma unroll
+    for (int q = 0; q < PW_R; q++)
+      if (keep[q] && oc[q] == ck) {
+        ov[q] = avos_sum<T>(L.l0v[k], ov[q]);
+        atomicOr(&L.hit, 1u << k);
+      }
+  }
+  int mine = 0;
+#pragma unroll
+  for (int q = 0; q < PW_R; q++) {
+    keep[q] = keep[q] && ov[q] != 0;
+    mine += keep[q] ? 1 : 0;
+  }
+  int tot;
+  const int excl = wave_excl_scan(mine, lane, tot);
+  if (lane == 0) L.sum[wv] = tot;
+  for (int k = 0; k < nd; k++) {
+    const int32_t ck = L.l0c[k];
+    int below = 0;
+#pragma unroll
+    for (int q = 0; q < PW_R; q++) below += __popcll(__ballot(keep[q] && oc[q] < ck));
+    if (lane == 0 && below) atomicAdd(&L.below[k], below);
+  }
+  __syncthreads();  // the staged lists are read: the buffers take the merged row
+  uint32_t l0mask = 0;
+  for (int k = 0; k < nd; k++)
+    if (!(L.hit >> k & 1) && L.l0v[k] != 0) l0mask |= 1u << k;
+  int pos = excl, out = __popc(l0mask);
+#pragma unroll
+  for (int w = 0; w < LV_WAVES; w++) {
+    pos += w < wv ? L.sum[w] : 0;
+    out += L.sum[w];
+  }
+#pragma unroll
+  for (int q = 0; q < PW_R; q++) {
+    if (keep[q]) {
+      int p = pos++;
+      for (int k = 0; k < nd; k++)
+        if ((l0mask >> k & 1) && L.l0c[k] < oc[q]) p++;
+      L.c[p] = oc[q];
+      L.v[p] = ov[q];
+      kept(ov[q]);
+    }
+  }
+  if (tid < nd && (l0mask >> tid & 1)) {
+    const int p = __popc(l0mask & ((1u << tid) - 1)) + L.below[tid];
+    L.c[p] = L.l0c[tid];
+    L.v[p] = L.l0v[tid];
+    kept(L.l0v[tid]);
+  }
+  __syncthreads();
+  return out;
+}
+
+// One long row by a workgroup of LV_NT threads: merged in LDS when it fits
+// (LV_BIG candidates, LV_MAXD direct entries), otherwise in its arena slot from
+// the lists in global memory.  S: the row (settled); dst: its reserved range.
+template <typename T>
+union LongLds {
+  struct {
+    int32_t lcol[LV_BIG];
+    int32_t mcol[LV_BIG];
+    T mval[LV_BIG];
+    RowMeta<T> meta;
+    int wsum[LV_WAVES];
+  };
+  PairLds<T> pair;
+};
+
+template <typename T>
+__device__ inline void merge_long_row(const int32_t* __restrict__ indices, const T* __restrict__ data,
+                                      const DagWork& ws, const DagArena<T>& ar, LongLds<T>& L, const SlotRegs& S,
+                                      int64_t dst, int width, T& cmax, T& fmax, uint32_t& evs) {
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t cnt = S.cnt;
+  const bool in_lds = cnt <= LV_BIG && S.nd <= LV_MAXD;
+  if (in_lds && (S.nl == 2 || S.nl == 3)) {
+    const int a_len = lane_i32(S.len, 0), b_len = S.nl > 2 ? lane_i32(S.len, 1) : 0;
+    const int out = pair_merge_wg<T>(indices, data, ar, L.pair, S.e0, S.nd, lane_i64(S.ro, 0), a_len,
+                                     (T)lane_i64(S.av, 0), lane_i64(S.ro, 1), b_len, (T)lane_i64(S.av, 1), width,
+                                     cmax, fmax, evs);
+    for (int q = threadIdx.x; q < out; q += LV_NT) {
+      ar.cols[dst + q] = L.pair.c[q];
+      ar.vals[dst + q] = L.pair.v[q];
+    }
+    if (threadIdx.x == 0) {
+      ws.row_off[S.v] = dst;
+      ws.row_len[S.v] = out;
+    }
+    __syncthreads();  // the next row restages the buffers
+    return;
+  }
+  if (in_lds && wv == 0) put_meta<T>(S, L.meta, lane);
+  __syncthreads();
+  int32_t* mcol = in_lds ? L.mcol : ar.cols + dst;
+  T* mval = in_lds ? L.mval : ar.vals + dst;
+  if (in_lds) {
+    merge_row_lds<T, LV_NT>(indices, data, ar, L.meta, S.e0, (int)cnt, 0, L.lcol, L.mcol, L.mval, threadIdx.x, width,
+                            cmax, evs);
+  } else {
+    RowJob<T> J;
+    J.v = S.v;
+    J.e0 = S.e0;
+    J.e1 = S.e0 + S.nd;
+    J.nd = S.nd;
+    J.cnt = cnt;
+    J.dst = dst;
+    merge_lists<T>(J, indices, data, ws, ar, nullptr, mcol, mval, threadIdx.x, LV_NT, width, cmax, evs);
+  }
+  __syncthreads();
+  int64_t out = 0;
+  for (int64_t b0 = 0; b0 < cnt; b0 += LV_NT) {
+    const int64_t i2 = b0 + threadIdx.x;
+    int32_t c = -1;
+    T val = 0;
+    bool keep = false;
+    if (i2 < cnt) {
+      if (in_lds) {
+        keep = lds_run_head<T>(L.mcol, L.mval, (int)i2, (int)cnt, c, val) && val != 0;
+      } else {
+        c = mcol[i2];
+        val = mval[i2];
+        keep = c >= 0;
+      }
+    }
+    const uint64_t msk = __ballot(keep);
+    if (lane == 0) L.wsum[wv] = __popcll(msk);
+    __syncthreads();
+    int64_t before = 0, total = 0;
+    for (int q = 0; q < LV_WAVES; q++) {
+      before += q < wv ? L.wsum[q] : 0;
+      total += L.wsum[q];
+    }
+    if (keep) {
+      const int64_t o = dst + out + before + __popcll(msk & ((1ull << lane) - 1ull));
+      ar.cols[o] = c;
+      ar.vals[o] = val;
+      const T a = val < 0 ? (T)-val : val;
+      if (a > 1 && a > fmax) fmax = a;
+    }
+    out += total;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    ws.row_off[S.v] = dst;
+    ws.row_len[S.v] = out;
+  }
+}
+
+// Round r, step 4: the long rows step 3 left, one per workgroup at a time.
 template <typename T>
 __global__ __launch_bounds__(LV_NT) void k_lvl_long(const int32_t* __restrict__ indices, const T* __restrict__ data,
                                                     DagWork ws, DagArena<T> ar, int width, rbg_status* st) {
-  __shared__ int32_t s_lcol[LV_BIG];
-  __shared__ int32_t s_mcol[LV_BIG];
-  __shared__ T s_mval[LV_BIG];
-  __shared__ RowMeta<T> s_meta;
-  __shared__ int s_wsum[LV_WAVES];
+  __shared__ LongLds<T> L;
   __shared__ int64_t s_cmax, s_fmax;
   int64_t* ctr = ws.counters;
   if (dag_halted(ctr) || ctr[C_CAP]) return;
   const int64_t nlong = ctr[C_LONG], Ls = ctr[C_PLACED] - ctr[C_LSTART], abase = ctr[C_ARENA];
   if (nlong == 0) return;
-  const int wv = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   if (threadIdx.x == 0) s_cmax = s_fmax = 0;
   T cmax = 0, fmax = 0;
@@ -1422,64 +1698,7 @@ __global__ __launch_bounds__(LV_NT) void k_lvl_long(const int32_t* __restrict__ 
     SlotRegs S;
     load_slot(ws, t, Ls, lane, S);
     settle_slot(S);
-    const int64_t cnt = S.cnt;
-    const int64_t dst = abase + S.seg;
-    const bool in_lds = cnt <= LV_BIG && S.nd <= LV_MAXD;
-    if (in_lds && wv == 0) put_meta<T>(S, s_meta, lane);
-    __syncthreads();
-    int32_t* mcol = in_lds ? s_mcol : ar.cols + dst;
-    T* mval = in_lds ? s_mval : ar.vals + dst;
-    if (in_lds) {
-      merge_row_lds<T, LV_NT>(indices, data, ar, s_meta, S.e0, (int)cnt, 0, s_lcol, s_mcol, s_mval,
-                              threadIdx.x, width, cmax, evs);
-    } else {
-      RowJob<T> J;
-      J.v = S.v;
-      J.e0 = S.e0;
-      J.e1 = S.e0 + S.nd;
-      J.nd = S.nd;
-      J.cnt = cnt;
-      J.dst = dst;
-      merge_lists<T>(J, indices, data, ws, ar, nullptr, mcol, mval, threadIdx.x, LV_NT, width, cmax, evs);
-    }
-    __syncthreads();
-    int64_t out = 0;
-    for (int64_t b0 = 0; b0 < cnt; b0 += LV_NT) {
-      const int64_t i2 = b0 + threadIdx.x;
-      int32_t c = -1;
-      T val = 0;
-      bool keep = false;
-      if (i2 < cnt) {
-        if (in_lds) {
-          keep = lds_run_head<T>(s_mcol, s_mval, (int)i2, (int)cnt, c, val) && val != 0;
-        } else {
-          c = mcol[i2];
-          val = mval[i2];
-          keep = c >= 0;
-        }
-      }
-      const uint64_t msk = __ballot(keep);
-      if (lane == 0) s_wsum[wv] = __popcll(msk);
-      __syncthreads();
-      int64_t before = 0, total = 0;
-      for (int q = 0; q < LV_WAVES; q++) {
-        before += q < wv ? s_wsum[q] : 0;
-        total += s_wsum[q];
-      }
-      if (keep) {
-        const int64_t o = dst + out + before + __popcll(msk & ((1ull << lane) - 1ull));
-        ar.cols[o] = c;
-        ar.vals[o] = val;
-        const T a = val < 0 ? (T)-val : val;
-        if (a > 1 && a > fmax) fmax = a;
-      }
-      out += total;
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      ws.row_off[S.v] = dst;
-      ws.row_len[S.v] = out;
-    }
+    merge_long_row<T>(indices, data, ws, ar, L, S, abase + S.seg, width, cmax, fmax, evs);
   }
   if (cmax) atomicMax((long long*)&s_cmax, (long long)cmax);
   if (fmax) atomicMax((long long*)&s_fmax, (long long)fmax);
@@ -1489,6 +1708,418 @@ __global__ __launch_bounds__(LV_NT) void k_lvl_long(const int32_t* __restrict__ 
     if (s_fmax) atomicMax((long long*)&ctr[C_FMAX], (long long)s_fmax);
   }
   if (evs) atomicOr(&st->events, evs);
+}
+
+__device__ inline void dag_report(const DagWork& ws, rbg_status* st) {
+  const int64_t* c = ws.counters;
+  if (c[C_CAP]) atomicOr(&st->flags, (uint32_t)RBG_F_CAPACITY);
+  st->aux[2] = c[C_CMAX];
+  st->aux[3] = c[C_FMAX];
+  st->aux[4] = c[C_ARENA];
+  st->aux[6] = c[C_NLEV];
+  st->aux[7] = c[C_DONE] && !c[C_CAP] && !c[C_HINT];
+}
+
+// ---- graphs of up to DS_MAX_N vertices --------------------------------------
+// Their closure is bound by launches and their round trips, not by bytes (n =
+// 21,162, 12 levels: some 120 launches and two waits, 1.04 ms, with the rounds
+// above; 0.44 ms so, 65 us of it the levels).  Every level comes first, from one workgroup that holds
+// a byte per vertex in LDS; then each level is one launch, whose workgroups
+// count their rows' candidates, reserve them in the arena with one atomic each
+// and merge.  A larger graph's levels do not fit one workgroup, and its levels
+// have rows enough to fill the launches above.
+constexpr int DS_MAX_N = 32640;
+constexpr int DS_LEVELS = 250;
+constexpr int DS_NT = 1024;
+constexpr int DS_ROWS = 64;   // rows of a workgroup at a time
+constexpr int DS_GRID = 512;  // two workgroups a CU
+constexpr uint32_t DS_NONE = 0x7fff, DS_MORE = 1u << 31;
+// a level had rows that k_lvl_units, or k_lvl_pairs, would leave to k_lvl_long
+// (the kinds recorded for a plan are the same whatever closed the graph)
+constexpr int DS_LONG_UNITS = 1, DS_LONG_PAIRS = 2;
+struct DsHints {
+  uint8_t kind[DS_LEVELS];
+  uint8_t given;
+};
+
+// Clears the counters and packs each row's first two non-self successors into
+// a word for the levels (ws.rem[0]).
+__global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ indptr,
+                                                 const int32_t* __restrict__ indices, DagWork ws, int32_t n) {
+  const int32_t v = blockIdx.x * 256 + threadIdx.x;
+  if (v < C_NCTR) {
+    // a workspace without room for the predecessor lists is left to the rounds, which refuse it
+    ws.counters[v] = v == C_CYCV ? -1 : v == C_DEEP ? indptr[n] > ws.ecap : 0;
+  }
+  if (v >= n) return;
+  uint32_t c[2] = {DS_NONE, DS_NONE};
+  int k = 0;
+  for (int64_t e = indptr[v], e1 = indptr[v + 1]; e < e1; e++) {
+    const int32_t w = indices[e];
+    if (w == v) continue;
+    if (k == 2) {
+      k++;
+      break;
+    }
+    c[k++] = (uint32_t)w;
+  }
+  ((uint32_t*)ws.rem[0])[v] = c[0] | c[1] << 15 | (k > 2 ? DS_MORE : 0);
+  ws.row_len[v] = 0;  // a row that is not reached has no entries
+  ws.cnt[v] = 0;      // by level: candidates reserved
+  ws.rem[1][v] = 0;   // by level: DS_LONG_* seen
+  ws.pptr[v] = 0;     // by workgroup: largest candidate, largest final value
+  if (v == n - 1) ws.pptr[n] = 0;
+}
+
+// Levels by sweeps over the rows, each row's level one above its highest
+// successor's, until none changes (a thread's rows see each other's news at
+// once).  Writes `order` by level and each level's first place (cand_loc).
+// C_DEEP where a level passes DS_LEVELS: too deep, or a cycle.
+template <int H>
+__global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__ indptr,
+                                                     const int32_t* __restrict__ indices, DagWork ws, int32_t n,
+                                                     int64_t* told) {
+  __shared__ __align__(16) uint8_t lev[4 * H * DS_NT + 16];
+  __shared__ int marks[4];  // of this sweep, read after its barrier; two sweeps on it is reused
+  __shared__ int hist[256], next[256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto tell = [&](int64_t levels) {
+    if (told) __hip_atomic_store(told, levels, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  if (ws.counters[C_DEEP]) {  // uniform: written by an earlier launch
+    if (tid == 0) tell(-1);
+    return;
+  }
+  if (tid < 4) marks[tid] = 0;
+  if (tid < 256) hist[tid] = 0;
+  uint32_t e[4 * H], lv[H];
+#pragma unroll
+  for (int h = 0; h < H; h++) {
+    const int row = 4 * (h * DS_NT + tid);
+    uint4 q = make_uint4(0, 0, 0, 0);
+    if (row < n) q = *(const uint4*)((const uint32_t*)ws.rem[0] + row);  // padded to 256 bytes
+    e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
+    *(uint32_t*)(lev + row) = 0;
+    lv[h] = 0;
+  }
+#pragma unroll
+  for (int x = 0; x < 4 * H; x++) {
+    const int row = 4 * ((x / 4) * DS_NT + tid) + x % 4;
+    if (row >= n) e[x] = DS_NONE | DS_NONE << 15;
+    const uint32_t c0 = e[x] & 0x7fff, c1 = (e[x] >> 15) & 0x7fff;
+    e[x] = (c0 == DS_NONE ? (uint32_t)n : c0) | (c1 == DS_NONE ? (uint32_t)n : c1) << 15 | (e[x] & DS_MORE);
+  }
+  __syncthreads();
+  if (tid == 0) lev[n] = 255;  // an absent successor's level: below 0
+  __syncthreads();
+  for (int it = 0;; it++) {
+    bool changed = false;
+    int worst = 0;
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+      if (4 * h * DS_NT >= n) continue;
+      // after s sweeps a level is at least min(s, the final one): smaller ones are final
+      if ((lv[h] & 0xff) < (uint32_t)it && (lv[h] >> 8 & 0xff) < (uint32_t)it && (lv[h] >> 16 & 0xff) < (uint32_t)it &&
+          lv[h] >> 24 < (uint32_t)it)
+        continue;
+      const int row = 4 * (h * DS_NT + tid);
+      uint32_t nv = 0;
+#pragma unroll
+      for (int x = 0; x < 4; x++) {
+        const uint32_t ex = e[4 * h + x];
+        const int l0 = (uint8_t)(lev[ex & 0x7fff] + 1), l1 = (uint8_t)(lev[(ex >> 15) & 0x7fff] + 1);
+        int nl = l0 > l1 ? l0 : l1;
+        if (ex & DS_MORE) {
+          const int v = row + x;
+          for (int64_t k = indptr[v]; k < indptr[v + 1]; k++) {
+            const int w = indices[k];
+            const int y = w == v ? 0 : lev[w] + 1;
+            nl = nl > y ? nl : y;
+          }
+        }
+        worst = nl > worst ? nl : worst;
+        nv |= (uint32_t)nl << (8 * x);
+      }
+      if (nv != lv[h] && row < n) {
+        lv[h] = nv;
+        changed = true;
+        if (row + 3 < n)
+          *(uint32_t*)(lev + row) = nv;
+        else
+          for (int x = 0; row + x < n; x++) lev[row + x] = (uint8_t)(nv >> (8 * x));
+      }
+    }
+    const int mark = (__any(changed) ? 1 : 0) | (__any(worst >= DS_LEVELS) ? 2 : 0);
+    if (mark && lane == 0) atomicOr(&marks[it & 3], mark);
+    if (tid == 0) marks[(it + 2) & 3] = 0;
+    __syncthreads();
+    const int m = marks[it & 3];  // the same for every thread
+    if (m & 2) {
+      if (tid == 0) {
+        ws.counters[C_DEEP] = 1;
+        tell(-1);
+      }
+      return;
+    }
+    if (!(m & 1)) break;
+  }
+  // rows of one level are mostly neighbours: one LDS atomic for all of a wave's
+  // lanes with the first lane's level, and so on
+  auto count = [&](int (&at)[256], int l, bool on) {
+    int place = 0;
+    for (uint64_t left = __ballot(on); left;) {
+      const int first = __builtin_ctzll(left), same = __builtin_amdgcn_readlane(l, first);
+      const uint64_t m = __ballot(on && l == same) & left;
+      int base = 0;
+      if (lane == first) base = atomicAdd(&at[same], __popcll(m));
+      base = __builtin_amdgcn_readlane(base, first);
+      if (on && l == same) place = base + __popcll(m & (((uint64_t)1 << lane) - 1));
+      left &= ~m;
+    }
+    return place;
+  };
+#pragma unroll 1
+  for (int i0 = 0; i0 < n; i0 += DS_NT) count(hist, i0 + tid < n ? lev[i0 + tid] : 0, i0 + tid < n);
+  __syncthreads();
+  if (tid < 64) {
+    int c[4], mine = 0;
+    for (int q = 0; q < 4; q++) mine += c[q] = hist[4 * lane + q];
+    int incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    int at = incl - mine;
+    for (int q = 0; q < 4; q++) {  // level L ends where L + 1 begins; no level is empty below the last
+      next[4 * lane + q] = at;
+      if (c[q]) {
+        ws.cand_loc[4 * lane + q] = at;
+        ws.cand_loc[4 * lane + q + 1] = at + c[q];
+        if (at + c[q] == n) {
+          ws.counters[C_NLEV] = 4 * lane + q + 1;
+          tell(4 * lane + q + 1);
+        }
+      }
+      at += c[q];
+    }
+    if (lane == 0) ws.counters[C_PLACED] = n;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int i0 = 0; i0 < n; i0 += DS_NT) {
+    const int i = i0 + tid;
+    const int at = count(next, i < n ? lev[i] : 0, i < n);
+    if (i < n) ws.order[at] = i;
+  }
+}
+
+// Level r: DS_ROWS rows or fewer per workgroup at a time, a quarter of them a
+// wave's (merge_unit), long rows by the whole workgroup behind them.
+template <typename T>
+__global__ __launch_bounds__(LV_NT) void k_ds_level(const int64_t* __restrict__ indptr,
+                                                    const int32_t* __restrict__ indices, const T* __restrict__ data,
+                                                    DagWork ws, DagArena<T> ar, int32_t r, int width,
+                                                    rbg_status* st) {
+  union Lds {
+    UnitLds<T> unit[LV_WAVES];
+    LongLds<T> row;
+  };
+  __shared__ Lds L;
+  __shared__ int32_t s_v[DS_ROWS], s_nd[DS_ROWS], s_nl[DS_ROWS];
+  __shared__ int64_t s_e0[DS_ROWS], s_cnt[DS_ROWS], s_seg[DS_ROWS];
+  __shared__ uint64_t s_long;
+  __shared__ int64_t s_base;
+  __shared__ long long s_cmax, s_fmax;
+  __shared__ int s_halt;
+  int64_t* ctr = ws.counters;
+  if (threadIdx.x == 0) s_halt = (ctr[C_DEEP] | ctr[C_CAP]) != 0 || r >= ctr[C_NLEV];
+  __syncthreads();
+  if (s_halt) return;
+  const int64_t l0 = ws.cand_loc[r], Ls = ws.cand_loc[r + 1] - l0;
+  const int tid = threadIdx.x, lane = tid & 63, wv = uni(tid >> 6);
+  if (tid == 0) s_cmax = s_fmax = 0;
+  T cmax = 0, fmax = 0;
+  uint32_t evs = 0;
+  // rows of a workgroup: the level is shared by as many of them as run at once
+  // where the level below had long rows (last levels of n = 21,162: 34 us, with
+  // half as many 47), else by half as many (11 us, 15 with all: each reserves
+  // its candidates by one atomic, one after another)
+  const bool fine = r > 0 && ws.cnt[r - 1] > 48 * (l0 - ws.cand_loc[r - 1]);
+  const int parts = fine ? DS_GRID : DS_GRID / 2;
+  int R = (int)((Ls + parts - 1) / parts);
+  R = R < LV_WAVES ? LV_WAVES : (R > DS_ROWS ? DS_ROWS : R);
+  const int64_t nch = (Ls + R - 1) / R;
+  int64_t lbase = 0;  // the level's first arena entry
+  if (wv == 0) {
+    for (int q = lane; q < r; q += 64) lbase += ws.cnt[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) lbase += __shfl_xor(lbase, o);
+  }
+  for (int64_t ch = blockIdx.x; ch < nch; ch += gridDim.x) {
+    const int64_t t0 = l0 + ch * R;
+    const int m = (int)(l0 + Ls - t0 < R ? l0 + Ls - t0 : R);
+    if (wv == 0) {
+      int64_t c = 0;
+      int32_t nd = 0, k = 0;
+      if (lane < m) {
+        const int64_t t = t0 + lane;
+        const int32_t v = ws.order[t];
+        const int64_t e0 = indptr[v], e1 = indptr[v + 1];
+        nd = (int32_t)(e1 - e0);
+        const bool keep = nd <= DagWork::SLOT_D;
+        for (int64_t e = e0; e < e1; e++) {
+          const int32_t w = indices[e];
+          c++;
+          if (w == v) continue;
+          const int64_t len = ws.row_len[w];
+          c += len;
+          if (keep) {
+            ws.slot_ro[t * DagWork::SLOT_D + k] = ws.row_off[w];
+            ws.slot_len[t * DagWork::SLOT_D + k] = (int32_t)len;
+            ws.slot_av[t * DagWork::SLOT_D + k] = (int64_t)data[e];
+          }
+          k++;
+        }
+        s_v[lane] = v;
+        s_nd[lane] = nd;
+        s_nl[lane] = 1 + k;
+        s_e0[lane] = e0;
+        s_cnt[lane] = c;
+      }
+      int64_t incl = c;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int64_t u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
+      }
+      if (lane < m) s_seg[lane] = incl - c;
+      const uint64_t lng = __ballot(lane < m && (nd > LV_MAXD || c > LU_CAND));
+      const bool lngp = __any(lane < m && (k < 1 || k > 2 || nd > LV_MAXD || c > LV_SMALL));
+      if (lane == 0 && (lng || lngp)) atomicOr(&ws.rem[1][r], (lng ? DS_LONG_UNITS : 0) | (lngp ? DS_LONG_PAIRS : 0));
+      if (lane == 63) {  // the workgroup's candidates
+        const int64_t base = lbase + (int64_t)atomicAdd((unsigned long long*)&ws.cnt[r], (unsigned long long)incl);
+        const bool fits = base + incl <= ar.cap;
+        if (!fits) ctr[C_CAP] = 1;
+        s_base = fits ? base : -1;
+        s_long = lng;
+      }
+    }
+    __syncthreads();
+    const int64_t abase = s_base;
+    const uint64_t longs = s_long;
+    if (abase >= 0) {
+      const int q = (m + LV_WAVES - 1) / LV_WAVES, b = wv * q, mw = m - b < q ? m - b : q;
+      if (mw > 0) {  // rows b ... b + mw - 1, row b + lane in lane `lane`
+        const int j = b + (lane < mw ? lane : 0);
+        const int64_t t = t0 + j, e0 = s_e0[j], seg = s_seg[j];
+        const int32_t v = s_v[j], nd = s_nd[j], nl = s_nl[j];
+        const uint64_t own = longs >> b;
+        const bool mine = lane < mw && !((own >> lane) & 1);
+        const int cw = mine ? (int)s_cnt[j] : 0, lw = mine ? nl : 0;
+        int totc, totl;
+        const int pc = wave_excl_scan(cw, lane, totc) + cw;
+        const int pl = wave_excl_scan(lw, lane, totl) + lw;
+        int s0 = 0;
+        while (s0 < mw) {  // units of consecutive rows, as in k_lvl_units
+          if ((own >> s0) & 1) {
+            s0++;
+            continue;
+          }
+          const uint64_t after = own >> s0;
+          const int nextlong = after ? s0 + __builtin_ctzll(after) : mw;
+          const int stop = nextlong < mw ? nextlong : mw;
+          const int bc = s0 > 0 ? __shfl(pc, s0 - 1) : 0, bl = s0 > 0 ? __shfl(pl, s0 - 1) : 0;
+          const uint64_t fit = __ballot(lane >= s0 && lane < stop && pc - bc <= LU_CAND && pl - bl <= LU_LISTS);
+          const int e = fit ? 63 - __builtin_clzll(fit) : s0;
+          const int src = s0 + lane < 64 ? s0 + lane : 63;
+          const int64_t tu = __shfl(t, src), e0u = __shfl(e0, src), cu = __shfl((int64_t)cw, src);
+          const int32_t vu = __shfl(v, src), ndu = __shfl(nd, src), nlu = __shfl(lw, src);
+          const int64_t segu = __shfl(seg, s0);
+          merge_unit<T>(indices, data, ws, ar, L.unit[wv], lane, e - s0 + 1, tu, vu, e0u, ndu, nlu, cu,
+                        __shfl(pc, e) - bc, __shfl(pl, e) - bl, abase + segu, width, cmax, fmax, evs);
+          s0 = e + 1;
+        }
+      }
+      for (uint64_t left = longs; left; left &= left - 1) {
+        const int j = __builtin_ctzll(left);
+        __syncthreads();  // the units' and the last long row's buffers
+        SlotRegs S;
+        S.v = s_v[j];
+        S.nd = s_nd[j];
+        S.nl = s_nl[j];
+        S.e0 = s_e0[j];
+        S.seg = s_seg[j];
+        S.cnt = s_cnt[j];
+        S.ro = S.av = 0;
+        S.len = 0;
+        if (lane < DagWork::SLOT_D && lane + 1 < S.nl && S.nd <= DagWork::SLOT_D) {
+          const int64_t k = (t0 + j) * DagWork::SLOT_D + lane;
+          S.ro = ws.slot_ro[k];
+          S.len = ws.slot_len[k];
+          S.av = ws.slot_av[k];
+        }
+        merge_long_row<T>(indices, data, ws, ar, L.row, S, abase + S.seg, width, cmax, fmax, evs);
+      }
+    }
+    __syncthreads();  // the next rows' tables
+  }
+  const long long wc = wave_max_i64((int64_t)cmax), wf = wave_max_i64((int64_t)fmax);
+  if (lane == 0 && wc > 0) atomicMax(&s_cmax, wc);
+  if (lane == 0 && wf > 0) atomicMax(&s_fmax, wf);
+  __syncthreads();
+  if (tid == 0) {
+    // the workgroup's own places, no atomics: every workgroup of a level may find
+    // larger values than the levels below
+    int64_t* top = ws.pptr + 2 * blockIdx.x;
+    if (s_cmax > top[0]) top[0] = s_cmax;
+    if (s_fmax > top[1]) top[1] = s_fmax;
+    if (blockIdx.x == 0 && r + 1 == ctr[C_NLEV]) ctr[C_DONE] = 1;
+  }
+  if (evs) atomicOr(&st->events, evs);
+}
+
+// The report, one thread per level: the arena's total, the levels' kinds, and
+// as the rounds would, a hint that left out what a level needs.
+__global__ __launch_bounds__(256) void k_ds_report(DagWork ws, int groups, DsHints hints, rbg_status* st) {
+  __shared__ unsigned long long s_arena;
+  __shared__ long long s_cmax, s_fmax;
+  __shared__ int s_wrong;
+  const int r = threadIdx.x, nlev = (int)ws.counters[C_NLEV];
+  if (r == 0) {
+    s_arena = 0;
+    s_cmax = s_fmax = 0;
+    s_wrong = 0;
+  }
+  __syncthreads();
+  long long cmax = 0, fmax = 0;
+  for (int b = r; b < groups; b += 256) {
+    const long long c = ws.pptr[2 * b], f = ws.pptr[2 * b + 1];
+    cmax = c > cmax ? c : cmax;
+    fmax = f > fmax ? f : fmax;
+  }
+  cmax = wave_max_i64(cmax);
+  fmax = wave_max_i64(fmax);
+  if ((r & 63) == 0) {
+    atomicMax(&s_cmax, cmax);
+    atomicMax(&s_fmax, fmax);
+  }
+  if (r < nlev && r < DS_LEVELS) {
+    const int64_t Ls = ws.cand_loc[r + 1] - ws.cand_loc[r], M = ws.cnt[r];
+    const bool units = (M + Ls - 1) / Ls <= LU_ROWS_MEAN;
+    const int kind = (units ? LK_UNITS : 0) | (ws.rem[1][r] & (units ? DS_LONG_UNITS : DS_LONG_PAIRS) ? LK_LONG : 0);
+    ws.kinds[r] = (uint8_t)kind;
+    const int hint = hints.kind[r];
+    if (hints.given && ((kind & LK_UNITS) != (hint & LK_UNITS) || (kind & ~hint & LK_LONG))) s_wrong = 1;
+    atomicAdd(&s_arena, (unsigned long long)M);
+  }
+  __syncthreads();
+  if (r == 0) {
+    ws.counters[C_ARENA] = (int64_t)s_arena;
+    ws.counters[C_CMAX] = s_cmax;
+    ws.counters[C_FMAX] = s_fmax;
+    if (s_wrong) ws.counters[C_HINT] = 1;
+    dag_report(ws, st);
+  }
 }
 
 // Round r, step 5 (single lane): advance the arena, count the level, detect a
@@ -1595,15 +2226,7 @@ __global__ void k_csr_triangles(const int64_t* __restrict__ indptr, const int32_
   }
 }
 
-__global__ void k_dag_report(DagWork ws, rbg_status* st) {
-  const int64_t* c = ws.counters;
-  if (c[C_CAP]) atomicOr(&st->flags, (uint32_t)RBG_F_CAPACITY);
-  st->aux[2] = c[C_CMAX];
-  st->aux[3] = c[C_FMAX];
-  st->aux[4] = c[C_ARENA];
-  st->aux[6] = c[C_NLEV];
-  st->aux[7] = c[C_DONE];
-}
+__global__ void k_dag_report(DagWork ws, rbg_status* st) { dag_report(ws, st); }
 
 // ---------------------------------------------------------------------------
 // wave-level helpers
@@ -1815,13 +2438,18 @@ __global__ void k_rows_init(int64_t* row_len, int64_t* counters, int32_t n) {
     for (int q = 0; q < C_NCTR; q++) counters[q] = 0;
 }
 
-// Segmented copy into CSR order: one wave moves 64 consecutive output rows,
-// which are contiguous in the output from out_ptr[r0].  Lane j holds row
+// Segmented copy into CSR order: one wave moves GROWS consecutive output rows,
+// which are contiguous in the output from out_ptr[r0] (the rows of the last
+// generations are long and neighbours: with 64, 32, 16, 8 and 4 rows a wave 61,
+// 36, 23, 16 and 15 us for n = 21,162 and 560, 525, 500, 486 and 486 for n =
+// 1,000,005).  Lane j holds row
 // r0 + j's source offset and length; the prefix of the lengths (in LDS) maps
 // every output entry of the group to its row, so stores are fully coalesced
 // and each lane keeps GC entries in flight.  src_of(r) / len_of(r) give a
 // row's source offset and length.
 constexpr int GC = 8;
+constexpr int GROWS = 8;
+
 template <typename T, typename SrcF, typename LenF>
 __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __restrict__ out_ptr, SrcF src_of,
                                      LenF len_of, const int32_t* __restrict__ in_idx, const T* __restrict__ in_val,
@@ -1830,7 +2458,7 @@ __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __res
   const int lane = threadIdx.x & 63;
   const int64_t r = r0 + lane;
   int64_t len = 0, src = 0;
-  if (r < n) {
+  if (lane < GROWS && r < n) {
     len = len_of(r);
     src = src_of(r);
   }
@@ -1880,6 +2508,10 @@ __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __res
 }
 
 constexpr int GATHER_NT = 256;
+static inline unsigned gather_grid(int64_t n) {
+  constexpr int rows = GATHER_NT / 64 * GROWS;
+  return (unsigned)((n + rows - 1) / rows);
+}
 template <typename T>
 __global__ __launch_bounds__(GATHER_NT) void k_dag_gather(const DagWork ws, const DagArena<T> ar,
                                                           const int64_t* __restrict__ out_ptr, int32_t n,
@@ -1892,19 +2524,68 @@ __global__ __launch_bounds__(GATHER_NT) void k_dag_gather(const DagWork ws, cons
     return;
   }
   const int w = threadIdx.x >> 6;
-  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * 64;
+  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * GROWS;
   if (r0 >= n) return;
   seg_copy_rows<T>(
       r0, n, out_ptr, [&](int64_t r) { return ws.row_off[r]; }, [&](int64_t r) { return ws.row_len[r]; }, ar.cols,
       ar.vals, out_idx, out_val, s_pre[w], s_src[w]);
 }
 
-__global__ void k_dag_finish_status(const DagWork ws, rbg_status* st) {
+__device__ inline void dag_status(const DagWork& ws, rbg_status* st) {
   st->aux[1] = ws.counters[C_NNZ];    // nnz of the gathered CSR
   st->aux[2] = ws.counters[C_CMAX];   // max |candidate|
   st->aux[3] = ws.counters[C_FMAX];   // max |final value| > 1
   st->aux[4] = ws.counters[C_ARENA];  // arena entries used
   st->aux[5] = ws.counters[C_TEMP];   // temp arena entries used
+}
+__global__ void k_dag_finish_status(const DagWork ws, rbg_status* st) { dag_status(ws, st); }
+
+// Row pointers and the status of a graph of up to DS_MAX_N rows by one
+// workgroup, in place of five launches.
+__global__ __launch_bounds__(DS_NT) void k_ds_ptr(const DagWork ws, int32_t n, int64_t* __restrict__ out,
+                                                  rbg_status* st) {
+  __shared__ int64_t wsum[DS_NT / 64];
+  constexpr int PASSES = (DS_MAX_N + 4 * DS_NT - 1) / (4 * DS_NT);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int64_t c[PASSES][4];  // every load in flight at once
+#pragma unroll
+  for (int b = 0; b < PASSES; b++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int32_t i = 4 * (b * DS_NT + tid) + q;
+      c[b][q] = i < n ? ws.row_len[i] : 0;
+    }
+  int64_t base = 0;
+#pragma unroll
+  for (int b = 0; b < PASSES; b++) {
+    if (4 * b * DS_NT >= n) break;
+    int64_t incl = c[b][0] + c[b][1] + c[b][2] + c[b][3];
+    const int64_t mine = incl;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t u = __shfl_up(incl, o);
+      if (lane >= o) incl += u;
+    }
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    int64_t at = base + incl - mine;
+    for (int w = 0; w < DS_NT / 64; w++) {
+      if (w < wv) at += wsum[w];
+      base += wsum[w];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int32_t i = 4 * (b * DS_NT + tid) + q;
+      if (i < n) out[i] = at;
+      at += c[b][q];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    out[n] = base;
+    ws.counters[C_NNZ] = base;
+    dag_status(ws, st);
+  }
 }
 
 __global__ void k_copy_i64(const int64_t* src, int64_t* dst, int64_t n) {
@@ -1965,7 +2646,7 @@ __global__ __launch_bounds__(GATHER_NT) void k_csr_compact(const int64_t* __rest
   __shared__ int64_t s_pre[GATHER_NT / 64][65];
   __shared__ int64_t s_src[GATHER_NT / 64][64];
   const int w = threadIdx.x >> 6;
-  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * 64;
+  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * GROWS;
   if (r0 >= n) return;
   seg_copy_rows<T>(
       r0, n, optr, [&](int64_t r) { return indptr[r]; }, [&](int64_t r) { return len[r]; }, idx, val, oidx, oval,
@@ -2042,6 +2723,103 @@ __global__ void k_csr_add_rows(const int64_t* __restrict__ ap, const int32_t* __
 
 using namespace rbg;
 
+// A pinned word that a kernel tells the host something through, without the
+// copy and the wait for the stream (a gap of 60 us in the queue, none so).  Words are kept
+// for the calls to come, no more of them than calls ran at once; a word goes
+// back when its kernel has written it or the stream was waited for.
+struct ToldWord {
+  int64_t* p = nullptr;
+  explicit ToldWord(bool wanted) {
+    if (!wanted) return;
+    {
+      std::lock_guard<std::mutex> g(lock());
+      if (!pool().empty()) {
+        p = pool().back();
+        pool().pop_back();
+      }
+    }
+    if (!p && hipHostMalloc((void**)&p, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+    }
+    if (p) *p = 0;
+  }
+  ~ToldWord() {
+    if (!p) return;
+    std::lock_guard<std::mutex> g(lock());
+    pool().push_back(p);
+  }
+  // what was told, or 0 after 2 ms
+  int64_t wait() const {
+    if (!p) return 0;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+      const int64_t v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+      if (v || std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) return v;
+    }
+  }
+  static std::mutex& lock() {
+    static std::mutex* m = new std::mutex;
+    return *m;
+  }
+  static std::vector<int64_t*>& pool() {
+    static std::vector<int64_t*>* v = new std::vector<int64_t*>;
+    return *v;
+  }
+};
+
+// The closure of a graph of up to DS_MAX_N vertices; *taken = false where its
+// levels are too many, it has a cycle or the workspace has no room for the
+// predecessor lists (known only where the host waits for it: rounds < 0 asks
+// for that many levels without a wait, and leaves C_DONE unset otherwise).
+template <typename T>
+static int dag_small(const int64_t* indptr, const int32_t* indices, const T* data, int32_t n, const DagWork& ws,
+                     const DagArena<T>& ar, int32_t rounds, const uint8_t* kinds, int width, rbg_status* st,
+                     hipStream_t s, bool* taken) {
+  const bool ask = rounds >= 0;
+  ToldWord word(ask);
+  hipLaunchKernelGGL(k_ds_prep, dim3((n + 255) / 256), dim3(256), 0, s, indptr, indices, ws, n);
+  RBG_CHECK_LAUNCH();
+  if (n <= 8 * DS_NT)
+    hipLaunchKernelGGL((k_ds_levels<2>), dim3(1), dim3(DS_NT), 0, s, indptr, indices, ws, n, word.p);
+  else if (n <= 24 * DS_NT)
+    hipLaunchKernelGGL((k_ds_levels<6>), dim3(1), dim3(DS_NT), 0, s, indptr, indices, ws, n, word.p);
+  else
+    hipLaunchKernelGGL((k_ds_levels<8>), dim3(1), dim3(DS_NT), 0, s, indptr, indices, ws, n, word.p);
+  RBG_CHECK_LAUNCH();
+  int64_t levels = -(int64_t)rounds;
+  if (ask) {
+    levels = word.wait();
+    if (levels == 0) {  // no word yet: the stream is busy
+      int64_t host[C_NCTR];
+      hipError_t e = hipMemcpyAsync(host, ws.counters, sizeof(host), hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e != hipSuccess) return (int)e;
+      levels = host[C_DEEP] ? -1 : host[C_NLEV];
+    }
+    if (levels < 0) {
+      *taken = false;
+      return 0;
+    }
+  }
+  *taken = true;
+  const int grid = (n + LV_WAVES - 1) / LV_WAVES < DS_GRID ? (n + LV_WAVES - 1) / LV_WAVES : DS_GRID;
+  for (int64_t r = 0; r < levels && r < DS_LEVELS; r++) {
+    int pi = prof_start(s);
+    hipLaunchKernelGGL((k_ds_level<T>), dim3(grid), dim3(LV_NT), 0, s, indptr, indices, data, ws, ar, (int32_t)r,
+                       width, st);
+    RBG_CHECK_LAUNCH();
+    prof_stop(2, pi, s);
+  }
+  DsHints hints{};
+  hints.given = rounds < 0 && kinds;
+  if (hints.given)
+    for (int64_t r = 0; r < levels && r < DS_LEVELS; r++) hints.kind[r] = kinds[r];
+  hipLaunchKernelGGL(k_ds_report, dim3(1), dim3(256), 0, s, ws, grid, hints, st);
+  RBG_CHECK_LAUNCH();
+  return 0;
+}
+
 extern "C" {
 
 int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(n > 0 ? n : 1, nnz); }
@@ -2059,6 +2837,12 @@ int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(
     DagWork ws = DagWork::carve(workspace, n);                                                                  \
     ws.ecap = ((char*)workspace + ws_bytes - (char*)ws.preds) / 4;                                              \
     DagArena<T> ar{arena_cols, arena_vals, arena_cap};                                                          \
+    if (n <= DS_MAX_N) {                                                                                        \
+      bool taken = false;                                                                                       \
+      const int rc = dag_small<T>(indptr, indices, data, n, ws, ar, exact ? batch : 0, level_kinds, width, st, \
+                                   s, &taken);                                                                  \
+      if (rc || taken) return rc;                                                                               \
+    }                                                                                                           \
     hipLaunchKernelGGL(k_dag_init, dim3((n + 255) / 256), dim3(256), 0, s, ws, n);                              \
     RBG_CHECK_LAUNCH();                                                                                         \
     const int gv = (int)((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048);                                      \
@@ -2117,6 +2901,19 @@ int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(
     RBG_CHECK_LAUNCH();                                                                                         \
     return 0;                                                                                                   \
   }                                                                                                             \
+  int rbg_dag_copy_rows_##SUF(void* workspace, int32_t n, const int32_t* arena_cols, const T* arena_vals,       \
+                              const int64_t* out_indptr, int32_t* out_indices, T* out_data, int64_t out_cap,    \
+                              rbg_status* st, rbg_stream_t stream) {                                            \
+    if (n <= 0 || !workspace || !out_indptr || out_cap < 0) return RBG_E_ARG;                                   \
+    if (out_cap == 0) return 0;                                                                                 \
+    if (!out_indices || !out_data) return RBG_E_ARG;                                                            \
+    DagWork ws = DagWork::carve(workspace, n);                                                                  \
+    DagArena<T> ar{(int32_t*)arena_cols, (T*)arena_vals, 0};                                                    \
+    hipLaunchKernelGGL((k_dag_gather<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0,            \
+                       (hipStream_t)stream, ws, ar, out_indptr, n, out_indices, out_data, out_cap, st);         \
+    RBG_CHECK_LAUNCH();                                                                                         \
+    return 0;                                                                                                   \
+  }                                                                                                             \
   int rbg_dag_gather_##SUF(void* workspace, int32_t n, const int32_t* arena_cols, const T* arena_vals,          \
                            int64_t* out_indptr, int32_t* out_indices, T* out_data, int64_t out_cap,             \
                            rbg_status* st, rbg_stream_t stream) {                                               \
@@ -2124,18 +2921,25 @@ int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(
     if (n <= 0 || !workspace || !out_indptr) return RBG_E_ARG;                                                  \
     DagWork ws = DagWork::carve(workspace, n);                                                                  \
     DagArena<T> ar{(int32_t*)arena_cols, (T*)arena_vals, 0};                                                    \
-    int rc = scan_exclusive(ws.row_len, out_indptr, n, ws.sums_a, ws.counters + C_NNZ, s);                      \
-    if (rc) return rc;                                                                                          \
-    hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n,                              \
-                       (const int64_t*)(ws.counters + C_NNZ));                                                  \
-    RBG_CHECK_LAUNCH();                                                                                         \
+    if (n <= DS_MAX_N) {                                                                                        \
+      hipLaunchKernelGGL(k_ds_ptr, dim3(1), dim3(DS_NT), 0, s, ws, n, out_indptr, st);                          \
+      RBG_CHECK_LAUNCH();                                                                                       \
+    } else {                                                                                                    \
+      int rc = scan_exclusive(ws.row_len, out_indptr, n, ws.sums_a, ws.counters + C_NNZ, s);                    \
+      if (rc) return rc;                                                                                        \
+      hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n,                            \
+                         (const int64_t*)(ws.counters + C_NNZ));                                                \
+      RBG_CHECK_LAUNCH();                                                                                       \
+    }                                                                                                           \
     if (out_indices && out_data) {                                                                              \
-      hipLaunchKernelGGL((k_dag_gather<T>), dim3((n + GATHER_NT - 1) / GATHER_NT), dim3(GATHER_NT), 0, s, ws, ar, \
+      hipLaunchKernelGGL((k_dag_gather<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s, ws, ar, \
                          (const int64_t*)out_indptr, n, out_indices, out_data, out_cap, st);                    \
       RBG_CHECK_LAUNCH();                                                                                       \
     }                                                                                                           \
-    hipLaunchKernelGGL(k_dag_finish_status, dim3(1), dim3(1), 0, s, ws, st);                                     \
-    RBG_CHECK_LAUNCH();                                                                                         \
+    if (n > DS_MAX_N) {                                                                                         \
+      hipLaunchKernelGGL(k_dag_finish_status, dim3(1), dim3(1), 0, s, ws, st);                                  \
+      RBG_CHECK_LAUNCH();                                                                                       \
+    }                                                                                                           \
     return 0;                                                                                                   \
   }
 
@@ -2229,7 +3033,7 @@ int64_t rbg_csr_tmp_bytes(int32_t n) { return 8 * ((int64_t)n + 1) + 8 * ((int64
     hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n, (const int64_t*)total);      \
     RBG_CHECK_LAUNCH();                                                                                         \
     if (out_idx && out_val) {                                                                                   \
-      hipLaunchKernelGGL((k_csr_compact<T>), dim3((n + GATHER_NT - 1) / GATHER_NT), dim3(GATHER_NT), 0, s, indptr, (const int32_t*)idx,     \
+      hipLaunchKernelGGL((k_csr_compact<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s, indptr, (const int32_t*)idx,     \
                          (const T*)val, (const int64_t*)len, (const int64_t*)out_indptr, n, out_idx, out_val);   \
       RBG_CHECK_LAUNCH();                                                                                       \
     }                                                                                                           \
@@ -2308,7 +3112,7 @@ extern "C" {
     hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n, (const int64_t*)total);      \
     RBG_CHECK_LAUNCH();                                                                                         \
     if (out_idx && out_val) {                                                                                   \
-      hipLaunchKernelGGL((k_csr_compact<T>), dim3((n + GATHER_NT - 1) / GATHER_NT), dim3(GATHER_NT), 0, s,          \
+      hipLaunchKernelGGL((k_csr_compact<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s,          \
                          cat_ptr, (const int32_t*)cat_idx,                                                      \
                          (const T*)cat_val, (const int64_t*)len, (const int64_t*)out_indptr, n, out_idx, out_val); \
       RBG_CHECK_LAUNCH();                                                                                       \

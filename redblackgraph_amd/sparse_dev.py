@@ -217,7 +217,7 @@ def dag_closure(A: DevCSR, width: int | None = None, stream=None, plan: DagPlan 
         else:
             oi = t.empty(nnz, dtype=t.int32, device=dev)
             ov = t.empty(nnz, dtype=vdt, device=dev)
-            _lib.call(f"rbg_dag_gather_{sfx}", _lib.ptr(plan.ws), n, _lib.ptr(plan.arena_cols),
+            _lib.call(f"rbg_dag_copy_rows_{sfx}", _lib.ptr(plan.ws), n, _lib.ptr(plan.arena_cols),
                       _lib.ptr(plan.arena_vals), _lib.ptr(optr), _lib.ptr(oi), _lib.ptr(ov), nnz, st.p, sh)
         info.nnz = nnz
         return DevCSR(optr, oi, ov, A.shape), info
@@ -268,7 +268,7 @@ def spgemm(A: DevCSR, B: DevCSR, mask_upper: bool = False, width: int | None = N
     nnz = int(s.aux[1])
     oi = t.empty(nnz, dtype=t.int32, device=dev)
     ov = t.empty(nnz, dtype=vdt, device=dev)
-    _lib.call(f"rbg_dag_gather_{sfx}", _lib.ptr(ws), m, _lib.ptr(ac), _lib.ptr(av), _lib.ptr(optr), _lib.ptr(oi),
+    _lib.call(f"rbg_dag_copy_rows_{sfx}", _lib.ptr(ws), m, _lib.ptr(ac), _lib.ptr(av), _lib.ptr(optr), _lib.ptr(oi),
               _lib.ptr(ov), nnz, st.p, sh)
     s = st.read(stream)
     return DevCSR(optr, oi, ov, (m, B.shape[1])), int(s.events)

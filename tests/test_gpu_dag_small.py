@@ -44,3 +44,118 @@ def test_long_rows_between_short_ones(orc, vdt, n):
     info = _check(orc, S, vdt)
     assert info.nlevels == 2 and info.cycle_vertex == -1
 
+
+def _layered(n, per, fan, rng, values=(2, 4)):
+    """Vertices numbered sinks first, `per` a level, `fan` successors in the
+    level below, and a diagonal."""
+    rows, cols = [np.arange(n)], [np.arange(n)]
+    v = np.arange(per, n)
+    for _ in range(fan):
+        rows.append(v)
+        cols.append((v // per - 1) * per + rng.integers(0, per, v.size))
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    _, first = np.unique(r * n + c, return_index=True)
+    r, c = r[first], c[first]
+    return sp.csr_matrix((np.where(r == c, rng.choice([-1, 1], r.size), rng.integers(*values, r.size)), (r, c)),
+                         shape=(n, n))
+
+
+@pytest.mark.parametrize("vdt", [np.int32, np.int64])
+@pytest.mark.parametrize("n,per,fan", [(1, 1, 1), (5, 1, 1), (63, 9, 1), (1000, 100, 3), (8192, 2048, 2),
+                                       (8193, 2048, 2), (32_640, 5000, 2), (32_641, 5000, 2), (900, 90, 9)])
+def test_sizes_of_the_one_workgroup_levels(orc, vdt, n, per, fan):
+    S = _layered(n, per, fan, np.random.default_rng(n))
+    info = _check(orc, S, vdt)
+    assert info.nlevels == -(-n // per)
+    perm = np.random.default_rng(1).permutation(n)  # any numbering
+    _check(orc, S[perm][:, perm], vdt)
+
+
+@pytest.mark.parametrize("levels", [249, 250, 251, 300])
+def test_levels_past_the_one_workgroup_limit(orc, levels):
+    """Deeper graphs take the rounds, with a plan (no wait) as without."""
+    n = 3 * levels  # three chains of ones: no product grows
+    v = np.arange(3, n)
+    S = sp.csr_matrix((np.ones(v.size, np.int64), (v, v - 3)), shape=(n, n))
+    A = sd.canonicalize(sd.from_scipy(S.astype(np.int64), np.int64))
+    plan = sd.DagPlan(n, A.data.dtype, 400 * n, A.nnz)
+    first, i1 = sd.dag_closure(A, plan=plan)
+    again, i2 = sd.dag_closure(A, plan=plan)
+    assert i1.nlevels == i2.nlevels == levels
+    assert sd.csr_equal(first, again)
+    want = orc.dag_closure(S, 64)
+    np.testing.assert_array_equal(sd.to_scipy(first).toarray(), want.toarray(n))
+
+
+@pytest.mark.parametrize("known", [False, True])
+def test_cycles_and_small_buffers(known):
+    """A cycle is named and a full arena grows, also with a plan whose level
+    count is known."""
+    n = 2000
+    S = _layered(n, 200, 2, np.random.default_rng(2))
+    A = sd.canonicalize(sd.from_scipy(S, np.int64))
+    plan = sd.DagPlan(n, A.data.dtype, 400_000, A.nnz + 10)
+    want, full = sd.dag_closure(A, plan=plan if known else None)
+    tight = sd.DagPlan(n, A.data.dtype, full.arena // 10, A.nnz)
+    if known:
+        tight.levels, tight.out_nnz, tight.kinds = plan.levels, plan.out_nnz, plan.kinds
+    got, info = sd.dag_closure(A, plan=tight)
+    assert sd.csr_equal(got, want) and info.cycle_vertex == -1
+    B = S.tolil()
+    B[0, n - 1] = 2  # the first level reaches the last
+    B = sd.canonicalize(sd.from_scipy(sp.csr_matrix(B), np.int64))
+    C, info = sd.dag_closure(B, plan=plan if known else None)
+    assert (C is None) == (info.cycle_vertex >= 0)
+    reach = want.indices.cpu().numpy()[int(want.indptr[n - 1]):int(want.indptr[n])]
+    assert (C is None) == (0 in reach)
+    # a workspace without the predecessor lists is refused as before
+    t = _lib.torch()
+    bare = sd.DagPlan(n, A.data.dtype, 400_000, 0)
+    from redblackgraph_amd.dense import status
+    for rounds in (8, -plan.levels if known else 8):
+        st = status()
+        st.reset(None)
+        _lib.call("rbg_dag_closure_i64", _lib.ptr(A.indptr), _lib.ptr(A.indices), _lib.ptr(A.data), n,
+                  _lib.ptr(bare.ws), int(_lib.load().rbg_dag_workspace_bytes(n, 0)), _lib.ptr(bare.arena_cols),
+                  _lib.ptr(bare.arena_vals), bare.arena_cols.numel(), rounds, None, 64, st.p,
+                  _lib.stream_handle(None))
+        s = st.read()
+        assert not s.aux[7]
+        assert rounds < 0 or s.flags & _lib.F_CAPACITY
+    t.cuda.synchronize()
+
+
+@pytest.mark.parametrize("vdt", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [6000, 40_000])
+@pytest.mark.parametrize("direct", [0, 1, 5])
+def test_long_rows_of_two_lists(orc, vdt, n, direct):
+    """Rows of one and two successors whose candidates reach from one wave's
+    share past the workgroup's, with shared columns, products that vanish
+    (values -1 and 1) and direct entries inside and outside the lists."""
+    rng = np.random.default_rng(direct)
+    sinks, mid, top = 3000, [], []
+    lengths = [1, 3, 255, 256, 257, 400, 500, 511, 512, 640, 1022, 1023, 1024, 1025, 1500, 2040]
+    rows, cols = [], []
+
+    def add(v, c):
+        rows.extend([v] * len(c))
+        cols.extend(int(x) for x in c)
+
+    for q, k in enumerate(lengths):
+        for rep in range(2):
+            v = sinks + len(mid)
+            mid.append(k)
+            add(v, rng.choice(sinks, k, replace=False))
+    for a in range(len(mid)):
+        for b in (a, a ^ 1, (a + 7) % len(mid), (a + 13) % len(mid)):
+            v = sinks + len(mid) + len(top)
+            top.append((a, b))
+            c = {sinks + a, sinks + b} | set(rng.choice(sinks, direct, replace=False).tolist())
+            add(v, sorted(c))
+    order = rng.permutation(sinks + len(mid) + len(top)) if direct == 1 else np.arange(n)
+    rows, cols = np.array(rows), np.array(cols)
+    if direct == 1:
+        rows, cols = order[rows], order[cols]
+    S = sp.csr_matrix((rng.choice([-1, 1, 2, 3], rows.size), (rows, cols)), shape=(n, n))
+    info = _check(orc, S, vdt)
+    assert info.nlevels == 3
