@@ -666,11 +666,11 @@ def bench_serve(args):
         b_total += 4 * n * anc + 4 * n + 8 * supp * aff + 4 * n
     assert bool((V2 == V).all().item())
     b_edge = b_total / len(edges)
-    roof = {"bound": "hbm", "kernel": "in-place edge insertion (k_edge_compose + k_edge_apply), N=4096 int32",
+    roof = {"bound": "hbm", "kernel": "in-place edge insertion (k_edge_step), N=4096 int32",
             "achieved": b_edge / per_edge_s / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
             "frac": b_edge / per_edge_s / PEAK_HBM, "traffic": None,
             "algorithmic_bytes_per_edge": b_edge, "ms_per_edge": per_edge_s * 1e3,
-            "note": "two small launches per edge: launch latency, not bytes, bounds an insertion into a pedigree "
+            "note": "one small launch per edge: launch latency, not bytes, bounds an insertion into a pedigree "
                     "closure (the rows that reach an edge's source are few)",
             "bytes_rule": "4 N (ancestor rows of the source) + 4 N (source column) + 8 |composed row| (rows that "
                           "reach the source) + 4 N (composed row written)"}

@@ -264,62 +264,112 @@ __global__ void k_zero_i64(int64_t* p, int64_t n) {
     p[i] = 0;
 }
 
-// Edge composition in place, two launches an edge (a composition into a
+// Edge composition in place, one launch an edge (a composition into a
 // pedigree's closure changes a few rows only, so its time is its launches and
-// their round trips to memory, not bytes: n = 4095, 64 edges, 1.43 -> 0.74 ms;
-// 6.3 us to compose and 4.3 to apply, where four launches took 22 an edge).
+// their round trips to memory, not bytes: n = 4095, 64 edges, 1.43 ms with four
+// launches an edge, 0.74 with two, 0.57 so).
 //
-// k_edge_compose: workgroup b computes the composed row u = lhs (x) W (lhs =
-// row alpha with entry beta replaced by the relationship) for columns [64 b,
-// 64 b + 64) and lists the rows m in [64 b, 64 b + 64) with W[m][alpha] != 0,
-// the vertices that reach alpha: the only rows the edge changes.  The present
+// A launch composes edge e and applies edge e - 1, at once: a cell that the
+// composition reads is taken as edge e - 1 leaves it, W[k][p] (+) col[k] (x)
+// u[p] (row alpha': u[p]), whether its own workgroup has stored that yet or not
+// -- the sum is a minimum, so adding a term twice changes nothing, and col, the
+// column alpha' before the edge, is kept beside the matrix.
+template <typename T>
+struct EdgeState {
+  T* u;           // the composed row
+  T* col;         // column alpha: the rows' values to alpha
+  int32_t* hit;   // the rows that reach alpha, the only ones the edge changes
+  int32_t* nhit;
+};
+
+// Workgroup b computes the composed row u = lhs (x) W (lhs = row alpha with
+// entry beta replaced by the relationship) for columns [64 b, 64 b + 64) and
+// lists the rows m in [64 b, 64 b + 64) with W[m][alpha] != 0.  The present
 // lefts of up to EC_SPAN columns are gathered in LDS at a time (16 loads in
 // flight per thread) and dealt to the four waves.
 constexpr int EC_SPAN = 4096;
 template <typename T>
-__global__ __launch_bounds__(256) void k_edge_compose(const T* __restrict__ W, int64_t n, int64_t alpha, int64_t beta,
-                                                      T np, T* __restrict__ u, int32_t* __restrict__ hit,
-                                                      int32_t* __restrict__ nhit, int width, int is_uns,
-                                                      rbg_status* st) {
-  __shared__ int32_t s_idx[EC_SPAN];
-  __shared__ T s_lhs[EC_SPAN];
-  __shared__ T s_part[4][64];
-  __shared__ int s_cnt;
+struct ComposeLds {
+  int32_t idx[EC_SPAN];
+  T lhs[EC_SPAN];
+  T term[EC_SPAN];  // col of the last edge
+  T part[4][64];
+  int cnt;
+};
+
+template <typename T>
+__device__ inline void edge_compose_block(ComposeLds<T>& L, const T* __restrict__ W, int64_t n, int64_t alpha,
+                                          int64_t beta, T np, EdgeState<T> now, int64_t last_alpha, EdgeState<T> last,
+                                          int width, int is_uns, rbg_status* st) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t p = (int64_t)blockIdx.x * 64 + lane;
-  if (wv == 0 && p < n && p != alpha && W[p * n + alpha] != 0) hit[atomicAdd(nhit, 1)] = (int32_t)p;
-  if (blockIdx.x == 0 && tid == 0 && W[beta * n + alpha] != 0) atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
-  T acc = 0;
+  const bool lazy = last_alpha >= 0;
   uint32_t evs = 0;
+  // a cell as the last edge leaves it: c its row's col, up u at its column
+  auto cell = [&](T w, T c, T up) {
+    if (c != 0 && up != 0) {
+      uint32_t ev = 0;
+      w = avos_sum<T>(w, avos_product<T>(c, up, width, is_uns != 0, ev));
+      evs |= ev;
+    }
+    return w;
+  };
+  const T ua = lazy ? last.u[alpha] : (T)0;
+  const T up = lazy && p < n ? last.u[p] : (T)0;
+  if (wv == 0 && p < n) {
+    T c = W[p * n + alpha];
+    if (lazy) c = p == last_alpha ? ua : cell(c, last.col[p], ua);
+    now.col[p] = c;
+    if (p != alpha && c != 0) now.hit[atomicAdd(now.nhit, 1)] = (int32_t)p;
+    if (p == beta && c != 0) atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
+  }
+  const bool replaced = lazy && alpha == last_alpha;
+  const T ca = lazy && !replaced ? last.col[alpha] : (T)0;
+  T acc = 0;
   for (int64_t k0 = 0; k0 < n; k0 += EC_SPAN) {
-    if (tid == 0) s_cnt = 0;
+    if (tid == 0) L.cnt = 0;
     __syncthreads();
-    T x[EC_SPAN / 256];
+    constexpr int Q = EC_SPAN / 256;
+    T x[Q], t[Q];
 #pragma unroll
-    for (int q = 0; q < EC_SPAN / 256; q++) {
+    for (int q = 0; q < Q; q++) {
       const int64_t k = k0 + 256 * q + tid;
-      x[q] = k < n ? W[alpha * n + k] : (T)0;
+      x[q] = k < n ? (replaced ? last.u[k] : W[alpha * n + k]) : (T)0;
+      t[q] = lazy && k < n ? last.col[k] : (T)0;
+    }
+    if (ca != 0) {
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        const int64_t k = k0 + 256 * q + tid;
+        if (k < n) x[q] = cell(x[q], ca, last.u[k]);
+      }
     }
 #pragma unroll
-    for (int q = 0; q < EC_SPAN / 256; q++) {
+    for (int q = 0; q < Q; q++) {
       const int64_t k = k0 + 256 * q + tid;
       if (k < n && k == beta && np != 0) x[q] = np;
       if (x[q] != 0) {
-        const int at = atomicAdd(&s_cnt, 1);
-        s_idx[at] = (int32_t)k;
-        s_lhs[at] = x[q];
+        const int at = atomicAdd(&L.cnt, 1);
+        L.idx[at] = (int32_t)k;
+        L.lhs[at] = x[q];
+        L.term[at] = t[q];
       }
     }
     __syncthreads();
-    const int cnt = s_cnt;
+    const int cnt = L.cnt;
     if (p < n)
       for (int e = wv; e < cnt; e += 16) {
         T y[4], l[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           const bool on = e + 4 * q < cnt;
-          l[q] = on ? s_lhs[e + 4 * q] : (T)0;
-          y[q] = on ? W[(int64_t)s_idx[e + 4 * q] * n + p] : (T)0;
+          l[q] = on ? L.lhs[e + 4 * q] : (T)0;
+          y[q] = on ? W[(int64_t)L.idx[e + 4 * q] * n + p] : (T)0;
+        }
+        if (lazy) {
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            if (e + 4 * q < cnt) y[q] = L.idx[e + 4 * q] == last_alpha ? up : cell(y[q], L.term[e + 4 * q], up);
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -330,33 +380,30 @@ __global__ __launch_bounds__(256) void k_edge_compose(const T* __restrict__ W, i
       }
     __syncthreads();  // the next span's lefts replace these
   }
-  s_part[wv][lane] = acc;
+  L.part[wv][lane] = acc;
   __syncthreads();
   if (wv == 0 && p < n)
-    u[p] = avos_sum<T>(avos_sum<T>(acc, s_part[1][lane]), avos_sum<T>(s_part[2][lane], s_part[3][lane]));
+    now.u[p] = avos_sum<T>(avos_sum<T>(acc, L.part[1][lane]), avos_sum<T>(L.part[2][lane], L.part[3][lane]));
   if (evs) atomicOr(&st->events, evs);
 }
 
-// The listed rows m: W[m][p] = W[m][p] (+) W[m][alpha] (x) u[p] where u is
-// present (relational_composition.c.in:110-137), and row alpha = u.
-// W[m][alpha] is unchanged by it: u[alpha] is alpha's own diagonal.  Also
-// clears the next edge's row counter.
+// The listed rows m: W[m][p] = W[m][p] (+) col[m] (x) u[p] where u is present
+// (relational_composition.c.in:110-137), and row alpha = u.  Workgroup `b` of
+// `groups`.
 template <typename T>
-__global__ __launch_bounds__(256) void k_edge_apply(T* __restrict__ W, int64_t n, int64_t alpha,
-                                                    const T* __restrict__ u, const int32_t* __restrict__ hit,
-                                                    const int32_t* __restrict__ nhit, int32_t* __restrict__ next_nhit,
-                                                    int width, int is_uns, rbg_status* st) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *next_nhit = 0;
-  for (int64_t p = blockIdx.x * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)gridDim.x * 256) W[alpha * n + p] = u[p];
+__device__ inline void edge_apply_block(T* __restrict__ W, int64_t n, int64_t alpha, EdgeState<T> e, int b, int groups,
+                                        int width, int is_uns, rbg_status* st) {
+  for (int64_t p = b * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)groups * 256) W[alpha * n + p] = e.u[p];
   uint32_t evs = 0;
-  const int nh = *nhit;
-  for (int h = blockIdx.x; h < nh; h += gridDim.x) {
-    T* Wm = W + (int64_t)hit[h] * n;
-    const T rma = Wm[alpha];
+  const int nh = *e.nhit;
+  for (int h = b; h < nh; h += groups) {
+    const int m = e.hit[h];
+    T* Wm = W + (int64_t)m * n;
+    const T rma = e.col[m];
     for (int64_t p0 = threadIdx.x; p0 < n; p0 += 256 * 8) {
       T up[8];
 #pragma unroll
-      for (int q = 0; q < 8; q++) up[q] = p0 + 256 * q < n ? u[p0 + 256 * q] : (T)0;
+      for (int q = 0; q < 8; q++) up[q] = p0 + 256 * q < n ? e.u[p0 + 256 * q] : (T)0;
 #pragma unroll
       for (int q = 0; q < 8; q++)
         if (up[q] != 0) {
@@ -368,6 +415,23 @@ __global__ __launch_bounds__(256) void k_edge_apply(T* __restrict__ W, int64_t n
     }
   }
   if (evs) atomicOr(&st->events, evs);
+}
+
+// Workgroups [0, ceil(n / 64)) compose an edge (alpha < 0: none), the others
+// apply the one before (last_alpha < 0: none).  `spare` counter: cleared for
+// the next launch.
+template <typename T>
+__global__ __launch_bounds__(256) void k_edge_step(T* W, int64_t n, int64_t alpha, int64_t beta, T np, EdgeState<T> now,
+                                                   int64_t last_alpha, EdgeState<T> last, int32_t* spare, int width,
+                                                   int is_uns, rbg_status* st) {
+  __shared__ ComposeLds<T> L;
+  const int cols = alpha < 0 ? 0 : (int)((n + 63) / 64);
+  if ((int)blockIdx.x < cols) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *spare = 0;
+    edge_compose_block<T>(L, W, n, alpha, beta, np, now, last_alpha, last, width, is_uns, st);
+  } else {
+    edge_apply_block<T>(W, n, last_alpha, last, (int)blockIdx.x - cols, (int)gridDim.x - cols, width, is_uns, st);
+  }
 }
 
 // Vertex composition, steps 3-4 (relational_composition.c.in:223-266).
@@ -445,34 +509,40 @@ static int edge_compose(const T* R, int64_t n, int64_t alpha, int64_t beta, T re
 }
 
 // `count` edges (alpha, beta, relationship) one after another.  scratch:
-// rbg_edge_compose_scratch_bytes(n) bytes (the composed row, two row counters
-// and the list of affected rows)
+// rbg_edge_compose_scratch_bytes(n) bytes (two edges' composed rows, columns
+// and lists of affected rows)
 template <typename T>
 static int edge_compose_many(T* W, int64_t n, const int64_t* edges, int64_t count, void* scratch, int width,
                              int is_uns, rbg_status* st, hipStream_t s) {
   if (!W || !scratch || !st || n <= 0 || n > 0x7fffffff || count < 0 || (count && !edges)) return RBG_E_ARG;
   for (int64_t e = 0; e < count; e++)
     if (edges[3 * e] < 0 || edges[3 * e] >= n || edges[3 * e + 1] < 0 || edges[3 * e + 1] >= n) return RBG_E_ARG;
+  if (!count) return 0;
   char* base = (char*)(((uintptr_t)scratch + 255) & ~(uintptr_t)255);
-  T* u = (T*)base;
-  int64_t* counters = (int64_t*)(base + ((n * (int64_t)sizeof(T) + 255) & ~(int64_t)255));
-  int32_t* hit = (int32_t*)(counters + 32);
-  if (count) {
-    hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(32), 0, s, counters, (int64_t)32);
+  auto take = [&](int64_t bytes) {
+    char* r = base;
+    base += (bytes + 255) & ~(int64_t)255;
+    return r;
+  };
+  // three counters on lines of their own: filled, read, and cleared for the next edge
+  int32_t* counters = (int32_t*)take(3 * 128);
+  EdgeState<T> state[2];
+  for (auto& e : state) e = EdgeState<T>{(T*)take(n * 8), (T*)take(n * 8), (int32_t*)take(n * 4), nullptr};
+  hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, s, (int64_t*)counters, (int64_t)48);
+  RBG_CHECK_LAUNCH();
+  const unsigned cols = (unsigned)((n + 63) / 64);
+  const unsigned rows = (unsigned)((n + 255) / 256 < 64 ? 64 : ((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048));
+  int64_t last = -1;
+  for (int64_t e = 0; e <= count; e++) {  // launch `count` applies the last edge
+    const bool some = e < count;
+    EdgeState<T>&now = state[e & 1], &before = state[(e + 1) & 1];
+    now.nhit = counters + 32 * (e % 3);
+    hipLaunchKernelGGL((k_edge_step<T>), dim3((some ? cols : 0) + (last >= 0 ? rows : 0)), dim3(256), 0, s, W, n,
+                       some ? edges[3 * e] : (int64_t)-1, some ? edges[3 * e + 1] : (int64_t)-1,
+                       some ? (T)edges[3 * e + 2] : (T)0, now, last, before, counters + 32 * ((e + 1) % 3), width,
+                       is_uns, st);
     RBG_CHECK_LAUNCH();
-  }
-  for (int64_t e = 0; e < count; e++) {
-    const int64_t alpha = edges[3 * e], beta = edges[3 * e + 1];
-    // on lines of their own: one is cleared while the other is read
-    int32_t* now = (int32_t*)(counters + 16 * (e & 1));
-    int32_t* next = (int32_t*)(counters + 16 * ((e + 1) & 1));
-    hipLaunchKernelGGL((k_edge_compose<T>), dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, W, n, alpha, beta,
-                       (T)edges[3 * e + 2], u, hit, now, width, is_uns, st);
-    RBG_CHECK_LAUNCH();
-    const unsigned grid = (unsigned)((n + 255) / 256 < 64 ? 64 : ((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048));
-    hipLaunchKernelGGL((k_edge_apply<T>), dim3(grid), dim3(256), 0, s, W, n, alpha, (const T*)u, (const int32_t*)hit,
-                       (const int32_t*)now, next, width, is_uns, st);
-    RBG_CHECK_LAUNCH();
+    last = some ? edges[3 * e] : -1;
   }
   return 0;
 }
@@ -584,7 +654,7 @@ int rbg_edge_compose_i64(const int64_t* R, int64_t n, int64_t alpha, int64_t bet
   return edge_compose<int64_t>(R, n, alpha, beta, rel, out, width, is_unsigned, st, (hipStream_t)stream);
 }
 int64_t rbg_edge_compose_scratch_bytes(int64_t n) {
-  return n <= 0 ? 0 : 256 + ((n * 8 + 255) & ~(int64_t)255) + 8 * 32 + 8 * n;
+  return n <= 0 ? 0 : 256 + 512 + 4 * (n * 8 + 255) + 2 * (n * 4 + 255);
 }
 int rbg_edge_compose_inplace_i32(int32_t* W, int64_t n, int64_t alpha, int64_t beta, int32_t rel, void* scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
