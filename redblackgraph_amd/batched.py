@@ -1,5 +1,5 @@
 """Batched dense closure: thousands of independent components closed by one
-launch schedule (recordable as one hipGraph) instead of one closure per graph.
+launch schedule (recordable as hipGraphs) instead of one closure per graph.
 
 The reference closes components one at a time
 (sparse/csgraph/transitive_closure.py:85-195, component_wise_closure, each
@@ -8,10 +8,11 @@ warshall.c.in:50-107).  Here every component is padded to a multiple of 128
 and laid out contiguously in one int32 pool in HBM; the C ABI
 (rbg_batch_create / run / capture / replay) walks all components' pivot
 blocks together, largest components first, with the phase-3 tile shape picked
-per size bucket (see autotune.py).  Lower triangular components (pedigrees
-numbered parents first) are instead closed together by one persistent launch:
-every component's work items in one grid, each waiting only on its own
-component's counters.
+per size bucket (see autotune.py), or by one persistent launch: every lower
+triangular component's work items in one grid, each waiting only on its own
+component's counters.  Before either, lower triangular components (pedigrees
+numbered parents first) up to order 4096 are closed from their rows' entries
+where these are few; the other launches follow only for what is left.
 
 Each component's result equals the single-matrix closure
 (dense.fw_closure): W, diameter, and the error behaviour.  Components whose

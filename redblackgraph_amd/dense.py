@@ -78,8 +78,9 @@ class FwOutcome:
     status: _lib.RbgStatus
     npad: int
     mode: str  # "fast" | "general"
-    # "full" | "lower" | "upper" (triangular schedules; "lower" is the
-    # persistent closure) | "lower-steps" (one launch per pivot step)
+    # the schedule that the entries' sides stand for: "full" | "lower" | "upper"
+    # (closed from the rows' entries, else by the blocked schedules; "lower" is
+    # then the persistent closure) | "lower-steps" (one launch per pivot step)
     schedule: str = "full"
 
     @property

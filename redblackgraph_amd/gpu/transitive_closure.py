@@ -1,8 +1,8 @@
 """GPU closures (gpu/transitive_closure.py:26-652 of the reference).
 
-transitive_closure_dag_gpu: on-device levels, then one launch per level that
-closes every vertex of the level (librbg_hip.so: rbg_dag_levels,
-rbg_dag_closure_levels_*, rbg_dag_gather_*).  Diameter: floor(log2) of the
+transitive_closure_dag_gpu: on-device levels, then each level's vertices closed
+together (librbg_hip.so: rbg_dag_closure_*, rbg_dag_gather_*,
+rbg_dag_copy_rows_*).  Diameter: floor(log2) of the
 largest |final value| above 1 (gpu/transitive_closure.py:639-646).
 
 transitive_closure_gpu: repeated squaring R <- R (+) R^2 with the reference's
