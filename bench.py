@@ -491,11 +491,11 @@ def bench_batched(args):
     if rows_closed == len(sizes):  # the tile launches found nothing left to do
         pool_bytes = 4.0 * sum(float(x) ** 2 for x in b.layout.npad)
         roof = {
-            "bound": "hbm", "kernel": "k_bfw_rows_close (every component's rows from their entries)",
+            "bound": "hbm", "kernel": "k_bfw_rows_scan ... k_bfw_rows_close (every component from its rows' entries)",
             "achieved": pool_bytes / (close_ms / 1e3) / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s",
             "frac": pool_bytes / (close_ms / 1e3) / PEAK_HBM,
-            "traffic": _read_traffic("bfw_rows_close_batched4096_pmc.txt"),
-            "bytes_rule": "every component's padded closure written once",
+            "traffic": _read_traffic("bfw_rows_batched4096_pmc.txt"),
+            "bytes_rule": "every component's padded matrix read once",
             "schedule": "from the rows' entries", "avg_launch_ms": close_ms,
             "idle_tile_launches": tile_launches, "idle_tile_ms": tile_ms,
             "kernel_share_of_step": close_ms / ms,
@@ -756,7 +756,7 @@ def bench_order(args):
     bytes_alg = 2 * (12 * nnz + 8 * (n + 1)) + 4 * n
     achieved = bytes_alg / (perm_ms / 1e3)
     roof = {
-        "bound": "hbm", "kernel": "rbg_permute_csr<long> (rows renamed and copied, then sorted per row)",
+        "bound": "hbm", "kernel": "rbg_permute_csr<long> (rows renamed and ranked, long rows sorted)",
         "achieved": achieved / 1e9, "peak": PEAK_HBM / 1e9, "unit": "GB/s", "frac": achieved / PEAK_HBM,
         "traffic": _read_traffic("permute_csr_order1m_pmc.txt"), "algorithmic_bytes_per_launch": bytes_alg,
         "avg_launch_ms": perm_ms,

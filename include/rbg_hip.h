@@ -148,7 +148,7 @@ int64_t rbg_fw_flow_waits(int64_t n, int32_t elem_bytes, int32_t edge, int64_t *
 int rbg_fw_prof_enable(int32_t on);
 /* Same facility for every timed launch kind: 0 FW panel, 1 FW tile, 5 FW small tile,
  * 6 FW persistent closure, 2 DAG level, 3 SpGEMM rows, 4 batched FW, 7 closure
- * from the rows' entries (single matrix and batch).  on = 1 starts recording afresh, 2
+ * from the rows' entries (the closing launch; of a batch, scan to close).  on = 1 starts recording afresh, 2
  * resumes and 0 pauses, both keeping what was recorded (so a caller can time
  * a sample of its launches).  rbg_prof_read returns (and clears) the summed
  * duration and count of one kind. */
@@ -532,7 +532,7 @@ int64_t rbg_batch_flow_tickets(const int32_t *npad, const int32_t *edge, int32_t
 int rbg_batch_create(const rbg_batch_comp *comps, int32_t count, rbg_batch **out);
 int rbg_batch_info(const rbg_batch *b, int64_t *info);
 /* Queues one run.  Outside a capture the call may wait, for no longer than
- * queueing every schedule's launches takes, for word that all components were
+ * loading the pool and the other schedules' idle launches take, for word that all components were
  * closed from their rows' entries; the launches behind are then not queued. */
 int rbg_batch_run(rbg_batch *b, rbg_stream_t stream);
 /* closed[i] = 1 where the last run closed component i from its rows' entries

@@ -413,11 +413,16 @@ static int64_t batch_step_launches(const rbg_batch* b) {
 
 // Whether every component is known to be closed from its rows, so that nothing
 // is left to launch.  The answer is there while the rows' last launch still
-// runs; it is awaited for about as long as queueing the idle launches would
-// take (4 us each), no longer: the call stays asynchronous where the stream is
-// busy (128 components, 260 idle launches: 1.75 -> 1.11 ms a replay).
+// runs; it is awaited for about as long as loading and scanning the pool and
+// then the idle launches take (4 us each and 1 ns a workgroup), no longer: the
+// call stays asynchronous where the stream is busy (with the input's copy in the
+// stream: 128 components, 260 idle launches, 1.75 -> 1.11 ms a replay; 4096, 27.0
+// -> 21.6 ms, in one persistent launch of 11 million items 30.4 -> 20.4).
 static bool batch_rows_told(const rbg_batch* b) {
-  const int64_t limit_us = 4 * batch_step_launches(b);
+  int64_t groups = 2 * b->n_chunk + b->n_tri128 + b->n_tri64 + b->classes.total;
+  for (int K = 0; K < b->stepnb; K++) groups += b->panel_cnt[K] + b->t128_cnt[K] + b->t64_cnt[K];
+  const int64_t pool_us = b->n_chunk * (4 * CHUNK * CHUNK / 1024) / 1900;  // written and read at 4 TB/s each
+  const int64_t limit_us = 4 * batch_step_launches(b) + groups / 1000 + pool_us;
   const auto t0 = std::chrono::steady_clock::now();
   for (;;) {
     const int64_t v = __atomic_load_n(b->told, __ATOMIC_ACQUIRE);
@@ -447,6 +452,7 @@ static int batch_launch_rows(rbg_batch* b, hipStream_t s) {
   const Item* scan = b->d_ritems;
   const Item* place = scan + b->n_rscan;
   const Item* close = place + b->n_rplace;
+  int pr = prof_start(s);
   hipLaunchKernelGGL(k_bfw_rows_scan, dim3((unsigned)b->n_rscan), dim3(NT), 0, s, b->d_comps, scan);
   RBG_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_bfw_rows_levels, dim3((unsigned)b->n_rows), dim3(ROWS_BATCH_NT), 0, s, b->d_comps, b->d_rows);
@@ -455,7 +461,6 @@ static int batch_launch_rows(rbg_batch* b, hipStream_t s) {
   RBG_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_bfw_rows_tell, dim3(1), dim3(NT), 0, s, b->d_comps, b->count, b->d_runs, b->told);
   RBG_CHECK_LAUNCH();
-  int pr = prof_start(s);
   hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_BATCH_CLOSE_NT), 0, s, b->d_comps, close);
   RBG_CHECK_LAUNCH();
   prof_stop(7, pr, s, 0.0);
