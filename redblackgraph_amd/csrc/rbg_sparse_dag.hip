@@ -1403,8 +1403,10 @@ __global__ __launch_bounds__(64) void k_lvl_pairs(const int32_t* __restrict__ in
 // A row of one or two successor lists by a workgroup: pair_merge's merge path
 // over LV_NT threads.  Every candidate placed by a binary search in every other
 // list took 113 us a level on average where this takes 100 (n = 1,000,005, the
-// four levels with long rows: 317 us the last, 263 so): bound by the chain of a
-// row's loads, at four workgroups a CU.
+// four levels with long rows: 317 us the last, 263 so).  Bound by reads of
+// parent rows at random places: the next row's slot read ahead changed nothing,
+// nor did LDS for six workgroups a CU in place of four, and more rows in flight
+// evict each other's lines (1536 workgroups: 15% slower).
 constexpr int PW_R = LV_BIG / LV_NT;  // merged positions per thread
 template <typename T>
 struct PairLds {
