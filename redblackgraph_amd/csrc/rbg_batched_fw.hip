@@ -1,5 +1,5 @@
 // Batched dense closure: many independent matrices ("components") closed by one
-// schedule of launches, recordable as a single hipGraph.
+// schedule of launches, recordable as hipGraphs.
 //
 // Reference: the per-graph closure is warshall.c.in:50-107 (through
 // core/redblack.py:49-50); the reference closes components one at a time
@@ -201,18 +201,15 @@ static __global__ __launch_bounds__(ROWS_BATCH_CLOSE_NT, 8) void k_bfw_rows_clos
   rows_close_slab<int32_t, 1, false, true>(L, rows_work(c), c.W, nullptr, c.npad, it.bid, 32, c.st);
 }
 
-// Tells the host whether every component is closed from its rows: the number
-// of the run, negative where one is not.
-static __global__ __launch_bounds__(NT) void k_bfw_rows_tell(const BComp* comps, int32_t count, int64_t* runs,
+// Tells the host whether every component is closed from its rows: the run's
+// ticket, negative where one is not.
+static __global__ __launch_bounds__(NT) void k_bfw_rows_tell(const BComp* comps, int32_t count, int64_t ticket,
                                                              int64_t* told) {
   bool left = false;
   for (int c = threadIdx.x; c < count; c += NT) left |= comps[c].done == 0;
   left = __syncthreads_or(left);
-  if (threadIdx.x == 0) {
-    const int64_t run = *runs + 1;
-    *runs = run;
-    __hip_atomic_store(told, left ? -run : run, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(told, left ? -ticket : ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Domain conversion of one 128 x 128 chunk, four cells per thread and pass.
@@ -388,16 +385,15 @@ struct rbg_batch {
   int32_t* d_rows = nullptr;
   Item* d_ritems = nullptr;
   int64_t n_rows = 0, n_rscan = 0, n_rplace = 0, n_rclose = 0;
-  int64_t* told = nullptr;    // pinned: k_bfw_rows_tell's answer
-  int64_t* d_runs = nullptr;  // runs told of; `runs`: launched
-  int64_t runs = 0;
+  int64_t* told = nullptr;  // pinned: k_bfw_rows_tell's answer
+  int64_t tickets = 0;      // handed out, one to each run the host waits for
   Item* d_prewalk = nullptr;  // (component, block) of the per-step components with dsnap
   int64_t n_prewalk = 0;
   std::vector<int64_t> panel_cnt, t128_cnt, t64_cnt;  // per step: items of running components
   std::vector<int64_t> tri128_off, tri64_off;         // per step: [off[K], off[K + 1]) of the step lists
   std::vector<double> work;                           // per step: relaxations its tile launches execute
   // captured: every launch of a run, or where rows are tried the launches up to
-  // theirs and, in graph 1, those behind
+  // the answer and the close pass and, in graph 1, those behind
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
 };
@@ -418,7 +414,9 @@ static int64_t batch_step_launches(const rbg_batch* b) {
 // call stays asynchronous where the stream is busy (with the input's copy in the
 // stream: 128 components, 260 idle launches, 1.75 -> 1.11 ms a replay; 4096, 27.0
 // -> 21.6 ms, in one persistent launch of 11 million items 30.4 -> 20.4).
-static bool batch_rows_told(const rbg_batch* b) {
+// A word of another run never has this run's ticket: the tickets are the
+// host's own, and a run that a caller's graph launches tells nothing.
+static bool batch_rows_told(const rbg_batch* b, int64_t ticket) {
   int64_t groups = 2 * b->n_chunk + b->n_tri128 + b->n_tri64 + b->classes.total;
   for (int K = 0; K < b->stepnb; K++) groups += b->panel_cnt[K] + b->t128_cnt[K] + b->t64_cnt[K];
   const int64_t pool_us = b->n_chunk * (4 * CHUNK * CHUNK / 1024) / 1900;  // written and read at 4 TB/s each
@@ -426,7 +424,7 @@ static bool batch_rows_told(const rbg_batch* b) {
   const auto t0 = std::chrono::steady_clock::now();
   for (;;) {
     const int64_t v = __atomic_load_n(b->told, __ATOMIC_ACQUIRE);
-    if (v == b->runs || v == -b->runs) return v > 0;
+    if (v == ticket || v == -ticket) return v > 0;
     if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(limit_us)) return false;
   }
 }
@@ -451,19 +449,27 @@ static int batch_init(rbg_batch* b, hipStream_t s) {
 static int batch_launch_rows(rbg_batch* b, hipStream_t s) {
   const Item* scan = b->d_ritems;
   const Item* place = scan + b->n_rscan;
-  const Item* close = place + b->n_rplace;
-  int pr = prof_start(s);
   hipLaunchKernelGGL(k_bfw_rows_scan, dim3((unsigned)b->n_rscan), dim3(NT), 0, s, b->d_comps, scan);
   RBG_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_bfw_rows_levels, dim3((unsigned)b->n_rows), dim3(ROWS_BATCH_NT), 0, s, b->d_comps, b->d_rows);
   RBG_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_bfw_rows_place, dim3((unsigned)b->n_rplace), dim3(NT), 0, s, b->d_comps, place);
   RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_bfw_rows_tell, dim3(1), dim3(NT), 0, s, b->d_comps, b->count, b->d_runs, b->told);
+  return 0;
+}
+
+// The close pass, and the answer ahead of it where the host will wait for one
+// (on a stream under capture it cannot: every launch is queued).
+static int batch_launch_close(rbg_batch* b, hipStream_t s, int64_t* ticket) {
+  *ticket = 0;
+  if (!stream_captures(s)) {
+    *ticket = ++b->tickets;
+    hipLaunchKernelGGL(k_bfw_rows_tell, dim3(1), dim3(NT), 0, s, b->d_comps, b->count, *ticket, b->told);
+    RBG_CHECK_LAUNCH();
+  }
+  hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_BATCH_CLOSE_NT), 0, s, b->d_comps,
+                     b->d_ritems + b->n_rscan + b->n_rplace);
   RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_bfw_rows_close, dim3((unsigned)b->n_rclose), dim3(ROWS_BATCH_CLOSE_NT), 0, s, b->d_comps, close);
-  RBG_CHECK_LAUNCH();
-  prof_stop(7, pr, s, 0.0);
   return 0;
 }
 
@@ -703,8 +709,6 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     if (e == hipSuccess) e = hipMalloc((void**)&b->d_ritems, sizeof(Item) * ritems.size());
     if (e == hipSuccess) e = hipHostMalloc((void**)&b->told, sizeof(int64_t), hipHostMallocMapped | hipHostMallocCoherent);
     if (e == hipSuccess) *b->told = 0;
-    if (e == hipSuccess) e = hipMalloc((void**)&b->d_runs, sizeof(int64_t));
-    if (e == hipSuccess) e = hipMemcpy(b->d_runs, b->told, sizeof(int64_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b->d_rows, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess)
       e = hipMemcpy(b->d_ritems, ritems.data(), sizeof(Item) * ritems.size(), hipMemcpyHostToDevice);
@@ -733,7 +737,6 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
     (void)hipFree(b->d_comps);
     (void)hipFree(b->d_items);
     (void)hipFree(b->d_rows);
-    (void)hipFree(b->d_runs);
     (void)hipFree(b->d_ritems);
     (void)hipFree(b->d_prewalk);
     (void)hipFree(b->d_flow);
@@ -769,11 +772,12 @@ int rbg_batch_run(rbg_batch* b, rbg_stream_t stream) {
   hipStream_t s = (hipStream_t)stream;
   int rc = batch_init(b, s);
   if (rc == 0 && batch_tries_rows(b)) {
+    int64_t ticket = 0;
+    const int pr = prof_start(s);
     rc = batch_launch_rows(b, s);
-    if (rc == 0 && !stream_captures(s)) {
-      b->runs++;
-      if (batch_rows_told(b)) return 0;
-    }
+    if (rc == 0) rc = batch_launch_close(b, s, &ticket);
+    prof_stop(7, pr, s, 0.0);
+    if (rc == 0 && ticket && batch_rows_told(b, ticket)) return 0;
   }
   return rc ? rc : batch_launch_steps(b, s);
 }
@@ -795,8 +799,8 @@ static void batch_drop_graphs(rbg_batch* b) {
   }
 }
 
-// part 0: the init and, where rows are tried, their launches; part 1: the
-// others; both in one graph where no rows are tried
+// part 0: the init and, where rows are tried, their launches up to the close
+// pass; part 1: the steps; all in one graph where no rows are tried
 static int batch_capture_part(rbg_batch* b, hipStream_t s, bool rows, int part) {
   hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return (int)e;
@@ -824,10 +828,9 @@ int rbg_batch_replay(rbg_batch* b, rbg_stream_t stream) {
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipGraphLaunch(b->exec[0], s);
   if (e != hipSuccess || !b->exec[1]) return (int)e;
-  if (!stream_captures(s)) {
-    b->runs++;
-    if (batch_rows_told(b)) return 0;
-  }
+  int64_t ticket = 0;
+  const int rc = batch_launch_close(b, s, &ticket);
+  if (rc || (ticket && batch_rows_told(b, ticket))) return rc;
   return (int)hipGraphLaunch(b->exec[1], s);
 }
 
@@ -837,7 +840,6 @@ int rbg_batch_destroy(rbg_batch* b) {
   (void)hipFree(b->d_comps);
   (void)hipFree(b->d_items);
   (void)hipFree(b->d_rows);
-  (void)hipFree(b->d_runs);
   (void)hipFree(b->d_ritems);
   (void)hipFree(b->d_prewalk);
   (void)hipFree(b->d_flow);

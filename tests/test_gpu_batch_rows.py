@@ -78,3 +78,67 @@ def test_batch_components_part_ways(kind, persistent):
             assert run[-1][i] == (alone[i][1].mode, alone[i][1].diameter)
     if kind == "mixed":
         assert told[0].any() and not told[0].all()
+
+
+def _alone(mats):
+    et = elem_type(np.int32)
+    out = [dense.fw_closure(_lib.to_device(m), et, schedule="steps") for m in mats]
+    return [w.cpu().numpy() for w, _ in out], [(o.mode, o.diameter) for _, o in out]
+
+
+def _check(b, mats, want):
+    b.stream.synchronize()
+    assert [(o.mode, o.diameter) for o in b.outcomes()] == want[1]
+    for i in range(len(mats)):
+        np.testing.assert_array_equal(b.result(i).cpu().numpy(), want[0][i])
+
+
+_INPUTS = {"closable": [_pedigree(200, 5), _pedigree(150, 6)], "mixed": [_pedigree(200, 7), _chain(150)],
+           "none": [_dense_lower(200), _chain(150)]}
+_INPUTS = {k: [np.tril(m) for m in v] for k, v in _INPUTS.items()}
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_input_changes_between_runs(graph, persistent):
+    """What one run found says nothing about the next one's input."""
+    want = {k: _alone(v) for k, v in _INPUTS.items()}
+    b = BatchedClosure([200, 150], tri=1, persistent=persistent)
+    try:
+        for kind in ("closable", "mixed", "closable", "none", "closable", "mixed", "mixed", "closable"):
+            b.load_dense(_INPUTS[kind])
+            b.run(graph=graph)
+            _check(b, _INPUTS[kind], want[kind])
+            np.testing.assert_array_equal(b.rows_closed(), {"closable": [1, 1], "mixed": [1, 0], "none": [0, 0]}[kind])
+    finally:
+        b.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("launches", [1, 2, 3])
+def test_batch_recorded_by_its_caller(launches, graph):
+    """A run recorded into the caller's own graph queues every launch, and what
+    it found is not taken for the answer of a later direct run."""
+    t = _lib.torch()
+    want = {k: _alone(v) for k, v in _INPUTS.items()}
+    b = BatchedClosure([200, 150], tri=1)
+    try:
+        outer = t.cuda.CUDAGraph()
+        t.cuda.synchronize()
+        with t.cuda.graph(outer, stream=b.stream):
+            b.run(graph=False)
+        for _ in range(launches):
+            b.load_dense(_INPUTS["closable"])
+            with t.cuda.stream(b.stream):
+                outer.replay()
+            _check(b, _INPUTS["closable"], want["closable"])
+        for kind in ("none", "mixed", "closable", "none"):
+            b.load_dense(_INPUTS[kind])
+            b.run(graph=graph)
+            _check(b, _INPUTS[kind], want[kind])
+        b.load_dense(_INPUTS["mixed"])
+        with t.cuda.stream(b.stream):
+            outer.replay()
+        _check(b, _INPUTS["mixed"], want["mixed"])
+    finally:
+        b.close()
