@@ -566,7 +566,8 @@ int64_t rbg_glue_temp_bytes(int64_t n);
  * the diagonal are left out.  _count writes N's row pointers (n + 1), st->aux[0]
  * != 0 when N differs from R and st->aux[1] = N's entries (whole status block;
  * temp: rbg_glue_temp_bytes(n)); RBG_F_CAPACITY: a row of N has more than 768
- * entries, and neither call's result holds.  _fill writes N's columns and values. */
+ * entries (or its columns share one place of the table), and neither call's
+ * result holds.  _fill writes N's columns and values. */
 int rbg_csr_square_count_i32(const int64_t *ap, const int32_t *aj, const int32_t *ax, int32_t n, int32_t upper,
                              int64_t *out_ptr, void *temp, int64_t temp_bytes, int32_t width, rbg_status *st,
                              rbg_stream_t stream);

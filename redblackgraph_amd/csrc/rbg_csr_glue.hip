@@ -71,11 +71,18 @@ static int rows_to_ptr(const int64_t* cnt, int64_t n, int64_t* out, void* temp, 
 // atomics.  Last steps of the closure of n = 11,012: 44 us to count and 42 to
 // write with two waves a row, 54 and 56 with four, 56 and 51 with one; the
 // product by folding lists and the merge took 277 + 81 us and the comparison
-// and three host waits came on top (whole closure 3.24 -> 0.62 ms).  A row with
-// more than SQ_COLUMNS columns sets RBG_F_CAPACITY.
+// and three host waits came on top (whole closure 3.24 -> 0.59 ms).  A row with
+// more than SQ_COLUMNS columns sets RBG_F_CAPACITY.  In a table that nears its
+// end a place is a walk through most of it, so a count whose walk passes
+// SQ_PROBES slots (at three quarters full they are tens) leaves the row, and
+// rows that could be as long are not begun: the counts of a closure of 4,000
+// vertices with rows past 1,024 columns took 35 ms a step before that, twice
+// the product and the merge that have to follow.  A counter of the columns in
+// place of the walk's length cost every row 10%.
 constexpr int SQ_SLOTS = 1024;
 constexpr int SQ_COLUMNS = 768;
 constexpr int SQ_NT = 128;
+constexpr int SQ_PROBES = 256;
 
 template <typename T>
 struct SquareRow {
@@ -84,7 +91,7 @@ struct SquareRow {
   U key[SQ_SLOTS];               // -1 -> 0, v -> v, nothing yet -> all ones
   int32_t cols[SQ_COLUMNS + 4];  // the columns together
   uint16_t slot[SQ_COLUMNS];
-  int total, m, full, changed;
+  int total, m, full, ended, changed;
 };
 
 template <typename T, bool FILL>
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
   const int64_t i = blockIdx.x;
   const int64_t r0 = ap[i];
   const int cnt = (int)(ap[i + 1] - r0);
-  if (tid == 0) L.total = L.m = L.full = L.changed = 0;
+  if (tid == 0) L.total = L.m = L.full = L.ended = L.changed = 0;
   __syncthreads();
   // the table's size from the row's products: at most three quarters full
   // where they are few, else SQ_SLOTS
@@ -121,16 +128,26 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
     L.col[q] = -1;
     L.key[q] = ~(U)0;
   }
+  const bool wide = !FILL && total > SQ_COLUMNS;  // else this row of N has no more columns than the table takes
+  if (wide && tid == 0)
+    L.ended = __hip_atomic_load(&st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & RBG_F_CAPACITY;
   __syncthreads();
-  bool full = false;
+  if (wide && L.ended) {
+    if (tid == 0) len[i] = 0;
+    return;
+  }
   uint32_t evs = 0;
-  auto place = [&](int32_t c) {  // c's slot, claimed if new; -1 when the table is full
+  auto stopped = [&]() {
+    return wide && __hip_atomic_load(&L.full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0;
+  };
+  auto place = [&](int32_t c) {  // c's slot, claimed if new; -1 when the table is crowded
     int h = (int)(((uint32_t)c * 0x9E3779B1u) >> shift);
-    for (int probe = 0; probe < slots; probe++) {
+    for (int probe = 0; probe < (FILL ? slots : SQ_PROBES); probe++) {
       const int32_t old = atomicCAS(&L.col[h], -1, c);
       if (old == -1 || old == c) return h;
       h = (h + 1) & (slots - 1);
     }
+    L.full = 1;
     return -1;
   };
   auto term = [&](T a, int32_t c, T b) {
@@ -140,10 +157,7 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
     evs |= ev;
     if (p == 0) return;
     const int h = place(c);
-    if (h < 0)
-      full = true;
-    else
-      atomicMin(&L.key[h], p == (T)-1 ? (U)0 : (U)p);
+    if (h >= 0) atomicMin(&L.key[h], p == (T)-1 ? (U)0 : (U)p);
   };
   // the waves take 16 of the row's entries at a time
   for (int e0 = (tid >> 6) * 16; e0 < cnt; e0 += SQ_NT / 64 * 16) {
@@ -153,7 +167,7 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
     const int64_t s = on ? ap[k] : 0;
     const int l = on ? (int)(ap[k + 1] - s) : 0;
     const int here = cnt - e0 < 16 ? cnt - e0 : 16;
-    for (int e = 0; e < here; e += 4) {
+    for (int e = 0; e < here && !stopped(); e += 4) {
       int le[4];
       int64_t at[4];
       T ae[4], b[4];
@@ -172,20 +186,17 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         if (lane < le[u]) term(ae[u], c[u], b[u]);
-        for (int t = 64; t < le[u]; t += 64)
+        for (int t = 64; t < le[u] && !stopped(); t += 64)
           if (t + lane < le[u]) term(ae[u], aj[at[u] + t], ax[at[u] + t]);
       }
     }
   }
   __syncthreads();
   bool changed = false;
-  for (int e = tid; e < cnt; e += SQ_NT) {  // R's own entries, each column once
+  for (int e = tid; e < cnt && !stopped(); e += SQ_NT) {  // R's own entries, each column once
     const T x = ax[r0 + e];
     const int h = place(aj[r0 + e]);
-    if (h < 0) {
-      full = true;
-      continue;
-    }
+    if (h < 0) break;
     const U k = L.key[h];
     T v = x;
     if (k != ~(U)0) {
@@ -196,7 +207,6 @@ __global__ __launch_bounds__(SQ_NT) void k_gl_square(const int64_t* __restrict__
     changed |= v != x;
     L.key[h] = v == (T)-1 ? (U)0 : (U)v;
   }
-  if (full) L.full = 1;
   if (changed) L.changed = 1;
   __syncthreads();
   for (int q = tid; q < slots; q += SQ_NT) {  // the taken slots, together (slots: a multiple of a wave)

@@ -61,11 +61,7 @@ def transitive_closure_gpu(A: CSRMatrixGPU, max_iterations: int = 64) -> Tuple[C
     R = sd.canonicalize(A._dev())
     tri = A.triangular
     diameter = 0
-    for iteration in range(max_iterations):
-        Rn = sd.square_step(R, mask_upper=tri)
-        if Rn is None:
-            break
-        R = Rn
+    for iteration, R in zip(range(max_iterations), sd.squaring_steps(R, mask_upper=tri)):
         diameter = iteration + 1
     d = _final_diameter(R)
     if d:

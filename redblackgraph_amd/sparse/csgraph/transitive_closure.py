@@ -107,11 +107,8 @@ def transitive_closure_squaring(A, max_iterations=64) -> TransitiveClosure:
     if _is_upper(A) or _is_lower(A):
         return transitive_closure_dag_sparse(A)
     R = sd.canonicalize(sd.from_scipy(A, np.int32))
-    for _ in range(max_iterations):
-        Rn = sd.square_step(R)
-        if Rn is None:
-            break
-        R = Rn
+    for _, R in zip(range(max_iterations), sd.squaring_steps(R)):
+        pass
     c = sd.to_scipy(R)
     diameter = 0
     if c.nnz:

@@ -319,36 +319,61 @@ def csr_equal(A: DevCSR, B: DevCSR) -> bool:
         bool(t.equal(A.data, B.data.to(A.data.dtype)))
 
 
-def square_step(R: DevCSR, mask_upper: bool = False, stream=None):
-    """One step of a squaring closure: R merged with R (x) R (min_abs), or None
-    when that is R itself.  Rows of up to 768 entries take one fused kernel
-    (rbg_csr_square_*); with longer ones the product, the merge and the
-    comparison run one after another."""
+def _square_step_fused(R: DevCSR, mask_upper: bool, stream):
+    """(True, the step's result or None where it is R itself) by one fused
+    kernel (rbg_csr_square_*); (False, None) where a row of the result has
+    more than 768 entries."""
     from .dense import status
     t = _lib.torch()
     n = R.n_rows
-    if n and R.shape[1] == n and R.nnz:
-        sfx = _sfx(R.data.dtype)
-        dev = R.indices.device
-        sh = _lib.stream_handle(stream)
-        st = status()
-        temp = glue_temp(n, dev)
-        optr = t.empty(n + 1, dtype=t.int64, device=dev)
-        width = 8 * R.data.element_size()
-        args = [_lib.ptr(R.indptr), _lib.ptr(R.indices), _lib.ptr(R.data), n, int(mask_upper)]
-        _lib.call(f"rbg_csr_square_count_{sfx}", *args, _lib.ptr(optr), _lib.ptr(temp), temp.numel(), width, st.p, sh)
-        s = st.read(stream)
-        if not s.flags & _lib.F_CAPACITY:
-            if not s.aux[0]:
-                return None
-            nnz = int(s.aux[1])
-            oi = t.empty(nnz, dtype=t.int32, device=dev)
-            ov = t.empty(nnz, dtype=R.data.dtype, device=dev)
-            _lib.call(f"rbg_csr_square_fill_{sfx}", *args, _lib.ptr(optr), _lib.ptr(oi), _lib.ptr(ov), width, st.p, sh)
-            return DevCSR(optr, oi, ov, R.shape)
-    R2, _ = spgemm(R, R, mask_upper=mask_upper, stream=stream)
-    N = avos_sum_csr(R, R2, min_abs=True, stream=stream)
-    return None if csr_equal(R, N) else N
+    sfx = _sfx(R.data.dtype)
+    dev = R.indices.device
+    sh = _lib.stream_handle(stream)
+    st = status()
+    temp = glue_temp(n, dev)
+    optr = t.empty(n + 1, dtype=t.int64, device=dev)
+    width = 8 * R.data.element_size()
+    args = [_lib.ptr(R.indptr), _lib.ptr(R.indices), _lib.ptr(R.data), n, int(mask_upper)]
+    _lib.call(f"rbg_csr_square_count_{sfx}", *args, _lib.ptr(optr), _lib.ptr(temp), temp.numel(), width, st.p, sh)
+    s = st.read(stream)
+    if s.flags & _lib.F_CAPACITY:
+        return False, None
+    if not s.aux[0]:
+        return True, None
+    nnz = int(s.aux[1])
+    oi = t.empty(nnz, dtype=t.int32, device=dev)
+    ov = t.empty(nnz, dtype=R.data.dtype, device=dev)
+    _lib.call(f"rbg_csr_square_fill_{sfx}", *args, _lib.ptr(optr), _lib.ptr(oi), _lib.ptr(ov), width, st.p, sh)
+    return True, DevCSR(optr, oi, ov, R.shape)
+
+
+def squaring_steps(R: DevCSR, mask_upper: bool = False, stream=None):
+    """The steps of a squaring closure: R merged with R (x) R (min_abs), then
+    that matrix with its own square, and so on, until a step changes nothing.
+    Steps whose rows have up to 768 entries take the fused kernel.  Rows only
+    grow, so once one is longer the product, the merge and the comparison run
+    one after another to the end."""
+    fused = True
+    while True:
+        N = None
+        if fused and R.n_rows and R.shape[1] == R.n_rows and R.nnz:
+            fused, N = _square_step_fused(R, mask_upper, stream)
+        else:
+            fused = False
+        if not fused:
+            R2, _ = spgemm(R, R, mask_upper=mask_upper, stream=stream)
+            N = avos_sum_csr(R, R2, min_abs=True, stream=stream)
+            if csr_equal(R, N):
+                N = None
+        if N is None:
+            return
+        R = N
+        yield R
+
+
+def square_step(R: DevCSR, mask_upper: bool = False, stream=None):
+    """The first of ``squaring_steps``, or None when it changes nothing."""
+    return next(squaring_steps(R, mask_upper, stream), None)
 
 
 # Largest dense form of a closure that edge_insert_many builds (bytes).

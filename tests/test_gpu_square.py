@@ -137,3 +137,70 @@ def test_components_one_pass(shape):
         least = np.full(comp.max() + 1, n)
         np.minimum.at(least, comp, np.arange(n))
         np.testing.assert_array_equal(lab, least[comp])
+
+
+def _crowded(dt):
+    """Rows of the closure past 1,024 columns: nearly every parent known."""
+    return synth.csr_pedigree(synth.PedigreeSpec(4000, 16, 0.95, 1), 0, dtype=dt)
+
+
+def test_squaring_closure_leaves_the_fused_step_for_good(monkeypatch):
+    """Rows only grow: after the first step with a row past the limit the
+    fused kernel is not tried again."""
+    from redblackgraph_amd.gpu import CSRMatrixGPU, transitive_closure_gpu
+    said = []
+    call = _lib.call
+
+    def counted(fn, *args):
+        if fn.startswith("rbg_csr_square") or fn.startswith("rbg_spgemm"):
+            said.append(fn[:16])
+        return call(fn, *args)
+
+    S = _crowded(np.int64)
+    monkeypatch.setattr(_lib, "call", counted)
+    C, _ = transitive_closure_gpu(CSRMatrixGPU.from_cpu(S))
+    monkeypatch.undo()
+    tried, plain = ([k for k, f in enumerate(said) if f.startswith(p)] for p in ("rbg_csr_square", "rbg_spgemm"))
+    assert len(plain) >= 2 and max(tried) < min(plain)
+    R = sd.canonicalize(sd.from_scipy(S, np.int64))
+    N = _plain(R, False)
+    while N is not None:
+        R, N = N, _plain(N, False)
+    assert sd.csr_equal(C._dev(), R)
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+def test_square_count_stops_at_the_limit(dt):
+    """Counting a step whose rows pass the limit costs less than half of the
+    product that then has to be computed (a tenth or so; a count that went on
+    to the end cost as much as the whole step)."""
+    from redblackgraph_amd.dense import status
+    t = _lib.torch()
+    R = sd.canonicalize(sd.from_scipy(_crowded(dt), dt))
+    sfx, n = "i32" if dt == np.int32 else "i64", R.n_rows
+    st, temp = status(), sd.glue_temp(n, R.indices.device)
+    ptr = t.empty(n + 1, dtype=t.int64, device=R.indices.device)
+
+    def count(M):
+        _lib.call(f"rbg_csr_square_count_{sfx}", _lib.ptr(M.indptr), _lib.ptr(M.indices), _lib.ptr(M.data), n, 0,
+                  _lib.ptr(ptr), _lib.ptr(temp), temp.numel(), 8 * np.dtype(dt).itemsize, st.p, _lib.stream_handle(None))
+
+    def ms(fn):
+        best = []
+        for _ in range(5):
+            a, b = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+            a.record()
+            fn()
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        return min(best)
+
+    declined = 0
+    while R is not None:  # the last step, which changes nothing, is declined too
+        count(R)
+        if st.read().flags & _lib.F_CAPACITY:
+            declined += 1
+            assert ms(lambda: count(R)) < 0.5 * ms(lambda: _plain(R, False))
+        R = _plain(R, False)
+    assert declined >= 2
