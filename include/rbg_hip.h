@@ -402,7 +402,9 @@ int rbg_dag_closure_i64(const int64_t *indptr, const int32_t *indices, const int
                         rbg_status *st, rbg_stream_t stream);
 /* No reference counterpart: the levels' kinds of the last closure in `workspace`
  * (count <= n bytes, one per level: 1 = merged by the unit kernel, else by the
- * pair kernel; | 2 = it had long rows), copied to host_dst (pinned) on `stream`.
+ * pair kernel; | 2 = it had long rows; | 4 = of a graph of up to 32,640 vertices that
+ * was closed by rounds, being too deep or having too many long rows for the launches
+ * that close such graphs otherwise), copied to host_dst (pinned) on `stream`.
  * Passed back as level_kinds with batch = -levels for the same graph, they
  * launch only the merge kernels each level needs.  A level that needs one the
  * hint left out stops the rounds (st->aux[7] = 0 without RBG_F_CYCLE or

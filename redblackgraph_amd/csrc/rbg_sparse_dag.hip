@@ -205,7 +205,7 @@ static int scan_dev(const int64_t* in, int64_t* local, int64_t* sums, const int6
 // ---------------------------------------------------------------------------
 enum {
   C_PLACED = 0,   // vertices placed so far
-  C_DEEP = 1,     // small graphs: not taken (too deep, a cycle, or a workspace sized without the nnz)
+  C_DEEP = 1,     // small graphs: not taken (too deep, long rows, a cycle, or a workspace sized without the nnz)
   C_UNUSED2 = 2,
   C_LSTART = 3,   // first index in `order` of the current level (its size: C_PLACED - C_LSTART)
   C_LPREV = 4,    // first index in `order` of the previous level
@@ -247,7 +247,7 @@ struct DagWork {
   int32_t* slot_len;   // [n * SLOT_D]
   int64_t* slot_av;    // [n * SLOT_D] (edge values, stored as int64)
   int32_t* long_list;  // [n] slots of the current level left to the long-row step
-  uint8_t* kinds;      // [n] per level: LK_UNITS (merged by k_lvl_units) | LK_LONG (it had long rows)
+  uint8_t* kinds;      // [n] per level: LK_UNITS (merged by k_lvl_units) | LK_LONG (it had long rows) | LK_ROUNDS
   int64_t* pptr;       // [n+1] predecessor lists (the reversed non-self edges) ...
   int32_t* preds;      // [ecap] ... carved from the workspace's tail by the closure
   int64_t ecap;
@@ -839,6 +839,7 @@ __device__ inline void put_meta(const SlotRegs& S, RowMeta<T>& M, int lane) {
 // reserved arena entry; each row lands at or below its own reserved range.
 constexpr int LK_UNITS = 1;  // level kinds: merged by k_lvl_units (else k_lvl_pairs)
 constexpr int LK_LONG = 2;   // the level had rows for k_lvl_long
+constexpr int LK_ROUNDS = 4;  // a graph of up to DS_MAX_N vertices that the rounds closed (every level)
 constexpr int LU_GRID = 4096;        // waves of k_lvl_pairs
 constexpr int LU_UNITS_GRID = 2048;  // waves of k_lvl_units
 constexpr int LU_ROWS_MEAN = 64;  // levels with a larger mean candidate count use k_lvl_pairs
@@ -1730,12 +1731,24 @@ __device__ inline void dag_report(const DagWork& ws, rbg_status* st) {
 // count their rows' candidates, reserve them in the arena with one atomic each
 // and merge.  A larger graph's levels do not fit one workgroup, and its levels
 // have rows enough to fill the launches above.
+// Rows of more than SLOT_D entries are merged by a workgroup one after another,
+// which takes time by the square of their entries (each list is searched for
+// every candidate), and a few neighbours of them are one workgroup's: graphs in
+// which these squares sum to more than DS_WORK go to the rounds, which deal
+// such rows out to 1,024 workgroups.  The line, in us here / by the rounds: n =
+// 500, a sixteenth of the rows with 30 entries (sum 30,000) 662 / 879; 2,000, a
+// quarter with 10 (60,000) 601 / 731; 32,000, a sixty-fourth with 10 (60,000)
+// 598 / 638; above it 32,000, a sixteenth with 10 (240,000) 913 / 719; sixteen
+// neighbours with 100 (160,000) 1641 / 1356, with 500 (4,000,000) 10,600 / 4,290;
+// a closed graph of 2,000 closed again 9,870 / 5,860.
 constexpr int DS_MAX_N = 32640;
+constexpr uint32_t DS_WORK = 1 << 16;
+constexpr uint32_t DS_ALONE = 257;  // entries of a row whose square alone passes DS_WORK
 constexpr int DS_LEVELS = 250;
 constexpr int DS_NT = 1024;
 constexpr int DS_ROWS = 64;   // rows of a workgroup at a time
 constexpr int DS_GRID = 512;  // two workgroups a CU
-constexpr uint32_t DS_NONE = 0x7fff, DS_MORE = 1u << 31;
+constexpr uint32_t DS_NONE = 0x7fff, DS_WIDE = 1u << 30, DS_MORE = 1u << 31;
 // a level had rows that k_lvl_units, or k_lvl_pairs, would leave to k_lvl_long
 // (the kinds recorded for a plan are the same whatever closed the graph)
 constexpr int DS_LONG_UNITS = 1, DS_LONG_PAIRS = 2;
@@ -1745,7 +1758,8 @@ struct DsHints {
 };
 
 // Clears the counters and packs each row's first two non-self successors into
-// a word for the levels (ws.rem[0]).
+// a word for the levels (ws.rem[0]), with DS_MORE where there are others and
+// DS_WIDE where the row has more than SLOT_D entries.
 __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ indptr,
                                                  const int32_t* __restrict__ indices, DagWork ws, int32_t n) {
   const int32_t v = blockIdx.x * 256 + threadIdx.x;
@@ -1756,7 +1770,8 @@ __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ ind
   if (v >= n) return;
   uint32_t c[2] = {DS_NONE, DS_NONE};
   int k = 0;
-  for (int64_t e = indptr[v], e1 = indptr[v + 1]; e < e1; e++) {
+  const int64_t e0 = indptr[v], e1 = indptr[v + 1];
+  for (int64_t e = e0; e < e1; e++) {
     const int32_t w = indices[e];
     if (w == v) continue;
     if (k == 2) {
@@ -1765,7 +1780,7 @@ __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ ind
     }
     c[k++] = (uint32_t)w;
   }
-  ((uint32_t*)ws.rem[0])[v] = c[0] | c[1] << 15 | (k > 2 ? DS_MORE : 0);
+  ((uint32_t*)ws.rem[0])[v] = c[0] | c[1] << 15 | (k > 2 ? DS_MORE : 0) | (e1 - e0 > DagWork::SLOT_D ? DS_WIDE : 0);
   ws.row_len[v] = 0;  // a row that is not reached has no entries
   ws.cnt[v] = 0;      // by level: candidates reserved
   ws.rem[1][v] = 0;   // by level: DS_LONG_* seen
@@ -1776,7 +1791,8 @@ __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ ind
 // Levels by sweeps over the rows, each row's level one above its highest
 // successor's, until none changes (a thread's rows see each other's news at
 // once).  Writes `order` by level and each level's first place (cand_loc).
-// C_DEEP where a level passes DS_LEVELS: too deep, or a cycle.
+// C_DEEP where a level passes DS_LEVELS (too deep, or a cycle) or the graph has
+// too many long rows (DS_WORK).
 template <int H>
 __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__ indptr,
                                                      const int32_t* __restrict__ indices, DagWork ws, int32_t n,
@@ -1784,6 +1800,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
   __shared__ __align__(16) uint8_t lev[4 * H * DS_NT + 16];
   __shared__ int marks[4];  // of this sweep, read after its barrier; two sweeps on it is reused
   __shared__ int hist[256], next[256];
+  __shared__ uint32_t work;  // squares of the long rows' entries
   const int tid = threadIdx.x, lane = tid & 63;
   auto tell = [&](int64_t levels) {
     if (told) __hip_atomic_store(told, levels, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1794,6 +1811,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
   }
   if (tid < 4) marks[tid] = 0;
   if (tid < 256) hist[tid] = 0;
+  if (tid == 0) work = 0;
   uint32_t e[4 * H], lv[H];
 #pragma unroll
   for (int h = 0; h < H; h++) {
@@ -1804,16 +1822,30 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
     *(uint32_t*)(lev + row) = 0;
     lv[h] = 0;
   }
+  uint32_t squares = 0;
 #pragma unroll
   for (int x = 0; x < 4 * H; x++) {
     const int row = 4 * ((x / 4) * DS_NT + tid) + x % 4;
     if (row >= n) e[x] = DS_NONE | DS_NONE << 15;
     const uint32_t c0 = e[x] & 0x7fff, c1 = (e[x] >> 15) & 0x7fff;
+    if (e[x] & DS_WIDE) {
+      const int64_t d = indptr[row + 1] - indptr[row];
+      const uint32_t q = d < DS_ALONE ? (uint32_t)d : DS_ALONE;
+      squares += q * q;
+    }
     e[x] = (c0 == DS_NONE ? (uint32_t)n : c0) | (c1 == DS_NONE ? (uint32_t)n : c1) << 15 | (e[x] & DS_MORE);
   }
   __syncthreads();
+  if (squares) atomicAdd(&work, squares);  // below 2^32: DS_MAX_N rows of DS_ALONE entries
   if (tid == 0) lev[n] = 255;  // an absent successor's level: below 0
   __syncthreads();
+  if (work > DS_WORK) {  // uniform: last written before the barrier
+    if (tid == 0) {
+      ws.counters[C_DEEP] = 1;
+      tell(-1);
+    }
+    return;
+  }
   for (int it = 0;; it++) {
     bool changed = false;
     int worst = 0;
@@ -2127,7 +2159,7 @@ __global__ __launch_bounds__(256) void k_ds_report(DagWork ws, int groups, DsHin
 // Round r, step 5 (single lane): advance the arena, count the level, detect a
 // cycle (nothing placed while vertices remain) and completion, and set up
 // round r + 1.
-__global__ void k_round_end(DagWork ws, int32_t r, int32_t n, int32_t hint) {
+__global__ void k_round_end(DagWork ws, int32_t r, int32_t n, int32_t hint, int32_t mark) {
   int64_t* ctr = ws.counters;
   if (dag_halted(ctr)) return;
   const int64_t placed_now = ctr[C_PLACED] - ctr[C_LSTART];
@@ -2135,7 +2167,7 @@ __global__ void k_round_end(DagWork ws, int32_t r, int32_t n, int32_t hint) {
   // that left out a merge kernel the level needed stops the rounds
   const int64_t mean = placed_now > 0 ? (ctr[C_M] + placed_now - 1) / placed_now : 1;
   const int kind = (mean <= LU_ROWS_MEAN ? LK_UNITS : 0) | (ctr[C_LONG] > 0 ? LK_LONG : 0);
-  ws.kinds[r < n ? r : n - 1] = (uint8_t)kind;
+  ws.kinds[r < n ? r : n - 1] = (uint8_t)(kind | mark);
   if (hint >= 0 && placed_now > 0 && ((kind & LK_UNITS) != (hint & LK_UNITS) || (kind & ~hint & LK_LONG))) {
     ctr[C_HINT] = 1;
     return;
@@ -2771,9 +2803,10 @@ struct ToldWord {
 };
 
 // The closure of a graph of up to DS_MAX_N vertices; *taken = false where its
-// levels are too many, it has a cycle or the workspace has no room for the
-// predecessor lists (known only where the host waits for it: rounds < 0 asks
-// for that many levels without a wait, and leaves C_DONE unset otherwise).
+// levels are too many or its rows too long, it has a cycle or the workspace has
+// no room for the predecessor lists (known only where the host waits for it:
+// rounds < 0 asks for that many levels without a wait, and leaves C_DONE unset
+// otherwise).
 template <typename T>
 static int dag_small(const int64_t* indptr, const int32_t* indices, const T* data, int32_t n, const DagWork& ws,
                      const DagArena<T>& ar, int32_t rounds, const uint8_t* kinds, int width, rbg_status* st,
@@ -2839,11 +2872,15 @@ int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(
     DagWork ws = DagWork::carve(workspace, n);                                                                  \
     ws.ecap = ((char*)workspace + ws_bytes - (char*)ws.preds) / 4;                                              \
     DagArena<T> ar{arena_cols, arena_vals, arena_cap};                                                          \
-    if (n <= DS_MAX_N) {                                                                                        \
+    /* without a wait, dag_small only where the kinds say that it closed the graph before */                    \
+    const bool known = exact && level_kinds;                                                                    \
+    int mark = known ? level_kinds[0] & LK_ROUNDS : 0;                                                          \
+    if (n <= DS_MAX_N && !mark && (known || !exact)) {                                                          \
       bool taken = false;                                                                                       \
       const int rc = dag_small<T>(indptr, indices, data, n, ws, ar, exact ? batch : 0, level_kinds, width, st, \
                                    s, &taken);                                                                  \
       if (rc || taken) return rc;                                                                               \
+      mark = LK_ROUNDS;                                                                                         \
     }                                                                                                           \
     hipLaunchKernelGGL(k_dag_init, dim3((n + 255) / 256), dim3(256), 0, s, ws, n);                              \
     RBG_CHECK_LAUNCH();                                                                                         \
@@ -2885,7 +2922,7 @@ int64_t rbg_dag_workspace_bytes(int32_t n, int64_t nnz) { return DagWork::bytes(
         RBG_CHECK_LAUNCH();                                                                                     \
       }                                                                                                         \
       prof_stop(2, pi, s);                                                                                      \
-      hipLaunchKernelGGL(k_round_end, dim3(1), dim3(1), 0, s, ws, r, n, hint);                                  \
+      hipLaunchKernelGGL(k_round_end, dim3(1), dim3(1), 0, s, ws, r, n, hint, mark);                            \
       RBG_CHECK_LAUNCH();                                                                                       \
       if (exact) {                                                                                              \
         if (r + 1 == -batch) break;                                                                             \

@@ -159,3 +159,85 @@ def test_long_rows_of_two_lists(orc, vdt, n, direct):
     S = sp.csr_matrix((rng.choice([-1, 1, 2, 3], rows.size), (rows, cols)), shape=(n, n))
     info = _check(orc, S, vdt)
     assert info.nlevels == 3
+
+
+def _row_lengths(lengths, n=3000):
+    """A sink per vertex but the last ones, which have rows of the given
+    numbers of entries (the diagonal among them)."""
+    S = sp.eye(n, dtype=np.int64).tolil()
+    for q, k in enumerate(lengths):
+        S[n - 1 - q, :k - 1] = 2
+    return S.tocsr()
+
+
+def _calls(monkeypatch, name):
+    said = []
+    call = _lib.call
+
+    def counted(fn, *args):
+        if fn.startswith(name):
+            said.append(fn)
+        return call(fn, *args)
+
+    monkeypatch.setattr(_lib, "call", counted)
+    return said
+
+
+# the squares of rows of more than 7 entries sum to at most 65,536
+@pytest.mark.parametrize("lengths,rounds", [([7] * 2000, False), ([256], False), ([257], True), ([1500], True),
+                                            ([64] * 16, False), ([64] * 16 + [8], True), ([8] * 1024, False),
+                                            ([8] * 1025, True), ([100] * 16, True)])
+def test_long_rows_are_the_rounds(orc, monkeypatch, lengths, rounds):
+    """Which launches close a graph shows in its plan's kinds, and the plan's
+    next closure takes the same ones at once."""
+    S = _row_lengths(lengths)
+    A = sd.canonicalize(sd.from_scipy(S, np.int64))
+    plan = sd.DagPlan(A.n_rows, A.data.dtype, 400_000, A.nnz)
+    want = orc.dag_closure(S, 64).toarray(A.n_rows)
+    said = _calls(monkeypatch, "rbg_dag_closure")
+    for _ in range(3):
+        C, _ = sd.dag_closure(A, plan=plan)
+        assert [bool(k & 4) for k in plan.kinds] == [rounds] * plan.levels
+        np.testing.assert_array_equal(sd.to_scipy(C).toarray(), want)
+    assert len(said) == 3
+
+
+def test_closed_graph_closed_again(orc):
+    """A closure is its own closure, and has rows too long for the launches of
+    small graphs."""
+    from redblackgraph_amd import synth
+    S = synth.csr_pedigree(synth.PedigreeSpec(2000, 11, 0.7, 1), 0)
+    C, _ = sd.dag_closure(sd.from_scipy(S, np.int64))
+    plan = sd.DagPlan(C.n_rows, C.data.dtype, 64 * C.nnz, C.nnz)
+    for _ in range(2):
+        again, _ = sd.dag_closure(C, plan=plan)
+        assert sd.csr_equal(again, C) and all(k & 4 for k in plan.kinds)
+
+
+@pytest.mark.parametrize("graph", ["deep", "long rows", "pedigree"])
+def test_rounds_without_a_wait(monkeypatch, graph):
+    """A level count alone closes any graph of so many levels without a wait;
+    a deep graph's plan does it by one call as well."""
+    from redblackgraph_amd import synth
+    from redblackgraph_amd.dense import status
+    n = 900
+    if graph == "deep":
+        v = np.arange(3, n)
+        S = sp.csr_matrix((np.ones(v.size, np.int64), (v, v - 3)), shape=(n, n))
+    elif graph == "long rows":
+        S = _row_lengths([300, 200], n)
+    else:
+        S = synth.csr_pedigree(synth.PedigreeSpec(n, 10, 0.7, 1), 0)
+    A = sd.canonicalize(sd.from_scipy(S.astype(np.int64), np.int64))
+    plan = sd.DagPlan(n, A.data.dtype, 400 * n, A.nnz)
+    said = _calls(monkeypatch, "rbg_dag_closure")
+    want, _ = sd.dag_closure(A, plan=plan)
+    got, _ = sd.dag_closure(A, plan=plan)
+    assert sd.csr_equal(got, want) and len(said) == 2
+    st = status()
+    st.reset(None)
+    _lib.call("rbg_dag_closure_i64", _lib.ptr(A.indptr), _lib.ptr(A.indices), _lib.ptr(A.data), n, _lib.ptr(plan.ws),
+              plan.ws.numel(), _lib.ptr(plan.arena_cols), _lib.ptr(plan.arena_vals), plan.arena_cols.numel(),
+              -plan.levels, None, 64, st.p, _lib.stream_handle(None))
+    s = st.read()
+    assert s.aux[7] == 1 and s.aux[6] == plan.levels
