@@ -205,7 +205,7 @@ static int scan_dev(const int64_t* in, int64_t* local, int64_t* sums, const int6
 // ---------------------------------------------------------------------------
 enum {
   C_PLACED = 0,   // vertices placed so far
-  C_DEEP = 1,     // small graphs: not taken (too deep, long rows, a cycle, or a workspace sized without the nnz)
+  C_DEEP = 1,     // small graphs: not taken (too deep, or too many long rows)
   C_UNUSED2 = 2,
   C_LSTART = 3,   // first index in `order` of the current level (its size: C_PLACED - C_LSTART)
   C_LPREV = 4,    // first index in `order` of the previous level
@@ -1723,6 +1723,44 @@ __device__ inline void dag_report(const DagWork& ws, rbg_status* st) {
   st->aux[7] = c[C_DONE] && !c[C_CAP] && !c[C_HINT];
 }
 
+// A vertex on a cycle among the unplaced ones: start at the smallest unplaced
+// vertex and keep following its first unplaced successor; the first vertex
+// met twice lies on a cycle.  One lane; returns at once unless C_STUCK.
+__device__ inline void dag_cycle_vertex(const int64_t* indptr, const int32_t* indices, const DagWork& ws, int32_t n,
+                                        int32_t* stamp, rbg_status* st) {
+  if (!ws.counters[C_STUCK]) return;
+  int32_t v = -1;
+  for (int32_t u = 0; u < n; u++)
+    if (ws.level[u] == INT32_MAX) {
+      v = u;
+      break;
+    }
+  if (v < 0) return;
+  for (int32_t u = 0; u < n; u++) stamp[u] = 0;
+  for (int64_t step = 0; step <= n; step++) {
+    if (stamp[v]) break;
+    stamp[v] = 1;
+    int32_t nxt = -1;
+    for (int64_t e = indptr[v]; e < indptr[v + 1]; e++) {
+      int32_t w = indices[e];
+      if (w != v && ws.level[w] == INT32_MAX) {
+        nxt = w;
+        break;
+      }
+    }
+    if (nxt < 0) break;
+    v = nxt;
+  }
+  st->aux[0] = v;
+  atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
+}
+
+// Launched after every closure by rounds.
+__global__ void k_dag_cycle_vertex(const int64_t* indptr, const int32_t* indices, DagWork ws, int32_t n,
+                                   int32_t* stamp, rbg_status* st) {
+  dag_cycle_vertex(indptr, indices, ws, n, stamp, st);
+}
+
 // ---- graphs of up to DS_MAX_N vertices --------------------------------------
 // Their closure is bound by launches and their round trips, not by bytes (n =
 // 21,162, 12 levels: some 120 launches and two waits, 1.04 ms, with the rounds
@@ -1751,6 +1789,7 @@ constexpr int DS_GRID = 512;  // two workgroups a CU
 constexpr uint32_t DS_NONE = 0x7fff, DS_WIDE = 1u << 30, DS_MORE = 1u << 31;
 // a level had rows that k_lvl_units, or k_lvl_pairs, would leave to k_lvl_long
 // (the kinds recorded for a plan are the same whatever closed the graph)
+constexpr int64_t DS_STUCK = -2;  // told: a cycle
 constexpr int DS_LONG_UNITS = 1, DS_LONG_PAIRS = 2;
 struct DsHints {
   uint8_t kind[DS_LEVELS];
@@ -1764,8 +1803,8 @@ __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ ind
                                                  const int32_t* __restrict__ indices, DagWork ws, int32_t n) {
   const int32_t v = blockIdx.x * 256 + threadIdx.x;
   if (v < C_NCTR) {
-    // a workspace without room for the predecessor lists is left to the rounds, which refuse it
-    ws.counters[v] = v == C_CYCV ? -1 : v == C_DEEP ? indptr[n] > ws.ecap : 0;
+    // a workspace without room for the predecessor lists is refused, as by the rounds
+    ws.counters[v] = v == C_CYCV ? -1 : v == C_CAP ? indptr[n] > ws.ecap : 0;
   }
   if (v >= n) return;
   uint32_t c[2] = {DS_NONE, DS_NONE};
@@ -1788,11 +1827,12 @@ __global__ __launch_bounds__(256) void k_ds_prep(const int64_t* __restrict__ ind
   if (v == n - 1) ws.pptr[n] = 0;
 }
 
-// Levels by sweeps over the rows, each row's level one above its highest
-// successor's, until none changes (a thread's rows see each other's news at
-// once).  Writes `order` by level and each level's first place (cand_loc).
-// C_DEEP where a level passes DS_LEVELS (too deep, or a cycle) or the graph has
-// too many long rows (DS_WORK).
+// Levels by sweeps over the rows: a row's level is known, one above its highest
+// successor's, once all of theirs are, until every one is (a thread's rows see
+// each other's news at once).  Writes `order` by level and each level's first
+// place (cand_loc).  C_DEEP where a level passes DS_LEVELS or the graph has too
+// many long rows (DS_WORK); C_STUCK where a sweep finds nothing new and rows
+// are left: a cycle, with `level` as the rounds leave it.
 template <int H>
 __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__ indptr,
                                                      const int32_t* __restrict__ indices, DagWork ws, int32_t n,
@@ -1805,7 +1845,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
   auto tell = [&](int64_t levels) {
     if (told) __hip_atomic_store(told, levels, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   };
-  if (ws.counters[C_DEEP]) {  // uniform: written by an earlier launch
+  if (ws.counters[C_CAP]) {  // uniform: written by an earlier launch
     if (tid == 0) tell(-1);
     return;
   }
@@ -1819,8 +1859,9 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
     uint4 q = make_uint4(0, 0, 0, 0);
     if (row < n) q = *(const uint4*)((const uint32_t*)ws.rem[0] + row);  // padded to 256 bytes
     e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
+    // a level + 2; 0: not known
     *(uint32_t*)(lev + row) = 0;
-    lv[h] = 0;
+    lv[h] = row < n ? 0 : 0x02020202;
   }
   uint32_t squares = 0;
 #pragma unroll
@@ -1837,7 +1878,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
   }
   __syncthreads();
   if (squares) atomicAdd(&work, squares);  // below 2^32: DS_MAX_N rows of DS_ALONE entries
-  if (tid == 0) lev[n] = 255;  // an absent successor's level: below 0
+  if (tid == 0) lev[n] = 1;  // an absent successor: known, below level 0
   __syncthreads();
   if (work > DS_WORK) {  // uniform: last written before the barrier
     if (tid == 0) {
@@ -1846,35 +1887,33 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
     }
     return;
   }
+  auto unknown = [](uint32_t q) { return ((q - 0x01010101u) & ~q & 0x80808080u) != 0; };  // a byte of 0
   for (int it = 0;; it++) {
-    bool changed = false;
+    bool changed = false, left = false;
     int worst = 0;
 #pragma unroll
     for (int h = 0; h < H; h++) {
-      if (4 * h * DS_NT >= n) continue;
-      // after s sweeps a level is at least min(s, the final one): smaller ones are final
-      if ((lv[h] & 0xff) < (uint32_t)it && (lv[h] >> 8 & 0xff) < (uint32_t)it && (lv[h] >> 16 & 0xff) < (uint32_t)it &&
-          lv[h] >> 24 < (uint32_t)it)
-        continue;
+      if (!unknown(lv[h])) continue;
       const int row = 4 * (h * DS_NT + tid);
       uint32_t nv = 0;
 #pragma unroll
       for (int x = 0; x < 4; x++) {
         const uint32_t ex = e[4 * h + x];
-        const int l0 = (uint8_t)(lev[ex & 0x7fff] + 1), l1 = (uint8_t)(lev[(ex >> 15) & 0x7fff] + 1);
-        int nl = l0 > l1 ? l0 : l1;
-        if (ex & DS_MORE) {
+        const int l0 = lev[ex & 0x7fff], l1 = lev[(ex >> 15) & 0x7fff];
+        int nl = l0 == 0 || l1 == 0 ? 0 : (l0 > l1 ? l0 : l1) + 1;
+        if (ex & DS_MORE && nl) {
           const int v = row + x;
-          for (int64_t k = indptr[v]; k < indptr[v + 1]; k++) {
+          const int64_t k1 = indptr[v + 1];
+          for (int64_t k = indptr[v]; k < k1 && nl; k++) {
             const int w = indices[k];
-            const int y = w == v ? 0 : lev[w] + 1;
-            nl = nl > y ? nl : y;
+            const int y = w == v ? 1 : lev[w];
+            nl = y == 0 ? 0 : (nl > y + 1 ? nl : y + 1);
           }
         }
         worst = nl > worst ? nl : worst;
-        nv |= (uint32_t)nl << (8 * x);
+        nv |= (uint32_t)(nl & 0xff) << (8 * x);
       }
-      if (nv != lv[h] && row < n) {
+      if (nv != lv[h]) {
         lv[h] = nv;
         changed = true;
         if (row + 3 < n)
@@ -1882,8 +1921,9 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
         else
           for (int x = 0; row + x < n; x++) lev[row + x] = (uint8_t)(nv >> (8 * x));
       }
+      left |= unknown(nv);
     }
-    const int mark = (__any(changed) ? 1 : 0) | (__any(worst >= DS_LEVELS) ? 2 : 0);
+    const int mark = (__any(changed) ? 1 : 0) | (__any(worst > DS_LEVELS + 1) ? 2 : 0) | (__any(left) ? 4 : 0);
     if (mark && lane == 0) atomicOr(&marks[it & 3], mark);
     if (tid == 0) marks[(it + 2) & 3] = 0;
     __syncthreads();
@@ -1895,7 +1935,23 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
       }
       return;
     }
-    if (!(m & 1)) break;
+    if (!(m & 4)) break;
+    if (!(m & 1)) {
+      int top = 1;
+      for (int i = tid; i < n; i += DS_NT) {
+        const int l = lev[i];
+        top = l > top ? l : top;
+        ws.level[i] = l ? l - 2 : INT32_MAX;
+      }
+      atomicMax(&hist[0], top - 1);
+      __syncthreads();
+      if (tid == 0) {
+        ws.counters[C_NLEV] = hist[0];  // levels that were placed
+        ws.counters[C_STUCK] = 1;
+        tell(DS_STUCK);
+      }
+      return;
+    }
   }
   // rows of one level are mostly neighbours: one LDS atomic for all of a wave's
   // lanes with the first lane's level, and so on
@@ -1913,7 +1969,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
     return place;
   };
 #pragma unroll 1
-  for (int i0 = 0; i0 < n; i0 += DS_NT) count(hist, i0 + tid < n ? lev[i0 + tid] : 0, i0 + tid < n);
+  for (int i0 = 0; i0 < n; i0 += DS_NT) count(hist, i0 + tid < n ? lev[i0 + tid] - 2 : 0, i0 + tid < n);
   __syncthreads();
   if (tid < 64) {
     int c[4], mine = 0;
@@ -1942,7 +1998,7 @@ __global__ __launch_bounds__(DS_NT) void k_ds_levels(const int64_t* __restrict__
 #pragma unroll 1
   for (int i0 = 0; i0 < n; i0 += DS_NT) {
     const int i = i0 + tid;
-    const int at = count(next, i < n ? lev[i] : 0, i < n);
+    const int at = count(next, i < n ? lev[i] - 2 : 0, i < n);
     if (i < n) ws.order[at] = i;
   }
 }
@@ -1966,7 +2022,7 @@ __global__ __launch_bounds__(LV_NT) void k_ds_level(const int64_t* __restrict__ 
   __shared__ long long s_cmax, s_fmax;
   __shared__ int s_halt;
   int64_t* ctr = ws.counters;
-  if (threadIdx.x == 0) s_halt = (ctr[C_DEEP] | ctr[C_CAP]) != 0 || r >= ctr[C_NLEV];
+  if (threadIdx.x == 0) s_halt = (ctr[C_DEEP] | ctr[C_CAP] | ctr[C_STUCK]) != 0 || r >= ctr[C_NLEV];
   __syncthreads();
   if (s_halt) return;
   const int64_t l0 = ws.cand_loc[r], Ls = ws.cand_loc[r + 1] - l0;
@@ -2114,11 +2170,14 @@ __global__ __launch_bounds__(LV_NT) void k_ds_level(const int64_t* __restrict__ 
 
 // The report, one thread per level: the arena's total, the levels' kinds, and
 // as the rounds would, a hint that left out what a level needs.
-__global__ __launch_bounds__(256) void k_ds_report(DagWork ws, int groups, DsHints hints, rbg_status* st) {
+__global__ __launch_bounds__(256) void k_ds_report(const int64_t* __restrict__ indptr,
+                                                   const int32_t* __restrict__ indices, int32_t n, DagWork ws,
+                                                   int groups, DsHints hints, rbg_status* st) {
   __shared__ unsigned long long s_arena;
   __shared__ long long s_cmax, s_fmax;
   __shared__ int s_wrong;
-  const int r = threadIdx.x, nlev = (int)ws.counters[C_NLEV];
+  const bool stuck = ws.counters[C_STUCK] != 0;
+  const int r = threadIdx.x, nlev = stuck ? 0 : (int)ws.counters[C_NLEV];  // levels merged
   if (r == 0) {
     s_arena = 0;
     s_cmax = s_fmax = 0;
@@ -2153,6 +2212,7 @@ __global__ __launch_bounds__(256) void k_ds_report(DagWork ws, int groups, DsHin
     ws.counters[C_FMAX] = s_fmax;
     if (s_wrong) ws.counters[C_HINT] = 1;
     dag_report(ws, st);
+    dag_cycle_vertex(indptr, indices, ws, n, ws.rem[0], st);
   }
 }
 
@@ -2183,39 +2243,6 @@ __global__ void k_round_end(DagWork ws, int32_t r, int32_t n, int32_t hint, int3
   ctr[C_LSTART] = ctr[C_PLACED];
   ctr[C_LONG] = 0;
   ctr[C_ROUND] = r + 1;
-}
-
-// A vertex on a cycle among the unplaced ones: start at the smallest unplaced
-// vertex and keep following its first unplaced successor; the first vertex
-// met twice lies on a cycle.  Single lane; launched after every closure and
-// returns at once unless a round found no vertex to place.
-__global__ void k_dag_cycle_vertex(const int64_t* indptr, const int32_t* indices, DagWork ws, int32_t n,
-                                   int32_t* stamp, rbg_status* st) {
-  if (!ws.counters[C_STUCK]) return;
-  int32_t v = -1;
-  for (int32_t u = 0; u < n; u++)
-    if (ws.level[u] == INT32_MAX) {
-      v = u;
-      break;
-    }
-  if (v < 0) return;
-  for (int32_t u = 0; u < n; u++) stamp[u] = 0;
-  for (int64_t step = 0; step <= n; step++) {
-    if (stamp[v]) break;
-    stamp[v] = 1;
-    int32_t nxt = -1;
-    for (int64_t e = indptr[v]; e < indptr[v + 1]; e++) {
-      int32_t w = indices[e];
-      if (w != v && ws.level[w] == INT32_MAX) {
-        nxt = w;
-        break;
-      }
-    }
-    if (nxt < 0) break;
-    v = nxt;
-  }
-  st->aux[0] = v;
-  atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
 }
 
 // Round r of the topological sort, last step (single lane): cycle and
@@ -2803,10 +2830,9 @@ struct ToldWord {
 };
 
 // The closure of a graph of up to DS_MAX_N vertices; *taken = false where its
-// levels are too many or its rows too long, it has a cycle or the workspace has
-// no room for the predecessor lists (known only where the host waits for it:
-// rounds < 0 asks for that many levels without a wait, and leaves C_DONE unset
-// otherwise).
+// levels are too many, its rows too long or the workspace has no room for the
+// predecessor lists (known only where the host waits for it: rounds < 0 asks
+// for that many levels without a wait, and leaves C_DONE unset otherwise).
 template <typename T>
 static int dag_small(const int64_t* indptr, const int32_t* indices, const T* data, int32_t n, const DagWork& ws,
                      const DagArena<T>& ar, int32_t rounds, const uint8_t* kinds, int width, rbg_status* st,
@@ -2830,8 +2856,9 @@ static int dag_small(const int64_t* indptr, const int32_t* indices, const T* dat
       hipError_t e = hipMemcpyAsync(host, ws.counters, sizeof(host), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       if (e != hipSuccess) return (int)e;
-      levels = host[C_DEEP] ? -1 : host[C_NLEV];
+      levels = host[C_DEEP] | host[C_CAP] ? -1 : host[C_STUCK] ? DS_STUCK : host[C_NLEV];
     }
+    if (levels == DS_STUCK) levels = 0;  // the report alone, which names a vertex on the cycle
     if (levels < 0) {
       *taken = false;
       return 0;
@@ -2850,7 +2877,7 @@ static int dag_small(const int64_t* indptr, const int32_t* indices, const T* dat
   hints.given = rounds < 0 && kinds;
   if (hints.given)
     for (int64_t r = 0; r < levels && r < DS_LEVELS; r++) hints.kind[r] = kinds[r];
-  hipLaunchKernelGGL(k_ds_report, dim3(1), dim3(256), 0, s, ws, grid, hints, st);
+  hipLaunchKernelGGL(k_ds_report, dim3(1), dim3(256), 0, s, indptr, indices, n, ws, grid, hints, st);
   RBG_CHECK_LAUNCH();
   return 0;
 }

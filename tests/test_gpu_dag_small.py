@@ -1,4 +1,6 @@
 """Levels that mix long and short closure rows, against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -241,3 +243,63 @@ def test_rounds_without_a_wait(monkeypatch, graph):
               -plan.levels, None, 64, st.p, _lib.stream_handle(None))
     s = st.read()
     assert s.aux[7] == 1 and s.aux[6] == plan.levels
+
+
+def _queued(A, plan, ws_bytes=None, kinds=None, batch=None):
+    """The status of a closure queued without a wait."""
+    from redblackgraph_amd.dense import status
+    st = status()
+    st.reset(None)
+    kinds = (ctypes.c_uint8 * plan.levels).from_buffer_copy(plan.kinds if kinds is None else kinds)
+    _lib.call("rbg_dag_closure_i64", _lib.ptr(A.indptr), _lib.ptr(A.indices), _lib.ptr(A.data), A.n_rows,
+              _lib.ptr(plan.ws), plan.ws.numel() if ws_bytes is None else ws_bytes, _lib.ptr(plan.arena_cols),
+              _lib.ptr(plan.arena_vals), plan.arena_cols.numel(), -plan.levels if batch is None else batch,
+              ctypes.cast(kinds, ctypes.c_void_p), 64, st.p, _lib.stream_handle(None))
+    return st.read()
+
+
+@pytest.mark.parametrize("n,per,fan", [(3, 1, 1), (2000, 200, 2), (9000, 900, 3), (32_640, 4000, 2)])
+@pytest.mark.parametrize("from_level", [0, 1, 2])
+def test_cycles_are_named_without_a_wait(n, per, fan, from_level):
+    """With an earlier graph's levels and kinds, a cycle is reported with a
+    vertex on it and the levels below it, as by the rounds; a workspace without
+    room for the predecessor lists is refused."""
+    S = _layered(n, per, fan, np.random.default_rng(n))
+    A = sd.canonicalize(sd.from_scipy(S, np.int64))
+    plan = sd.DagPlan(n, A.data.dtype, 1 << 24, A.nnz + 10)
+    sd.dag_closure(A, plan=plan)
+    s = _queued(A, plan)
+    assert s.aux[7] == 1 and s.aux[6] == plan.levels and not s.flags & (_lib.F_CYCLE | _lib.F_CAPACITY)
+    if n > 3:  # three vertices' lists fit what the sizes are rounded up by
+        s = _queued(A, plan, ws_bytes=int(_lib.load().rbg_dag_workspace_bytes(n, 0)))
+        assert not s.aux[7] and s.flags & _lib.F_CAPACITY
+    low = from_level * per  # a vertex of that level, and one above it that reaches it
+    v = n - 1
+    while v >= low + per:
+        v = int(S.indices[S.indptr[v]:S.indptr[v + 1]][0])
+    top = n - 1
+    B = S.tolil()
+    B[v, top] = 2
+    B = sp.csr_matrix(B)
+    B = sd.canonicalize(sd.from_scipy(B, np.int64))
+    s = _queued(B, plan)
+    C, info = sd.dag_closure(B, plan=plan)
+    from scipy.sparse.csgraph import connected_components
+    H = sd.to_scipy(B)
+    H = sp.csr_matrix((np.abs(H.data), H.indices, H.indptr), shape=H.shape)
+    _, comp = connected_components(H, directed=True, connection="strong")
+    size = np.bincount(comp)
+    if v == top:  # an entry on the diagonal
+        assert size.max() == 1 and s.aux[7] == 1 and not s.flags & _lib.F_CYCLE and C is not None
+        return
+    assert s.flags & _lib.F_CYCLE and not s.aux[7] and size[comp[int(s.aux[0])]] > 1
+    assert C is None and size[comp[info.cycle_vertex]] > 1
+    # the levels placed: the longest paths among the vertices that reach no cycle
+    inside = size[comp] > 1
+    bad = inside.copy()
+    for _ in range(n):
+        more = bad | (np.asarray((H != 0).astype(np.int64) @ bad).ravel() > 0)
+        if (more == bad).all():
+            break
+        bad = more
+    assert s.aux[6] == info.nlevels == max((x // per + 1 for x in np.nonzero(~bad)[0]), default=0)
