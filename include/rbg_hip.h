@@ -54,6 +54,7 @@ enum {
   RBG_F_HAS_UPPER = 32,   /* precheck: some off-diagonal entry lies above the diagonal       */
   RBG_F_STALLED = 64,     /* a bounded wait of the persistent closure ran out (set with
                              RBG_F_NEED_GENERAL): rerun, e.g. with tri = 3                  */
+  RBG_F_KINDS = 128,      /* DAG closure: level_kinds were another graph's                   */
 };
 
 /*
@@ -408,7 +409,10 @@ int rbg_dag_closure_i64(const int64_t *indptr, const int32_t *indices, const int
  * Passed back as level_kinds with batch = -levels for the same graph, they
  * launch only the merge kernels each level needs.  A level that needs one the
  * hint left out stops the rounds (st->aux[7] = 0 without RBG_F_CYCLE or
- * RBG_F_CAPACITY: call again with batch > 0); a cycle is still reported. */
+ * RBG_F_CAPACITY: call again with batch > 0); a cycle is still reported.  The
+ * launches for graphs of up to 32,640 vertices depend on no hint but the 4: with
+ * another graph's kinds or level count the closure holds and RBG_F_KINDS asks for
+ * the levels' kinds to be read again. */
 int rbg_dag_level_kinds(void *workspace, int32_t n, uint8_t *host_dst, int32_t count, rbg_stream_t stream);
 /* Topological sort (_topological_sort.pyx:30-163, topological_sort), by the
  * closure's Kahn levels: level_out[v] = the longest path from v to a vertex

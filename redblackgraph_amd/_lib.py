@@ -39,6 +39,7 @@ EV_OVERFLOW_WIDTH, EV_OVERFLOW_RED, EV_INVALID, EV_SIGN = 1, 2, 4, 8
 F_NEED_GENERAL, F_PRECOND_FAIL, F_CYCLE, F_CAPACITY = 1, 2, 4, 8
 F_HAS_LOWER, F_HAS_UPPER = 16, 32
 F_STALLED = 64
+F_KINDS = 128
 NO_KEY = (1 << 64) - 1
 
 # (name, restype, argtypes) of every exported symbol; include/rbg_hip.h is the

@@ -1793,7 +1793,7 @@ constexpr int64_t DS_STUCK = -2;  // told: a cycle
 constexpr int DS_LONG_UNITS = 1, DS_LONG_PAIRS = 2;
 struct DsHints {
   uint8_t kind[DS_LEVELS];
-  uint8_t given;
+  int32_t levels;  // 0: none given
 };
 
 // Clears the counters and packs each row's first two non-self successors into
@@ -2169,7 +2169,8 @@ __global__ __launch_bounds__(LV_NT) void k_ds_level(const int64_t* __restrict__ 
 }
 
 // The report, one thread per level: the arena's total, the levels' kinds, and
-// as the rounds would, a hint that left out what a level needs.
+// whether the hint was another graph's (the closure holds all the same: no
+// launch here depends on it).
 __global__ __launch_bounds__(256) void k_ds_report(const int64_t* __restrict__ indptr,
                                                    const int32_t* __restrict__ indices, int32_t n, DagWork ws,
                                                    int groups, DsHints hints, rbg_status* st) {
@@ -2202,7 +2203,7 @@ __global__ __launch_bounds__(256) void k_ds_report(const int64_t* __restrict__ i
     const int kind = (units ? LK_UNITS : 0) | (ws.rem[1][r] & (units ? DS_LONG_UNITS : DS_LONG_PAIRS) ? LK_LONG : 0);
     ws.kinds[r] = (uint8_t)kind;
     const int hint = hints.kind[r];
-    if (hints.given && ((kind & LK_UNITS) != (hint & LK_UNITS) || (kind & ~hint & LK_LONG))) s_wrong = 1;
+    if (hints.levels && ((kind & LK_UNITS) != (hint & LK_UNITS) || (kind & ~hint & LK_LONG))) s_wrong = 1;
     atomicAdd(&s_arena, (unsigned long long)M);
   }
   __syncthreads();
@@ -2210,8 +2211,8 @@ __global__ __launch_bounds__(256) void k_ds_report(const int64_t* __restrict__ i
     ws.counters[C_ARENA] = (int64_t)s_arena;
     ws.counters[C_CMAX] = s_cmax;
     ws.counters[C_FMAX] = s_fmax;
-    if (s_wrong) ws.counters[C_HINT] = 1;
     dag_report(ws, st);
+    if (s_wrong || (hints.levels && hints.levels != nlev)) atomicOr(&st->flags, (uint32_t)RBG_F_KINDS);
     dag_cycle_vertex(indptr, indices, ws, n, ws.rem[0], st);
   }
 }
@@ -2874,9 +2875,10 @@ static int dag_small(const int64_t* indptr, const int32_t* indices, const T* dat
     prof_stop(2, pi, s);
   }
   DsHints hints{};
-  hints.given = rounds < 0 && kinds;
-  if (hints.given)
+  if (rounds < 0 && kinds) {
+    hints.levels = -rounds;
     for (int64_t r = 0; r < levels && r < DS_LEVELS; r++) hints.kind[r] = kinds[r];
+  }
   hipLaunchKernelGGL(k_ds_report, dim3(1), dim3(256), 0, s, indptr, indices, n, ws, grid, hints, st);
   RBG_CHECK_LAUNCH();
   return 0;

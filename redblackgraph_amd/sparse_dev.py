@@ -139,6 +139,14 @@ class DagPlan:
         self.kinds = None   # one byte per level of that graph: which merge kernels it needed
         self.kinds_host = None
 
+    def queue_kinds(self, sh) -> None:
+        """Copy the last closure's level kinds to kinds_host, on the stream."""
+        t = _lib.torch()
+        count = min(self.n, _KINDS_MAX)
+        if self.kinds_host is None or self.kinds_host.numel() < count:
+            self.kinds_host = t.empty(count, dtype=t.uint8, pin_memory=True)
+        _lib.call("rbg_dag_level_kinds", _lib.ptr(self.ws), self.n, _lib.ptr(self.kinds_host), count, sh)
+
 
 def dag_closure(A: DevCSR, width: int | None = None, stream=None, plan: DagPlan | None = None,
                 arena_factor: float = 48.0, batch: int = 0):
@@ -191,10 +199,7 @@ def dag_closure(A: DevCSR, width: int | None = None, stream=None, plan: DagPlan 
                   _lib.ptr(plan.arena_vals), _lib.ptr(optr), _lib.ptr(oi) if cap else None,
                   _lib.ptr(ov) if cap else None, cap, st.p, sh)
         if not hinted:
-            kcount = min(n, _KINDS_MAX)
-            if plan.kinds_host is None or plan.kinds_host.numel() < kcount:
-                plan.kinds_host = t.empty(kcount, dtype=t.uint8, pin_memory=True)
-            _lib.call("rbg_dag_level_kinds", _lib.ptr(plan.ws), n, _lib.ptr(plan.kinds_host), kcount, sh)
+            plan.queue_kinds(sh)
         s = st.read(stream)
         if s.flags & _lib.F_CYCLE:
             return None, DagInfo(0, 0, 0, int(s.aux[0]), int(s.aux[6]), 0)
@@ -210,7 +215,10 @@ def dag_closure(A: DevCSR, width: int | None = None, stream=None, plan: DagPlan 
         info.arena = int(s.aux[4])
         plan.levels = info.nlevels
         plan.out_nnz = nnz
-        if not hinted:
+        if hinted and s.flags & _lib.F_KINDS:  # closed, but the plan's kinds were another graph's
+            plan.queue_kinds(sh)
+            (t.cuda.current_stream() if stream is None else stream).synchronize()
+        if not hinted or s.flags & _lib.F_KINDS:
             plan.kinds = bytes(plan.kinds_host[:info.nlevels].numpy()) if info.nlevels <= _KINDS_MAX else None
         if cap and nnz <= cap:
             oi, ov = oi[:nnz], ov[:nnz]

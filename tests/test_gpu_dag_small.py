@@ -303,3 +303,29 @@ def test_cycles_are_named_without_a_wait(n, per, fan, from_level):
             break
         bad = more
     assert s.aux[6] == info.nlevels == max((x // per + 1 for x in np.nonzero(~bad)[0]), default=0)
+
+
+def test_plan_reused_for_another_graph(orc, monkeypatch):
+    """Kinds of another graph of the same size cost a small graph no second
+    closure, and the plan then holds its own."""
+    n = 3000
+    rng = np.random.default_rng(4)
+    graphs = [_layered(n, 300, 1, rng), _layered(n, 300, 3, rng), _layered(n, 500, 3, rng)]
+    As = [sd.canonicalize(sd.from_scipy(S, np.int64)) for S in graphs]
+    plan = sd.DagPlan(n, As[0].data.dtype, 1 << 24, max(A.nnz for A in As))
+    kinds = []
+    for S, A in zip(graphs, As):
+        own = sd.DagPlan(n, A.data.dtype, 1 << 24, A.nnz)
+        sd.dag_closure(A, plan=own)
+        kinds.append((own.levels, own.kinds))
+    assert kinds[0][0] == kinds[1][0] > kinds[2][0] and kinds[0][1] != kinds[1][1]
+    sd.dag_closure(As[0], plan=plan)
+    said = _calls(monkeypatch, "rbg_dag_closure")
+    for q in (1, 2):
+        C, info = sd.dag_closure(As[q], plan=plan)
+        want = orc.dag_closure(graphs[q], 64)
+        np.testing.assert_array_equal(C.indptr.cpu().numpy(), want.indptr)
+        np.testing.assert_array_equal(C.indices.cpu().numpy(), want.indices)
+        np.testing.assert_array_equal(C.data.cpu().numpy(), want.data)
+        assert (plan.levels, plan.kinds) == kinds[q] and info.nlevels == kinds[q][0]
+    assert len(said) == 2
