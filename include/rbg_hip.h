@@ -324,8 +324,8 @@ int rbg_edge_compose_inplace_i32(int32_t *W, int64_t n, int64_t alpha, int64_t b
 int rbg_edge_compose_inplace_i64(int64_t *W, int64_t n, int64_t alpha, int64_t beta, int64_t rel, void *scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
 /* `count` edges one after another, each as rbg_edge_compose_inplace_*: edges
- * (host memory) holds alpha, beta and the relationship of each.  Two launches
- * an edge; nothing is read by the host. */
+ * (host memory) holds alpha, beta and the relationship of each.  One launch an
+ * edge, one before the first and one behind the last; nothing is read by the host. */
 int rbg_edge_compose_many_i32(int32_t *W, int64_t n, const int64_t *edges, int64_t count, void *scratch,
                               int32_t width, int32_t is_unsigned, rbg_status *st, rbg_stream_t stream);
 int rbg_edge_compose_many_i64(int64_t *W, int64_t n, const int64_t *edges, int64_t count, void *scratch,

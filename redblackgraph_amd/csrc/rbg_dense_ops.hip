@@ -259,15 +259,10 @@ __global__ __launch_bounds__(256) void k_edge_update(const T* __restrict__ R, in
   if (evs) atomicOr(&st->events, evs);
 }
 
-__global__ void k_zero_i64(int64_t* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0;
-}
-
 // Edge composition in place, one launch an edge (a composition into a
 // pedigree's closure changes a few rows only, so its time is its launches and
 // their round trips to memory, not bytes: n = 4095, 64 edges, 1.43 ms with four
-// launches an edge, 0.74 with two, 0.57 so).
+// launches an edge, 0.74 with two, 0.39 so).
 //
 // A launch composes edge e and applies edge e - 1, at once: a cell that the
 // composition reads is taken as edge e - 1 leaves it, W[k][p] (+) col[k] (x)
@@ -276,33 +271,56 @@ __global__ void k_zero_i64(int64_t* p, int64_t n) {
 // column alpha' before the edge, is kept beside the matrix.
 template <typename T>
 struct EdgeState {
-  T* u;           // the composed row
-  T* col;         // column alpha: the rows' values to alpha
-  int32_t* hit;   // the rows that reach alpha, the only ones the edge changes
+  typename unsigned_of<T>::type* u;  // the composed row, as sum keys
+  T* col;                            // column alpha: the rows' values to alpha
+  int32_t* hit;                      // the rows that reach alpha, the only ones the edge changes
   int32_t* nhit;
 };
 
-// Workgroup b computes the composed row u = lhs (x) W (lhs = row alpha with
-// entry beta replaced by the relationship) for columns [64 b, 64 b + 64) and
-// lists the rows m in [64 b, 64 b + 64) with W[m][alpha] != 0.  The present
-// lefts of up to EC_SPAN columns are gathered in LDS at a time (16 loads in
-// flight per thread) and dealt to the four waves.
-constexpr int EC_SPAN = 4096;
+// Workgroup (x, y): the terms of the composed row u = lhs (x) W (lhs = row
+// alpha with entry beta replaced by the relationship) for columns [64 x, 64 x +
+// 64) from the lefts in [span y, span y + span), combined by a minimum of sum
+// keys; y = 0 also lists the rows m in [64 x, 64 x + 64) with W[m][alpha] != 0.
+// The present lefts are gathered in LDS, up to EC_SPAN at a time, and dealt to
+// the four waves.  A pedigree's row holds a few lefts and most workgroups leave
+// after the gather; where rows are full of them it is the spans that fill the
+// chip: 16 edges, n = 4095, 0.2, 5, 30 and 100% of the cells below the diagonal
+// 139, 467, 773 and 787 us; with the columns' workgroups alone, each over all lefts, and 64
+// workgroups for the rows' updates 156, 1384, 4444, 6196; with seven launches an
+// edge 384, 1140, 2344, 2830.  Spans are as narrow as EC_GROUPS workgroups allow,
+// which all run at once.
+constexpr int EC_SPAN = 1024;
+constexpr int EC_GROUPS = 4096;
+// The updates: a row's EC_CHUNK columns by a workgroup at a time, EC_APPLY of
+// them (n = 8192, 0.2%: a whole row at a time 463 us, 2048 columns 301, 1024 290).
+constexpr int EC_APPLY = 1024;
+constexpr int EC_CHUNK = 1024;
+static inline int edge_spans(int64_t n) {
+  const int64_t cols = (n + 63) / 64, most = (n + 255) / 256, s = EC_GROUPS / cols;
+  return (int)(s < 1 ? 1 : (s < most ? s : most));
+}
+static inline int64_t edge_span(int64_t n) {  // whole passes of the workgroup
+  return ((n + edge_spans(n) - 1) / edge_spans(n) + 255) & ~(int64_t)255;
+}
+
 template <typename T>
 struct ComposeLds {
   int32_t idx[EC_SPAN];
   T lhs[EC_SPAN];
   T term[EC_SPAN];  // col of the last edge
   T part[4][64];
+  T ca;  // col of the last edge at alpha
   int cnt;
 };
 
 template <typename T>
 __device__ inline void edge_compose_block(ComposeLds<T>& L, const T* __restrict__ W, int64_t n, int64_t alpha,
-                                          int64_t beta, T np, EdgeState<T> now, int64_t last_alpha, EdgeState<T> last,
-                                          int width, int is_uns, rbg_status* st) {
+                                          int64_t beta, T np, int x, int y, int64_t span, EdgeState<T> now, int64_t last_alpha,
+                                          EdgeState<T> last, typename unsigned_of<T>::type* spare_u, int width,
+                                          int is_uns, rbg_status* st) {
+  using U = typename unsigned_of<T>::type;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int64_t p = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t p = (int64_t)x * 64 + lane;
   const bool lazy = last_alpha >= 0;
   uint32_t evs = 0;
   // a cell as the last edge leaves it: c its row's col, up u at its column
@@ -314,76 +332,83 @@ __device__ inline void edge_compose_block(ComposeLds<T>& L, const T* __restrict_
     }
     return w;
   };
-  const T ua = lazy ? last.u[alpha] : (T)0;
-  const T up = lazy && p < n ? last.u[p] : (T)0;
-  if (wv == 0 && p < n) {
+  const T up = lazy && p < n ? sum_unkey<T>(last.u[p]) : (T)0;
+  if (y == 0 && wv == 0 && p < n) {
     T c = W[p * n + alpha];
-    if (lazy) c = p == last_alpha ? ua : cell(c, last.col[p], ua);
+    if (lazy) {
+      const T ua = sum_unkey<T>(last.u[alpha]);
+      c = p == last_alpha ? ua : cell(c, last.col[p], ua);
+    }
     now.col[p] = c;
     if (p != alpha && c != 0) now.hit[atomicAdd(now.nhit, 1)] = (int32_t)p;
     if (p == beta && c != 0) atomicOr(&st->flags, (uint32_t)RBG_F_CYCLE);
+    spare_u[p] = ~(U)0;
   }
   const bool replaced = lazy && alpha == last_alpha;
-  const T ca = lazy && !replaced ? last.col[alpha] : (T)0;
+  if (tid == 0) L.ca = lazy && !replaced ? last.col[alpha] : (T)0;
+  constexpr int Q = EC_SPAN / 256, FLY = 4;
+  const int64_t k1 = span * (y + 1) < n ? span * (y + 1) : n;
   T acc = 0;
-  for (int64_t k0 = 0; k0 < n; k0 += EC_SPAN) {
+  for (int64_t k0 = span * y; k0 < k1; k0 += EC_SPAN) {
     if (tid == 0) L.cnt = 0;
-    __syncthreads();
-    constexpr int Q = EC_SPAN / 256;
-    T x[Q], t[Q];
+    T v[Q], t[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) {
       const int64_t k = k0 + 256 * q + tid;
-      x[q] = k < n ? (replaced ? last.u[k] : W[alpha * n + k]) : (T)0;
-      t[q] = lazy && k < n ? last.col[k] : (T)0;
+      v[q] = k < k1 ? (replaced ? sum_unkey<T>(last.u[k]) : W[alpha * n + k]) : (T)0;
+      t[q] = lazy && k < k1 ? last.col[k] : (T)0;
     }
+    __syncthreads();
+    const T ca = L.ca;
     if (ca != 0) {
 #pragma unroll
       for (int q = 0; q < Q; q++) {
         const int64_t k = k0 + 256 * q + tid;
-        if (k < n) x[q] = cell(x[q], ca, last.u[k]);
+        if (k < k1) v[q] = cell(v[q], ca, sum_unkey<T>(last.u[k]));
       }
     }
 #pragma unroll
     for (int q = 0; q < Q; q++) {
       const int64_t k = k0 + 256 * q + tid;
-      if (k < n && k == beta && np != 0) x[q] = np;
-      if (x[q] != 0) {
+      if (k < k1 && k == beta && np != 0) v[q] = np;
+      if (v[q] != 0) {
         const int at = atomicAdd(&L.cnt, 1);
         L.idx[at] = (int32_t)k;
-        L.lhs[at] = x[q];
+        L.lhs[at] = v[q];
         L.term[at] = t[q];
       }
     }
     __syncthreads();
     const int cnt = L.cnt;
     if (p < n)
-      for (int e = wv; e < cnt; e += 16) {
-        T y[4], l[4];
+      for (int e = wv; e < cnt; e += 4 * FLY) {
+        T w[FLY], l[FLY];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < FLY; q++) {
           const bool on = e + 4 * q < cnt;
           l[q] = on ? L.lhs[e + 4 * q] : (T)0;
-          y[q] = on ? W[(int64_t)L.idx[e + 4 * q] * n + p] : (T)0;
+          w[q] = on ? W[(int64_t)L.idx[e + 4 * q] * n + p] : (T)0;
         }
         if (lazy) {
 #pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (e + 4 * q < cnt) y[q] = L.idx[e + 4 * q] == last_alpha ? up : cell(y[q], L.term[e + 4 * q], up);
+          for (int q = 0; q < FLY; q++)
+            if (e + 4 * q < cnt) w[q] = L.idx[e + 4 * q] == last_alpha ? up : cell(w[q], L.term[e + 4 * q], up);
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < FLY; q++) {
           uint32_t ev = 0;
-          if (y[q] != 0) acc = avos_sum<T>(acc, avos_product<T>(l[q], y[q], width, is_uns != 0, ev));
+          if (w[q] != 0) acc = avos_sum<T>(acc, avos_product<T>(l[q], w[q], width, is_uns != 0, ev));
           evs |= ev;
         }
       }
-    __syncthreads();  // the next span's lefts replace these
+    __syncthreads();  // the next lefts replace these
   }
   L.part[wv][lane] = acc;
   __syncthreads();
-  if (wv == 0 && p < n)
-    now.u[p] = avos_sum<T>(avos_sum<T>(acc, L.part[1][lane]), avos_sum<T>(L.part[2][lane], L.part[3][lane]));
+  if (wv == 0 && p < n) {
+    const T sum = avos_sum<T>(avos_sum<T>(acc, L.part[1][lane]), avos_sum<T>(L.part[2][lane], L.part[3][lane]));
+    if (sum != 0) atomicMin(&now.u[p], sum_key<T>(sum));
+  }
   if (evs) atomicOr(&st->events, evs);
 }
 
@@ -393,45 +418,58 @@ __device__ inline void edge_compose_block(ComposeLds<T>& L, const T* __restrict_
 template <typename T>
 __device__ inline void edge_apply_block(T* __restrict__ W, int64_t n, int64_t alpha, EdgeState<T> e, int b, int groups,
                                         int width, int is_uns, rbg_status* st) {
-  for (int64_t p = b * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)groups * 256) W[alpha * n + p] = e.u[p];
+  for (int64_t p = b * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)groups * 256)
+    W[alpha * n + p] = sum_unkey<T>(e.u[p]);
   uint32_t evs = 0;
-  const int nh = *e.nhit;
-  for (int h = b; h < nh; h += groups) {
-    const int m = e.hit[h];
+  // a row's chunk of columns at a time
+  const int64_t chunks = (n + EC_CHUNK - 1) / EC_CHUNK, units = *e.nhit * chunks;
+  for (int64_t c = b; c < units; c += groups) {
+    const int m = e.hit[c / chunks];
     T* Wm = W + (int64_t)m * n;
     const T rma = e.col[m];
-    for (int64_t p0 = threadIdx.x; p0 < n; p0 += 256 * 8) {
-      T up[8];
+    const int64_t p0 = c % chunks * EC_CHUNK + threadIdx.x;
+    constexpr int Q = EC_CHUNK / 256;
+    T up[Q], w[Q];
 #pragma unroll
-      for (int q = 0; q < 8; q++) up[q] = p0 + 256 * q < n ? e.u[p0 + 256 * q] : (T)0;
-#pragma unroll
-      for (int q = 0; q < 8; q++)
-        if (up[q] != 0) {
-          const int64_t p = p0 + 256 * q;
-          uint32_t ev = 0;
-          Wm[p] = avos_sum<T>(Wm[p], avos_product<T>(rma, up[q], width, is_uns != 0, ev));
-          evs |= ev;
-        }
+    for (int q = 0; q < Q; q++) {
+      up[q] = p0 + 256 * q < n ? sum_unkey<T>(e.u[p0 + 256 * q]) : (T)0;
+      w[q] = p0 + 256 * q < n ? Wm[p0 + 256 * q] : (T)0;
     }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      if (up[q] != 0) {
+        uint32_t ev = 0;
+        Wm[p0 + 256 * q] = avos_sum<T>(w[q], avos_product<T>(rma, up[q], width, is_uns != 0, ev));
+        evs |= ev;
+      }
   }
   if (evs) atomicOr(&st->events, evs);
 }
 
-// Workgroups [0, ceil(n / 64)) compose an edge (alpha < 0: none), the others
-// apply the one before (last_alpha < 0: none).  `spare` counter: cleared for
-// the next launch.
+// Workgroups [0, compose) compose an edge, the others apply the one before.
+// `spare` counter and row: cleared for the next launch.
 template <typename T>
-__global__ __launch_bounds__(256) void k_edge_step(T* W, int64_t n, int64_t alpha, int64_t beta, T np, EdgeState<T> now,
-                                                   int64_t last_alpha, EdgeState<T> last, int32_t* spare, int width,
-                                                   int is_uns, rbg_status* st) {
+__global__ __launch_bounds__(256) void k_edge_step(T* W, int64_t n, int64_t alpha, int64_t beta, T np, int compose,
+                                                   int64_t span, EdgeState<T> now, int64_t last_alpha, EdgeState<T> last, int32_t* spare,
+                                                   typename unsigned_of<T>::type* spare_u, int width, int is_uns,
+                                                   rbg_status* st) {
   __shared__ ComposeLds<T> L;
-  const int cols = alpha < 0 ? 0 : (int)((n + 63) / 64);
-  if ((int)blockIdx.x < cols) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *spare = 0;
-    edge_compose_block<T>(L, W, n, alpha, beta, np, now, last_alpha, last, width, is_uns, st);
+  const int cols = (int)((n + 63) / 64), b = (int)blockIdx.x;
+  if (b < compose) {
+    if (b == 0 && threadIdx.x == 0) *spare = 0;
+    edge_compose_block<T>(L, W, n, alpha, beta, np, b % cols, b / cols, span, now, last_alpha, last, spare_u, width,
+                          is_uns, st);
   } else {
-    edge_apply_block<T>(W, n, last_alpha, last, (int)blockIdx.x - cols, (int)gridDim.x - cols, width, is_uns, st);
+    edge_apply_block<T>(W, n, last_alpha, last, b - compose, (int)gridDim.x - compose, width, is_uns, st);
   }
+}
+
+// Before the first edge: the counters and its row.
+template <typename T>
+__global__ __launch_bounds__(256) void k_edge_clear(int64_t n, typename unsigned_of<T>::type* u, int32_t* counters) {
+  using U = typename unsigned_of<T>::type;
+  if (blockIdx.x == 0 && threadIdx.x < 96) counters[threadIdx.x] = 0;
+  for (int64_t p = blockIdx.x * (int64_t)256 + threadIdx.x; p < n; p += (int64_t)gridDim.x * 256) u[p] = ~(U)0;
 }
 
 // Vertex composition, steps 3-4 (relational_composition.c.in:223-266).
@@ -524,23 +562,30 @@ static int edge_compose_many(T* W, int64_t n, const int64_t* edges, int64_t coun
     base += (bytes + 255) & ~(int64_t)255;
     return r;
   };
-  // three counters on lines of their own: filled, read, and cleared for the next edge
+  // three counters on lines of their own and three rows: filled, read, and
+  // cleared for the next edge
   int32_t* counters = (int32_t*)take(3 * 128);
+  using U = typename unsigned_of<T>::type;
+  U* u[3];
+  for (auto& q : u) q = (U*)take(n * 8);
   EdgeState<T> state[2];
-  for (auto& e : state) e = EdgeState<T>{(T*)take(n * 8), (T*)take(n * 8), (int32_t*)take(n * 4), nullptr};
-  hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, s, (int64_t*)counters, (int64_t)48);
-  RBG_CHECK_LAUNCH();
+  for (auto& e : state) e = EdgeState<T>{nullptr, (T*)take(n * 8), (int32_t*)take(n * 4), nullptr};
   const unsigned cols = (unsigned)((n + 63) / 64);
-  const unsigned rows = (unsigned)((n + 255) / 256 < 64 ? 64 : ((n + 255) / 256 < 2048 ? (n + 255) / 256 : 2048));
+  hipLaunchKernelGGL(k_edge_clear<T>, dim3((unsigned)((n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024)), dim3(256), 0,
+                     s, n, u[0], counters);
+  RBG_CHECK_LAUNCH();
+  const unsigned rows = (unsigned)(n / 8 < 64 ? 64 : (n / 8 < EC_APPLY ? n / 8 : EC_APPLY));
   int64_t last = -1;
   for (int64_t e = 0; e <= count; e++) {  // launch `count` applies the last edge
     const bool some = e < count;
     EdgeState<T>&now = state[e & 1], &before = state[(e + 1) & 1];
     now.nhit = counters + 32 * (e % 3);
-    hipLaunchKernelGGL((k_edge_step<T>), dim3((some ? cols : 0) + (last >= 0 ? rows : 0)), dim3(256), 0, s, W, n,
+    now.u = u[e % 3];
+    const unsigned compose = some ? cols * (unsigned)edge_spans(n) : 0;
+    hipLaunchKernelGGL((k_edge_step<T>), dim3(compose + (last >= 0 ? rows : 0)), dim3(256), 0, s, W, n,
                        some ? edges[3 * e] : (int64_t)-1, some ? edges[3 * e + 1] : (int64_t)-1,
-                       some ? (T)edges[3 * e + 2] : (T)0, now, last, before, counters + 32 * ((e + 1) % 3), width,
-                       is_uns, st);
+                       some ? (T)edges[3 * e + 2] : (T)0, (int)compose, edge_span(n), now, last, before, counters + 32 * ((e + 1) % 3),
+                       u[(e + 1) % 3], width, is_uns, st);
     RBG_CHECK_LAUNCH();
     last = some ? edges[3 * e] : -1;
   }
@@ -654,7 +699,7 @@ int rbg_edge_compose_i64(const int64_t* R, int64_t n, int64_t alpha, int64_t bet
   return edge_compose<int64_t>(R, n, alpha, beta, rel, out, width, is_unsigned, st, (hipStream_t)stream);
 }
 int64_t rbg_edge_compose_scratch_bytes(int64_t n) {
-  return n <= 0 ? 0 : 256 + 512 + 4 * (n * 8 + 255) + 2 * (n * 4 + 255);
+  return n <= 0 ? 0 : 256 + 512 + 5 * (n * 8 + 255) + 2 * (n * 4 + 255);
 }
 int rbg_edge_compose_inplace_i32(int32_t* W, int64_t n, int64_t alpha, int64_t beta, int32_t rel, void* scratch,
                                  int32_t width, int32_t is_unsigned, rbg_status* st, rbg_stream_t stream) {
