@@ -288,7 +288,7 @@ struct EdgeState {
 // 139, 467, 773 and 787 us; with the columns' workgroups alone, each over all lefts, and 64
 // workgroups for the rows' updates 156, 1384, 4444, 6196; with seven launches an
 // edge 384, 1140, 2344, 2830.  Spans are as narrow as EC_GROUPS workgroups allow,
-// which all run at once.
+// two rounds of the chip.
 constexpr int EC_SPAN = 1024;
 constexpr int EC_GROUPS = 4096;
 // The updates: a row's EC_CHUNK columns by a workgroup at a time, EC_APPLY of

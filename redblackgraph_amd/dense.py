@@ -275,8 +275,9 @@ def edge_compose_many(R, edges, et: ElemType, stream=None, inplace: bool = False
     sh = _lib.stream_handle(stream)
     cur = R if (inplace and R.is_contiguous()) else R.contiguous().clone()
     scratch = t.empty(int(_lib.load().rbg_edge_compose_scratch_bytes(n)), dtype=t.uint8, device=R.device)
-    flat = (ctypes.c_int64 * (3 * len(edges)))(*(int(x) for edge in edges for x in edge))
-    _lib.call(fn, _lib.ptr(cur), n, flat, len(edges), _lib.ptr(scratch), et.width, int(et.unsigned), st.p, sh)
+    listed = [int(x) for a, b, rel in edges for x in (a, b, rel)]
+    flat = (ctypes.c_int64 * len(listed))(*listed)
+    _lib.call(fn, _lib.ptr(cur), n, flat, len(listed) // 3, _lib.ptr(scratch), et.width, int(et.unsigned), st.p, sh)
     return cur, st.read(stream)
 
 

@@ -115,3 +115,20 @@ def test_edges_into_full_rows_cost_less_than_one_by_one():
         return min(best)
 
     assert ms(lambda: dense.edge_compose_many(R, edges, et)) < ms(lambda: _one_by_one(R, edges, et))
+
+
+def test_edges_of_any_iterable():
+    """Edges come from a generator, an array or rows of one, and each has three
+    numbers."""
+    t = _lib.torch()
+    et = elem_type(np.int32)
+    R = _full(300, 0.1, t.int32, 2)
+    edges = [(290, 10, 2), (200, 20, 3), (299, 200, 2)]
+    want, _ = dense.edge_compose_many(R, edges, et)
+    for form in ((e for e in edges), np.array(edges), [np.array(e, dtype=np.uint8 if max(e) < 256 else np.int64) for e in edges],
+                 map(list, edges), dict.fromkeys(edges), zip(*zip(*edges))):
+        got, _ = dense.edge_compose_many(R, form, et)
+        assert t.equal(got, want)
+    for wrong in ([(290, 10)], [(290, 10, 2, 1)], [(290, 10), (2, 200, 20, 3)], [290, 10, 2]):
+        with pytest.raises((TypeError, ValueError)):
+            dense.edge_compose_many(R, wrong, et)
