@@ -52,7 +52,8 @@ struct MmWork {
   MmList<T> a, b;
 };
 
-static inline int64_t mm_slots(int64_t cols) { return cols / 4 < 64 ? 64 : cols / 4; }
+// a quarter of a row, and of rows up to 256 columns 64 or all
+static inline int64_t mm_slots(int64_t cols) { return cols / 4 < 64 ? (cols < 64 ? cols : 64) : cols / 4; }
 
 template <typename T>
 static int64_t mm_layout(int64_t M, int64_t K, int64_t N, char* base, MmWork<T>* w) {

@@ -47,3 +47,13 @@ def test_host_scalar_entry_points():
     with pytest.raises(OverflowError):
         rb.avos_product(9223372036854775807, 3)
     assert rb.avos_sum(-1, 1) == -1
+
+
+@pytest.mark.parametrize("elem", [4, 8])
+@pytest.mark.parametrize("M,K,N", [(1 << 22, 4, 4), (4, 1 << 22, 1), (1 << 20, 1, 16), (1000, 63, 70), (300, 300, 300)])
+def test_matmul_rows_workspace_of_narrow_operands(elem, M, K, N):
+    """No more room than the operands' own entries can take, but for what the
+    arrays' starts are rounded up by."""
+    from redblackgraph_amd import _lib
+    need = _lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, elem)
+    assert need <= (4 + elem) * (M * K + K * N) + 4 * (M + K) + 2048 + 7 * 256
