@@ -265,13 +265,17 @@ int rbg_matmul_i64(const int64_t *A, int64_t lda, const int64_t *B, int64_t ldb,
  * only the present pairs A[i][k] (x) B[k][j] are computed, with the full
  * arithmetic.  st->aux[5] = 1: C is written, unless RBG_F_NEED_GENERAL is set
  * (a term overflows: rbg_matmul_* must run instead).  st->aux[5] = 0: not
- * taken (more than 1 present pair in 64 of the M K N terms, a row with more
+ * taken (more than 1 present pair in 64 of the M K N terms, or so many that the blocked
+ * kernels are faster for the shape; a row with more
  * entries than a quarter of its length, or a value below -1), C is untouched,
  * and RBG_F_PRECOND_FAIL says what rbg_matmul_precheck_* would say of the two
  * operands.  Writes the whole status block.  Native widths only.  workspace:
  * rbg_matmul_rows_workspace_bytes(M, K, N, elem_bytes) bytes, 256-byte
  * aligned. */
 int64_t rbg_matmul_rows_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t elem_bytes);
+/* 0 where no operands of this shape are faster this way (many short rows of C, or a
+ * few very long rows): rbg_matmul_precheck_* and the blocked kernels instead. */
+int32_t rbg_matmul_rows_fits(int64_t M, int64_t K, int64_t N, int32_t elem_bytes);
 int rbg_matmul_rows_i32(const int32_t *A, int64_t lda, const int32_t *B, int64_t ldb, int32_t *C, int64_t ldc,
                         int64_t M, int64_t K, int64_t N, void *workspace, int64_t workspace_bytes, rbg_status *st,
                         rbg_stream_t stream);

@@ -85,6 +85,7 @@ SIGNATURES = {
     "rbg_matmul_i32": (I32, [P, I64, P, I64, P, I64, I64, I64, I64, I32, I32, P, P]),
     "rbg_matmul_i64": (I32, [P, I64, P, I64, P, I64, I64, I64, I64, I32, I32, P, P]),
     "rbg_matmul_rows_workspace_bytes": (I64, [I64, I64, I64, I32]),
+    "rbg_matmul_rows_fits": (I32, [I64, I64, I64, I32]),
     "rbg_matmul_rows_i32": (I32, [P, I64, P, I64, P, I64, I64, I64, I64, P, I64, P, P]),
     "rbg_matmul_rows_i64": (I32, [P, I64, P, I64, P, I64, I64, I64, I64, P, I64, P, P]),
     "rbg_matmul_fast_workspace_bytes": (I64, [I64, I64, I64, I32]),

@@ -22,8 +22,9 @@
 namespace rbg {
 
 // Taken when the present pairs are at most 1 in ROWS_MM_PAIRS of the M K N
-// terms, no row has more entries than a quarter of its length (or 64), and no
-// value is below -1.  Near that line (both operands 12% full) it takes, against
+// terms, no row has more entries than a quarter of its length (or 64), no value
+// is below -1, and the pairs take less time than the blocked kernels would
+// (mm_limits).  Near the first line (both operands 12% full) it takes, against
 // the blocked kernel (us): int32 63 / 277 at n = 512, 239 / 705 at 2048, 14640
 // / 27490 at 8192; int64 2218 / 11120 at 4096.  Operands not taken pay for the
 // scan in place of rbg_matmul_precheck_* (within 2%, n = 256 to 8192).
@@ -74,6 +75,48 @@ static int64_t mm_layout(int64_t M, int64_t K, int64_t N, char* base, MmWork<T>*
   const MmList<T> a = list(M, K), b = list(K, N);
   if (w) *w = MmWork<T>{(unsigned long long*)pairs, a, b};
   return o;
+}
+
+// The most present pairs for which the entries are faster, where the blocked
+// fast kernel would follow (operands in its domain) and where the general one
+// would, in ns of what was measured: here 2.5 + K / 100 a row of C and, on each
+// of the workgroups that run at once, 3 a pair (4, and once for every part,
+// where a row of C does not fit the LDS); there 50,000, 200 (int64 650; general
+// 2,000 and 3,000) a k for every round of 256 tiles, and the operands'
+// conversion.  Times (us, entries / blocked fast / general), int32: 10% full
+// 2^18 x 64 x 64 924 / 490 / 838, 2^16 x 16 x 16 195 / 104 / 150, 2^13 x 32 x 64
+// 61 / 97 / 151, 2^17 x 256 x 8 800 / 869 / 1281; 12% 300 x 1024 x 16000 800 /
+// 600 / 4595; 10% 2000 x 500 x 40000 14500 / 2340 / 27100, 2% 767 / 2250 / 18300;
+// 5% 64 x 64 x 262144 7290 / 256 / 677; 64 x 2^18 x 64 1910 / 65100 / 489000.
+// `fits`: the entries may be faster also with operands in the domain, and their
+// scan, a wave a row (2.3 ns a column), is no large part of the product.
+struct MmLimits {
+  int64_t cells, parts;  // of a row of C in LDS, and how often
+  size_t lds;
+  unsigned long long fast, general;
+  bool fits;
+};
+template <typename T>
+static MmLimits mm_limits(int64_t M, int64_t K, int64_t N) {
+  MmLimits l;
+  const int64_t fit = ROWS_MM_LDS / (int64_t)sizeof(T) - 16, V = 16 / (int64_t)sizeof(T);
+  l.cells = N < fit ? N : fit;
+  l.parts = (N + l.cells - 1) / l.cells;
+  l.lds = (size_t)((l.cells + V - 1) / V * 16);
+  const double a_cu = l.lds > 20 * 1024 ? 160 * 1024 / (double)l.lds : 8, slots = 256 * (double)(int)a_cu;
+  const double few = (double)M * (double)K * (double)N / ROWS_MM_PAIRS;
+  const double tiles = (double)((M + 127) / 128) * (double)((N + 127) / 128), rounds = tiles > 256 ? tiles / 256 : 1;
+  const double cells = sizeof(T) * ((double)M * (double)K + (double)K * (double)N), out = sizeof(T) * (double)M * (double)N;
+  auto most = [&](double blocked) {
+    const double left = blocked - (2.5 + 0.01 * (double)K) * (double)M;
+    const double p = left * ((double)M < slots ? (double)M : slots) / (l.parts > 1 ? 4.0 * (double)l.parts : 3.0);
+    return p <= 0 ? 0ull : (unsigned long long)(p < few ? p : few);
+  };
+  const double fast = 50e3 + (sizeof(T) == 8 ? 650.0 : 200.0) * (double)K * rounds + (4 * cells + out) / 4000;
+  l.fast = most(fast);
+  l.general = most(50e3 + (sizeof(T) == 8 ? 3000.0 : 2000.0) * (double)K * rounds + (cells + out) / 4000);
+  l.fits = l.fast != 0 && 2.3 * (double)(K > N ? K : N) < 0.15 * fast;
+  return l;
 }
 
 // A row's entries in column order, by one wave: 16-byte loads, eight in
@@ -208,7 +251,8 @@ static __global__ __launch_bounds__(MM_PLAN_NT) void k_mm_plan(int64_t M, int64_
 // Row blockIdx.x of C.  `cells` of N in LDS at a time.  aux[5] = 1: written.
 template <typename T>
 static __global__ __launch_bounds__(ROWS_MM_NT) void k_mm_rows(MmWork<T> w, T* C, int64_t ldc, int64_t N, int64_t cells,
-                                                              unsigned long long most, rbg_status* st) {
+                                                              unsigned long long fast, unsigned long long general,
+                                                              rbg_status* st) {
   using U = typename unsigned_of<T>::type;
   constexpr int V = 16 / (int)sizeof(T);
   extern __shared__ __align__(16) unsigned char lds[];
@@ -217,7 +261,8 @@ static __global__ __launch_bounds__(ROWS_MM_NT) void k_mm_rows(MmWork<T> w, T* C
   unsigned long long pairs = lane < ROWS_MM_COUNTERS ? w.pairs[16 * lane] : 0;
   for (int o = 8; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o, 64);
   pairs = __shfl(pairs, 0, 64);
-  if (pairs > most || (st->flags & RBG_F_CAPACITY)) return;
+  const uint32_t flags = st->flags;
+  if (pairs > (flags & RBG_F_PRECOND_FAIL ? general : fast) || (flags & RBG_F_CAPACITY)) return;
   if (tid == 0 && blockIdx.x == 0) st->aux[5] = 1;
   const int64_t i = blockIdx.x;
   const int count = (int)(w.a.head[i] & MM_COUNT);
@@ -322,11 +367,9 @@ static int matmul_rows(const T* A, int64_t lda, const T* B, int64_t ldb, T* C, i
   hipLaunchKernelGGL((k_mm_plan<T>), dim3((unsigned)((rows + MM_PLAN_NT / 64 - 1) / (MM_PLAN_NT / 64))),
                      dim3(MM_PLAN_NT), 0, s, M, K, w, st);
   RBG_CHECK_LAUNCH();
-  const int64_t fit = ROWS_MM_LDS / (int64_t)sizeof(T) - 16;
-  const int64_t cells = N < fit ? N : fit;
-  const unsigned long long most = (unsigned long long)((double)M * (double)K * (double)N / ROWS_MM_PAIRS);
-  const size_t lds = (size_t)((cells + V - 1) / V * 16);
-  hipLaunchKernelGGL((k_mm_rows<T>), dim3((unsigned)M), dim3(ROWS_MM_NT), lds, s, w, C, ldc, N, cells, most, st);
+  const MmLimits l = mm_limits<T>(M, K, N);
+  hipLaunchKernelGGL((k_mm_rows<T>), dim3((unsigned)M), dim3(ROWS_MM_NT), l.lds, s, w, C, ldc, N, l.cells, l.fast,
+                     l.general, st);
   RBG_CHECK_LAUNCH();
   return 0;
 }
@@ -341,6 +384,10 @@ int64_t rbg_matmul_rows_workspace_bytes(int64_t M, int64_t K, int64_t N, int32_t
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   return elem_bytes == 8 ? mm_layout<int64_t>(M, K, N, nullptr, nullptr)
                          : mm_layout<int32_t>(M, K, N, nullptr, nullptr);
+}
+int32_t rbg_matmul_rows_fits(int64_t M, int64_t K, int64_t N, int32_t elem_bytes) {
+  if (M <= 0 || K <= 0 || N <= 0) return 0;
+  return (elem_bytes == 8 ? mm_limits<int64_t>(M, K, N) : mm_limits<int32_t>(M, K, N)).fits;
 }
 int rbg_matmul_rows_i32(const int32_t* A, int64_t lda, const int32_t* B, int64_t ldb, int32_t* C, int64_t ldc,
                         int64_t M, int64_t K, int64_t N, void* workspace, int64_t workspace_bytes, rbg_status* st,

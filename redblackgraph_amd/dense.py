@@ -206,7 +206,8 @@ MATMUL_FAST_MIN_TERMS = 1 << 24
 
 def matmul(A, B, et: ElemType, stream=None, force_general: bool = False):
     """C = A (x) B for device matrices (M x K) and (K x N).  Native-width
-    operands with few entries (closures) take rbg_matmul_rows_*; others inside
+    operands with few entries (closures) take rbg_matmul_rows_* where their
+    shape is one for it (rbg_matmul_rows_fits); others inside
     the fast domain (rbg_matmul_precheck's rules) rbg_matmul_fast_*; others,
     and a fast run whose MSB guard fails, take the general kernel with the
     full arithmetic and events."""
@@ -221,19 +222,26 @@ def matmul(A, B, et: ElemType, stream=None, force_general: bool = False):
     A = A.contiguous()
     B = B.contiguous()
     if et.native and not force_general and M * K * N >= MATMUL_FAST_MIN_TERMS:
-        # from the operands' entries, where they are few
-        ws = t.empty(int(_lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, A.element_size())), dtype=t.uint8,
-                     device=A.device)
-        _lib.call(f"rbg_matmul_rows_{sfx}", _lib.ptr(A), K, _lib.ptr(B), N, _lib.ptr(C), N, M, K, N, _lib.ptr(ws),
-                  ws.numel(), st.p, sh)
-        s = st.read(stream)
-        taken = bool(s.aux[5])
-        s.aux[5] = 0
-        if taken and not s.flags & _lib.F_NEED_GENERAL:
-            s.flags = 0
-            return C, s
-        if not taken and not s.flags & _lib.F_PRECOND_FAIL:
+        if _lib.load().rbg_matmul_rows_fits(M, K, N, A.element_size()):
+            # from the operands' entries, where they are few
+            ws = t.empty(int(_lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, A.element_size())), dtype=t.uint8,
+                         device=A.device)
+            _lib.call(f"rbg_matmul_rows_{sfx}", _lib.ptr(A), K, _lib.ptr(B), N, _lib.ptr(C), N, M, K, N,
+                      _lib.ptr(ws), ws.numel(), st.p, sh)
+            s = st.read(stream)
+            taken = bool(s.aux[5])
+            s.aux[5] = 0
+            if taken and not s.flags & _lib.F_NEED_GENERAL:
+                s.flags = 0
+                return C, s
+            blocked = not taken and not s.flags & _lib.F_PRECOND_FAIL
             del ws
+        else:
+            st.reset(stream)
+            _lib.call(f"rbg_matmul_precheck_{sfx}", _lib.ptr(A), K, M, K, st.p, sh)
+            _lib.call(f"rbg_matmul_precheck_{sfx}", _lib.ptr(B), N, K, N, st.p, sh)
+            blocked = not st.read(stream).flags & _lib.F_PRECOND_FAIL
+        if blocked:
             ws = t.empty(int(_lib.load().rbg_matmul_fast_workspace_bytes(M, K, N, A.element_size())),
                          dtype=t.uint8, device=A.device)
             st.reset(stream)

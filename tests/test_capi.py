@@ -57,3 +57,18 @@ def test_matmul_rows_workspace_of_narrow_operands(elem, M, K, N):
     from redblackgraph_amd import _lib
     need = _lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, elem)
     assert need <= (4 + elem) * (M * K + K * N) + 4 * (M + K) + 2048 + 7 * 256
+
+
+@pytest.mark.parametrize("elem", [4, 8])
+def test_matmul_shapes_for_the_entries(elem):
+    """Shapes measured: many short rows of C, or few very long ones, are the
+    blocked kernels' whatever the operands hold; closures and their blocks, and
+    short rows with many terms, are tried from the entries."""
+    from redblackgraph_amd import _lib
+    fits = _lib.load().rbg_matmul_rows_fits
+    for shape in ((1 << 22, 4, 4), (1 << 20, 16, 16), (1 << 18, 64, 64), (1 << 17, 32, 32), (4, 4, 1 << 22),
+                  (64, 64, 1 << 18)):
+        assert fits(*shape, elem) == 0, shape
+    for shape in ((300, 300, 300), (1000, 3000, 2000), (8192, 8192, 8192), (20_000, 2000, 20_000), (64, 1 << 18, 64),
+                  (4096, 64, 64), (256, 4096, 4096), (1 << 16, 256, 256), (32_000, 32_000, 32_000)):
+        assert fits(*shape, elem) == 1, shape

@@ -116,3 +116,21 @@ def test_matmul_of_closures_vs_general(dt, n):
     C, s = dense.matmul(W, W, et)
     G, g = dense.matmul(W, W, et, force_general=True)
     assert bool((C == G).all()) and s.events == g.events == 0 and s.flags == 0
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("M,K,N", [(1 << 20, 4, 4), (3, 5, 1 << 20), (300, 300, 300)])
+def test_matmul_by_shape(orc, dt, M, K, N):
+    """Products that the shape leaves to the blocked kernels, and one that it
+    does not, by the facade."""
+    rng = np.random.default_rng(M)
+    A = ((rng.random((M, K)) < 0.2) * rng.integers(2, 90, (M, K))).astype(dt)
+    B = ((rng.random((K, N)) < 0.2) * rng.integers(2, 90, (K, N))).astype(dt)
+    for diagonal in (True, False):
+        if not diagonal:  # inside the fast kernels' domain
+            np.fill_diagonal(A, 0)
+            np.fill_diagonal(B, 0)
+        C, st = dense.matmul(_lib.to_device(A), _lib.to_device(B), elem_type(dt))
+        ref, ev = orc.matmul(A, B)
+        assert int(st.events) == ev == 0
+        np.testing.assert_array_equal(C.cpu().numpy(), ref)
