@@ -14,6 +14,7 @@ from ._dtypes import ElemType, msb
 
 FW_TILE = 128
 ROWS_MAX_N = 32640  # rbg_fw_rows_max_n(): the largest order rbg_fw_rows_* takes
+ROWS_ANY_MAX_N = 16384  # and the largest with entries above the diagonal
 _tls = threading.local()
 
 

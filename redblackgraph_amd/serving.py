@@ -80,11 +80,17 @@ class Resident:
 
 
 def _dense_bytes(n: int) -> int:
-    from .dense import padded_order
+    from .dense import ROWS_ANY_MAX_N, ROWS_MAX_N, padded_order
     p = padded_order(n)
     # input copy, padded work matrix, snapshot workspace (four snapshot
-    # buffers and the persistent closure's counters)
-    return 4 * n * n + 4 * p * p + 8 * 4 * 32 * p + 4 * (p // 64) ** 2
+    # buffers and the persistent closure's counters), the rows' workspace and
+    # the second matrix of an upper triangular or unordered closure from them
+    need = 4 * n * n + 4 * p * p + 8 * 4 * 32 * p + 4 * (p // 64) ** 2
+    if n <= ROWS_MAX_N:
+        need += int(_lib.load().rbg_fw_rows_workspace_bytes(n, 4))
+    if n <= ROWS_ANY_MAX_N:
+        need += 4 * p * p
+    return need
 
 
 def _sparse_close_bytes(nnz: int, n: int) -> int:

@@ -4,7 +4,7 @@ budget."""
 import numpy as np
 import pytest
 
-from redblackgraph_amd import _lib, dense
+from redblackgraph_amd import _lib, dense, synth
 from redblackgraph_amd._dtypes import elem_type
 from redblackgraph_amd.serving import ClosureServer, synthetic_trace, summarize
 
@@ -101,3 +101,33 @@ def test_admission_within_budget():
     finally:
         alone.close()
     assert [r.digest for r in res] == [r.digest for r in res1]
+
+
+@pytest.mark.parametrize("numbering", ["lower", "upper", "any", "full"])
+@pytest.mark.parametrize("n", [100, 1500, 3000])
+def test_footprint_covers_a_dense_closure(numbering, n):
+    """What a worker allocates for a closure, its workspaces among it, is no
+    more than the footprint that admission reserved."""
+    import threading
+    from redblackgraph_amd import dense, serving
+    from redblackgraph_amd._dtypes import elem_type
+    A = synth.dense_pedigree(synth.component_spec(n), n)
+    if numbering != "lower":
+        A = synth.reverse_vertices(A) if numbering == "upper" else synth.shuffle_vertices(A, 1)
+    t = _lib.torch()
+    peak = []
+
+    def worker():  # a thread's first closure allocates its workspaces
+        stream = t.cuda.Stream()
+        with t.cuda.stream(stream):
+            t.cuda.synchronize()
+            t.cuda.reset_peak_memory_stats()
+            before = t.cuda.memory_allocated()
+            W = _lib.to_device(A)
+            dense.fw_closure(W, elem_type(np.int32), stream=stream, schedule="full" if numbering == "full" else "auto")
+            peak.append(t.cuda.max_memory_allocated() - before)
+
+    th = threading.Thread(target=worker)
+    th.start()
+    th.join()
+    assert peak[0] <= serving._dense_bytes(n) + 64 * 512  # allocations are rounded up to 512 bytes
