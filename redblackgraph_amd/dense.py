@@ -41,29 +41,42 @@ def _cached_bytes(name: str, key: tuple, nbytes, t, dev):
     return ws
 
 
+def _spare(make):
+    """The buffer that ``make`` allocates, or None where it does not fit the
+    memory: for those that a slower path does without."""
+    try:
+        return make()
+    except _lib.torch().OutOfMemoryError:
+        return None
+
+
 _ROWS_SIDES = {1: "lower", 2: "upper", 3: "full"}
 
 
 def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
     """rbg_fw_rows_* / rbg_fw_rows_any_*: the closure from the rows' direct
     entries.  Returns (closed or not, the schedule the entries' sides stand
-    for or None when they are not known, status)."""
+    for or None when they are not known, status); status None where there is
+    no room for the workspace."""
     t = _lib.torch()
     dev = _lib.device()
     elem = work.element_size()
-    ws = _cached_bytes("rows_cache", (dev.index, n, elem),
-                       lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev)
+    ws = _spare(lambda: _cached_bytes("rows_cache", (dev.index, n, elem),
+                                      lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev))
+    if ws is None:
+        return False, None, None
     sfx = "i32" if elem == 4 else "i64"
     sh = _lib.stream_handle(stream)
     _lib.call(f"rbg_fw_rows_{sfx}", _lib.ptr(src), n, src.stride(0), _lib.ptr(work), npad, _lib.ptr(ws), ws.numel(),
               st.p, sh)
     s = st.read(stream)
     if s.aux[5] > 1:
-        largest = t.empty_like(work)
-        _lib.call(f"rbg_fw_rows_any_{sfx}", n, _lib.ptr(work), _lib.ptr(largest), npad, _lib.ptr(ws), ws.numel(),
-                  st.p, sh)
-        s = st.read(stream)
-        if s.flags & _lib.F_NEED_GENERAL:
+        largest = _spare(lambda: t.empty_like(work))
+        if largest is not None:
+            _lib.call(f"rbg_fw_rows_any_{sfx}", n, _lib.ptr(work), _lib.ptr(largest), npad, _lib.ptr(ws), ws.numel(),
+                      st.p, sh)
+            s = st.read(stream)
+        if largest is None or s.flags & _lib.F_NEED_GENERAL:
             s.aux[5] = s.flags = 0
     closed, sched = bool(s.aux[5]), _ROWS_SIDES.get(int(s.aux[6]))
     s.aux[5] = s.aux[6] = 0
@@ -154,7 +167,7 @@ def fw_closure(W, et: ElemType, stream=None, force_general: bool = False, schedu
             closed, known, s = _rows_closure(src, work, n, npad, st, stream)
             if closed and not s.flags & _lib.F_NEED_GENERAL:
                 return work[:n, :n], FwOutcome(s, npad, "fast", known)
-            if closed or s.flags & _lib.F_PRECOND_FAIL:
+            if closed or (s is not None and s.flags & _lib.F_PRECOND_FAIL):
                 fast = False
     st.reset(stream)
     if fast:
@@ -223,10 +236,12 @@ def matmul(A, B, et: ElemType, stream=None, force_general: bool = False):
     A = A.contiguous()
     B = B.contiguous()
     if et.native and not force_general and M * K * N >= MATMUL_FAST_MIN_TERMS:
+        ws = None
         if _lib.load().rbg_matmul_rows_fits(M, K, N, A.element_size()):
+            size = int(_lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, A.element_size()))
+            ws = _spare(lambda: t.empty(size, dtype=t.uint8, device=A.device))
+        if ws is not None:
             # from the operands' entries, where they are few
-            ws = t.empty(int(_lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, A.element_size())), dtype=t.uint8,
-                         device=A.device)
             _lib.call(f"rbg_matmul_rows_{sfx}", _lib.ptr(A), K, _lib.ptr(B), N, _lib.ptr(C), N, M, K, N,
                       _lib.ptr(ws), ws.numel(), st.p, sh)
             s = st.read(stream)

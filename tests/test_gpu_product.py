@@ -134,3 +134,29 @@ def test_matmul_by_shape(orc, dt, M, K, N):
         ref, ev = orc.matmul(A, B)
         assert int(st.events) == ev == 0
         np.testing.assert_array_equal(C.cpu().numpy(), ref)
+
+
+def test_matmul_without_room_for_the_entries(orc, monkeypatch):
+    """Where the entries' workspace does not fit the memory the product takes
+    the kernels that need none of it."""
+    t = _lib.torch()
+    rng = np.random.default_rng(1)
+    n = 300
+    A, B = _few(rng, n, n, 3, np.int32), _few(rng, n, n, 4, np.int32)
+    size = int(_lib.load().rbg_matmul_rows_workspace_bytes(n, n, n, 4))
+    empty = t.empty
+    refused = []
+
+    def no_room(shape, *args, **kw):
+        if shape == size and kw.get("dtype") == t.uint8:
+            refused.append(shape)
+            raise t.OutOfMemoryError("no room")
+        return empty(shape, *args, **kw)
+
+    Ad, Bd = _lib.to_device(A), _lib.to_device(B)
+    monkeypatch.setattr(t, "empty", no_room)
+    C, st = dense.matmul(Ad, Bd, elem_type(np.int32))
+    monkeypatch.undo()
+    ref, ev = orc.matmul(A, B)
+    assert refused and int(st.events) == ev
+    np.testing.assert_array_equal(C.cpu().numpy(), ref)

@@ -203,3 +203,42 @@ def test_rows_closure_declines_cycles():
     Wf, outf = _full(A)
     assert out2.mode == outf.mode == "general"
     assert out2.status.cycle_last_key == outf.status.cycle_last_key
+
+
+@pytest.mark.parametrize("what", ["workspace", "second matrix"])
+@pytest.mark.parametrize("numbering", ["lower", "any"])
+def test_closure_without_room_for_the_rows(monkeypatch, what, numbering):
+    """Where the rows' workspace or the second matrix does not fit the memory
+    the blocked schedules close the matrix, as they did before."""
+    t = _lib.torch()
+    n = 700
+    A = synth.dense_pedigree(synth.PedigreeSpec(n, 10, 0.8, 2), 5)
+    if numbering == "any":
+        A = synth.shuffle_vertices(A, 3)
+    et = elem_type(np.int32)
+    Ad = _lib.to_device(A)
+    want, full = dense.fw_closure(Ad, et, schedule="full")
+    size = int(_lib.load().rbg_fw_rows_workspace_bytes(n, 4))
+    empty, like = t.empty, t.empty_like
+    refused = []
+
+    def no_room(shape, *args, **kw):
+        if what == "workspace" and shape == size and kw.get("dtype") == t.uint8:
+            refused.append(shape)
+            raise t.OutOfMemoryError("no room")
+        return empty(shape, *args, **kw)
+
+    def no_second(x, *args, **kw):
+        if what == "second matrix":
+            refused.append(tuple(x.shape))
+            raise t.OutOfMemoryError("no room")
+        return like(x, *args, **kw)
+
+    dense._tls.__dict__.pop("rows_cache", None)
+    monkeypatch.setattr(t, "empty", no_room)
+    monkeypatch.setattr(t, "empty_like", no_second)
+    W, out = dense.fw_closure(Ad, et)
+    monkeypatch.undo()
+    assert t.equal(W, want) and (out.mode, out.diameter) == (full.mode, full.diameter)
+    assert bool(refused) == (what == "workspace" or numbering == "any")
+    assert out.schedule == ("lower" if numbering == "lower" else "full")
