@@ -16,7 +16,7 @@
 // of the blocked schedules, almost all of which have an absent operand: the
 // closure is bound by reading the input and writing the result.
 //
-// Four launches, no waits between workgroups and nothing read by the host:
+// Four launches (three up to ROWS_PLACE_HERE rows), no waits between workgroups and nothing read by the host:
 //   scan    one wave per row: reads the matrix once, checks the fast domain,
 //           keeps each row's off-diagonal entries in ascending column order;
 //   levels  one workgroup: each row's level (1 + the largest level among its
@@ -33,7 +33,11 @@
 // closure) 151 / 157 at n = 100 with 12, 231 / 246 at 300 with 24, 274 / 563
 // at 1000 with 25, 451 / 1489 at 2000 with 50, 1511 / 3747 at 4000 with 100
 // and 7603 / 10283 at 8000 with 200, each growing with the entries.  A matrix
-// not taken pays for the scan and the level pass, 2-20 us.  A path of L edges
+// not taken pays for the scan, which the blocked closure's load then repeats, and
+// for the level pass: 20 us of 250 at n = 300 with 28, 70 of 10270 at 8000 with
+// 204, and up to 110 of 305 where rows of ten entries lie in 28 levels (n = 200,
+// unordered); one of another numbering that is tried and has too many cells above
+// its largest value (rows_first_value) for two passes more, 10 to 20%.  A path of L edges
 // has a value of L bits at least, so a graph deeper than 64 levels overflows
 // (general mode) unless it is full of shortcuts, which are entries.
 #include "fw_kernels.hpp"
@@ -63,6 +67,7 @@ enum : uint32_t {
   STOP_WIDE = 16,        // more than rows_slots(n) entries
   ROW_BELOW = 32,        // with ROW_STOP: an entry below the diagonal
   ROW_ABOVE = 64,        // above it
+  ROW_THIRD = 128,       // (level pass) some row has more than two entries
   REC_UPPER = 1u << 26,  // in RowRec::p1_cnt: an entry above the diagonal
 };
 __host__ __device__ inline int rec_cnt(uint32_t w) { return (int)((w >> 16) & 0xff); }
@@ -254,7 +259,7 @@ struct LevelShared {
 // 93 us with one row per thread and pass, chunk by chunk, and 66 us with the
 // records moved here, eight unrolled; N = 512: 12 us).  Returns the STOP_*
 // reasons (or 2: too deep), 0 when the positions are in w.pos; `sides` has 1
-// when entries lie below the diagonal, 2 above.
+// when entries lie below the diagonal, 2 above, 4 when a row has more than two.
 template <typename T, int H>
 __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev, int& sides) {
   const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, n = (int)n64;
@@ -273,7 +278,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
     lv[h] = 0;
   }
-  int facts = 0;  // STOP_*, ROW_BELOW, ROW_ABOVE
+  int facts = 0;  // STOP_*, ROW_BELOW, ROW_ABOVE, ROW_THIRD
   bool more = false;
 #pragma unroll
   for (int x = 0; x < 4 * H; x++) {
@@ -287,6 +292,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     }
     const bool m = (e[x] & ROW_MORE) != 0;
     more |= m;
+    if (m) facts |= ROW_THIRD;
     if (c0 != ROW_NONE) facts |= (int)c0 < row ? ROW_BELOW : ROW_ABOVE;
     if (c1 != ROW_NONE) facts |= (int)c1 < row ? ROW_BELOW : ROW_ABOVE;
     if (m && (w.rec0[row].p1_cnt & REC_UPPER)) facts |= ROW_ABOVE;
@@ -329,7 +335,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
       }
     }
     int mark = (__any(changed) ? 1 : 0) | (__any(worst >= ROWS_MAX_LEVELS) ? 2 : 0);
-    for (int k = 3; k < 7; k++) mark |= __any(facts & (1 << k)) ? 1 << k : 0;
+    for (int k = 3; k < 8; k++) mark |= __any(facts & (1 << k)) ? 1 << k : 0;
     if (mark && lane == 0) atomicOr(&L.marks[it & 3], mark);
     if (tid == 0) L.marks[(it + 2) & 3] = 0;  // read two sweeps ago, marked two sweeps on
     __syncthreads();

@@ -15,18 +15,47 @@ static __global__ __launch_bounds__(NT) void k_rows_scan(const T* A, int64_t n, 
 // 127.6 -> 131.3, where one CU moves too many records).
 constexpr int64_t ROWS_PLACE_HERE = 2048;
 
+// Entries times levels above which a matrix of another numbering with a row of
+// more than two entries is not tried:
+// the more paths and the longer, the more cells have a largest path value above
+// the largest final value (see rows_first_value), and the passes that find out
+// that they are too many take up to half of the blocked closure's time again.
+// Rows of k entries, unordered int32, us by the rows / blocked (f: tried and not
+// closed, the blocked closure's included): n = 200, 6 levels, k = 10 (49 n) 185 /
+// 307; 14 levels, k = 6 (76 n) 213 / 306, k = 8 (101 n) 362 / 308; n = 300, 14
+// levels, k = 8 (103 n) 413 / 418, k = 10 (128 n) 616 / 415; n = 1000, 14 levels,
+// k = 5 (65 n) 345 / 1005, k = 6 (78 n) 1195 f / 1002; n = 6000, 6 levels, k = 10
+// (50 n) 849 / 24220, 14 levels, k = 6 (78 n) 24930 f / 24250; n = 8000, 6
+// levels, k = 200 (1000 n) 84070 f / 52110.
+// (int64, whose blocked closure takes half as long again: n = 200, 14 levels, k =
+// 8 (101 n) 367 / 452, k = 10 (128 n) 622 / 453.)
+template <typename T>
+static int64_t rows_any_work(int64_t n) {
+  return (n < 1000 ? (sizeof(T) == 8 ? 110 : 100) : 70) * n;
+}
+
 // Also writes the whole status block.  aux[6]: 1 the matrix is lower
 // triangular, 2 upper, 3 has entries on both sides (0: not looked at).  ctl[0]
 // and aux[5]: the same where it is closed from its rows, else 0.
 template <typename T, int H>
 static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n, RowsWork<T> w, bool allowed,
-                                                                     rbg_status* st) {
+                                                                     int64_t any_work, rbg_status* st) {
   extern __shared__ __align__(16) uint8_t lev[];
   __shared__ LevelShared L;
+  __shared__ int entries;
   int sides = 0;
   const int stop = allowed ? rows_levels<T, H>(w, n, L, lev, sides) : 1;
   const int side = sides & 2 ? (sides & 1 ? 3 : 2) : 1;
-  const int code = stop || (side > 1 && n > ROWS_ANY_MAX_N) ? 0 : side;
+  int code = stop || (side > 1 && n > ROWS_ANY_MAX_N) ? 0 : side;
+  if (code > 1 && (sides & 4)) {  // uniform, as is what follows
+    if (threadIdx.x == 0) entries = 0;
+    __syncthreads();
+    int mine = 0;
+    for (int64_t i = threadIdx.x; i < n; i += ROWS_LEVEL_NT) mine += rec_cnt(w.rec0[i].p1_cnt);
+    if (mine) atomicAdd(&entries, mine);
+    __syncthreads();
+    if ((int64_t)entries * w.ctl[1] > any_work) code = 0;
+  }
   if (code && n <= ROWS_PLACE_HERE) {
     __syncthreads();  // every row's position
     for (int64_t i = threadIdx.x; i < n; i += ROWS_LEVEL_NT) rows_place<T>(w, i);
@@ -70,23 +99,38 @@ static __global__ __launch_bounds__(ROWS_CLOSE_NT, LARGEST ? 4 : 8) void k_rows_
   rows_close_slab<T, 1, LARGEST, false>(L, w, W, W2, ld, rows_slab_of(blockIdx.x, gridDim.x), width, st);
 }
 
-// The slab's cells whose largest path value is above the largest final value.
+// The slab's cells whose largest path value is above the largest final value;
+// a wave's at a time, and no more once they are too many.
 template <typename T>
 static __global__ __launch_bounds__(NT) void k_rows_select(int64_t n, RowsWork<T> w, const T* W2, int64_t ld,
                                                           const rbg_status* st) {
   constexpr int V = 16 / (int)sizeof(T);
   const T top = (T)st->diameter_max;
   if (w.ctl[0] < 2 || w.slab_top[blockIdx.x] <= top) return;
+  const int lane = threadIdx.x & 63;
   const int64_t j = blockIdx.x * rows_slab<T>() + (threadIdx.x % ROWS_LANES) * V;
   for (int64_t i = threadIdx.x / ROWS_LANES; i < n; i += NT / ROWS_LANES) {
     T z[V];
     rows_ld<T, V>(W2 + i * ld + j, z);
+    uint64_t above[V];
+    int all = 0;
 #pragma unroll
-    for (int x = 0; x < V; x++)
-      if (z[x] > top) {
-        const uint32_t at = atomicAdd(&w.cells[0], 1u);
-        if (at < ROWS_MAX_CELLS) w.cells[1 + at] = (uint32_t)i | (uint32_t)(j + x) << 16;
-      }
+    for (int x = 0; x < V; x++) {
+      above[x] = __ballot(z[x] > top);
+      all += __popcll(above[x]);
+    }
+    if (all == 0) continue;
+    // the lanes at row i < n are the wave's first ones
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&w.cells[0], (uint32_t)all);
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (at >= ROWS_MAX_CELLS) return;
+#pragma unroll
+    for (int x = 0; x < V; x++) {
+      const uint32_t mine = at + (uint32_t)__popcll(above[x] & (((uint64_t)1 << lane) - 1));
+      if (z[x] > top && mine < ROWS_MAX_CELLS) w.cells[1 + mine] = (uint32_t)i | (uint32_t)(j + x) << 16;
+      at += (uint32_t)__popcll(above[x]);
+    }
   }
 }
 
@@ -144,11 +188,14 @@ static int fw_rows(const T* A, int64_t n, int64_t lda, T* W, int64_t npad, void*
   const bool allowed = g_flow_limit_override.load() == 0;
   const size_t lds = (size_t)(n + 4);
   if (n <= 8 * ROWS_LEVEL_NT)
-    hipLaunchKernelGGL((k_rows_levels<T, 2>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
+    hipLaunchKernelGGL((k_rows_levels<T, 2>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed,
+                       rows_any_work<T>(n), st);
   else if (n <= 16 * ROWS_LEVEL_NT)
-    hipLaunchKernelGGL((k_rows_levels<T, 4>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
+    hipLaunchKernelGGL((k_rows_levels<T, 4>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed,
+                       rows_any_work<T>(n), st);
   else
-    hipLaunchKernelGGL((k_rows_levels<T, 8>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed, st);
+    hipLaunchKernelGGL((k_rows_levels<T, 8>), dim3(1), dim3(ROWS_LEVEL_NT), lds, s, n, w, allowed,
+                       rows_any_work<T>(n), st);
   RBG_CHECK_LAUNCH();
   if (n > ROWS_PLACE_HERE) {
     hipLaunchKernelGGL((k_rows_place<T>), dim3((unsigned)((n + NT - 1) / NT)), dim3(NT), 0, s, n, w);

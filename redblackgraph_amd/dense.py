@@ -41,15 +41,6 @@ def _cached_bytes(name: str, key: tuple, nbytes, t, dev):
     return ws
 
 
-def _spare(make):
-    """The buffer that ``make`` allocates, or None where it does not fit the
-    memory: for those that a slower path does without."""
-    try:
-        return make()
-    except _lib.torch().OutOfMemoryError:
-        return None
-
-
 _ROWS_SIDES = {1: "lower", 2: "upper", 3: "full"}
 
 
@@ -61,9 +52,10 @@ def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
     t = _lib.torch()
     dev = _lib.device()
     elem = work.element_size()
-    ws = _spare(lambda: _cached_bytes("rows_cache", (dev.index, n, elem),
-                                      lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev))
-    if ws is None:
+    try:
+        ws = _cached_bytes("rows_cache", (dev.index, n, elem),
+                           lambda: int(_lib.load().rbg_fw_rows_workspace_bytes(n, elem)), t, dev)
+    except t.OutOfMemoryError:
         return False, None, None
     sfx = "i32" if elem == 4 else "i64"
     sh = _lib.stream_handle(stream)
@@ -71,13 +63,16 @@ def _rows_closure(src, work, n: int, npad: int, st: _lib.Status, stream):
               st.p, sh)
     s = st.read(stream)
     if s.aux[5] > 1:
-        largest = _spare(lambda: t.empty_like(work))
-        if largest is not None:
+        try:
+            largest = t.empty_like(work)
+        except t.OutOfMemoryError:
+            s.aux[5] = 0
+        else:
             _lib.call(f"rbg_fw_rows_any_{sfx}", n, _lib.ptr(work), _lib.ptr(largest), npad, _lib.ptr(ws), ws.numel(),
                       st.p, sh)
             s = st.read(stream)
-        if largest is None or s.flags & _lib.F_NEED_GENERAL:
-            s.aux[5] = s.flags = 0
+            if s.flags & _lib.F_NEED_GENERAL:
+                s.aux[5] = s.flags = 0
     closed, sched = bool(s.aux[5]), _ROWS_SIDES.get(int(s.aux[6]))
     s.aux[5] = s.aux[6] = 0
     return closed, sched, s
@@ -239,7 +234,10 @@ def matmul(A, B, et: ElemType, stream=None, force_general: bool = False):
         ws = None
         if _lib.load().rbg_matmul_rows_fits(M, K, N, A.element_size()):
             size = int(_lib.load().rbg_matmul_rows_workspace_bytes(M, K, N, A.element_size()))
-            ws = _spare(lambda: t.empty(size, dtype=t.uint8, device=A.device))
+            try:
+                ws = t.empty(size, dtype=t.uint8, device=A.device)
+            except t.OutOfMemoryError:
+                pass
         if ws is not None:
             # from the operands' entries, where they are few
             _lib.call(f"rbg_matmul_rows_{sfx}", _lib.ptr(A), K, _lib.ptr(B), N, _lib.ptr(C), N, M, K, N,

@@ -242,3 +242,86 @@ def test_closure_without_room_for_the_rows(monkeypatch, what, numbering):
     assert t.equal(W, want) and (out.mode, out.diameter) == (full.mode, full.diameter)
     assert bool(refused) == (what == "workspace" or numbering == "any")
     assert out.schedule == ("lower" if numbering == "lower" else "full")
+
+
+def _closed(A):
+    """(closed from the rows or not, W) of the rows' launches alone, and the
+    whole closure against the full schedule's."""
+    t = _lib.torch()
+    et = elem_type(A.dtype)
+    n, npad = len(A), dense.padded_order(len(A))
+    Ad = _lib.to_device(A)
+    work = t.empty((npad, npad), dtype=Ad.dtype, device=Ad.device)
+    closed, sched, st = dense._rows_closure(Ad, work, n, npad, dense.status(), None)
+    want, full = dense.fw_closure(Ad, et, schedule="full")
+    got, out = dense.fw_closure(Ad, et)
+    assert t.equal(got, want) and (out.mode, out.diameter) == (full.mode, full.diameter)
+    if closed:
+        assert t.equal(work[:n, :n], want) and int(st.diameter_max) == int(out.status.diameter_max)
+    return closed
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("many,closed", [(4096, True), (4097, False), (6000, False)])
+def test_rows_closure_cells_above_the_largest_value(dt, many, closed):
+    """A chain of ten, and vertices that reach its head both at once and by
+    the whole chain: the longer way's value is above every final one, a cell
+    for each; up to 4,096 such cells have their first values looked up."""
+    m = 10
+    n = m + 1 + many
+    A = np.zeros((n, n), dtype=dt)
+    i = np.arange(1, m + 1)
+    A[i, i - 1] = 3
+    A[m + 1:, m] = 3
+    A[m + 1:, 0] = 2
+    A[np.arange(n), np.arange(n)] = 1
+    assert _closed(synth.shuffle_vertices(A, 1)) == closed
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("depth,closed", [(8, True), (9, True), (10, False)])
+def test_rows_closure_vertices_between(dt, depth, closed):
+    """A vertex that reaches another at once and through a binary tree: up to
+    1,024 vertices between the two are looked through for the first value."""
+    tree = 2 ** (depth + 1) - 1  # vertex 0 its root
+    leaf, j = tree, tree + 1
+    A = np.zeros((tree + 2, tree + 2), dtype=dt)
+    v = np.arange(2 ** depth - 1)
+    A[v, 2 * v + 1] = 2
+    A[v, 2 * v + 2] = 3
+    A[2 ** depth - 1:tree, leaf] = 2
+    A[leaf, j] = 3
+    A[0, j] = 2
+    A[np.arange(tree + 2), np.arange(tree + 2)] = -1
+    assert (tree - 1 + 1 <= 1024) == closed
+    assert _closed(synth.shuffle_vertices(A, 2)) == closed
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("n,layers,lookback", [(40, 5, 1), (100, 7, 3), (700, 10, 2), (1500, 24, 4), (3000, 12, 1)])
+def test_rows_closure_takes_pedigrees(dt, n, layers, lookback):
+    """Pedigrees are closed from their rows in every numbering."""
+    A = synth.dense_pedigree(synth.PedigreeSpec(n, layers, 0.8, lookback), n, dtype=dt)
+    for M in (A, synth.reverse_vertices(A), synth.shuffle_vertices(A, 1), synth.shuffle_vertices(A, 2)):
+        assert _closed(M)
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("n,layers,entries,tried", [(1200, 6, 8, True), (1200, 14, 12, False), (300, 6, 10, True),
+                                                    (300, 20, 12, False)])
+def test_rows_closure_of_many_paths(monkeypatch, dt, n, layers, entries, tried):
+    """Rows of many entries: with few levels closed from them in every
+    numbering, with many only where it is lower triangular, and then the passes
+    for the other numberings are not run in vain."""
+    rng = np.random.default_rng(n)
+    bounds = np.linspace(0, n, layers + 1).astype(int)
+    A = np.zeros((n, n), dtype=dt)
+    for lo, hi in zip(bounds[1:-1], bounds[2:]):
+        for i in range(lo, hi):
+            A[i, rng.integers(0, lo, entries)] = rng.integers(2, 4, entries)
+    A[np.arange(n), np.arange(n)] = -1
+    assert _closed(A)
+    said, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda fn, *args: (said.append(fn), call(fn, *args))[1])
+    assert _closed(synth.shuffle_vertices(A, 3)) == _closed(synth.reverse_vertices(A)) == tried
+    assert any(fn.startswith("rbg_fw_rows_any") for fn in said) == tried
