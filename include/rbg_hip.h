@@ -181,8 +181,8 @@ int rbg_fw_load_i64(const int64_t *A, int64_t n, int64_t lda, int64_t *W, int64_
  * st->aux[5] = 1 (every off-diagonal entry below the diagonal), 2 (above) or 3
  * (both), and with
  *   1  the closure (natural values) is written into columns [0, n) of rows
- *      [0, n) of W (row stride npad, a multiple of 128, 16-byte aligned; the
- *      rest of W is unspecified) and st->diameter_max = the max trajectory
+ *      [0, n) of W (row stride npad, a multiple of 128, 16-byte aligned, n rows
+ *      within 64 GiB; the rest of W is unspecified) and st->diameter_max = the max trajectory
  *      value; RBG_F_NEED_GENERAL then asks for mode 1 as for rbg_fw_dense_*;
  *   2, 3  rbg_fw_rows_any_*, with the same W, workspace and st, writes them.
  *      W2 is a second matrix like W (scratch).  st->aux[5] = 0 after it, or

@@ -165,6 +165,8 @@ static int rows_args(const void* A, int64_t n, const T* W, int64_t npad, void* w
   if (!A || !W || !wsp || !st || n <= 0 || n > ROWS_MAX_N || npad < n || npad % TILE || ((uintptr_t)W & 15) ||
       ((uintptr_t)wsp & 255))
     return RBG_E_ARG;
+  // the close pass counts 16-byte units in 32 bits
+  if (npad / (16 / (int64_t)sizeof(T)) > 0xffffffffll / n) return RBG_E_ARG;
   return ws_bytes < rows_layout<T>(n, (char*)wsp, w) ? RBG_E_WORKSPACE : 0;
 }
 

@@ -72,3 +72,20 @@ def test_matmul_shapes_for_the_entries(elem):
     for shape in ((300, 300, 300), (1000, 3000, 2000), (8192, 8192, 8192), (20_000, 2000, 20_000), (64, 1 << 18, 64),
                   (4096, 64, 64), (256, 4096, 4096), (1 << 16, 256, 256), (32_000, 32_000, 32_000)):
         assert fits(*shape, elem) == 1, shape
+
+
+@pytest.mark.parametrize("sfx,elem", [("i32", 4), ("i64", 8)])
+def test_rows_closure_refuses_a_row_stride_past_its_indices(sfx, elem):
+    """The close pass counts 16-byte units of the matrix in 32 bits: a stride
+    that carries n rows past them is an argument error, with no launch."""
+    from redblackgraph_amd import _lib
+    L = _lib.load()
+    n = 32_640
+    fake = 1 << 20  # never read: the arguments are refused
+    room = int(L.rbg_fw_rows_workspace_bytes(n, elem))
+    stride = (1 << 32) // n * (16 // elem) // 128 * 128
+    over = stride + 256
+    for npad in (over, 1 << 31):
+        assert getattr(L, f"rbg_fw_rows_{sfx}")(fake, n, n, fake, npad, fake, room, fake, None) == -1
+    over = (1 << 32) // 16_384 * (16 // elem) // 128 * 128 + 256
+    assert getattr(L, f"rbg_fw_rows_any_{sfx}")(16_384, fake, fake, over, fake, room, fake, None) == -1
