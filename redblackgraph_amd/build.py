@@ -53,9 +53,16 @@ def shift_hazards(asm: str):
     return found
 
 
-def _check_asm(src: str, objdir: str) -> None:
+def _asm_paths(src: str, objdir: str):
     stem = os.path.splitext(os.path.basename(src))[0]
-    for path in glob.glob(os.path.join(objdir, f"{stem}-hip-amdgcn-*gfx950*.s")):
+    return glob.glob(os.path.join(objdir, f"{stem}-hip-amdgcn-*gfx950*.s"))
+
+
+def _check_asm(src: str, objdir: str) -> None:
+    paths = _asm_paths(src, objdir)
+    if not paths:
+        raise RuntimeError(f"{src}: no device assembly to check in {objdir}")
+    for path in paths:
         with open(path) as f:
             bad = shift_hazards(f.read())
         if bad:
@@ -75,6 +82,8 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
     for src in sources():
         obj = os.path.join(objdir, os.path.basename(src) + ".o")
         objs.append(obj)
+        for old in _asm_paths(src, objdir):  # the check reads this build's
+            os.remove(old)
         cmd = [HIPCC, *FLAGS, "--save-temps=obj", "-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

@@ -1,5 +1,7 @@
 """The build's check of the device assembly.  CPU only."""
-from redblackgraph_amd.build import shift_hazards
+import pytest
+
+from redblackgraph_amd.build import _check_asm, shift_hazards
 
 _ASM = """
 _Z3fooPl:
@@ -22,3 +24,16 @@ def test_other_shifts_pass():
     assert shift_hazards(_ASM.format(amount=135, vgprs=144)) == []
     assert shift_hazards(_ASM.format(amount=131, vgprs=132)) == []
     assert shift_hazards(_ASM.replace("v{amount}", "s4").format(vgprs=136)) == []
+
+
+def test_check_needs_the_assembly(tmp_path):
+    """A build whose temporaries have other names is not passed unchecked."""
+    src = str(tmp_path / "rbg_foo.hip")
+    with pytest.raises(RuntimeError, match="no device assembly"):
+        _check_asm(src, str(tmp_path))
+    asm = tmp_path / "rbg_foo-hip-amdgcn-amd-amdhsa-gfx950.s"
+    asm.write_text(_ASM.format(amount=134, vgprs=136))
+    _check_asm(src, str(tmp_path))
+    asm.write_text(_ASM.format(amount=135, vgprs=136))
+    with pytest.raises(RuntimeError, match="64-bit shift"):
+        _check_asm(src, str(tmp_path))
