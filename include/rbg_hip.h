@@ -8,8 +8,9 @@
  *   - Every call is asynchronous on `stream` and performs no host
  *     synchronisation, so it may be captured into a hipGraph -- except the
  *     ones whose comment says they wait (the DAG closure's completion test,
- *     the topological sort's round test, the components' round test, the
- *     batched plan's descriptor upload).
+ *     the topological sort's round test, the batched plan's descriptor upload,
+ *     rbg_batch_run and rbg_batch_replay outside a capture,
+ *     rbg_batch_rows_closed).
  *   - Return value: 0 on success, an RBG_E_* code for argument errors, or a
  *     hipError_t (>0) from a failed launch.
  *   - Arithmetic errors (cycles, overflow) are reported through the device
@@ -541,9 +542,11 @@ int64_t rbg_batch_flow_tickets(const int32_t *npad, const int32_t *edge, int32_t
                                int64_t cap);
 int rbg_batch_create(const rbg_batch_comp *comps, int32_t count, rbg_batch **out);
 int rbg_batch_info(const rbg_batch *b, int64_t *info);
-/* Queues one run.  Outside a capture the call may wait, for no longer than
- * loading the pool and the other schedules' idle launches take, for word that all components were
- * closed from their rows' entries; the launches behind are then not queued. */
+/* Queues one run.  Outside a capture the call (like rbg_batch_replay) may wait,
+ * yielding the processor, for no longer than loading the pool and the other
+ * schedules' idle launches take, for word that all components were closed from
+ * their rows' entries; the launches behind are then not queued.  A run that the
+ * caller records into a graph of its own never waits: every launch is queued. */
 int rbg_batch_run(rbg_batch *b, rbg_stream_t stream);
 /* closed[i] = 1 where the last run closed component i from its rows' entries
  * (count entries, host memory); waits for the stream. */

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <chrono>
 #include <numeric>
+#include <thread>
 
 #include "fw_rows.hpp"
 
@@ -426,6 +427,7 @@ static bool batch_rows_told(const rbg_batch* b, int64_t ticket) {
     const int64_t v = __atomic_load_n(b->told, __ATOMIC_ACQUIRE);
     if (v == ticket || v == -ticket) return v > 0;
     if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(limit_us)) return false;
+    std::this_thread::yield();
   }
 }
 

@@ -17,6 +17,7 @@
 
 #include <chrono>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 namespace rbg {
@@ -2818,6 +2819,7 @@ struct ToldWord {
     for (;;) {
       const int64_t v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
       if (v || std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) return v;
+      std::this_thread::yield();
     }
   }
   static std::mutex& lock() {
