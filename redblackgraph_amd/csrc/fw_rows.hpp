@@ -67,7 +67,6 @@ enum : uint32_t {
   STOP_WIDE = 16,        // more than rows_slots(n) entries
   ROW_BELOW = 32,        // with ROW_STOP: an entry below the diagonal
   ROW_ABOVE = 64,        // above it
-  ROW_THIRD = 128,       // (level pass) some row has more than two entries
   REC_UPPER = 1u << 26,  // in RowRec::p1_cnt: an entry above the diagonal
 };
 __host__ __device__ inline int rec_cnt(uint32_t w) { return (int)((w >> 16) & 0xff); }
@@ -245,6 +244,7 @@ struct LevelShared {
   int hist[ROWS_MAX_LEVELS];
   int next[ROWS_MAX_LEVELS];
   int marks[4];
+  int third;
 };
 
 // Level and position of every row, by one workgroup of at least 64 threads
@@ -259,11 +259,13 @@ struct LevelShared {
 // 93 us with one row per thread and pass, chunk by chunk, and 66 us with the
 // records moved here, eight unrolled; N = 512: 12 us).  Returns the STOP_*
 // reasons (or 2: too deep), 0 when the positions are in w.pos; `sides` has 1
-// when entries lie below the diagonal, 2 above, 4 when a row has more than two.
+// when entries lie below the diagonal, 2 above; L.third tells whether a row has
+// more than two.
 template <typename T, int H>
 __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, uint8_t* lev, int& sides) {
   const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, n = (int)n64;
   if (tid < 4) L.marks[tid] = 0;
+  if (tid == 0) L.third = 0;
   if (tid < ROWS_MAX_LEVELS) L.hist[tid] = 0;
   uint32_t e[4 * H];
   uint32_t lv[H];  // four levels each
@@ -278,7 +280,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     e[4 * h] = q.x, e[4 * h + 1] = q.y, e[4 * h + 2] = q.z, e[4 * h + 3] = q.w;
     lv[h] = 0;
   }
-  int facts = 0;  // STOP_*, ROW_BELOW, ROW_ABOVE, ROW_THIRD
+  int facts = 0;  // STOP_*, ROW_BELOW, ROW_ABOVE
   bool more = false;
 #pragma unroll
   for (int x = 0; x < 4 * H; x++) {
@@ -292,7 +294,6 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     }
     const bool m = (e[x] & ROW_MORE) != 0;
     more |= m;
-    if (m) facts |= ROW_THIRD;
     if (c0 != ROW_NONE) facts |= (int)c0 < row ? ROW_BELOW : ROW_ABOVE;
     if (c1 != ROW_NONE) facts |= (int)c1 < row ? ROW_BELOW : ROW_ABOVE;
     if (m && (w.rec0[row].p1_cnt & REC_UPPER)) facts |= ROW_ABOVE;
@@ -300,6 +301,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
   }
   __syncthreads();
   if (tid == 0) lev[n] = 255;  // an absent entry's level: below 0
+  if (more) L.third = 1;
   __syncthreads();
   for (int it = 0;; it++) {
     bool changed = false;
@@ -335,7 +337,7 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
       }
     }
     int mark = (__any(changed) ? 1 : 0) | (__any(worst >= ROWS_MAX_LEVELS) ? 2 : 0);
-    for (int k = 3; k < 8; k++) mark |= __any(facts & (1 << k)) ? 1 << k : 0;
+    for (int k = 3; k < 7; k++) mark |= __any(facts & (1 << k)) ? 1 << k : 0;
     if (mark && lane == 0) atomicOr(&L.marks[it & 3], mark);
     if (tid == 0) L.marks[(it + 2) & 3] = 0;  // read two sweeps ago, marked two sweeps on
     __syncthreads();

@@ -47,7 +47,7 @@ static __global__ __launch_bounds__(ROWS_LEVEL_NT) void k_rows_levels(int64_t n,
   const int stop = allowed ? rows_levels<T, H>(w, n, L, lev, sides) : 1;
   const int side = sides & 2 ? (sides & 1 ? 3 : 2) : 1;
   int code = stop || (side > 1 && n > ROWS_ANY_MAX_N) ? 0 : side;
-  if (code > 1 && (sides & 4)) {  // uniform, as is what follows
+  if (code > 1 && L.third) {  // uniform, as is what follows
     if (threadIdx.x == 0) entries = 0;
     __syncthreads();
     int mine = 0;
