@@ -310,22 +310,39 @@ __device__ inline int rows_levels(RowsWork<T> w, int64_t n64, LevelShared& L, ui
     for (int h = 0; h < H; h++) {
       if (4 * h * nt >= n) continue;  // no row of any thread
       const int row = 4 * (h * nt + tid);
-      uint32_t nv = 0;
+      uint32_t nv = 0, third = 0;
 #pragma unroll
       for (int x = 0; x < 4; x++) {
         const uint32_t ex = e[4 * h + x];
         const int l0 = (uint8_t)(lev[ex & 0xffff] + 1), l1 = (uint8_t)(lev[(ex >> 16) & 0x7fff] + 1);
-        int nl = l0 > l1 ? l0 : l1;
-        if (more && ex >> 31) {
-          const int cnt = rec_cnt(w.rec0[row + x].p1_cnt);
-          const int32_t* ec = w.ecol + (int64_t)(row + x) * w.slots;
-          for (int k = 2; k < cnt; k++) {
-            const int y = lev[ec[k]] + 1;
+        const int nl = l0 > l1 ? l0 : l1;
+        third |= (ex >> 31) << x;
+        worst = nl > worst ? nl : worst;
+        nv |= (uint32_t)nl << (8 * x);
+      }
+      while (third) {  // rows with further entries, four by a load
+        const int x = __builtin_ctz(third);
+        third &= third - 1;
+        int nl = (int)(nv >> (8 * x) & 0xff);
+        const int cnt = rec_cnt(w.rec0[row + x].p1_cnt);
+        const int32_t* ec = w.ecol + (int64_t)(row + x) * w.slots;
+        int k = 2;
+        for (; k + 4 <= cnt; k += 4) {
+          int c[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++) c[q] = ec[k + q];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int y = lev[c[q]] + 1;
             nl = nl > y ? nl : y;
           }
         }
+        for (; k < cnt; k++) {
+          const int y = lev[ec[k]] + 1;
+          nl = nl > y ? nl : y;
+        }
         worst = nl > worst ? nl : worst;
-        nv |= (uint32_t)nl << (8 * x);
+        nv = (nv & ~(0xffu << (8 * x))) | (uint32_t)(nl & 0xff) << (8 * x);
       }
       if (nv != lv[h]) {
         lv[h] = nv;
