@@ -18,6 +18,8 @@
 namespace rbg {
 
 constexpr int CC_HOOKS = 2;  // hooking passes before the join (100 + 115 us; one: 56 + 296, three: 110 + 114)
+constexpr int32_t CC_SMALL = 1024;  // vertices up to which they cost more than they save (n = 300: 45 us without, 80 with; 4096, 8 edges each: 448, 78)
+constexpr int CC_STEPS = 64;  // of a compression before the last
 
 // A first forest: each vertex under the first vertex of its row, if smaller
 // (in a closed graph numbered parents first, a founder of its own).
@@ -116,10 +118,14 @@ static __global__ __launch_bounds__(256) void k_cc_join(const int64_t* __restric
   }
 }
 
-static __global__ void k_cc_compress(int32_t* lab, int32_t n) {
+// Every vertex under its root, or `most` labels up its way: a first forest may
+// be one long path (vertices in a row, each under the one before), whose walk
+// to the root would be as long for the last of them.  64 a pass shorten the path
+// 64 times a pass, and a vertex left on the way is under one of its own tree.
+static __global__ void k_cc_compress(int32_t* lab, int32_t n, int32_t most) {
   for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
     int32_t x = cc_load(&lab[v]), p = cc_load(&lab[x]);
-    while (p != x) {
+    for (int32_t step = 1; p != x && step < most; step++) {
       x = p;
       p = cc_load(&lab[x]);
     }
@@ -143,17 +149,17 @@ int rbg_components(const int64_t* indptr, const int32_t* indices, int32_t n, int
   const int join_grid = (int)((n + 3) / 4 < 8192 ? (n + 3) / 4 : 8192);  // a wave per vertex
   hipLaunchKernelGGL(k_cc_init, dim3(grid), dim3(256), 0, s, indptr, indices, labels, n);
   RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n);
+  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n, CC_STEPS);
   RBG_CHECK_LAUNCH();
-  for (int32_t r = 0; r < CC_HOOKS; r++) {
+  for (int32_t r = 0; r < CC_HOOKS && n > CC_SMALL; r++) {
     hipLaunchKernelGGL(k_cc_hook, dim3(grid), dim3(256), 0, s, indptr, indices, n, 1 + r % 2, labels);
     RBG_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n);
+    hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n, CC_STEPS);
     RBG_CHECK_LAUNCH();
   }
   hipLaunchKernelGGL(k_cc_join, dim3(join_grid), dim3(256), 0, s, indptr, indices, n, labels);
   RBG_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n);
+  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(256), 0, s, labels, n, 0x7fffffff);
   RBG_CHECK_LAUNCH();
   if (rounds) *rounds = 1;
   return 0;

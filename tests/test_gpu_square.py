@@ -204,3 +204,52 @@ def test_square_count_stops_at_the_limit(dt):
             assert ms(lambda: count(R)) < 0.5 * ms(lambda: _plain(R, False))
         R = _plain(R, False)
     assert declined >= 2
+
+
+@pytest.mark.parametrize("n", [5, 1024, 1025, 4097, 300_000])
+@pytest.mark.parametrize("shape", ["path", "path down", "two paths", "comb", "random"])
+def test_components_of_long_paths(n, shape):
+    """Vertices in a row, each joined to the one before: first forests as deep
+    as the graph, alone, two of them crossing, with teeth, and none."""
+    from scipy.sparse.csgraph import connected_components
+    rng = np.random.default_rng(n)
+    r, c = np.arange(1, n), np.arange(n - 1)
+    if shape == "path down":
+        r, c = c, r
+    elif shape == "two paths":  # even and odd vertices, joined by the last edge
+        r, c = np.r_[np.arange(2, n), n - 1], np.r_[np.arange(n - 2), n - 2]
+    elif shape == "comb":  # every third vertex hangs from the first third's path
+        k = max(1, n // 3)
+        r, c = np.r_[np.arange(1, k), np.arange(k, n)], np.r_[np.arange(k - 1), np.arange(n - k) % k]
+    elif shape == "random":
+        r, c = rng.integers(0, n, n // 2), rng.integers(0, n, n // 2)
+    S = sp.csr_matrix((np.ones(len(r), np.int32), (r, c)), shape=(n, n))
+    S.sort_indices()
+    lab = _labels(S)
+    _, comp = connected_components(S, directed=False)
+    least = np.full(comp.max() + 1, n)
+    np.minimum.at(least, comp, np.arange(n))
+    np.testing.assert_array_equal(lab, least[comp])
+
+
+def test_components_of_a_long_path_cost_no_walk():
+    """A path of a million vertices in their order takes about as long as one in
+    a shuffled order (a walk down the whole path took ten times)."""
+    from redblackgraph_amd.sparse.csgraph._components import _device_labels_dev
+    t = _lib.torch()
+    n = 1_000_000
+    q = np.random.default_rng(1).permutation(n)
+
+    def ms(r, c):
+        A = sd.from_scipy(sp.csr_matrix((np.ones(n - 1, np.int32), (r, c)), shape=(n, n)), np.int32)
+        best = []
+        for _ in range(6):
+            a, b = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+            a.record()
+            _device_labels_dev(A)
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        return min(best)
+
+    assert ms(np.arange(1, n), np.arange(n - 1)) < 3 * ms(q[1:], q[:-1])
