@@ -180,7 +180,9 @@ __global__ void k_perm_inverse(const int32_t* __restrict__ p, int32_t n, int32_t
 // copied renamed to the staging buffer and listed (its output range) for the
 // segmented sort.  Bound by the comparisons (closure of 300,007 vertices, 15 M
 // entries: 361 us and 46 us of segmented sort; up to 256 columns 350 + 174, up
-// to 1024 890 + 25; tie-breaking in every comparison 450 + 174).
+// to 1024 890 + 25; tie-breaking in every comparison 450 + 174).  Rows of up to
+// 64 entries, one a lane, are ranked from registers: a million rows of one
+// entry 311 us, of three 380 (through the LDS and eight columns a lane 565, 613).
 constexpr int PS_MAX = 512;
 template <typename T>
 __global__ __launch_bounds__(ORD_NT) void k_permute_csr_fused(const int64_t* __restrict__ indptr,
@@ -199,7 +201,8 @@ __global__ __launch_bounds__(ORD_NT) void k_permute_csr_fused(const int64_t* __r
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // a wave's row is uniform
   int32_t* kw = keys[wv];
   const int64_t waves = (int64_t)gridDim.x * (ORD_NT / 64);
   for (int64_t i = (int64_t)blockIdx.x * (ORD_NT / 64) + wv; i < n; i += waves) {
@@ -217,6 +220,21 @@ __global__ __launch_bounds__(ORD_NT) void k_permute_csr_fused(const int64_t* __r
       continue;
     }
     const int L = (int)len;
+    if (L <= 64) {  // an entry a lane: no LDS, ties broken as it goes
+      int32_t key = 0;
+      T val = 0;
+      if (lane < L) {
+        key = pinv[indices[s + lane]];
+        val = data[s + lane];
+      }
+      int r = 0;
+      for (int m = 0; m < L; m++) r += __builtin_amdgcn_readlane(key, m) < key + (int)(lane > m);
+      if (lane < L) {
+        out_idx[d + r] = key;
+        out_val[d + r] = val;
+      }
+      continue;
+    }
     constexpr int Q = PS_MAX / 64;
     int32_t key[Q];
     T val[Q];
@@ -245,23 +263,25 @@ __global__ __launch_bounds__(ORD_NT) void k_permute_csr_fused(const int64_t* __r
     for (int q = 0; q < Q; q++) sum += 64 * q + lane < L ? r[q] : 0;
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
     if (sum != L * (L - 1) / 2) {
-      for (int q = 0; 64 * q < L; q++) {  // repeated columns keep their order in the row
-        const int k = 64 * q + lane;
-        if (k < L) {
-          int t = 0;
-          for (int m = 0; m < L; m++) t += (kw[m] < kw[k] || (kw[m] == kw[k] && m < k)) ? 1 : 0;
-          out_idx[d + t] = kw[k];
-          out_val[d + t] = data[s + k];
+#pragma unroll
+      for (int q = 0; q < Q; q++) r[q] = 0;
+      for (int m = 0; m < L; m += 4) {  // repeated columns keep their order in the row
+        const int4 o = *(const int4*)(kw + m);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+          if (64 * q >= L) break;
+          const int k = 64 * q + lane;
+          r[q] += (int)(o.x < key[q] + (int)(k > m)) + (int)(o.y < key[q] + (int)(k > m + 1)) +
+                  (int)(o.z < key[q] + (int)(k > m + 2)) + (int)(o.w < key[q] + (int)(k > m + 3));
         }
       }
-    } else {
-#pragma unroll
-      for (int q = 0; q < Q; q++)
-        if (64 * q + lane < L) {
-          out_idx[d + r[q]] = key[q];
-          out_val[d + r[q]] = val[q];
-        }
     }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      if (64 * q + lane < L) {
+        out_idx[d + r[q]] = key[q];
+        out_val[d + r[q]] = val[q];
+      }
     wsync();  // the next row restages the keys
   }
 }
