@@ -2501,7 +2501,7 @@ __global__ void k_rows_init(int64_t* row_len, int64_t* counters, int32_t n) {
     for (int q = 0; q < C_NCTR; q++) counters[q] = 0;
 }
 
-// Segmented copy into CSR order: one wave moves GROWS consecutive output rows,
+// Segmented copy into CSR order: one wave moves ROWS consecutive output rows,
 // which are contiguous in the output from out_ptr[r0] (the rows of the last
 // generations are long and neighbours: with 64, 32, 16, 8 and 4 rows a wave 61,
 // 36, 23, 16 and 15 us for n = 21,162 and 560, 525, 500, 486 and 486 for n =
@@ -2512,8 +2512,12 @@ __global__ void k_rows_init(int64_t* row_len, int64_t* counters, int32_t n) {
 // row's source offset and length.
 constexpr int GC = 8;
 constexpr int GROWS = 8;
+// The merged rows of two matrices are short more often than not, and from so
+// many rows on 64 a wave fill the chip as well (avos_sum of a million rows of one
+// entry 169 us, with 8 a wave 184, of three 234 and 251).
+constexpr int32_t GROWS_MANY = 1 << 18;
 
-template <typename T, typename SrcF, typename LenF>
+template <typename T, int ROWS, typename SrcF, typename LenF>
 __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __restrict__ out_ptr, SrcF src_of,
                                      LenF len_of, const int32_t* __restrict__ in_idx, const T* __restrict__ in_val,
                                      int32_t* __restrict__ out_idx, T* __restrict__ out_val, int64_t* s_pre,
@@ -2521,7 +2525,7 @@ __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __res
   const int lane = threadIdx.x & 63;
   const int64_t r = r0 + lane;
   int64_t len = 0, src = 0;
-  if (lane < GROWS && r < n) {
+  if (lane < ROWS && r < n) {
     len = len_of(r);
     src = src_of(r);
   }
@@ -2571,8 +2575,8 @@ __device__ inline void seg_copy_rows(int64_t r0, int32_t n, const int64_t* __res
 }
 
 constexpr int GATHER_NT = 256;
-static inline unsigned gather_grid(int64_t n) {
-  constexpr int rows = GATHER_NT / 64 * GROWS;
+static inline unsigned gather_grid(int64_t n, int wave_rows = GROWS) {
+  const int rows = GATHER_NT / 64 * wave_rows;
   return (unsigned)((n + rows - 1) / rows);
 }
 template <typename T>
@@ -2589,7 +2593,7 @@ __global__ __launch_bounds__(GATHER_NT) void k_dag_gather(const DagWork ws, cons
   const int w = threadIdx.x >> 6;
   const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * GROWS;
   if (r0 >= n) return;
-  seg_copy_rows<T>(
+  seg_copy_rows<T, GROWS>(
       r0, n, out_ptr, [&](int64_t r) { return ws.row_off[r]; }, [&](int64_t r) { return ws.row_len[r]; }, ar.cols,
       ar.vals, out_idx, out_val, s_pre[w], s_src[w]);
 }
@@ -2700,7 +2704,7 @@ __global__ void k_csr_sort_rows(const int64_t* __restrict__ indptr, int32_t* __r
   len[r] = out - a;
 }
 
-template <typename T>
+template <typename T, int ROWS>
 __global__ __launch_bounds__(GATHER_NT) void k_csr_compact(const int64_t* __restrict__ indptr,
                                                            const int32_t* __restrict__ idx, const T* __restrict__ val,
                                                            const int64_t* __restrict__ len,
@@ -2709,11 +2713,24 @@ __global__ __launch_bounds__(GATHER_NT) void k_csr_compact(const int64_t* __rest
   __shared__ int64_t s_pre[GATHER_NT / 64][65];
   __shared__ int64_t s_src[GATHER_NT / 64][64];
   const int w = threadIdx.x >> 6;
-  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * GROWS;
+  const int64_t r0 = ((int64_t)blockIdx.x * (GATHER_NT / 64) + w) * ROWS;
   if (r0 >= n) return;
-  seg_copy_rows<T>(
+  seg_copy_rows<T, ROWS>(
       r0, n, optr, [&](int64_t r) { return indptr[r]; }, [&](int64_t r) { return len[r]; }, idx, val, oidx, oval,
       s_pre[w], s_src[w]);
+}
+
+template <typename T>
+static int csr_compact(const int64_t* indptr, const int32_t* idx, const T* val, const int64_t* len, const int64_t* optr,
+                       int32_t n, int32_t* oidx, T* oval, hipStream_t s) {
+  if (n < GROWS_MANY)
+    hipLaunchKernelGGL((k_csr_compact<T, GROWS>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s, indptr, idx, val, len,
+                       optr, n, oidx, oval);
+  else
+    hipLaunchKernelGGL((k_csr_compact<T, 64>), dim3(gather_grid(n, 64)), dim3(GATHER_NT), 0, s, indptr, idx, val, len,
+                       optr, n, oidx, oval);
+  RBG_CHECK_LAUNCH();
+  return 0;
 }
 
 // Rows that are not canonical (columns not strictly increasing, or an
@@ -3103,9 +3120,8 @@ int64_t rbg_csr_tmp_bytes(int32_t n) { return 8 * ((int64_t)n + 1) + 8 * ((int64
     hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n, (const int64_t*)total);      \
     RBG_CHECK_LAUNCH();                                                                                         \
     if (out_idx && out_val) {                                                                                   \
-      hipLaunchKernelGGL((k_csr_compact<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s, indptr, (const int32_t*)idx,     \
-                         (const T*)val, (const int64_t*)len, (const int64_t*)out_indptr, n, out_idx, out_val);   \
-      RBG_CHECK_LAUNCH();                                                                                       \
+      rc = csr_compact<T>(indptr, idx, val, len, out_indptr, n, out_idx, out_val, s);                           \
+      if (rc) return rc;                                                                                        \
     }                                                                                                           \
     return 0;                                                                                                   \
   }
@@ -3182,10 +3198,8 @@ extern "C" {
     hipLaunchKernelGGL(k_set_last, dim3(1), dim3(1), 0, s, out_indptr, (int64_t)n, (const int64_t*)total);      \
     RBG_CHECK_LAUNCH();                                                                                         \
     if (out_idx && out_val) {                                                                                   \
-      hipLaunchKernelGGL((k_csr_compact<T>), dim3(gather_grid(n)), dim3(GATHER_NT), 0, s,          \
-                         cat_ptr, (const int32_t*)cat_idx,                                                      \
-                         (const T*)cat_val, (const int64_t*)len, (const int64_t*)out_indptr, n, out_idx, out_val); \
-      RBG_CHECK_LAUNCH();                                                                                       \
+      rc = csr_compact<T>(cat_ptr, cat_idx, cat_val, len, out_indptr, n, out_idx, out_val, s);                  \
+      if (rc) return rc;                                                                                        \
     }                                                                                                           \
     return 0;                                                                                                   \
   }

@@ -253,3 +253,25 @@ def test_components_of_a_long_path_cost_no_walk():
         return min(best)
 
     assert ms(np.arange(1, n), np.arange(n - 1)) < 3 * ms(q[1:], q[:-1])
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [1, 31, 33, 262_143, 262_144, 262_209])
+def test_sum_of_short_and_empty_rows(dt, n):
+    """Either side of the row count from which a wave moves 64 rows: rows of
+    none to three entries, columns of both, one and neither matrix."""
+    rng = np.random.default_rng(n)
+
+    def some():
+        k = rng.integers(0, 4, n)
+        return sp.csr_matrix((rng.integers(1, 9, k.sum()).astype(dt), (np.repeat(np.arange(n), k),
+                                                                       rng.integers(0, min(n, 5), k.sum()))),
+                             shape=(n, n))
+
+    A, B = some(), some()
+    C = sd.to_scipy(sd.avos_sum_csr(sd.canonicalize(sd.from_scipy(A, dt)), sd.canonicalize(sd.from_scipy(B, dt))))
+    assert C.has_sorted_indices
+    a, b = A[:, :5].toarray(), B[:, :5].toarray()
+    want = np.where(a == 0, b, np.where(b == 0, a, np.minimum(a, b)))
+    np.testing.assert_array_equal(C[:, :5].toarray(), want)
+    assert C.nnz == np.count_nonzero(want)
