@@ -787,9 +787,13 @@ int rbg_batch_run(rbg_batch* b, rbg_stream_t stream) {
 int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stream) {
   if (!b || !closed) return RBG_E_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const hipError_t e = hipMemcpy2DAsync(closed, sizeof(int32_t), &b->d_comps->done, sizeof(BComp), sizeof(int32_t),
-                                        (size_t)b->count, hipMemcpyDeviceToHost, s);
-  return e == hipSuccess ? (int)hipStreamSynchronize(s) : (int)e;
+  // whole descriptors (a strided copy to the caller's memory came back empty under a profiler)
+  std::vector<BComp> comps((size_t)b->count);
+  hipError_t e = hipMemcpyAsync(comps.data(), b->d_comps, sizeof(BComp) * comps.size(), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return (int)e;
+  for (size_t i = 0; i < comps.size(); i++) closed[i] = comps[i].done;
+  return 0;
 }
 
 static void batch_drop_graphs(rbg_batch* b) {
