@@ -393,6 +393,7 @@ struct rbg_batch {
   std::vector<int64_t> panel_cnt, t128_cnt, t64_cnt;  // per step: items of running components
   std::vector<int64_t> tri128_off, tri64_off;         // per step: [off[K], off[K + 1]) of the step lists
   std::vector<double> work;                           // per step: relaxations its tile launches execute
+  std::vector<int32_t> from;                          // the caller's index of each descriptor (largest first)
   // captured: every launch of a run, or where rows are tried the launches up to
   // the answer and the close pass and, in graph 1, those behind
   hipGraph_t graph[2] = {nullptr, nullptr};
@@ -592,7 +593,14 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
                  room && !flow ? (char*)q.snap + dsnap_offset(q.npad, 4) : nullptr, rows, 0};
   }
   // largest first: the components running at step K are a prefix
-  std::stable_sort(c.begin(), c.end(), [](const BComp& a, const BComp& b) { return a.npad > b.npad; });
+  std::vector<int32_t> from(count);
+  std::iota(from.begin(), from.end(), 0);
+  std::stable_sort(from.begin(), from.end(), [&](int32_t x, int32_t y) { return c[x].npad > c[y].npad; });
+  {
+    std::vector<BComp> sorted;
+    for (int32_t i : from) sorted.push_back(c[i]);
+    c.swap(sorted);
+  }
   // the persistent launch: lower triangular components with its workspace,
   // in classes of equal order and tile edge (else they take the per-step
   // launches)
@@ -608,6 +616,7 @@ int rbg_batch_create(const rbg_batch_comp* comps, int32_t count, rbg_batch** out
   }
   auto* b = new rbg_batch();
   b->count = count;
+  b->from = std::move(from);
   b->maxnb = c[0].npad / BLK;
   b->classes = classes;
   std::vector<BFlow> fl;
@@ -792,7 +801,7 @@ int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stre
   hipError_t e = hipMemcpyAsync(comps.data(), b->d_comps, sizeof(BComp) * comps.size(), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return (int)e;
-  for (size_t i = 0; i < comps.size(); i++) closed[i] = comps[i].done;
+  for (size_t i = 0; i < comps.size(); i++) closed[b->from[i]] = comps[i].done;
   return 0;
 }
 

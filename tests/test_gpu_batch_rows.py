@@ -142,3 +142,14 @@ def test_batch_recorded_by_its_caller(launches, graph):
         _check(b, _INPUTS["mixed"], want["mixed"])
     finally:
         b.close()
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+def test_rows_closed_names_the_callers_components(persistent):
+    """Components in no order of size: the flags are in the caller's order."""
+    mats = [_pedigree(60, 1), _dense_lower(200), _pedigree(900, 2), _chain(130), _pedigree(300, 3), _dense_lower(500),
+            _pedigree(1500, 4), _chain(150)]
+    mats = [np.tril(m) for m in mats]
+    _, told = _close(mats, 1, persistent)
+    for t in told:
+        assert list(t) == [True, False, True, False, True, False, True, False]
