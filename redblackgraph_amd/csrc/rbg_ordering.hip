@@ -179,10 +179,11 @@ __global__ void k_perm_inverse(const int32_t* __restrict__ p, int32_t n, int32_t
 // and is ranked again with ties broken by place.  A row longer than PS_MAX is
 // copied renamed to the staging buffer and listed (its output range) for the
 // segmented sort.  Bound by the comparisons (closure of 300,007 vertices, 15 M
-// entries: 361 us and 46 us of segmented sort; up to 256 columns 350 + 174, up
-// to 1024 890 + 25; tie-breaking in every comparison 450 + 174).  Rows of up to
-// 64 entries, one a lane, are ranked from registers: a million rows of one
-// entry 311 us, of three 380 (through the LDS and eight columns a lane 565, 613).
+// entries, every row through the LDS: 361 us and 46 us of segmented sort; up to
+// 256 columns 350 + 174, up to 1024 890 + 25; tie-breaking in every comparison
+// 450 + 174).  Rows of up to 64 entries, one a lane, are ranked from registers:
+// that closure 292 + 46; a million rows of one entry 311 us, of three 380
+// (through the LDS and eight columns a lane 565, 613).
 constexpr int PS_MAX = 512;
 template <typename T>
 __global__ __launch_bounds__(ORD_NT) void k_permute_csr_fused(const int64_t* __restrict__ indptr,

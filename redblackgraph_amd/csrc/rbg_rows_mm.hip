@@ -14,7 +14,7 @@
 //   rows  a workgroup per row of C: N cells in LDS, a wave per entry of A's
 //         row, lanes over the entries of B's row, LDS atomic min.
 // N = 8192 int32, W @ W of the closure of a 24-generation pedigree (0.56% of
-// the cells): scan 123 us (0.54 GB, 4.4 TB/s), plan 8, rows 173, of which 35
+// the cells): scan 123 us (0.54 GB, 4.4 TB/s), plan 8, rows 177, of which 35
 // write C, about 90 wait for B's rows and the rest is the terms' arithmetic
 // (all avos_product: 227; one of B's rows at a time: 267); 26.1 ms blocked.
 #include "fw_kernels.hpp"
