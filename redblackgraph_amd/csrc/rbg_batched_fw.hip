@@ -25,6 +25,8 @@
 // path.
 #include <algorithm>
 #include <chrono>
+#include <memory>
+#include <new>
 #include <numeric>
 #include <thread>
 
@@ -797,11 +799,12 @@ int rbg_batch_rows_closed(const rbg_batch* b, int32_t* closed, rbg_stream_t stre
   if (!b || !closed) return RBG_E_ARG;
   hipStream_t s = (hipStream_t)stream;
   // whole descriptors (a strided copy to the caller's memory came back empty under a profiler)
-  std::vector<BComp> comps((size_t)b->count);
-  hipError_t e = hipMemcpyAsync(comps.data(), b->d_comps, sizeof(BComp) * comps.size(), hipMemcpyDeviceToHost, s);
+  const std::unique_ptr<BComp[]> comps(new (std::nothrow) BComp[b->count]);
+  if (!comps) return (int)hipErrorOutOfMemory;
+  hipError_t e = hipMemcpyAsync(comps.get(), b->d_comps, sizeof(BComp) * b->count, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return (int)e;
-  for (size_t i = 0; i < comps.size(); i++) closed[b->from[i]] = comps[i].done;
+  for (int32_t i = 0; i < b->count; i++) closed[b->from[i]] = comps[i].done;
   return 0;
 }
 
